@@ -41,7 +41,7 @@ struct zpic_batch {
     zk_bsim *dsims;     /* device descriptors */
     zk_bspec *dspecs;
     int *ditems;        /* device item table (int pairs) */
-    item_range fill, node, yee, guard, sort;
+    item_range fill, node, yee, sort;
     item_range *tile, *glob; /* per species index */
     int *gblocks;            /* per species: blocks of the out-of-window pass */
     int *ntiles;             /* per simulation, at creation */
@@ -224,7 +224,6 @@ static void build_items(zpic_batch *b, table *T)
     GRID_PHASE(b->fill, blocks_of(3 * (size_t)(M->nx + 3) * (M->ny + 3), 256));
     GRID_PHASE(b->node, blocks_of((size_t)(M->nx + 3) * (M->ny + 3), 256));
     GRID_PHASE(b->yee, ((M->nx + 3 + ZK_YEE_BX - 1) / ZK_YEE_BX) * ((M->ny + 3 + ZK_YEE_BY - 1) / ZK_YEE_BY));
-    GRID_PHASE(b->guard, blocks_of(3 * (size_t)(M->nx + 3) + 3 * (size_t)M->ny, 256));
 #undef GRID_PHASE
 
     /* particle phases: species by particles per tile (the tile pass) or
@@ -284,7 +283,7 @@ static void enqueue_step(zpic_batch *b, int with_sort)
     if (with_sort) ZCHECK(zk_batch_sort(b->dspecs, b->nspecs, ITEMS(b->sort), s));
     /* current_update, emf_advance */
     ZCHECK(zk_batch_current(b->dsims, ITEMS(b->node), b->max_passes, s));
-    ZCHECK(zk_batch_fields(b->dsims, ITEMS(b->yee), ITEMS(b->guard), s));
+    ZCHECK(zk_batch_fields(b->dsims, ITEMS(b->yee), s));
     if (with_sort) ZCHECK(zk_batch_end_step_sorted(b->dsims, b->nsims, b->dspecs, b->nspecs, s));
     else ZCHECK(zk_batch_end_step(b->dsims, b->nsims, b->dspecs, b->nspecs, s));
 }

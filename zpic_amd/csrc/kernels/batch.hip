@@ -4,7 +4,7 @@
  * A batch runs the reference step sequence (em2d/simulation.c:45-56) of
  * every simulation, but each phase of the step (current reset, push of the
  * k-th species, out-of-window push, energy, current reduction, filter
- * passes, Yee update, guard cells) is a single kernel launch over an item
+ * passes, Yee update) is a single kernel launch over an item
  * table of (simulation or species, block) pairs, so simulations of uneven
  * size share the GPU and a whole step is a fixed sequence of launches that
  * a HIP graph captures once and replays.
@@ -108,14 +108,7 @@ __global__ void __launch_bounds__(256) yee_batch(const zk_bsim *sims, const int 
     const zk_bsim &M = sims[s];
     const int ntx = (M.nx + 3 + BX - 1) / BX;
     yee_tile(M.E[M.ecur], M.B[M.ecur], j_after(M, M.npass), M.E[1 - M.ecur], M.B[1 - M.ecur], M.nx, M.ny, M.nrow,
-             M.yk, t % ntx, t / ntx);
-}
-
-__global__ void guards_batch(const zk_bsim *sims, const int *items)
-{
-    const zk_bsim &M = sims[items[2 * blockIdx.x]];
-    guard_node(M.E[1 - M.ecur], M.B[1 - M.ecur], M.nx, M.ny, M.nrow, 1,
-               items[2 * blockIdx.x + 1] * blockDim.x + threadIdx.x);
+             M.yk, t % ntx, t / ntx, 1);
 }
 
 /* The re-sort of the single-simulation path (zk_sort_tiles: stayers in
@@ -222,11 +215,9 @@ extern "C" int zk_batch_current(const zk_bsim *sims, const int *node_items, int 
     ZK_LAUNCH_CHECK();
 }
 
-extern "C" int zk_batch_fields(const zk_bsim *sims, const int *yee_items, int nyee, const int *guard_items,
-                               int nguard, zk_stream_t s)
+extern "C" int zk_batch_fields(const zk_bsim *sims, const int *yee_items, int nyee, zk_stream_t s)
 {
     LAUNCH_ITEMS(yee_batch, nyee, sims, yee_items);
-    LAUNCH_ITEMS(guards_batch, nguard, sims, guard_items);
     ZK_LAUNCH_CHECK();
 }
 

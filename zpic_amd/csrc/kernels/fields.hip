@@ -7,10 +7,11 @@
  * B += dt/2 curl E again, into one pass over LDS tiles.  Each node is
  * computed with the reference's expressions and update ranges, so with the
  * same J the result is bit-identical.  Inputs and outputs are distinct
- * buffers (the host swaps them).
+ * buffers (the host swaps them).  The guard cells of the outputs are
+ * written by the nodes they are images of (emf_update_gc, :573-637).
  *
- * zk_field_guards copies guard cells from their periodic images
- * (emf_update_gc, :573-637); zk_move_window shifts the grid one cell left
+ * zk_field_guards copies guard cells from their periodic images on its own
+ * (grids edited outside the step); zk_move_window shifts the grid one cell left
  * and clears the last columns (emf_move_window, :648-675); zk_add_ext
  * forms the fields seen by particles (emf_update_part_fld, :838-914);
  * zk_emf_energy sums E_c^2 and B_c^2 in FP64 (emf_get_energy, :729-750);
@@ -33,9 +34,9 @@ namespace {
 __global__ void __launch_bounds__(256) yee_kernel(const float *__restrict__ E, const float *__restrict__ B,
                                                   const float *__restrict__ J, float *__restrict__ Eo,
                                                   float *__restrict__ Bo, int nx, int ny, int nrow, YeeK k,
-                                                  int open_y, int shift)
+                                                  int periodic_x, int open_y, int shift)
 {
-    yee_tile(E, B, J, Eo, Bo, nx, ny, nrow, k, blockIdx.x, blockIdx.y, open_y, shift);
+    yee_tile(E, B, J, Eo, Bo, nx, ny, nrow, k, blockIdx.x, blockIdx.y, periodic_x, open_y, shift);
 }
 
 __global__ void guard_kernel(float *E, float *B, int nx, int ny, int nrow, int periodic_x, int open_y)
@@ -306,7 +307,7 @@ extern "C" int zk_pha(const zk_parts *p, int np_upper, const zk_spec_ctr *ctr, i
 }
 
 extern "C" int zk_yee(const float *E, const float *B, const float *J, float *Eo, float *Bo, int nx, int ny,
-                             int nrow, float dt, float dx, float dy, int open_y, int shift, zk_stream_t s)
+                             int nrow, float dt, float dx, float dy, int periodic_x, int open_y, int shift, zk_stream_t s)
 {
     YeeK k;
     const float dt2 = dt / 2.0f;
@@ -317,7 +318,8 @@ extern "C" int zk_yee(const float *E, const float *B, const float *J, float *Eo,
     k.dt = dt;
     k.mur_y = (dt - dy) / (dt + dy);
     dim3 grid((nx + 3 + BX - 1) / BX, (ny + 3 + BY - 1) / BY);
-    hipLaunchKernelGGL(yee_kernel, grid, dim3(256), 0, s, E, B, J, Eo, Bo, nx, ny, nrow, k, open_y, shift);
+    hipLaunchKernelGGL(yee_kernel, grid, dim3(256), 0, s, E, B, J, Eo, Bo, nx, ny, nrow, k, periodic_x,
+                       open_y, shift);
     ZK_LAUNCH_CHECK();
 }
 

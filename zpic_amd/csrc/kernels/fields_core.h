@@ -34,12 +34,42 @@ typedef zk_yee_k YeeK; /* (dt/2)/dx, (dt/2)/dy, dt/dx, dt/dy, dt, Mur coefficien
 /* shift: the step ends in a window move (em2d/emf.c:646-676): every node
  * is written one column to the left, the leftmost guard column's values
  * are dropped and raw columns nx - 1 .. nx + 1 are zeroed, as the
- * reference's shift after the step leaves them (the y guards, copied after
- * this kernel, commute with the shift). */
+ * reference's shift after the step leaves them (the y guards commute with
+ * the shift). */
+/* Guard cells (emf_update_gc, em2d/emf.c:573-637): a node that is the
+ * periodic image of guards is also written to those guards, and guards
+ * with an image are written by it alone, so no copy pass follows the step
+ * (a launch of 3.5-4.5 us at any grid size: 11 % of a 32 x 32 step's
+ * kernels, 5 % of a vacuum step at 2000 x 512).  Tiles away from the edges
+ * keep the plain store. */
+__device__ inline void yee_store(float *__restrict__ Eo, float *__restrict__ Bo, int nx, int nrow, int bi, int bj,
+                                 const float *e, const float *b, int shift)
+{
+    if (shift) {
+        /* buffer column bi goes to bi - 1 (raw i - 1); raw columns from
+         * nx - 1 on are zero, the last one written by the last node */
+        if (bi == 0) return;
+        const size_t g = 3 * ((size_t)(bi - 1) + (size_t)bj * nrow);
+        const bool zero = bi - 1 >= nx;
+        for (int c = 0; c < 3; c++) {
+            Bo[g + c] = zero ? 0.0f : b[c];
+            Eo[g + c] = zero ? 0.0f : e[c];
+        }
+        if (bi == nx + 2)
+            for (int c = 0; c < 3; c++) Bo[g + 3 + c] = Eo[g + 3 + c] = 0.0f;
+        return;
+    }
+    const size_t g = 3 * ((size_t)bi + (size_t)bj * nrow);
+    for (int c = 0; c < 3; c++) {
+        Bo[g + c] = b[c];
+        Eo[g + c] = e[c];
+    }
+}
+
 __device__ inline void yee_tile(const float *__restrict__ E, const float *__restrict__ B,
                                 const float *__restrict__ J, float *__restrict__ Eo, float *__restrict__ Bo, int nx,
-                                int ny, int nrow, const YeeK &k, const int tx, const int ty, const int open_y = 0,
-                                const int shift = 0)
+                                int ny, int nrow, const YeeK &k, const int tx, const int ty, const int periodic_x,
+                                const int open_y = 0, const int shift = 0)
 {
     __shared__ float e[3][LY][LX], b[3][LY][LX], jj[3][LY][LX];
     const int bw = nx + 3, bh = ny + 3;
@@ -99,6 +129,8 @@ __device__ inline void yee_tile(const float *__restrict__ E, const float *__rest
         }
         __syncthreads();
     }
+    /* tiles holding guards, or nodes that guards are images of */
+    const bool edge = (periodic_x && (bi0 <= 2 || bi0 + BX > nx)) || (!open_y && (bj0 <= 2 || bj0 + BY > ny));
     /* B2 = B1 + dt/2 * (-curl E1) and outputs on u in [1, BX+1), v in [OY, BY+OY) */
     for (int m = tid; m < BX * BY; m += blockDim.x) {
         const int u = 1 + m % BX, v = OY + m / BX;
@@ -111,29 +143,22 @@ __device__ inline void yee_tile(const float *__restrict__ E, const float *__rest
             by += (k.dtx2 * (e[2][v][u + 1] - e[2][v][u]));
             bz += (-k.dtx2 * (e[1][v][u + 1] - e[1][v][u]) + k.dty2 * (e[0][v + 1][u] - e[0][v][u]));
         }
-        if (shift) {
-            /* buffer column bi goes to bi - 1 (raw i - 1); raw columns from
-             * nx - 1 on are zero, the last one written by the last node */
-            if (bi == 0) continue;
-            const size_t g = 3 * ((size_t)(bi - 1) + (size_t)bj * nrow);
-            const bool zero = bi - 1 >= nx;
-            Bo[g + 0] = zero ? 0.0f : bx;
-            Bo[g + 1] = zero ? 0.0f : by;
-            Bo[g + 2] = zero ? 0.0f : bz;
-            Eo[g + 0] = zero ? 0.0f : e[0][v][u];
-            Eo[g + 1] = zero ? 0.0f : e[1][v][u];
-            Eo[g + 2] = zero ? 0.0f : e[2][v][u];
-            if (bi == bw - 1)
-                for (int c = 0; c < 3; c++) Bo[g + 3 + c] = Eo[g + 3 + c] = 0.0f;
+        const float bn[3] = {bx, by, bz}, en[3] = {e[0][v][u], e[1][v][u], e[2][v][u]};
+        if (!edge) {
+            yee_store(Eo, Bo, nx, nrow, bi, bj, en, bn, shift);
             continue;
         }
-        const size_t g = 3 * ((size_t)bi + (size_t)bj * nrow);
-        Bo[g + 0] = bx;
-        Bo[g + 1] = by;
-        Bo[g + 2] = bz;
-        Eo[g + 0] = e[0][v][u];
-        Eo[g + 1] = e[1][v][u];
-        Eo[g + 2] = e[2][v][u];
+        /* the images of an interior index c on a periodic axis of n cells:
+         * c - n when that is the lower guard, c, and c + n, ... up to n + 1 */
+        const bool cy = !open_y;
+        if ((periodic_x && (i < 0 || i >= nx)) || (cy && (j < 0 || j >= ny))) continue;
+        for (int gj = cy && j - ny >= -1 ? j - ny : j; gj <= ny + 1; gj += ny) {
+            for (int gi = periodic_x && i - nx >= -1 ? i - nx : i; gi <= nx + 1; gi += nx) {
+                yee_store(Eo, Bo, nx, nrow, gi + 1, gj + 1, en, bn, shift);
+                if (!periodic_x) break;
+            }
+            if (!cy) break;
+        }
     }
 }
 

@@ -210,11 +210,12 @@ int zk_smooth_x_passes(const float *in, float *out, int nx, int ny, int nrow, in
                        const float *sb, int periodic_x, zk_stream_t s);
 
 /* fields */
-/* open_y: first-order Mur absorbing boundaries at the y edges; shift: the
+/* One field step, guard cells of the outputs included (periodic_x: along
+ * x; along y unless open_y).  open_y: first-order Mur absorbing boundaries at the y edges; shift: the
  * output is the grid after the step and a window move (one column left,
  * the rightmost columns zeroed), as zk_move_window would make it */
 int zk_yee(const float *E, const float *B, const float *J, float *Eo, float *Bo,
-                  int nx, int ny, int nrow, float dt, float dx, float dy, int open_y, int shift,
+                  int nx, int ny, int nrow, float dt, float dx, float dy, int periodic_x, int open_y, int shift,
                   zk_stream_t s);
 int zk_field_guards(float *E, float *B, int nx, int ny, int nrow, int periodic_x,
                            int open_y, zk_stream_t s);
@@ -361,8 +362,7 @@ int zk_batch_push(const zk_bspec *specs, const zk_bsim *sims, const int *tile_it
                   const int *global_items, int nglobal, size_t lds, int waves, int fixed, zk_stream_t s);
 int zk_batch_finalize(const zk_bspec *specs, int nspecs, zk_stream_t s);
 int zk_batch_current(const zk_bsim *sims, const int *node_items, int n, int max_passes, zk_stream_t s);
-int zk_batch_fields(const zk_bsim *sims, const int *yee_items, int nyee, const int *guard_items, int nguard,
-                    zk_stream_t s);
+int zk_batch_fields(const zk_bsim *sims, const int *yee_items, int nyee, zk_stream_t s);
 int zk_batch_sort(const zk_bspec *specs, int nspecs, const int *items, int n, zk_stream_t s);
 int zk_batch_end_step(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_stream_t s);
 int zk_batch_end_step_sorted(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_stream_t s);
