@@ -251,6 +251,7 @@ static void save_state(zpic_diff *D, int c)
         spec_ckpt *C = CS(D, c, k);
         parts_copy(&C->p, &d->set[d->cur], D->np[k]);
         zpic_d2d_async(C->tile_off, d->tile_off, sizeof(int) * (size_t)(d->t.ntiles + 2));
+        zpic_spec_settle(d);
         zpic_d2h(&C->ctr, d->ctr, sizeof(zk_spec_ctr));
         if (C->ctr.np_total != D->np[k] || C->ctr.n_sorted != C->ctr.np_total || C->ctr.n_dead)
             zpic_fatal("zpic_diff: species '%s' changed its particle count", s->name);
@@ -267,6 +268,7 @@ static void restore_state(zpic_diff *D, int c, int iter)
         t_species *s = &sim->species[k];
         struct zpic_dev_species *d = s->dev;
         spec_ckpt *C = CS(D, c, k);
+        zpic_spec_settle(d);
         parts_copy(&d->set[d->cur], &C->p, D->np[k]);
         zpic_d2d_async(d->tile_off, C->tile_off, sizeof(int) * (size_t)(d->t.ntiles + 2));
         zpic_h2d(d->ctr, &C->ctr, sizeof(zk_spec_ctr));

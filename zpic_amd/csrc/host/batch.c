@@ -41,7 +41,7 @@ struct zpic_batch {
     zk_bsim *dsims;     /* device descriptors */
     zk_bspec *dspecs;
     int *ditems;        /* device item table (int pairs) */
-    item_range fill, node, yee, sort;
+    item_range fill, fold, node, yee, sort;
     item_range *tile, *glob; /* per species index */
     int *gblocks;            /* per species: blocks of the out-of-window pass */
     int *ntiles;             /* per simulation, at creation */
@@ -155,6 +155,7 @@ static void refresh(zpic_batch *b)
         t_species *s = b->spec[k];
         zpic_species_ensure(s);
         struct zpic_dev_species *d = s->dev;
+        zpic_spec_settle(d);
         if (d->moved_since_sort) zpic_fatal("batch: species '%s' has an unsorted window shift", s->name);
         /* the batched re-sort keeps tile ranges only: no unsorted tail */
         if (d->tail_upper > 0 || d->n_slack > 0) zpic_spec_sort(s);
@@ -222,6 +223,7 @@ static void build_items(zpic_batch *b, table *T)
         (range).n = T->n - (range).off;                                                                                \
     } while (0)
     GRID_PHASE(b->fill, blocks_of(3 * (size_t)(M->nx + 3) * (M->ny + 3), 256));
+    GRID_PHASE(b->fold, zk_batch_reduce_blocks(M));
     GRID_PHASE(b->node, blocks_of((size_t)(M->nx + 3) * (M->ny + 3), 256));
     GRID_PHASE(b->yee, ((M->nx + 3 + ZK_YEE_BX - 1) / ZK_YEE_BX) * ((M->ny + 3 + ZK_YEE_BY - 1) / ZK_YEE_BY));
 #undef GRID_PHASE
@@ -282,7 +284,7 @@ static void enqueue_step(zpic_batch *b, int with_sort)
     ZCHECK(zk_batch_finalize(b->dspecs, b->nspecs, s));
     if (with_sort) ZCHECK(zk_batch_sort(b->dspecs, b->nspecs, ITEMS(b->sort), s));
     /* current_update, emf_advance */
-    ZCHECK(zk_batch_current(b->dsims, ITEMS(b->node), b->max_passes, s));
+    ZCHECK(zk_batch_current(b->dsims, ITEMS(b->fold), ITEMS(b->node), b->max_passes, s));
     ZCHECK(zk_batch_fields(b->dsims, ITEMS(b->yee), s));
     if (with_sort) ZCHECK(zk_batch_end_step_sorted(b->dsims, b->nsims, b->dspecs, b->nspecs, s));
     else ZCHECK(zk_batch_end_step(b->dsims, b->nsims, b->dspecs, b->nspecs, s));

@@ -50,6 +50,7 @@ void current_delete(t_current *c)
 {
     struct zpic_dev_current *d = c->dev;
     if (d) {
+        zpic_current_settle(d);
         zpic_sync();
         zpic_dfree(d->J[0]);
         zpic_dfree(d->J[1]);
@@ -60,6 +61,20 @@ void current_delete(t_current *c)
     }
     free(c->J_buf);
     c->J_buf = NULL;
+}
+
+/* the launch that follows finishes the pushes in the list */
+static void fin_done(struct zpic_dev_current *d)
+{
+    for (int k = 0; k < d->fin.n; k++) d->fin_owner[k]->fin_cur = NULL;
+    d->fin.n = 0;
+}
+
+void zpic_current_settle(struct zpic_dev_current *d)
+{
+    if (!d || d->fin.n == 0) return;
+    ZCHECK(zk_spec_finalize_set(&d->fin, zpic_stream()));
+    fin_done(d);
 }
 
 void zpic_current_ensure(t_current *c, const zk_tiles *t)
@@ -175,8 +190,10 @@ void current_update(t_current *c)
     a.t = d->t;
     a.periodic_x = !c->moving_window;
     a.open_y = d->open_y;
+    a.fin = d->fin;
     zpic_ktimer_begin(ZPIC_T_CURRENT);
     ZCHECK(zk_current_reduce(&a, zpic_stream()));
+    fin_done(d);
     const int maxp = 2 * (c->smooth.xlevel > 0 ? c->smooth.xlevel : 0) + 2;
     int axis[maxp];
     float sa[maxp], sb[maxp];

@@ -490,12 +490,14 @@ static void ctr_check(const zk_spec_ctr *c)
 
 static void ctr_read(struct zpic_dev_species *d, zk_spec_ctr *c)
 {
+    zpic_spec_settle(d);
     zpic_d2h(c, d->ctr, sizeof(*c));
     ctr_check(c);
 }
 
 static void species_free_device(struct zpic_dev_species *d)
 {
+    zpic_spec_settle(d);
     if (d->ready) {
         zk_spec_ctr c;
         zpic_d2h(&c, d->ctr, sizeof(c));
@@ -785,6 +787,7 @@ static void upload(t_species *s)
 {
     struct zpic_dev_species *d = s->dev;
     const int np = s->np > 0 ? s->np : 0;
+    zpic_spec_settle(d);
     grow_sets(d, np);
     ensure_stage(d, sizeof(t_part) * (size_t)(np > 0 ? np : 1));
     zpic_h2d(d->stage, s->part, sizeof(t_part) * (size_t)np);
@@ -1071,6 +1074,7 @@ static void push_args(t_species *s, t_emf *emf, t_current *cur, zk_push_args *pa
 {
     struct zpic_dev_species *d = s->dev;
     struct zpic_dev_current *dc = cur->dev;
+    zpic_spec_settle(d); /* a push not finished yet: its partials are overwritten now */
     zk_push_args a;
     memset(&a, 0, sizeof(a));
     a.p = d->set[d->cur];
@@ -1108,10 +1112,11 @@ static void push_args(t_species *s, t_emf *emf, t_current *cur, zk_push_args *pa
     *pa = a;
 }
 
-/* The rest of spec_advance after its push: iteration count, window
- * injection and energy (push_done; with fin set the energy is left to
- * the caller's zk_spec_finalize_set, which gets this species' entry). */
-static void push_done(t_species *s, int move, int tb, zk_finalize_set *fin)
+/* The rest of spec_advance after its push: iteration count and window
+ * injection.  The energy sum and the push count are left to the launch of
+ * the current_update that follows (zpic_current_settle when something
+ * reads the counters first); a sort in between changes neither. */
+static void push_done(t_species *s, int move, int tb, struct zpic_dev_current *dc)
 {
     struct zpic_dev_species *d = s->dev;
     s->iter++;
@@ -1121,19 +1126,23 @@ static void push_done(t_species *s, int move, int tb, zk_finalize_set *fin)
         d->moved_since_sort++;
     }
     const float qm = s->q * s->m_q;
-    if (fin) {
-        const int k = fin->n++;
-        fin->ctr[k] = d->ctr;
-        fin->epart[k] = d->epart;
-        fin->nparts[k] = d->t.ntiles + tb;
-        fin->qm[k] = (double)qm;
-        fin->dx0[k] = (double)s->dx[0];
-        fin->dx1[k] = (double)s->dx[1];
-    } else {
-        ZCHECK(zk_spec_finalize(d->ctr, d->epart, d->t.ntiles + tb, (double)qm, (double)s->dx[0],
-                                (double)s->dx[1], zpic_stream()));
-    }
+    if (dc->fin.n == ZK_FUSE_MAX) zpic_current_settle(dc);
+    zk_finalize_set *fin = &dc->fin;
+    const int k = fin->n++;
+    fin->ctr[k] = d->ctr;
+    fin->epart[k] = d->epart;
+    fin->nparts[k] = d->t.ntiles + tb;
+    fin->qm[k] = (double)qm;
+    fin->dx0[k] = (double)s->dx[0];
+    fin->dx1[k] = (double)s->dx[1];
+    dc->fin_owner[k] = d;
+    d->fin_cur = dc;
     d->host_valid = 0;
+}
+
+void zpic_spec_settle(struct zpic_dev_species *d)
+{
+    if (d && d->fin_cur) zpic_current_settle(d->fin_cur);
 }
 
 /* Whether the tiles are sorted after the push of this step (move: the
@@ -1219,7 +1228,7 @@ void spec_advance(t_species *s, t_emf *emf, t_current *cur)
     /* a staged re-sort completes before the window's injections are
      * appended to the (new) set */
     if (staged) resort_staged(s);
-    push_done(s, move, a.global_blocks, NULL);
+    push_done(s, move, a.global_blocks, cur->dev);
     if (staged) {
         s->dev->moved_since_sort = 0;
         s->dev->steps_since_sort = 0;
@@ -1271,10 +1280,7 @@ void zpic_spec_advance_all(t_species *spec, int n, t_emf *emf, t_current *cur)
             cur->dev->fresh = 0;
             for (int k = 0; k < n; k++)
                 if (staged[k]) resort_staged(&spec[k]);
-            zk_finalize_set fin;
-            memset(&fin, 0, sizeof(fin));
-            for (int k = 0; k < n; k++) push_done(&spec[k], move[k], m.s[k].global_blocks, &fin);
-            ZCHECK(zk_spec_finalize_set(&fin, zpic_stream()));
+            for (int k = 0; k < n; k++) push_done(&spec[k], move[k], m.s[k].global_blocks, cur->dev);
             for (int k = 0; k < n; k++) {
                 if (staged[k]) {
                     spec[k].dev->moved_since_sort = 0;

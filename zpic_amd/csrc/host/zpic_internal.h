@@ -88,6 +88,7 @@ struct zpic_dev_species {
     int n_slack;          /* free slots of the ranges at the last sort */
     int np_live;          /* upper bound of the particles (not slots) */
     int *sstay, *sleave;  /* per tile: stayers written, leavers staged */
+    struct zpic_dev_current *fin_cur; /* holds this species' unfinished push */
 };
 
 struct zpic_dev_current {
@@ -103,6 +104,10 @@ struct zpic_dev_current {
     int fresh;            /* no deposit since current_zero */
     int pref[3];          /* preferred tile (tx, ty, halo), 0: process-wide setting */
     int open_y;           /* no fold along y (open y boundaries) */
+    /* pushes whose energy and push count the next current_update finishes
+     * in its own launch, and the species they belong to */
+    zk_finalize_set fin;
+    struct zpic_dev_species *fin_owner[ZK_FUSE_MAX];
 };
 
 struct zpic_dev_emf {
@@ -135,6 +140,10 @@ void zpic_current_jov_register(t_current *cur, float q);
 float zpic_current_jov_scale(const t_current *cur);   /* 2^(40 - jov_k) */
 float zpic_current_jov_unscale(const t_current *cur); /* 2^(jov_k - 40) */
 
+/* finish the energy and push counts a current density still holds; the
+ * same for one species (before its counters are read or replaced) */
+void zpic_current_settle(struct zpic_dev_current *dc);
+void zpic_spec_settle(struct zpic_dev_species *d);
 void zpic_spec_sync_energy(t_species *s);
 void zpic_spec_sort(t_species *s); /* tile sort of the device particles now */
 int zpic_current_passes(const t_current *c, int axis[], float sa[], float sb[], int max);

@@ -91,7 +91,10 @@ __global__ void reduce_batch(const zk_bsim *sims, const int *items)
     r.t = M.t;
     r.periodic_x = 1;
     r.open_y = 0;
-    reduce_node(r, items[2 * blockIdx.x + 1] * blockDim.x + threadIdx.x);
+    const int b = items[2 * blockIdx.x + 1], span = reduce_span(r.t), nbx = reduce_blocks_x(M.nx);
+    if (span == 2) reduce_block<2>(r, b % nbx, b / nbx);
+    else if (span == 3) reduce_block<3>(r, b % nbx, b / nbx);
+    else reduce_node(r, b * blockDim.x + threadIdx.x);
 }
 
 __global__ void smooth_batch(const zk_bsim *sims, const int *items, int pass)
@@ -208,9 +211,16 @@ extern "C" int zk_batch_finalize(const zk_bspec *specs, int nspecs, zk_stream_t 
     ZK_LAUNCH_CHECK();
 }
 
-extern "C" int zk_batch_current(const zk_bsim *sims, const int *node_items, int n, int max_passes, zk_stream_t s)
+extern "C" int zk_batch_reduce_blocks(const zk_bsim *M)
 {
-    LAUNCH_ITEMS(reduce_batch, n, sims, node_items);
+    if (reduce_span(M->t)) return reduce_blocks_x(M->nx) * reduce_blocks_y(M->ny);
+    return ((M->nx + 3) * (M->ny + 3) + 255) / 256;
+}
+
+extern "C" int zk_batch_current(const zk_bsim *sims, const int *reduce_items, int nreduce, const int *node_items, int n,
+                                int max_passes, zk_stream_t s)
+{
+    LAUNCH_ITEMS(reduce_batch, nreduce, sims, reduce_items);
     for (int p = 0; p < max_passes; p++) LAUNCH_ITEMS(smooth_batch, n, sims, node_items, p);
     ZK_LAUNCH_CHECK();
 }

@@ -16,12 +16,36 @@
  * handling of kernel_x / kernel_y (em2d/current.c:316-413).
  */
 #include "current_core.h"
+#include "finalize_core.h"
 
 using namespace zk;
 
 namespace {
 
-__global__ void reduce_kernel(zk_reduce_args a) { reduce_node(a, blockIdx.x * blockDim.x + threadIdx.x); }
+/* The first RED_FIN blocks finish the push's bookkeeping (energy and push
+ * count of a.fin's species, one block each), which was a launch of its own
+ * (4 us of a small grid's step) and has nothing to do with J; the others
+ * take 32 x 8 nodes each, in contiguous runs per XCD like the tiles that
+ * wrote the windows.  RED_FIN is 8 so that it does not shift those runs. */
+constexpr int RED_FIN = 8;
+
+template <int N>
+__global__ void __launch_bounds__(256) reduce_kernel(zk_reduce_args a, int nbx, int nblocks)
+{
+    const int b = (int)blockIdx.x - RED_FIN;
+    if (b < 0) {
+        const int k = blockIdx.x;
+        if (k < a.fin.n)
+            finalize_body(a.fin.ctr[k], a.fin.epart[k], a.fin.nparts[k], a.fin.qm[k], a.fin.dx0[k], a.fin.dx1[k]);
+        return;
+    }
+    if constexpr (N == 0) {
+        reduce_node(a, b * blockDim.x + threadIdx.x);
+    } else {
+        const int item = zk_xcd_item(b, nblocks);
+        reduce_block<N>(a, item % nbx, item / nbx);
+    }
+}
 
 __global__ void smooth_kernel(const float *__restrict__ in, float *__restrict__ out, int nx, int ny, int nrow,
                               int axis, float sa, float sb, int periodic_x, int open_y)
@@ -138,8 +162,13 @@ extern "C" int zk_smooth_x_passes(const float *in, float *out, int nx, int ny, i
 
 extern "C" int zk_current_reduce(const zk_reduce_args *a, zk_stream_t s)
 {
-    const int nodes = (a->t.nx + 3) * (a->t.ny + 3);
-    hipLaunchKernelGGL(reduce_kernel, dim3((nodes + 255) / 256), dim3(256), 0, s, *a);
+    const int span = reduce_span(a->t);
+    const int nbx = reduce_blocks_x(a->t.nx), nodes = (a->t.nx + 3) * (a->t.ny + 3);
+    const int nb = span ? nbx * reduce_blocks_y(a->t.ny) : (nodes + 255) / 256;
+    const dim3 grid(RED_FIN + nb);
+    if (span == 2) hipLaunchKernelGGL(reduce_kernel<2>, grid, dim3(256), 0, s, *a, nbx, nb);
+    else if (span == 3) hipLaunchKernelGGL(reduce_kernel<3>, grid, dim3(256), 0, s, *a, nbx, nb);
+    else hipLaunchKernelGGL(reduce_kernel<0>, grid, dim3(256), 0, s, *a, nbx, nb);
     ZK_LAUNCH_CHECK();
 }
 

@@ -6,6 +6,7 @@
 #define ZK_CURRENT_CORE_H
 
 #include "common.h"
+#include "reduce_index.h"
 
 namespace zk {
 
@@ -16,6 +17,8 @@ __device__ inline int floor_div(int a, int b)
     return (a % b != 0 && ((a < 0) != (b < 0))) ? q - 1 : q;
 }
 
+/* One node by itself, for any tiling and any grid: the windows one after
+ * the other.  reduce_block below is its faster form. */
 __device__ inline void reduce_node(const zk_reduce_args &a, const int node)
 {
     const zk_tiles &t = a.t;
@@ -58,6 +61,81 @@ __device__ inline void reduce_node(const zk_reduce_args &a, const int node)
     out[0] = sx;
     out[1] = sy;
     out[2] = sz;
+}
+
+/* Nodes [32 bx, 32 bx + 32) x [8 by, 8 by + 8) of the buffer, one thread
+ * each, for grids of at least 3 x 3 cells whose windows span at most N
+ * tiles per axis (W <= N T).
+ *
+ * The work is a handful of loads per node, and what bounds it is their
+ * latency: reduce_node walks the windows with integer divisions and waits
+ * for each load before the next (10 us on grids of any size up to 256 x
+ * 256).  Here the N x N candidate windows are found with one product per
+ * axis, all their loads are issued together, and the sums are then taken in
+ * reduce_node's order, so J is the same bit for bit: a window that does not
+ * cover the node adds 0 to a sum that starts at +0. */
+template <int N>
+__device__ inline void reduce_block(const zk_reduce_args &a, const int bx, const int by)
+{
+    const zk_tiles &t = a.t;
+    const int i = bx * ZK_RED_BX + (int)(threadIdx.x % ZK_RED_BX) - 1;
+    const int j = by * ZK_RED_BY + (int)(threadIdx.x / ZK_RED_BX) - 1;
+    if (i > t.nx + 1 || j > t.ny + 1) return;
+    const int fx = a.periodic_x, fy = !a.open_y;
+    const int ci = !fx ? i : i < 0 ? i + t.nx : i >= t.nx ? i - t.nx : i;
+    const int cj = !fy ? j : j < 0 ? j + t.ny : j >= t.ny ? j - t.ny : j;
+    const float invx = 1.0f / t.TX, invy = 1.0f / t.TY;
+    const int n = t.WX * t.WY;
+    int rxs[2], rys[2];
+    const int nix = axis_images(ci, t.nx, fx, rxs), niy = axis_images(cj, t.ny, fy, rys);
+    float s[3] = {0.0f, 0.0f, 0.0f};
+    for (int gy = 0; gy < niy; gy++) {
+        const int ry = gy ? rys[1] : rys[0];
+        const int ky = last_tile(ry, t.H, invy);
+        for (int gx = 0; gx < nix; gx++) {
+            const int rx = gx ? rxs[1] : rxs[0];
+            const int kx = last_tile(rx, t.H, invx);
+            const long long *o = a.Jov + 3 * ((rx + 1) + (size_t)(ry + 1) * a.nrow);
+            const long long o0 = o[0], o1 = o[1], o2 = o[2];
+            if (a.region) {
+                float v[N * N][3];
+#pragma unroll
+                for (int d = 0; d < N * N; d++) {
+                    const int ty = ky - (N - 1) + d / N, tx = kx - (N - 1) + d % N;
+                    const int w = window_offset(ry, t.H, t.TY, ty), u = window_offset(rx, t.H, t.TX, tx);
+                    const bool ok = window_covers(ty, t.nty, w, t.WY) && window_covers(tx, t.ntx, u, t.WX);
+                    const float *p = a.region + (ok ? (size_t)(tx + ty * t.ntx) * 3 * n + u + w * t.WX : 0);
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        const float q = p[c * n];
+                        v[d][c] = ok ? q : 0.0f;
+                    }
+                }
+#pragma unroll
+                for (int d = 0; d < N * N; d++)
+#pragma unroll
+                    for (int c = 0; c < 3; c++) s[c] += v[d][c];
+            }
+            s[0] += (float)o0 * a.jov_unscale;
+            s[1] += (float)o1 * a.jov_unscale;
+            s[2] += (float)o2 * a.jov_unscale;
+        }
+    }
+    float *out = a.J + 3 * ((size_t)(i + 1) + (size_t)(j + 1) * (t.nx + 3));
+    out[0] = s[0];
+    out[1] = s[1];
+    out[2] = s[2];
+}
+
+/* blocks of reduce_block over the buffer, and the N it needs (0: only
+ * reduce_node can take the grid or the tiling) */
+__host__ __device__ inline int reduce_blocks_x(int nx) { return (nx + 3 + ZK_RED_BX - 1) / ZK_RED_BX; }
+__host__ __device__ inline int reduce_blocks_y(int ny) { return (ny + 3 + ZK_RED_BY - 1) / ZK_RED_BY; }
+__host__ __device__ inline int reduce_span(const zk_tiles &t)
+{
+    if (t.nx < 3 || t.ny < 3) return 0;
+    if (t.WX <= 2 * t.TX && t.WY <= 2 * t.TY) return 2;
+    return t.WX <= 3 * t.TX && t.WY <= 3 * t.TY ? 3 : 0;
 }
 
 __device__ inline void stencil(float sa, float sb, const float *l, const float *m, const float *u, float *o)

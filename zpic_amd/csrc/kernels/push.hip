@@ -80,12 +80,6 @@ __global__ void __launch_bounds__(256) push_global_kernel(zk_push_args a)
     push_global_body(a, blockIdx.x, gridDim.x);
 }
 
-__global__ void __launch_bounds__(1024) finalize_kernel(zk_spec_ctr *ctr, const double *epart, int nparts, double qm, double dx0,
-                                double dx1)
-{
-    finalize_body(ctr, epart, nparts, qm, dx0, dx1);
-}
-
 /* one block per species */
 __global__ void __launch_bounds__(1024) finalize_set_kernel(zk_finalize_set f)
 {
@@ -167,13 +161,6 @@ extern "C" int zk_push_species(const zk_push_multi *m, zk_stream_t s)
     for (int k = 0; k < m->n; k++)
         if (m->s[k].global_blocks > 0)
             hipLaunchKernelGGL(push_global_kernel, dim3(m->s[k].global_blocks), dim3(256), 0, s, m->s[k]);
-    ZK_LAUNCH_CHECK();
-}
-
-extern "C" int zk_spec_finalize(zk_spec_ctr *ctr, const double *epart, int nparts, double qm,
-                                       double dx0, double dx1, zk_stream_t s)
-{
-    hipLaunchKernelGGL(finalize_kernel, dim3(1), dim3(1024), 0, s, ctr, epart, nparts, qm, dx0, dx1);
     ZK_LAUNCH_CHECK();
 }
 

@@ -9,6 +9,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "finalize_core.h"
 
 
 /* 1: the fixed-point push defers the deposits of cell-crossing particles
@@ -954,29 +955,6 @@ __device__ inline void push_global_body(const zk_push_args &a, const int block, 
     if (threadIdx.x == 0) {
         if (ndead_blk) atomicAdd(&a.ctr->n_dead, ndead_blk);
         if (nov_blk) atomicAdd(&a.ctr->n_overflow, nov_blk);
-    }
-}
-
-/* Sum the energy partials and count the pushes (em2d/particles.c:1231,
- * 1267).  The order of the sum is fixed (thread t adds partials t, t + B,
- * t + 2B, ... with coalesced loads, then a tree over the B threads; B a
- * power of two up to 1024), so every run sums alike. */
-__device__ inline void finalize_body(zk_spec_ctr *ctr, const double *epart, int nparts, double qm, double dx0,
-                                     double dx1)
-{
-    __shared__ double part[1024];
-    double s = 0.0;
-    for (int i = threadIdx.x; i < nparts; i += blockDim.x) s += epart[i];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = (int)blockDim.x / 2; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) part[threadIdx.x] += part[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const double tot = part[0];
-        ctr->energy = qm * tot * dx0 * dx1;
-        ctr->npush += (unsigned long long)(ctr->np_total - ctr->n_dead - ctr->n_slack);
     }
 }
 

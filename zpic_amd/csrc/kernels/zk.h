@@ -143,8 +143,6 @@ typedef struct zk_finalize_set {
     double qm[ZK_FUSE_MAX], dx0[ZK_FUSE_MAX], dx1[ZK_FUSE_MAX];
 } zk_finalize_set;
 int zk_spec_finalize_set(const zk_finalize_set *f, zk_stream_t s);
-int zk_spec_finalize(zk_spec_ctr *ctr, const double *epart, int nparts,
-                            double qm, double dx0, double dx1, zk_stream_t s);
 
 /* Tile ranges.  Range t of a sorted set starts at off[t]; its first
  * tile_n[t] slots hold the tile's particles and the rest, up to
@@ -196,7 +194,11 @@ typedef struct zk_reduce_args {
     zk_tiles t;
     int periodic_x;
     int open_y;                 /* no fold along y: the raw guard rows are kept */
+    zk_finalize_set fin;        /* species whose last push is finished along with it */
 } zk_reduce_args;
+/* nodes of the buffer per block of the reduction */
+#define ZK_RED_BX 32
+#define ZK_RED_BY 8
 int zk_current_reduce(const zk_reduce_args *a, zk_stream_t s);
 int zk_smooth(const float *in, float *out, int nx, int ny, int nrow, int axis,
                      float sa, float sb, int periodic_x, int open_y, zk_stream_t s);
@@ -361,7 +363,9 @@ int zk_batch_prepare_push(size_t lds);
 int zk_batch_push(const zk_bspec *specs, const zk_bsim *sims, const int *tile_items, int ntile,
                   const int *global_items, int nglobal, size_t lds, int waves, int fixed, zk_stream_t s);
 int zk_batch_finalize(const zk_bspec *specs, int nspecs, zk_stream_t s);
-int zk_batch_current(const zk_bsim *sims, const int *node_items, int n, int max_passes, zk_stream_t s);
+int zk_batch_reduce_blocks(const zk_bsim *M); /* blocks of the current fold of one simulation */
+int zk_batch_current(const zk_bsim *sims, const int *reduce_items, int nreduce, const int *node_items, int n,
+                     int max_passes, zk_stream_t s);
 int zk_batch_fields(const zk_bsim *sims, const int *yee_items, int nyee, zk_stream_t s);
 int zk_batch_sort(const zk_bspec *specs, int nspecs, const int *items, int n, zk_stream_t s);
 int zk_batch_end_step(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_stream_t s);
