@@ -452,7 +452,7 @@ void emf_advance(t_emf *emf, const t_current *ccur)
     zpic_emf_ensure(emf);
     zpic_current_ensure(cur, NULL);
     struct zpic_dev_emf *d = emf->dev;
-    zpic_timer_begin(ZPIC_T_EMF);
+    const zk_stamp st = zpic_phase_begin(ZPIC_T_EMF);
     const int o = 1 - d->cur;
     /* a window move after this step (em2d/emf.c:648-650, with the
      * iteration count the step ends with) is written by the field update
@@ -463,7 +463,7 @@ void emf_advance(t_emf *emf, const t_current *ccur)
                       emf->ext_fld.B_type == EMF_FLD_TYPE_NONE;
     zpic_ktimer_begin(ZPIC_T_FIELD);
     ZCHECK(zk_yee(d->E[d->cur], d->B[d->cur], zpic_current_J(cur), d->E[o], d->B[o], emf->nx[0], emf->nx[1],
-                  emf->nrow, emf->dt, emf->dx[0], emf->dx[1], !emf->moving_window, d->open_y, fused,
+                  emf->nrow, emf->dt, emf->dx[0], emf->dx[1], !emf->moving_window, d->open_y, fused, st,
                   zpic_stream()));
     zpic_ktimer_end(ZPIC_T_FIELD);
     d->cur = o;
@@ -478,7 +478,8 @@ void emf_advance(t_emf *emf, const t_current *ccur)
         d->cur = m;
         emf->n_move++;
     }
-    zpic_timer_end(ZPIC_T_EMF);
+    zpic_phase_end(ZPIC_T_EMF, (move && !fused) || emf->ext_fld.E_type != EMF_FLD_TYPE_NONE ||
+                                   emf->ext_fld.B_type != EMF_FLD_TYPE_NONE);
     d->host_valid = 0;
 }
 

@@ -726,7 +726,7 @@ static void sort_now_from(t_species *s, int spread, int slack, const int *before
         /* the particles are in tile ranges (plus a tail): keep the stayers */
         ZCHECK(zk_sort_tiles(&d->set[d->cur], &d->set[other], d->ctr, d->cnt, d->stay, d->nbr, d->tailn, d->tile_off,
                              d->counted ? d->tile_n : NULL, before, d->tile_off2, d->tile_n2, d->cursor, &d->t,
-                             d->tail_upper, slack, d->cap, zpic_stream()));
+                             d->tail_upper, slack, d->cap, zpic_phase_stamp(ZPIC_T_SPEC), zpic_stream()));
         int *tmp = d->tile_off;
         d->tile_off = d->tile_off2;
         d->tile_off2 = tmp;
@@ -992,13 +992,15 @@ static void inject_column(t_species *s)
     if (n > 0) {
         grow_sets(d, d->np_upper + n);
         if (n <= ZK_APPEND_MAX) {
-            ZCHECK(zk_unpack_append(d->pin_dev[k], n, &d->set[d->cur], d->next_id, d->ctr, zpic_stream()));
+            ZCHECK(zk_unpack_append(d->pin_dev[k], n, &d->set[d->cur], d->next_id, d->ctr,
+                                    zpic_phase_stamp(ZPIC_T_SPEC), zpic_stream()));
             zpic_event_record(d->pin_ev[k]);
         } else {
             ensure_stage(d, sizeof(t_part) * (size_t)n);
             zpic_h2d_async(d->stage, tmp, sizeof(t_part) * (size_t)n);
             zpic_event_record(d->pin_ev[k]);
             ZCHECK(zk_unpack(d->stage, n, &d->set[d->cur], d->next_id, d->ctr, 1, zpic_stream()));
+            ZCHECK(zk_stamp_end(zpic_phase_stamp(ZPIC_T_SPEC), zpic_stream()));
         }
         d->next_id += n;
         d->np_upper += n;
@@ -1060,6 +1062,7 @@ static void inject_column_device(t_species *s, int k, zk_rng_state *rng)
         a.rng = rng;
         ZCHECK(zk_inject_column(&a, zpic_stream()));
         zpic_event_record(d->pin_ev[k]);
+        ZCHECK(zk_stamp_end(zpic_phase_stamp(ZPIC_T_SPEC), zpic_stream()));
         d->next_id += n;
         d->np_upper += n;
         d->tail_upper += n;
@@ -1214,10 +1217,10 @@ void spec_advance(t_species *s, t_emf *emf, t_current *cur)
     zpic_emf_ensure(emf);
     zpic_current_ensure(cur, &s->dev->t);
 
-    zpic_timer_begin(ZPIC_T_SPEC);
     zk_push_args a;
     int move;
     push_args(s, emf, cur, &a, &move);
+    a.stamp = zpic_phase_begin(ZPIC_T_SPEC);
     const int sort = sort_due(s, move);
     const int staged = sort && staged_ready(s->dev) && a.fixed;
     if (staged) push_sorting(s, &a);
@@ -1236,7 +1239,7 @@ void spec_advance(t_species *s, t_emf *emf, t_current *cur)
         sort_now(s, 0, 1);
     }
     probe_prefetch(s);
-    zpic_timer_end(ZPIC_T_SPEC);
+    zpic_phase_end(ZPIC_T_SPEC, staged);
 }
 
 static int same_tiles(const zk_tiles *a, const zk_tiles *b)
@@ -1265,7 +1268,10 @@ void zpic_spec_advance_all(t_species *spec, int n, t_emf *emf, t_current *cur)
         for (int k = 1; k < n && fuse; k++)
             fuse = same_tiles(&m.s[k].t, &m.s[0].t) && m.s[k].fx_scale == m.s[0].fx_scale;
         if (fuse) {
-            zpic_timer_begin(ZPIC_T_SPEC);
+            const zk_stamp st = zpic_phase_begin(ZPIC_T_SPEC);
+            m.s[0].stamp = st;
+            for (int k = 1; k < n; k++) m.s[k].stamp = zpic_phase_stamp(ZPIC_T_SPEC);
+            int extra = 0;
             /* the sort decisions (whose counter reads wait for the queue)
              * are taken before the push, which sorts where it can */
             int due[ZK_FUSE_MAX], staged[ZK_FUSE_MAX];
@@ -1290,7 +1296,8 @@ void zpic_spec_advance_all(t_species *spec, int n, t_emf *emf, t_current *cur)
                 }
             }
             for (int k = 0; k < n; k++) probe_prefetch(&spec[k]);
-            zpic_timer_end(ZPIC_T_SPEC);
+            for (int k = 0; k < n; k++) extra |= staged[k];
+            zpic_phase_end(ZPIC_T_SPEC, extra);
             return;
         }
     }

@@ -78,5 +78,12 @@ void zpic_ktimer_end(int which);
 void zpic_timer_begin(int which);
 void zpic_timer_end(int which);
 double zpic_timer_total(int which);
+/* The phases ZPIC_T_SPEC and ZPIC_T_EMF are timed by their own kernels
+ * (zk_clock): zpic_phase_begin gives the stamp of the phase's first launch,
+ * zpic_phase_stamp that of a later one (an untimed stamp when the phase is
+ * not open); extra ends a phase whose last launches took none. */
+zk_stamp zpic_phase_begin(int which);
+zk_stamp zpic_phase_stamp(int which);
+void zpic_phase_end(int which, int extra);
 
 #endif

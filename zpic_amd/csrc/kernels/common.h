@@ -64,6 +64,22 @@ __device__ inline int zk_cell_ix(int c, int cbits) { return c < 0 ? ZK_DEAD : (c
 __device__ inline int zk_cell_iy(int c, int cbits) { return c >> cbits; }
 __device__ inline int zk_cell(int ix, int iy, int cbits) { return ix == ZK_DEAD ? -1 : (ix | (iy << cbits)); }
 
+/* Clock readings of a timed phase (zk_clock): zk_stamp_first at the start of
+ * a launch, zk_stamp_last at its end; every thread may call them. */
+__device__ inline void zk_stamp_first(const zk_stamp &s)
+{
+    if (!s.clk || !s.open || blockIdx.x + blockIdx.y != 0 || threadIdx.x != 0) return;
+    const int o = 1 - s.slot;
+    if (s.clk->t1[o] > s.clk->t0[o]) s.clk->total += s.clk->t1[o] - s.clk->t0[o];
+    s.clk->t0[s.slot] = wall_clock64();
+}
+
+__device__ inline void zk_stamp_last(const zk_stamp &s)
+{
+    if (!s.clk || blockIdx.x + 1 != gridDim.x || blockIdx.y + 1 != gridDim.y || threadIdx.x != 0) return;
+    s.clk->t1[s.slot] = wall_clock64();
+}
+
 /* Floor modulo for periodic wrap. */
 __device__ inline int zk_wrap(int i, int n)
 {

@@ -34,9 +34,11 @@ namespace {
 __global__ void __launch_bounds__(256) yee_kernel(const float *__restrict__ E, const float *__restrict__ B,
                                                   const float *__restrict__ J, float *__restrict__ Eo,
                                                   float *__restrict__ Bo, int nx, int ny, int nrow, YeeK k,
-                                                  int periodic_x, int open_y, int shift)
+                                                  int periodic_x, int open_y, int shift, zk_stamp st)
 {
+    zk_stamp_first(st);
     yee_tile(E, B, J, Eo, Bo, nx, ny, nrow, k, blockIdx.x, blockIdx.y, periodic_x, open_y, shift);
+    zk_stamp_last(st);
 }
 
 __global__ void guard_kernel(float *E, float *B, int nx, int ny, int nrow, int periodic_x, int open_y)
@@ -307,7 +309,8 @@ extern "C" int zk_pha(const zk_parts *p, int np_upper, const zk_spec_ctr *ctr, i
 }
 
 extern "C" int zk_yee(const float *E, const float *B, const float *J, float *Eo, float *Bo, int nx, int ny,
-                             int nrow, float dt, float dx, float dy, int periodic_x, int open_y, int shift, zk_stream_t s)
+                             int nrow, float dt, float dx, float dy, int periodic_x, int open_y, int shift, zk_stamp st,
+                      zk_stream_t s)
 {
     YeeK k;
     const float dt2 = dt / 2.0f;
@@ -319,7 +322,7 @@ extern "C" int zk_yee(const float *E, const float *B, const float *J, float *Eo,
     k.mur_y = (dt - dy) / (dt + dy);
     dim3 grid((nx + 3 + BX - 1) / BX, (ny + 3 + BY - 1) / BY);
     hipLaunchKernelGGL(yee_kernel, grid, dim3(256), 0, s, E, B, J, Eo, Bo, nx, ny, nrow, k, periodic_x,
-                       open_y, shift);
+                       open_y, shift, st);
     ZK_LAUNCH_CHECK();
 }
 

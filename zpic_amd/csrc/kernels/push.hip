@@ -59,26 +59,33 @@ constexpr int ZK_WIN_DEFAULT = 25; /* 16 x 16 tiles, 3-cell margin */
 template <int MIN_WAVES, int PAIR, bool FX, int WC = 0>
 __global__ void __launch_bounds__(256, MIN_WAVES) push_tile_kernel(zk_push_args a)
 {
-    if ((int)blockIdx.x >= a.t.ntiles) {
+    zk_stamp_first(a.stamp);
+    if ((int)blockIdx.x >= a.t.ntiles)
         push_global_body(a, (int)blockIdx.x - a.t.ntiles, a.global_blocks);
-        return;
-    }
-    push_tile_body<PAIR, FX, OneSpecies, WC>(OneSpecies{a}, zk_xcd_item(blockIdx.x, a.t.ntiles));
+    else
+        push_tile_body<PAIR, FX, OneSpecies, WC>(OneSpecies{a}, zk_xcd_item(blockIdx.x, a.t.ntiles));
+    zk_stamp_last(a.stamp);
 }
 
 /* every species of a simulation in one launch (shared staging and window) */
 template <int WC>
 __global__ void __launch_bounds__(256, ZK_SPECIES_OCC) push_species_kernel(zk_push_multi m)
 {
+    zk_stamp_first(m.s[0].stamp);
     push_tile_body<1, true, SpeciesSet, WC>(SpeciesSet{m}, zk_xcd_item(blockIdx.x, m.s[0].t.ntiles));
+    zk_stamp_last(m.s[0].stamp);
 }
 
 bool default_window(const zk_tiles &t) { return t.WX == ZK_WIN_DEFAULT && t.WY == ZK_WIN_DEFAULT; }
 
 __global__ void __launch_bounds__(256) push_global_kernel(zk_push_args a)
 {
+    zk_stamp_first(a.stamp);
     push_global_body(a, blockIdx.x, gridDim.x);
+    zk_stamp_last(a.stamp);
 }
+
+__global__ void stamp_kernel(zk_stamp st) { zk_stamp_last(st); }
 
 /* one block per species */
 __global__ void __launch_bounds__(1024) finalize_set_kernel(zk_finalize_set f)
@@ -177,6 +184,12 @@ extern "C" int zk_fill_f32(float *p, size_t n, float v, zk_stream_t s)
     size_t blocks = (n + 255) / 256;
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(fill_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p, n, v);
+    ZK_LAUNCH_CHECK();
+}
+
+extern "C" int zk_stamp_end(zk_stamp st, zk_stream_t s)
+{
+    hipLaunchKernelGGL(stamp_kernel, dim3(1), dim3(64), 0, s, st);
     ZK_LAUNCH_CHECK();
 }
 

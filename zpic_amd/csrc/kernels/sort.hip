@@ -70,9 +70,10 @@ __global__ void __launch_bounds__(1024) scan_stay_kernel(const int *stay, int *m
 
 __global__ void __launch_bounds__(ZK_SORT_THREADS)
     scatter_stay_kernel(zk_parts src, zk_parts dst, const int *old_off, const int *old_n, const int *new_off,
-                        const int *stay, const int *nbr, int *cursor, zk_tiles t)
+                        const int *stay, const int *nbr, int *cursor, zk_tiles t, zk_stamp st)
 {
     scatter_stay_body(src, dst, old_off, old_n, new_off, stay, nbr, cursor, t, blockIdx.x, gridDim.x);
+    zk_stamp_last(st);
 }
 
 __global__ void __launch_bounds__(ZK_SORT_THREADS)
@@ -120,7 +121,7 @@ __global__ void unpack_kernel(const int *__restrict__ aos, int n, zk_parts dst, 
  * no copy on the stream) and commits the new count itself, so one launch
  * replaces a copy, the unpack and the commit. */
 __global__ void __launch_bounds__(1024) unpack_append_kernel(const int *__restrict__ aos, int n, zk_parts dst,
-                                                             int64_t id0, zk_spec_ctr *ctr)
+                                                             int64_t id0, zk_spec_ctr *ctr, zk_stamp st)
 {
     __shared__ int base_s;
     if (threadIdx.x == 0) base_s = ctr->np_total;
@@ -142,6 +143,7 @@ __global__ void __launch_bounds__(1024) unpack_append_kernel(const int *__restri
     }
     __syncthreads();
     if (threadIdx.x == 0) ctr->np_total = base + n;
+    zk_stamp_last(st);
 }
 
 __global__ void unpack_commit(zk_spec_ctr *ctr, int n, int append)
@@ -205,7 +207,7 @@ extern "C" int zk_sort(const zk_parts *src, const zk_parts *dst, zk_spec_ctr *ct
 extern "C" int zk_sort_tiles(const zk_parts *src, const zk_parts *dst, zk_spec_ctr *ctr, int *move, int *stay,
                              int *nbr, int *tailn, int *old_off, const int *old_n, const int *before,
                              int *new_off, int *new_n, int *cursor, const zk_tiles *t, int tail_upper, int slack,
-                             int cap_slots, zk_stream_t s)
+                             int cap_slots, zk_stamp st, zk_stream_t s)
 {
     const unsigned tb = tail_upper > 0 ? grid_for(tail_upper, 1024, 4096) : 0;
     const unsigned g = (unsigned)t->ntiles + tb;
@@ -215,7 +217,7 @@ extern "C" int zk_sort_tiles(const zk_parts *src, const zk_parts *dst, zk_spec_c
     hipLaunchKernelGGL(scan_stay_kernel, dim3(1), dim3(1024), 0, s, stay, move, tailn, new_off, new_n, cursor, ctr,
                        t->ntiles, slack, cap_slots, before);
     hipLaunchKernelGGL(scatter_stay_kernel, dim3(g), dim3(ZK_SORT_THREADS), 0, s, *src, *dst, old_off, old_n,
-                       new_off, stay, nbr, cursor, *t);
+                       new_off, stay, nbr, cursor, *t, st);
     if (t->ntiles > 0 && new_n && slack)
         hipLaunchKernelGGL(mark_free_kernel, dim3(t->ntiles), dim3(256), 0, s, dst->cell, new_off, new_n);
     ZK_LAUNCH_CHECK();
@@ -246,11 +248,12 @@ extern "C" int zk_unpack(const void *aos, int n, const zk_parts *dst, int64_t id
 }
 
 extern "C" int zk_unpack_append(const void *aos, int n, const zk_parts *dst, int64_t id0, zk_spec_ctr *ctr,
-                                 zk_stream_t s)
+                                zk_stamp st, zk_stream_t s)
 {
     if (n <= 0) return 0;
     if (n > ZK_APPEND_MAX) return 1;
-    hipLaunchKernelGGL(unpack_append_kernel, dim3(1), dim3(1024), 0, s, (const int *)aos, n, *dst, id0, ctr);
+    hipLaunchKernelGGL(unpack_append_kernel, dim3(1), dim3(1024), 0, s, (const int *)aos, n, *dst, id0, ctr,
+                       st);
     ZK_LAUNCH_CHECK();
 }
 

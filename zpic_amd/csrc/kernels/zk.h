@@ -41,6 +41,21 @@ extern "C" {
  * free slots included). */
 #define ZK_FX_TILE_MAX ((1 << 18) - 16)
 
+/* Time the GPU spends in a phase of the step (spec_time, emf_time), kept by
+ * the phase's own kernels: the first block of its first launch reads the
+ * constant-rate clock into t0[slot] and adds the previous phase's interval
+ * to total; the last block of each of its launches reads it into t1[slot].
+ * Phases alternate slots, so the two never touch the same entry in one
+ * launch. */
+typedef struct zk_clock {
+    unsigned long long t0[2], t1[2], total; /* ticks */
+} zk_clock;
+typedef struct zk_stamp {
+    zk_clock *clk;              /* NULL: the launch is not timed */
+    int slot;
+    int open;                   /* 1: this launch begins the phase */
+} zk_stamp;
+
 /* Per-species counters kept in device memory. */
 typedef struct zk_spec_ctr {
     int np_total;               /* slots in use: tile ranges + unsorted tail */
@@ -117,6 +132,7 @@ typedef struct zk_push_args {
     int sorting;
     zk_parts sdst;
     int *sstay, *sleave;
+    zk_stamp stamp;
 } zk_push_args;
 
 /* Species of one simulation pushed by one tile launch: same tiling,
@@ -128,6 +144,8 @@ typedef struct zk_push_multi {
 } zk_push_multi;
 
 int zk_fill_f32(float *p, size_t n, float v, zk_stream_t s);
+/* reads the clock into a phase's end on its own */
+int zk_stamp_end(zk_stamp st, zk_stream_t s);
 /* divide the n fixed-point values of p by 2^shift (arithmetic shift) */
 int zk_rescale_fx(long long *p, size_t n, int shift, zk_stream_t s);
 int zk_push(const zk_push_args *a, zk_stream_t s);
@@ -163,7 +181,8 @@ int zk_sort(const zk_parts *src, const zk_parts *dst, zk_spec_ctr *ctr,
  * nbr (13 ntiles) */
 int zk_sort_tiles(const zk_parts *src, const zk_parts *dst, zk_spec_ctr *ctr, int *move, int *stay, int *nbr,
                   int *tailn, int *old_off, const int *old_n, const int *before, int *new_off, int *new_n,
-                  int *cursor, const zk_tiles *t, int tail_upper, int slack, int cap_slots, zk_stream_t s);
+                  int *cursor, const zk_tiles *t, int tail_upper, int slack, int cap_slots, zk_stamp st,
+                  zk_stream_t s);
 /* Second half of a staged re-sort, after a push with `sorting` set: the
  * staged leavers of every tile (sleave[t] of them in the staging region of
  * dst) go to the free slots of their new tile's range behind its sstay[t]
@@ -182,7 +201,8 @@ int zk_pack(const zk_parts *src, int n, void *aos, zk_stream_t s);
 /* append n <= ZK_APPEND_MAX particles (t_part AoS, device-accessible, e.g.
  * page-locked host memory) to the unsorted tail in one launch */
 #define ZK_APPEND_MAX 16384
-int zk_unpack_append(const void *aos, int n, const zk_parts *dst, int64_t id0, zk_spec_ctr *ctr, zk_stream_t s);
+int zk_unpack_append(const void *aos, int n, const zk_parts *dst, int64_t id0, zk_spec_ctr *ctr, zk_stamp st,
+                     zk_stream_t s);
 
 /* current: window reduction + raw overflow -> folded J; smoothing passes */
 typedef struct zk_reduce_args {
@@ -218,7 +238,7 @@ int zk_smooth_x_passes(const float *in, float *out, int nx, int ny, int nrow, in
  * the rightmost columns zeroed), as zk_move_window would make it */
 int zk_yee(const float *E, const float *B, const float *J, float *Eo, float *Bo,
                   int nx, int ny, int nrow, float dt, float dx, float dy, int periodic_x, int open_y, int shift,
-                  zk_stream_t s);
+                  zk_stamp st, zk_stream_t s);
 int zk_field_guards(float *E, float *B, int nx, int ny, int nrow, int periodic_x,
                            int open_y, zk_stream_t s);
 int zk_move_window(const float *E, const float *B, float *Eo, float *Bo, int nx,
