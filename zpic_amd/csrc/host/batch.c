@@ -68,7 +68,7 @@ static void fill_sim(zpic_batch *b, int i)
     }
     M->region = dc->region;
     for (int k = 0; k < sim->n_species; k++) zpic_current_jov_register(cur, sim->species[k].q);
-    M->Jov = dc->Jov;
+    M->Jov = zpic_current_jov(cur, 0);
     M->jov_unscale = zpic_current_jov_unscale(cur);
     M->ecur = de->cur;
     M->jcur = dc->jcur;
@@ -104,7 +104,7 @@ static void fill_spec(zpic_batch *b, int k)
     a->nrow = cur->nrow;
     a->region = dc->region;
     a->fresh = (b->spec_k[k] == 0);
-    a->Jov = dc->Jov;
+    a->Jov = zpic_current_jov(cur, 0);
     a->jov_scale = zpic_current_jov_scale(cur);
     a->epart = d->epart;
     a->t = d->t;

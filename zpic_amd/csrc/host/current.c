@@ -55,12 +55,39 @@ void current_delete(t_current *c)
         zpic_dfree(d->J[0]);
         zpic_dfree(d->J[1]);
         zpic_dfree(d->region);
-        zpic_dfree(d->Jov);
+        for (int k = 0; k < 2; k++) {
+            zpic_dfree(d->Jov2[k]);
+            zpic_dfree(d->jflag[k]);
+        }
         free(d);
         c->dev = NULL;
     }
     free(c->J_buf);
     c->J_buf = NULL;
+}
+
+static size_t jflag_bytes(const t_current *c)
+{
+    const size_t n = (size_t)zk_red_blocks_x(c->nx[0]) * (size_t)zk_red_blocks_y(c->nx[1]);
+    return (n + 3) / 4 * 4;
+}
+
+/* overflow grid k all zero (zero bits are the fixed-point zero) */
+static void jov_clear(t_current *c, int k)
+{
+    struct zpic_dev_current *d = c->dev;
+    if (d->jov_state[k] == ZPIC_JOV_CLEAN) return;
+    ZCHECK(zk_fill_f32((float *)d->Jov2[k], 6 * zpic_grid_nodes(c->nx), 0.0f, zpic_stream()));
+    ZCHECK(zk_fill_f32((float *)d->jflag[k], jflag_bytes(c) / 4, 0.0f, zpic_stream()));
+    d->jov_state[k] = ZPIC_JOV_CLEAN;
+}
+
+long long *zpic_current_jov(t_current *c, int flagged)
+{
+    struct zpic_dev_current *d = c->dev;
+    int *st = &d->jov_state[d->jov_cur];
+    *st = flagged && *st != ZPIC_JOV_DIRTY ? ZPIC_JOV_FLAGGED : ZPIC_JOV_DIRTY;
+    return d->Jov2[d->jov_cur];
 }
 
 /* the launch that follows finishes the pushes in the list */
@@ -89,10 +116,15 @@ void zpic_current_ensure(t_current *c, const zk_tiles *t)
         const size_t nodes = zpic_grid_nodes(c->nx);
         d->J[0] = zpic_dmalloc(sizeof(float3) * nodes);
         d->J[1] = zpic_dmalloc(sizeof(float3) * nodes);
-        d->Jov = zpic_dmalloc(sizeof(long long) * 3 * nodes);
+        for (int k = 0; k < 2; k++) {
+            d->Jov2[k] = zpic_dmalloc(sizeof(long long) * 3 * nodes);
+            d->jflag[k] = zpic_dmalloc(jflag_bytes(c));
+            d->jov_state[k] = ZPIC_JOV_DIRTY;
+        }
+        d->jov_cur = 0;
+        jov_clear(c, 0);
         d->region = zpic_dmalloc(sizeof(float) * 3 * (size_t)tt.WX * (size_t)tt.WY * (size_t)tt.ntiles);
         ZCHECK(zk_fill_f32(d->J[0], 3 * nodes, 0.0f, zpic_stream()));
-        ZCHECK(zk_fill_f32((float *)d->Jov, 6 * nodes, 0.0f, zpic_stream()));
         d->jcur = 0;
         d->ready = 1;
     } else if (t && (t->TX != d->t.TX || t->TY != d->t.TY || t->H != d->t.H || t->nx != d->t.nx ||
@@ -106,8 +138,8 @@ void current_zero(t_current *c)
     /* em2d/current.c:98-107: every deposit of the step starts from zero */
     zpic_current_ensure(c, NULL);
     struct zpic_dev_current *d = c->dev;
-    /* zero bits are the fixed-point zero */
-    ZCHECK(zk_fill_f32((float *)d->Jov, 6 * zpic_grid_nodes(c->nx), 0.0f, zpic_stream()));
+    if (d->jov_state[d->jov_cur] != ZPIC_JOV_CLEAN) d->jov_cur ^= 1;
+    jov_clear(c, d->jov_cur);
     d->fresh = 1;
     d->host_valid = 0;
 }
@@ -124,7 +156,7 @@ void zpic_current_jov_register(t_current *c, float q)
     const int k = zpic_fixed_point_exp(q);
     if (d->jov_set && k <= d->jov_k) return;
     if (d->jov_set && d->ready)
-        ZCHECK(zk_rescale_fx(d->Jov, 3 * zpic_grid_nodes(c->nx), k - d->jov_k, zpic_stream()));
+        ZCHECK(zk_rescale_fx(d->Jov2[d->jov_cur], 3 * zpic_grid_nodes(c->nx), k - d->jov_k, zpic_stream()));
     d->jov_k = k;
     d->jov_set = 1;
 }
@@ -183,7 +215,12 @@ void current_update(t_current *c)
     struct zpic_dev_current *d = c->dev;
     zk_reduce_args a;
     a.region = d->fresh ? NULL : d->region;
-    a.Jov = d->Jov;
+    a.Jov = d->Jov2[d->jov_cur];
+    a.jflag = d->jov_state[d->jov_cur] == ZPIC_JOV_DIRTY ? NULL : d->jflag[d->jov_cur];
+    const int other = 1 - d->jov_cur;
+    const int clears = d->jov_state[other] == ZPIC_JOV_FLAGGED && zk_current_clears(&d->t);
+    a.Jov_next = clears ? d->Jov2[other] : NULL;
+    a.jflag_next = clears ? d->jflag[other] : NULL;
     a.jov_unscale = zpic_current_jov_unscale(c);
     a.J = d->J[d->jcur];
     a.nrow = c->nrow;
@@ -193,6 +230,7 @@ void current_update(t_current *c)
     a.fin = d->fin;
     zpic_ktimer_begin(ZPIC_T_CURRENT);
     ZCHECK(zk_current_reduce(&a, zpic_stream()));
+    if (clears) d->jov_state[other] = ZPIC_JOV_CLEAN;
     fin_done(d);
     const int maxp = 2 * (c->smooth.xlevel > 0 ? c->smooth.xlevel : 0) + 2;
     int axis[maxp];

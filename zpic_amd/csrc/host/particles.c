@@ -1090,7 +1090,8 @@ static void push_args(t_species *s, t_emf *emf, t_current *cur, zk_push_args *pa
     a.region = dc->region;
     a.fresh = dc->fresh;
     zpic_current_jov_register(cur, s->q);
-    a.Jov = dc->Jov;
+    a.Jov = zpic_current_jov(cur, 1);
+    a.jflag = dc->jflag[dc->jov_cur];
     a.jov_scale = zpic_current_jov_scale(cur);
     a.epart = d->epart;
     a.t = d->t;

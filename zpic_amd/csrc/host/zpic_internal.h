@@ -91,6 +91,12 @@ struct zpic_dev_species {
     struct zpic_dev_current *fin_cur; /* holds this species' unfinished push */
 };
 
+enum {
+    ZPIC_JOV_DIRTY = 0,   /* anything: cleared as a whole before it is used */
+    ZPIC_JOV_CLEAN = 1,   /* all zero, no flag set */
+    ZPIC_JOV_FLAGGED = 2, /* zero but for the flagged blocks */
+};
+
 struct zpic_dev_current {
     int ready;
     int host_valid;
@@ -98,7 +104,13 @@ struct zpic_dev_current {
     float *J[2];
     int jcur;
     float *region;        /* per-tile current windows */
-    long long *Jov;       /* raw current of out-of-window pushes (fixed point) */
+    /* raw current of out-of-window pushes (fixed point): two grids that take
+     * turns, so that the fold of one step can clear the other for the next;
+     * jov_state says what each holds */
+    long long *Jov2[2];
+    unsigned char *jflag[2]; /* blocks deposited to (zk_red_blocks) */
+    int jov_state[2];     /* ZPIC_JOV_* */
+    int jov_cur;
     int jov_k;            /* Jov holds multiples of 2^(jov_k - 40) */
     int jov_set;          /* jov_k was set by a species */
     int fresh;            /* no deposit since current_zero */
@@ -137,6 +149,9 @@ const float *zpic_current_J(t_current *cur);
 /* the overflow grid's fixed-point scale covers a species of charge q
  * (raised, with the grid's sums rescaled exactly, when q needs more) */
 void zpic_current_jov_register(t_current *cur, float q);
+/* the overflow grid of this step, about to be deposited to: by a push that
+ * flags what it touches, or (flagged 0) by one that does not */
+long long *zpic_current_jov(t_current *cur, int flagged);
 float zpic_current_jov_scale(const t_current *cur);   /* 2^(40 - jov_k) */
 float zpic_current_jov_unscale(const t_current *cur); /* 2^(jov_k - 40) */
 

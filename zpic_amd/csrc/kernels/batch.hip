@@ -85,13 +85,15 @@ __global__ void reduce_batch(const zk_bsim *sims, const int *items)
     zk_reduce_args r;
     r.region = M.deposited ? M.region : nullptr;
     r.Jov = M.Jov;
+    r.jflag = nullptr;
+    r.jflag_next = nullptr;
     r.jov_unscale = M.jov_unscale;
     r.J = j_after(M, 0);
     r.nrow = M.nrow;
     r.t = M.t;
     r.periodic_x = 1;
     r.open_y = 0;
-    const int b = items[2 * blockIdx.x + 1], span = reduce_span(r.t), nbx = reduce_blocks_x(M.nx);
+    const int b = items[2 * blockIdx.x + 1], span = reduce_span(r.t), nbx = zk_red_blocks_x(M.nx);
     if (span == 2) reduce_block<2>(r, b % nbx, b / nbx);
     else if (span == 3) reduce_block<3>(r, b % nbx, b / nbx);
     else reduce_node(r, b * blockDim.x + threadIdx.x);
@@ -213,7 +215,7 @@ extern "C" int zk_batch_finalize(const zk_bspec *specs, int nspecs, zk_stream_t 
 
 extern "C" int zk_batch_reduce_blocks(const zk_bsim *M)
 {
-    if (reduce_span(M->t)) return reduce_blocks_x(M->nx) * reduce_blocks_y(M->ny);
+    if (reduce_span(M->t)) return zk_red_blocks_x(M->nx) * zk_red_blocks_y(M->ny);
     return ((M->nx + 3) * (M->ny + 3) + 255) / 256;
 }
 

@@ -160,11 +160,13 @@ extern "C" int zk_smooth_x_passes(const float *in, float *out, int nx, int ny, i
     ZK_LAUNCH_CHECK();
 }
 
+extern "C" int zk_current_clears(const zk_tiles *t) { return reduce_span(*t) != 0; }
+
 extern "C" int zk_current_reduce(const zk_reduce_args *a, zk_stream_t s)
 {
     const int span = reduce_span(a->t);
-    const int nbx = reduce_blocks_x(a->t.nx), nodes = (a->t.nx + 3) * (a->t.ny + 3);
-    const int nb = span ? nbx * reduce_blocks_y(a->t.ny) : (nodes + 255) / 256;
+    const int nbx = zk_red_blocks_x(a->t.nx), nodes = (a->t.nx + 3) * (a->t.ny + 3);
+    const int nb = span ? nbx * zk_red_blocks_y(a->t.ny) : (nodes + 255) / 256;
     const dim3 grid(RED_FIN + nb);
     if (span == 2) hipLaunchKernelGGL(reduce_kernel<2>, grid, dim3(256), 0, s, *a, nbx, nb);
     else if (span == 3) hipLaunchKernelGGL(reduce_kernel<3>, grid, dim3(256), 0, s, *a, nbx, nb);

@@ -78,9 +78,22 @@ template <int N>
 __device__ inline void reduce_block(const zk_reduce_args &a, const int bx, const int by)
 {
     const zk_tiles &t = a.t;
+    /* the other overflow grid, deposited to in the step before: its flagged
+     * blocks are cleared for the next step */
+    bool clear = false;
+    if (a.jflag_next) {
+        unsigned char *f = a.jflag_next + bx + by * zk_red_blocks_x(t.nx);
+        clear = *f != 0;
+        __syncthreads();
+        if (clear && threadIdx.x == 0) *f = 0;
+    }
     const int i = bx * ZK_RED_BX + (int)(threadIdx.x % ZK_RED_BX) - 1;
     const int j = by * ZK_RED_BY + (int)(threadIdx.x / ZK_RED_BX) - 1;
     if (i > t.nx + 1 || j > t.ny + 1) return;
+    if (clear) {
+        long long *z = a.Jov_next + 3 * ((size_t)(i + 1) + (size_t)(j + 1) * a.nrow);
+        z[0] = z[1] = z[2] = 0;
+    }
     const int fx = a.periodic_x, fy = !a.open_y;
     const int ci = !fx ? i : i < 0 ? i + t.nx : i >= t.nx ? i - t.nx : i;
     const int cj = !fy ? j : j < 0 ? j + t.ny : j >= t.ny ? j - t.ny : j;
@@ -95,8 +108,13 @@ __device__ inline void reduce_block(const zk_reduce_args &a, const int bx, const
         for (int gx = 0; gx < nix; gx++) {
             const int rx = gx ? rxs[1] : rxs[0];
             const int kx = last_tile(rx, t.H, invx);
-            const long long *o = a.Jov + 3 * ((rx + 1) + (size_t)(ry + 1) * a.nrow);
-            const long long o0 = o[0], o1 = o[1], o2 = o[2];
+            long long o0 = 0, o1 = 0, o2 = 0;
+            if (!a.jflag || a.jflag[(rx + 1) / ZK_RED_BX + (ry + 1) / ZK_RED_BY * zk_red_blocks_x(t.nx)]) {
+                const long long *o = a.Jov + 3 * ((rx + 1) + (size_t)(ry + 1) * a.nrow);
+                o0 = o[0];
+                o1 = o[1];
+                o2 = o[2];
+            }
             if (a.region) {
                 float v[N * N][3];
 #pragma unroll
@@ -127,10 +145,8 @@ __device__ inline void reduce_block(const zk_reduce_args &a, const int bx, const
     out[2] = s[2];
 }
 
-/* blocks of reduce_block over the buffer, and the N it needs (0: only
- * reduce_node can take the grid or the tiling) */
-__host__ __device__ inline int reduce_blocks_x(int nx) { return (nx + 3 + ZK_RED_BX - 1) / ZK_RED_BX; }
-__host__ __device__ inline int reduce_blocks_y(int ny) { return (ny + 3 + ZK_RED_BY - 1) / ZK_RED_BY; }
+/* the N that reduce_block needs (0: only reduce_node can take the grid or
+ * the tiling; it reads the whole overflow grid and clears none) */
 __host__ __device__ inline int reduce_span(const zk_tiles &t)
 {
     if (t.nx < 3 || t.ny < 3) return 0;

@@ -96,6 +96,27 @@ struct GlobalCurrent {
     long long *J;
     int nrow;
     float scale;
+    unsigned char *flag; /* zk_push_args.jflag */
+    int nfx;
+    __device__ static GlobalCurrent of(const zk_push_args &a)
+    {
+        return {a.Jov, a.nrow, a.jov_scale, a.jflag, zk_red_blocks_x(a.t.nx)};
+    }
+    /* flags the nodes that a particle starting in buffer cell (ci, cj) can
+     * reach: it crosses at most one cell edge per axis, so nodes
+     * [c - 1, c + 2].  The reduction reads, and the step after the next one
+     * clears, only flagged blocks: a grid of 24 bytes per node that is
+     * nearly empty is not read and rewritten every step. */
+    __device__ void touch(int ci, int cj) const
+    {
+        if (!flag) return;
+        const int x0 = (ci - 1) / ZK_RED_BX, x1 = (ci + 2) / ZK_RED_BX;
+        const int y0 = (cj - 1) / ZK_RED_BY * nfx, y1 = (cj + 2) / ZK_RED_BY * nfx;
+        flag[x0 + y0] = 1;
+        flag[x1 + y0] = 1;
+        flag[x0 + y1] = 1;
+        flag[x1 + y1] = 1;
+    }
     __device__ void add(int a, int b, int c, float v) const
     {
         atomicAdd((unsigned long long *)&J[3 * (a + b * nrow) + c], zk_fx(v, scale));
@@ -809,7 +830,7 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
             if (threadIdx.x == 0) nls[sp] = nl;
         } else if (nl > 0) {
             const GlobalFields gf = {a.E, a.B, a.nrow};
-            const GlobalCurrent gj = {a.Jov, a.nrow, a.jov_scale};
+            const GlobalCurrent gj = GlobalCurrent::of(a);
             /* whole waves per round: the sorting store needs every lane */
             for (int qb = 0; qb < nl; qb += blockDim.x) {
                 const int q = qb + (int)threadIdx.x;
@@ -819,6 +840,7 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
                     i = a.ovf_list[i0 + q];
                     c = load_part(P, i);
                     int di, dj;
+                    gj.touch(c.ix + 1, c.iy + 1);
                     kin += push_one(gf, gj, c.ix + 1, c.iy + 1, c.x, c.y, c.ux, c.uy, c.uz, di, dj, k);
                     c.ix += di;
                     c.iy += dj;
@@ -860,7 +882,7 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
                 const Consts k = {a.tem, a.dt_dx, a.dt_dy, a.qnx, a.qny, a.q};
                 const zk_parts P = a.p;
                 const GlobalFields gf = {a.E, a.B, a.nrow};
-                const GlobalCurrent gj = {a.Jov, a.nrow, a.jov_scale};
+                const GlobalCurrent gj = GlobalCurrent::of(a);
                 const int i0 = a.tile_off[tile];
                 for (int qb = 0; qb < nl; qb += ZK_WAVE) {
                     const int q = qb + (int)__lane_id();
@@ -870,6 +892,7 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
                         i = a.ovf_list[i0 + q];
                         c = load_part(P, i);
                         int di, dj;
+                        gj.touch(c.ix + 1, c.iy + 1);
                         kin += push_one(gf, gj, c.ix + 1, c.iy + 1, c.x, c.y, c.ux, c.uy, c.uz, di, dj, k);
                         c.ix += di;
                         c.iy += dj;
@@ -927,7 +950,7 @@ __device__ inline void push_global_body(const zk_push_args &a, const int block, 
     const zk_tiles &t = a.t;
     const Consts k = {a.tem, a.dt_dx, a.dt_dy, a.qnx, a.qny, a.q};
     const GlobalFields gf = {a.E, a.B, a.nrow};
-    const GlobalCurrent gj = {a.Jov, a.nrow, a.jov_scale};
+    const GlobalCurrent gj = GlobalCurrent::of(a);
     zk_parts P = a.p;
     double kin = 0.0;
     int ndead = 0, nov = 0;
@@ -941,6 +964,7 @@ __device__ inline void push_global_body(const zk_push_args &a, const int block, 
         if (c.ix == ZK_DEAD) continue;
         int di, dj;
         nov++;
+        gj.touch(c.ix + 1, c.iy + 1);
         kin += push_one(gf, gj, c.ix + 1, c.iy + 1, c.x, c.y, c.ux, c.uy, c.uz, di, dj, k);
         c.ix += di;
         c.iy += dj;

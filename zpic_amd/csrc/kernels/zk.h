@@ -76,6 +76,14 @@ typedef struct zk_spec_ctr {
     double energy;              /* kinetic energy of the last push            */
 } zk_spec_ctr;
 
+/* Nodes of the buffer per block of the current reduction, and per flag of
+ * the overflow grid: block (bx, by) holds buffer nodes [32 bx, 32 bx + 32) x
+ * [8 by, 8 by + 8), and its flag is bx + by * zk_red_blocks_x(nx). */
+#define ZK_RED_BX 32
+#define ZK_RED_BY 8
+#define zk_red_blocks_x(nx) (((nx) + 3 + ZK_RED_BX - 1) / ZK_RED_BX)
+#define zk_red_blocks_y(ny) (((ny) + 3 + ZK_RED_BY - 1) / ZK_RED_BY)
+
 /* Particle arrays of one buffer set: the cell index pair is packed into
  * one word, cell = ix | iy << cbits (nx <= 2^cbits, cbits + bits of ny <=
  * 31), -1 for a removed particle; 24 bytes per particle. */
@@ -107,6 +115,8 @@ typedef struct zk_push_args {
     int fresh;                  /* 1: overwrite region, 0: accumulate    */
     long long *Jov;             /* raw current of out-of-window pushes, 64-bit
                                    fixed point at jov_scale (order-free sums) */
+    unsigned char *jflag;       /* set for the zk_red_blocks of Jov deposited to
+                                   (NULL: not kept) */
     double *epart;              /* energy partials, one per block        */
     zk_tiles t;
     int moving_window;          /* x absorbing + window shift           */
@@ -208,6 +218,9 @@ int zk_unpack_append(const void *aos, int n, const zk_parts *dst, int64_t id0, z
 typedef struct zk_reduce_args {
     const float *region;
     const long long *Jov;
+    const unsigned char *jflag; /* blocks of Jov that may be nonzero (NULL: all) */
+    long long *Jov_next;        /* overflow grid of the next step, cleared here where */
+    unsigned char *jflag_next;  /* its flags say so (NULL: not cleared) */
     float jov_unscale;          /* Q_J / 2^40 */
     float *J;
     int nrow;
@@ -216,9 +229,8 @@ typedef struct zk_reduce_args {
     int open_y;                 /* no fold along y: the raw guard rows are kept */
     zk_finalize_set fin;        /* species whose last push is finished along with it */
 } zk_reduce_args;
-/* nodes of the buffer per block of the reduction */
-#define ZK_RED_BX 32
-#define ZK_RED_BY 8
+/* whether the reduction of this tiling clears Jov_next (and reads flags) */
+int zk_current_clears(const zk_tiles *t);
 int zk_current_reduce(const zk_reduce_args *a, zk_stream_t s);
 int zk_smooth(const float *in, float *out, int nx, int ny, int nrow, int axis,
                      float sa, float sb, int periodic_x, int open_y, zk_stream_t s);
