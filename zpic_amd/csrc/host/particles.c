@@ -1334,6 +1334,22 @@ void spec_move_window(t_species *s)
  * diagnostics
  * ---------------------------------------------------------------------- */
 
+static zk_charge_args charge_args(const t_species *s, float *rho)
+{
+    const struct zpic_dev_species *d = s->dev;
+    zk_charge_args a;
+    memset(&a, 0, sizeof(a));
+    a.p = d->set[d->cur];
+    a.tile_off = d->tile_off;
+    a.tile_n = d->counted ? d->tile_n : NULL;
+    a.ctr = d->ctr;
+    a.q = s->q;
+    zpic_fixed_point_scale(s->q, &a.fx_scale, &a.fx_unscale);
+    a.t = d->t;
+    a.rho = rho;
+    return a;
+}
+
 /* spec_deposit_charge without any allocation: the deposit and the caller's
  * density are staged in the library's file-scope scratch array (two grids
  * of at most ZK_NOALLOC_CHARGE_MAX nodes); the species must already be on
@@ -1366,7 +1382,7 @@ int spec_deposit_charge_noalloc(const t_species *cs, float *charge)
     zpic_h2d_async(acc, charge, sizeof(float) * n);
     /* the scratch keeps the previous call's contents: clear the deposit */
     ZCHECK(zk_fill_f32(rho, n, 0.0f, zpic_stream()));
-    ZCHECK(zk_charge(&d->set[d->cur], d->np_upper, d->ctr, s->q, s->nx[0], rho, zpic_stream()));
+    ZCHECK(zk_charge(charge_args(s, rho), d->tail_upper, zpic_stream()));
     ZCHECK(zk_add_f32(acc, rho, n, zpic_stream()));
     zpic_d2h(charge, acc, sizeof(float) * n);
     if (!s->moving_window)
@@ -1384,12 +1400,12 @@ void spec_deposit_charge(const t_species *cs, float *charge)
     struct zpic_dev_species *d = s->dev;
     const int nrow = s->nx[0] + 1;
     const size_t n = (size_t)nrow * (size_t)(s->nx[1] + 1);
-    float *rho = zpic_dmalloc(sizeof(float) * n);
+    ensure_stage(d, sizeof(float) * n);
+    float *rho = d->stage;
     ZCHECK(zk_fill_f32(rho, n, 0.0f, zpic_stream()));
-    ZCHECK(zk_charge(&d->set[d->cur], d->np_upper, d->ctr, s->q, s->nx[0], rho, zpic_stream()));
+    ZCHECK(zk_charge(charge_args(s, rho), d->tail_upper, zpic_stream()));
     float *h = malloc(sizeof(float) * n);
     zpic_d2h(h, rho, sizeof(float) * n);
-    zpic_dfree(rho);
     for (size_t k = 0; k < n; k++) charge[k] += h[k];
     free(h);
     if (!s->moving_window)
@@ -1447,13 +1463,12 @@ void spec_deposit_pha(const t_species *cs, const int rep_type, const int pha_nx[
     }
     zpic_species_ensure(s);
     const size_t n = (size_t)na * (size_t)nb;
-    float *dbuf = zpic_dmalloc(sizeof(float) * n);
-    ZCHECK(zk_fill_f32(dbuf, n, 0.0f, zpic_stream()));
+    ensure_stage(d, sizeof(float) * n + zk_pha_scratch(d->np_upper, na, nb));
+    float *dbuf = d->stage;
     ZCHECK(zk_pha(&d->set[d->cur], d->np_upper, d->ctr, qa, qb, s->dx[0], s->dx[1], na, nb, amin, bmin, ra, rb, s->q,
-                  dbuf, zpic_stream()));
+                  dbuf, dbuf + n, zpic_stream()));
     float *h = malloc(sizeof(float) * n);
     zpic_d2h(h, dbuf, sizeof(float) * n);
-    zpic_dfree(dbuf);
     for (size_t k = 0; k < n; k++) buf[k] += h[k];
     free(h);
 }

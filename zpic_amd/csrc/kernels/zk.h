@@ -268,8 +268,19 @@ int zk_add_ext(const float *F, const float *ext, float ux, float uy, float uz,
                       float *out, size_t nodes, zk_stream_t s);
 int zk_emf_energy(const float *E, const float *B, int nx, int ny, int nrow,
                          double *partial, int nblk, double *out6, double scale, zk_stream_t s);
-int zk_charge(const zk_parts *p, int np_upper, const zk_spec_ctr *ctr, float q,
-                     int nx, float *rho, zk_stream_t s);
+/* CIC charge of a tile-sorted species (ranges as in zk_push_args, and an
+ * unsorted tail of at most tail_upper slots) added to rho, (nx + 1) x
+ * (ny + 1) nodes; splits and tail are set by zk_charge */
+typedef struct zk_charge_args {
+    zk_parts p;
+    const int *tile_off, *tile_n;
+    const zk_spec_ctr *ctr;
+    float q, fx_scale, fx_unscale;
+    zk_tiles t;
+    int splits, tail;
+    float *rho;
+} zk_charge_args;
+int zk_charge(zk_charge_args a, int tail_upper, zk_stream_t s);
 /* Scratch of the allocation-free charge deposit: a file-scope device array
  * of 2 * ZK_NOALLOC_CHARGE_MAX floats (64 MiB) on every device the library
  * runs on.  zk_noalloc_scratch returns its address on the current device
@@ -277,11 +288,12 @@ int zk_charge(const zk_parts *p, int np_upper, const zk_spec_ctr *ctr, float q,
 #define ZK_NOALLOC_CHARGE_MAX (8 << 20)
 int zk_noalloc_scratch(float **ptr);
 int zk_add_f32(float *acc, const float *v, size_t n, zk_stream_t s);
-/* out (na x nb, row length na) += phase-space density of quantities qa, qb
+/* out (na x nb, row length na) = phase-space density of quantities qa, qb
  * (em2d/particles.c:1569-1632 weights): amin/bmin the lower range bounds,
  * ra/rb the bins per unit */
 int zk_pha(const zk_parts *p, int np_upper, const zk_spec_ctr *ctr, int qa, int qb, float dx0, float dx1, int na,
-           int nb, float amin, float bmin, float ra, float rb, float q, float *out, zk_stream_t s);
+           int nb, float amin, float bmin, float ra, float rb, float q, float *out, float *scratch, zk_stream_t s);
+size_t zk_pha_scratch(int np_upper, int na, int nb); /* bytes of scratch zk_pha needs */
 
 /* ---- particle initialisation on the device (init.hip) ---- */
 typedef struct zk_init_args {
