@@ -40,13 +40,18 @@ struct zpic_batch {
     zk_bspec *hspecs;
     zk_bsim *dsims;     /* device descriptors */
     zk_bspec *dspecs;
+    zk_push_multi *hsets;    /* push arguments of each simulation pushed in one launch */
+    zk_push_multi *dsets;
+    int *fused;              /* per simulation */
     int *ditems;        /* device item table (int pairs) */
     item_range fill, fold, node, yee, sort;
-    item_range *tile, *glob; /* per species index */
+    item_range *tile, *glob; /* per species index, of the species pushed on their own */
+    item_range fuse;         /* the simulations whose species are pushed together */
     int *gblocks;            /* per species: blocks of the out-of-window pass */
     int *ntiles;             /* per simulation, at creation */
     size_t lds;
     int waves, fixed;
+    int win;            /* every tile has the default window */
     void *graph[2];     /* 0: plain step, 1: step with the tile sort */
 };
 
@@ -68,7 +73,9 @@ static void fill_sim(zpic_batch *b, int i)
     }
     M->region = dc->region;
     for (int k = 0; k < sim->n_species; k++) zpic_current_jov_register(cur, sim->species[k].q);
-    M->Jov = zpic_current_jov(cur, 0);
+    zpic_current_jov_tidy(cur);
+    M->Jov = zpic_current_jov(cur, 1);
+    M->jflag = dc->jflag[dc->jov_cur];
     M->jov_unscale = zpic_current_jov_unscale(cur);
     M->ecur = de->cur;
     M->jcur = dc->jcur;
@@ -104,7 +111,8 @@ static void fill_spec(zpic_batch *b, int k)
     a->nrow = cur->nrow;
     a->region = dc->region;
     a->fresh = (b->spec_k[k] == 0);
-    a->Jov = zpic_current_jov(cur, 0);
+    a->Jov = zpic_current_jov(cur, 1);
+    a->jflag = dc->jflag[dc->jov_cur];
     a->jov_scale = zpic_current_jov_scale(cur);
     a->epart = d->epart;
     a->t = d->t;
@@ -136,6 +144,7 @@ static void fill_spec(zpic_batch *b, int k)
     S->stay = d->stay;
     S->nbr = d->nbr;
     S->tailn = d->tailn;
+    S->fset = -1;
     const float qm = s->q * s->m_q;
     S->qm = qm;
     S->dx0 = s->dx[0];
@@ -164,6 +173,34 @@ static void refresh(zpic_batch *b)
     }
     for (int i = 0; i < b->nsims; i++) fill_sim(b, i);
     for (int k = 0; k < b->nspecs; k++) fill_spec(b, k);
+    /* one launch pushes the species of a simulation where sim_iter does so
+     * (decided once: the item tables depend on it) */
+    for (int i = 0, k = 0; i < b->nsims; i++) {
+        const int n = b->sims[i]->n_species;
+        if (!b->ditems) {
+            b->fused[i] = n >= 2 && n <= ZK_FUSE_MAX && b->fixed && zpic_species_fusion();
+            for (int j = 1; j < n && b->fused[i]; j++)
+                b->fused[i] = b->hspecs[k + j].a.fx_scale == b->hspecs[k].a.fx_scale;
+        }
+        if (b->fused[i]) {
+            zk_push_multi *m = &b->hsets[i];
+            memset(m, 0, sizeof(*m));
+            m->n = n;
+            for (int j = 0; j < n; j++) {
+                zk_bspec *S = &b->hspecs[k + j];
+                S->fset = i;
+                S->fk = j;
+                m->s[j] = S->a;
+                m->s[j].fresh = 1;
+                m->s[j].p = S->set[S->pcur];
+                m->s[j].tile_off = S->offs[S->ocur];
+                m->s[j].E = b->hsims[i].E[b->hsims[i].ecur];
+                m->s[j].B = b->hsims[i].B[b->hsims[i].ecur];
+            }
+        }
+        k += n;
+    }
+    zpic_h2d(b->dsets, b->hsets, sizeof(zk_push_multi) * (size_t)b->nsims);
     zpic_h2d(b->dsims, b->hsims, sizeof(zk_bsim) * (size_t)b->nsims);
     if (b->nspecs) zpic_h2d(b->dspecs, b->hspecs, sizeof(zk_bspec) * (size_t)b->nspecs);
 }
@@ -185,6 +222,15 @@ static void put(table *t, int desc, int block)
     t->v[2 * t->n] = desc;
     t->v[2 * t->n + 1] = block;
     t->n++;
+}
+
+/* Position b of the n tiles of a simulation: consecutive workgroups go to
+ * the 8 XCDs in turn, so they take tiles from 8 contiguous runs and
+ * neighbouring tiles share an L2 (zk_xcd_item of the kernels). */
+static int xcd_tile(int b, int n)
+{
+    const int x = b % 8, base = n / 8, rem = n % 8;
+    return x * base + (x < rem ? x : rem) + b / 8;
 }
 
 static int blocks_of(size_t n, int per) { return (int)((n + (size_t)per - 1) / (size_t)per); }
@@ -222,7 +268,7 @@ static void build_items(zpic_batch *b, table *T)
         }                                                                                                              \
         (range).n = T->n - (range).off;                                                                                \
     } while (0)
-    GRID_PHASE(b->fill, blocks_of(3 * (size_t)(M->nx + 3) * (M->ny + 3), 256));
+    GRID_PHASE(b->fill, zk_red_blocks_x(M->nx) * zk_red_blocks_y(M->ny));
     GRID_PHASE(b->fold, zk_batch_reduce_blocks(M));
     GRID_PHASE(b->node, blocks_of((size_t)(M->nx + 3) * (M->ny + 3), 256));
     GRID_PHASE(b->yee, ((M->nx + 3 + ZK_YEE_BX - 1) / ZK_YEE_BX) * ((M->ny + 3 + ZK_YEE_BY - 1) / ZK_YEE_BY));
@@ -239,8 +285,8 @@ static void build_items(zpic_batch *b, table *T)
         b->tile[p].off = T->n;
         for (int q = 0; q < b->nspecs; q++) {
             const int k = order[q];
-            if (b->spec_k[k] != p) continue;
-            for (int t = 0; t < b->hspecs[k].a.t.ntiles; t++) put(T, k, t);
+            if (b->spec_k[k] != p || b->fused[b->spec_sim[k]]) continue;
+            for (int t = 0, nt = b->hspecs[k].a.t.ntiles; t < nt; t++) put(T, k, xcd_tile(t, nt));
         }
         b->tile[p].n = T->n - b->tile[p].off;
         b->glob[p].off = T->n;
@@ -251,6 +297,13 @@ static void build_items(zpic_batch *b, table *T)
         }
         b->glob[p].n = T->n - b->glob[p].off;
     }
+    b->fuse.off = T->n;
+    for (int q = 0; q < b->nspecs; q++) {
+        const int k = order[q], i = b->spec_sim[k];
+        if (b->spec_k[k] != 0 || !b->fused[i]) continue;
+        for (int t = 0, nt = b->hspecs[k].a.t.ntiles; t < nt; t++) put(T, i, xcd_tile(t, nt));
+    }
+    b->fuse.n = T->n - b->fuse.off;
     for (int k = 0; k < b->nspecs; k++) {
         order[k] = k;
         w[k] = (double)b->spec[k]->np;
@@ -260,7 +313,7 @@ static void build_items(zpic_batch *b, table *T)
     b->sort.off = T->n;
     for (int q = 0; q < b->nspecs; q++) {
         const int k = order[q];
-        for (int t = 0; t < b->hspecs[k].a.t.ntiles; t++) put(T, k, t);
+        for (int t = 0, nt = b->hspecs[k].a.t.ntiles; t < nt; t++) put(T, k, xcd_tile(t, nt));
     }
     b->sort.n = T->n - b->sort.off;
     free(order);
@@ -276,18 +329,19 @@ static void enqueue_step(zpic_batch *b, int with_sort)
     const zk_stream_t s = zpic_stream();
     /* current_zero (em2d/current.c:98-107) */
     ZCHECK(zk_batch_fill_jov(b->dsims, ITEMS(b->fill), s));
-    /* spec_advance of the p-th species of every simulation; the species
+    /* spec_advance: all species of a simulation at once where they share a
+     * launch, then the p-th species of every other simulation; the species
      * of one simulation deposit into one set of windows, in order */
+    ZCHECK(zk_batch_push_sets(b->dsets, ITEMS(b->fuse), b->lds, b->win, s));
     for (int p = 0; p < b->max_spec; p++)
-        ZCHECK(zk_batch_push(b->dspecs, b->dsims, ITEMS(b->tile[p]), ITEMS(b->glob[p]), b->lds, b->waves, b->fixed,
+        ZCHECK(zk_batch_push(b->dspecs, b->dsims, ITEMS(b->tile[p]), ITEMS(b->glob[p]), b->lds, b->win, b->waves, b->fixed,
                              s));
     ZCHECK(zk_batch_finalize(b->dspecs, b->nspecs, s));
     if (with_sort) ZCHECK(zk_batch_sort(b->dspecs, b->nspecs, ITEMS(b->sort), s));
     /* current_update, emf_advance */
     ZCHECK(zk_batch_current(b->dsims, ITEMS(b->fold), ITEMS(b->node), b->max_passes, s));
     ZCHECK(zk_batch_fields(b->dsims, ITEMS(b->yee), s));
-    if (with_sort) ZCHECK(zk_batch_end_step_sorted(b->dsims, b->nsims, b->dspecs, b->nspecs, s));
-    else ZCHECK(zk_batch_end_step(b->dsims, b->nsims, b->dspecs, b->nspecs, s));
+    ZCHECK(zk_batch_end_step(b->dsims, b->nsims, b->dspecs, b->nspecs, b->dsets, with_sort, s));
 }
 
 zpic_batch *zpic_batch_new(t_simulation *const *sims, int n)
@@ -328,6 +382,9 @@ zpic_batch *zpic_batch_new(t_simulation *const *sims, int n)
     b->glob = calloc((size_t)(b->max_spec > 0 ? b->max_spec : 1), sizeof(item_range));
     b->hsims = calloc((size_t)n, sizeof(zk_bsim));
     b->hspecs = calloc((size_t)ns, sizeof(zk_bspec));
+    b->hsets = calloc((size_t)n, sizeof(zk_push_multi));
+    b->fused = calloc((size_t)n, sizeof(int));
+    b->dsets = zpic_dmalloc(sizeof(zk_push_multi) * (size_t)n);
     b->dsims = zpic_dmalloc(sizeof(zk_bsim) * (size_t)n);
     b->dspecs = zpic_dmalloc(sizeof(zk_bspec) * (size_t)ns);
     b->waves = zpic_push_waves();
@@ -342,11 +399,13 @@ zpic_batch *zpic_batch_new(t_simulation *const *sims, int n)
     b->ntiles = malloc(sizeof(int) * (size_t)n);
     for (int i = 0; i < n; i++) b->ntiles[i] = b->hsims[i].t.ntiles;
     b->lds = 0;
+    b->win = 1;
     for (int k = 0; k < b->nspecs; k++) {
         const zk_tiles *t = &b->hspecs[k].a.t;
         /* E, B window and the current window (64-bit with the fixed-point deposit) */
         const size_t l = (size_t)t->WX * t->WY * (6 * sizeof(float) + 3 * (b->fixed ? 8 : 4));
         if (l > b->lds) b->lds = l;
+        if (!zk_batch_default_window(t)) b->win = 0;
     }
     for (int i = 0; i < n; i++)
         if (b->hsims[i].npass > b->max_passes) b->max_passes = b->hsims[i].npass;
@@ -432,6 +491,9 @@ void zpic_batch_delete(zpic_batch *b)
     zpic_graph_free(b->graph[1]);
     zpic_dfree(b->dsims);
     zpic_dfree(b->dspecs);
+    zpic_dfree(b->dsets);
+    free(b->hsets);
+    free(b->fused);
     zpic_dfree(b->ditems);
     free(b->sims);
     free(b->spec);

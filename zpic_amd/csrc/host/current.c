@@ -82,6 +82,11 @@ static void jov_clear(t_current *c, int k)
     d->jov_state[k] = ZPIC_JOV_CLEAN;
 }
 
+void zpic_current_jov_tidy(t_current *c)
+{
+    if (c->dev->jov_state[c->dev->jov_cur] == ZPIC_JOV_DIRTY) jov_clear(c, c->dev->jov_cur);
+}
+
 long long *zpic_current_jov(t_current *c, int flagged)
 {
     struct zpic_dev_current *d = c->dev;

@@ -1070,6 +1070,16 @@ static void inject_column_device(t_species *s, int k, zk_rng_state *rng)
     }
 }
 
+/* Blocks of the global pass for a tail of at most n particles: one per 256,
+ * in multiples of 8 so that the tiles that follow them in the launch keep
+ * their XCDs. */
+static int tail_blocks(int n)
+{
+    if (n <= 0) return 0;
+    const int b = ((n - 1) / 256 / 8 + 1) * 8;
+    return b < ZPIC_GLOBAL_BLOCKS ? b : ZPIC_GLOBAL_BLOCKS;
+}
+
 /* Arguments of the push of species s (em2d/particles.c:1104-1117); sets
  * *move when the window moves this step.  The species, fields and current
  * must be on the device. */
@@ -1109,7 +1119,7 @@ static void push_args(t_species *s, t_emf *emf, t_current *cur, zk_push_args *pa
     a.shift = *move;
     /* the global pass pushes the unsorted tail (injected particles), if any */
     a.ovf_list = d->ovf_list;
-    a.global_blocks = d->tail_upper > 0 ? ZPIC_GLOBAL_BLOCKS : 0;
+    a.global_blocks = tail_blocks(d->tail_upper);
     a.waves = zpic_push_waves();
     a.fixed = zpic_fixed_deposit();
     zpic_fixed_point_scale(s->q, &a.fx_scale, &a.fx_unscale);

@@ -152,6 +152,8 @@ void zpic_current_jov_register(t_current *cur, float q);
 /* the overflow grid of this step, about to be deposited to: by a push that
  * flags what it touches, or (flagged 0) by one that does not */
 long long *zpic_current_jov(t_current *cur, int flagged);
+/* its contents are zero but for the flagged blocks afterwards */
+void zpic_current_jov_tidy(t_current *cur);
 float zpic_current_jov_scale(const t_current *cur);   /* 2^(40 - jov_k) */
 float zpic_current_jov_unscale(const t_current *cur); /* 2^(jov_k - 40) */
 

@@ -51,18 +51,42 @@ __global__ void fill_jov_kernel(const zk_bsim *sims, const int *items)
 {
     const int s = items[2 * blockIdx.x], b = items[2 * blockIdx.x + 1];
     const zk_bsim &M = sims[s];
-    const size_t n = 3 * (size_t)(M.nx + 3) * (M.ny + 3);
-    const size_t i = (size_t)b * blockDim.x + threadIdx.x;
-    if (i < n) M.Jov[i] = 0;
+    /* block b of the overflow grid, where the step before deposited to it */
+    unsigned char *f = M.jflag + b;
+    const bool dirty = *f != 0;
+    __syncthreads();
+    if (!dirty) return;
+    if (threadIdx.x == 0) *f = 0;
+    const int nbx = zk_red_blocks_x(M.nx);
+    const int i = b % nbx * ZK_RED_BX + (int)(threadIdx.x % ZK_RED_BX);
+    const int j = b / nbx * ZK_RED_BY + (int)(threadIdx.x / ZK_RED_BX);
+    if (i > M.nx + 2 || j > M.ny + 2) return;
+    long long *z = M.Jov + 3 * ((size_t)i + (size_t)j * M.nrow);
+    z[0] = z[1] = z[2] = 0;
 }
 
-template <int MIN_WAVES, bool FX>
+/* WC: every member has the default window (compile-time LDS offsets), or 0 */
+template <int MIN_WAVES, bool FX, int WC = 0>
 __global__ void __launch_bounds__(256, MIN_WAVES) push_tile_batch(const zk_bspec *specs, const zk_bsim *sims,
                                                                   const int *items)
 {
     const zk_bspec &S = specs[items[2 * blockIdx.x]];
     const zk_push_args a = spec_args(S, sims[S.sim]);
-    push_tile_body<1, FX>(OneSpecies{a}, items[2 * blockIdx.x + 1]);
+    push_tile_body<1, FX, OneSpecies, WC>(OneSpecies{a}, items[2 * blockIdx.x + 1]);
+}
+
+/* All species of a simulation in one workgroup per tile, as sim_iter pushes
+ * them: one staging of the fields and one store of the window.  The
+ * arguments are read through the constant address space, as a kernel's own
+ * are: no store of the push can change them, so they need no registers.
+ * (Held as values, or read as ordinary memory, they spilled 140-228 bytes
+ * per lane.) */
+template <int WC>
+__global__ void __launch_bounds__(256, ZK_PUSH_OCC) push_species_batch(const zk_push_multi *sets, const int *items)
+{
+    typedef const __attribute__((address_space(4))) zk_push_multi const_set;
+    const_set *m = (const_set *)(unsigned long long)(sets + items[2 * blockIdx.x]);
+    push_tile_body<1, true, SpeciesSet, WC>(SpeciesSet{*(const zk_push_multi *)m}, items[2 * blockIdx.x + 1]);
 }
 
 __global__ void __launch_bounds__(256) push_global_batch(const zk_bspec *specs, const zk_bsim *sims,
@@ -85,7 +109,7 @@ __global__ void reduce_batch(const zk_bsim *sims, const int *items)
     zk_reduce_args r;
     r.region = M.deposited ? M.region : nullptr;
     r.Jov = M.Jov;
-    r.jflag = nullptr;
+    r.jflag = M.jflag;
     r.jflag_next = nullptr;
     r.jov_unscale = M.jov_unscale;
     r.J = j_after(M, 0);
@@ -152,7 +176,7 @@ __global__ void __launch_bounds__(ZK_SORT_THREADS) scatter_batch(const zk_bspec 
 /* Advance the buffer indices of every simulation and species so the next
  * replay reads this step's results: new fields, filtered current, and the
  * sorted particle set of species sorted this step. */
-__global__ void end_step_batch(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, int sorted)
+__global__ void __launch_bounds__(1024) end_step_batch(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_push_multi *sets, int sorted)
 {
     for (int s = threadIdx.x; s < nsims; s += blockDim.x) {
         sims[s].ecur ^= 1;
@@ -164,6 +188,18 @@ __global__ void end_step_batch(zk_bsim *sims, int nsims, zk_bspec *specs, int ns
             specs[k].ocur ^= 1;
         }
         specs[k].iter++;
+    }
+    /* the fused push's arguments follow */
+    __syncthreads();
+    for (int k = threadIdx.x; k < nspecs; k += blockDim.x) {
+        const zk_bspec &S = specs[k];
+        if (S.fset < 0) continue;
+        const zk_bsim &M = sims[S.sim];
+        zk_push_args &a = sets[S.fset].s[S.fk];
+        a.p = S.set[S.pcur];
+        a.tile_off = S.offs[S.ocur];
+        a.E = M.E[M.ecur];
+        a.B = M.B[M.ecur];
     }
 }
 
@@ -180,11 +216,24 @@ extern "C" int zk_batch_fill_jov(const zk_bsim *sims, const int *items, int n, z
     ZK_LAUNCH_CHECK();
 }
 
+extern "C" int zk_batch_push_sets(const zk_push_multi *sets, const int *items, int n, size_t lds, int win, zk_stream_t s)
+{
+    if (n > 0) {
+        if (win) hipLaunchKernelGGL(push_species_batch<ZK_WIN_DEFAULT>, dim3(n), dim3(256), lds, s, sets, items);
+        else hipLaunchKernelGGL(push_species_batch<0>, dim3(n), dim3(256), lds, s, sets, items);
+    }
+    ZK_LAUNCH_CHECK();
+}
+
 extern "C" int zk_batch_push(const zk_bspec *specs, const zk_bsim *sims, const int *tile_items, int ntile,
-                             const int *global_items, int nglobal, size_t lds, int waves, int fixed, zk_stream_t s)
+                             const int *global_items, int nglobal, size_t lds, int win, int waves, int fixed,
+                             zk_stream_t s)
 {
     if (ntile > 0) {
-        if (fixed)
+        if (fixed && win)
+            hipLaunchKernelGGL((push_tile_batch<ZK_PUSH_OCC, true, ZK_WIN_DEFAULT>), dim3(ntile), dim3(256), lds, s, specs,
+                               sims, tile_items);
+        else if (fixed)
             hipLaunchKernelGGL((push_tile_batch<ZK_PUSH_OCC, true>), dim3(ntile), dim3(256), lds, s, specs, sims, tile_items);
         else if (waves == 8)
             hipLaunchKernelGGL((push_tile_batch<8, false>), dim3(ntile), dim3(256), lds, s, specs, sims, tile_items);
@@ -195,12 +244,14 @@ extern "C" int zk_batch_push(const zk_bspec *specs, const zk_bsim *sims, const i
     ZK_LAUNCH_CHECK();
 }
 
+extern "C" int zk_batch_default_window(const zk_tiles *t) { return default_window(*t); }
+
 extern "C" int zk_batch_prepare_push(size_t lds)
 {
     if (lds <= 65536) return 0;
-    const void *fns[3] = {(const void *)push_tile_batch<1, false>, (const void *)push_tile_batch<8, false>,
-                          (const void *)push_tile_batch<ZK_PUSH_OCC, true>};
-    for (int k = 0; k < 3; k++) {
+    const void *fns[4] = {(const void *)push_tile_batch<1, false>, (const void *)push_tile_batch<8, false>,
+                          (const void *)push_tile_batch<ZK_PUSH_OCC, true>, (const void *)push_species_batch<0>};
+    for (int k = 0; k < 4; k++) {
         const int e = (int)hipFuncSetAttribute(fns[k], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e) return e;
     }
@@ -234,7 +285,7 @@ extern "C" int zk_batch_fields(const zk_bsim *sims, const int *yee_items, int ny
 }
 
 /* The sort of the species whose schedule asks for it this step; a graph
- * holding these launches must end its step with zk_batch_end_step_sorted. */
+ * holding these launches must end its step with zk_batch_end_step. */
 extern "C" int zk_batch_sort(const zk_bspec *specs, int nspecs, const int *items, int n, zk_stream_t s)
 {
     if (nspecs <= 0) return 0;
@@ -245,14 +296,9 @@ extern "C" int zk_batch_sort(const zk_bspec *specs, int nspecs, const int *items
     ZK_LAUNCH_CHECK();
 }
 
-extern "C" int zk_batch_end_step(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_stream_t s)
+extern "C" int zk_batch_end_step(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_push_multi *sets, int sorted,
+                                 zk_stream_t s)
 {
-    hipLaunchKernelGGL(end_step_batch, dim3(1), dim3(256), 0, s, sims, nsims, specs, nspecs, 0);
-    ZK_LAUNCH_CHECK();
-}
-
-extern "C" int zk_batch_end_step_sorted(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_stream_t s)
-{
-    hipLaunchKernelGGL(end_step_batch, dim3(1), dim3(256), 0, s, sims, nsims, specs, nspecs, 1);
+    hipLaunchKernelGGL(end_step_batch, dim3(1), dim3(1024), 0, s, sims, nsims, specs, nspecs, sets, sorted);
     ZK_LAUNCH_CHECK();
 }

@@ -48,35 +48,42 @@ using namespace zk;
 
 namespace {
 
-/* WC: the window is WC x WC nodes (compile-time LDS offsets), 0 any */
-constexpr int ZK_WIN_DEFAULT = 25; /* 16 x 16 tiles, 3-cell margin */
 
-/* Blocks past the tiles push the unsorted tail (the global pass) in the
- * same launch: the two touch disjoint particles, deposit into disjoint
- * windows or with exact atomics into the overflow grid, and write their own
- * energy partials, so they may run side by side (one launch and its gap
- * less per step while a moving window's injected columns wait for a sort). */
-template <int MIN_WAVES, int PAIR, bool FX, int WC = 0>
-__global__ void __launch_bounds__(256, MIN_WAVES) push_tile_kernel(zk_push_args a)
+/* Threads per tile workgroup.  256 where the tiles fill the GPU: five such
+ * workgroups share a CU's LDS and registers.  With fewer tiles than that the
+ * waves of a tile decide how many the CU runs: up to one tile per CU, 1024
+ * threads. */
+constexpr int ZK_CUS = 256;
+
+inline int tile_threads(int ntiles) { return ntiles <= ZK_CUS ? 1024 : ntiles <= 2 * ZK_CUS ? 512 : 256; }
+
+/* The first global_blocks blocks push the unsorted tail (the global pass)
+ * in the same launch: the two touch disjoint particles, deposit into
+ * disjoint windows or with exact atomics into the overflow grid, and write
+ * their own energy partials, so they may run side by side (one launch and
+ * its gap less per step while a moving window's injected columns wait for a
+ * sort).  They come first because each is a long chain of dependent global
+ * accesses. */
+template <int MIN_WAVES, int PAIR, bool FX, int WC = 0, int NT = 256>
+__global__ void __launch_bounds__(NT, MIN_WAVES) push_tile_kernel(zk_push_args a)
 {
     zk_stamp_first(a.stamp);
-    if ((int)blockIdx.x >= a.t.ntiles)
-        push_global_body(a, (int)blockIdx.x - a.t.ntiles, a.global_blocks);
+    const int b = (int)blockIdx.x - a.global_blocks;
+    if (b < 0)
+        push_global_body(a, blockIdx.x, a.global_blocks);
     else
-        push_tile_body<PAIR, FX, OneSpecies, WC>(OneSpecies{a}, zk_xcd_item(blockIdx.x, a.t.ntiles));
+        push_tile_body<PAIR, FX, OneSpecies, WC, NT>(OneSpecies{a}, zk_xcd_item(b, a.t.ntiles));
     zk_stamp_last(a.stamp);
 }
 
 /* every species of a simulation in one launch (shared staging and window) */
-template <int WC>
-__global__ void __launch_bounds__(256, ZK_SPECIES_OCC) push_species_kernel(zk_push_multi m)
+template <int WC, int NT>
+__global__ void __launch_bounds__(NT, NT == 256 ? ZK_SPECIES_OCC : 4) push_species_kernel(zk_push_multi m)
 {
     zk_stamp_first(m.s[0].stamp);
-    push_tile_body<1, true, SpeciesSet, WC>(SpeciesSet{m}, zk_xcd_item(blockIdx.x, m.s[0].t.ntiles));
+    push_tile_body<1, true, SpeciesSet, WC, NT>(SpeciesSet{m}, zk_xcd_item(blockIdx.x, m.s[0].t.ntiles));
     zk_stamp_last(m.s[0].stamp);
 }
-
-bool default_window(const zk_tiles &t) { return t.WX == ZK_WIN_DEFAULT && t.WY == ZK_WIN_DEFAULT; }
 
 __global__ void __launch_bounds__(256) push_global_kernel(zk_push_args a)
 {
@@ -108,39 +115,55 @@ __global__ void fill_kernel(float *p, size_t n, float v)
 
 } // namespace
 
+namespace {
+
+typedef void (*tile_kernel)(zk_push_args);
+typedef void (*species_kernel)(zk_push_multi);
+
+template <int WC>
+tile_kernel fixed_kernel(int nt)
+{
+    return nt == 1024  ? push_tile_kernel<4, 1, true, WC, 1024>
+           : nt == 512 ? push_tile_kernel<4, 1, true, WC, 512>
+                       : push_tile_kernel<ZK_PUSH_OCC, 1, true, WC, 256>;
+}
+
+template <int WC>
+species_kernel set_kernel(int nt)
+{
+    return nt == 1024 ? push_species_kernel<WC, 1024>
+           : nt == 512 ? push_species_kernel<WC, 512>
+                       : push_species_kernel<WC, 256>;
+}
+
+/* windows of large tiles need more than the default 64 KiB of LDS */
+int allow_lds(const void *fn, size_t lds)
+{
+    return lds > 65536 ? (int)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) : 0;
+}
+
+} // namespace
+
 extern "C" int zk_push(const zk_push_args *a, zk_stream_t s)
 {
     const int n = a->t.WX * a->t.WY;
     /* E, B window (6 n floats) and the current window: 3 n floats, or 3 n
      * 64-bit integers with the fixed-point deposit */
     const size_t lds = (size_t)6 * n * sizeof(float) + (size_t)3 * n * (a->fixed ? 8 : 4);
-    /* variants: 0 lets the compiler keep every value in registers (about
-     * 6 waves per SIMD); 8 asks for 8 waves per SIMD at the price of a few
-     * register spills; 2 pushes two particles per thread and iteration */
-    const bool dw = default_window(a->t);
-    const void *fn = a->fixed ? (dw ? (const void *)push_tile_kernel<ZK_PUSH_OCC, 1, true, ZK_WIN_DEFAULT>
-                                    : (const void *)push_tile_kernel<ZK_PUSH_OCC, 1, true>)
-                     : a->waves == 8 ? (const void *)push_tile_kernel<8, 1, false>
-                     : a->waves == 2 ? (const void *)push_tile_kernel<1, 2, false>
-                                     : (const void *)push_tile_kernel<1, 1, false>;
-    if (lds > 65536) {
-        /* windows of large tiles need more than the default 64 KiB of LDS */
-        const int e = (int)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e) return e;
-    }
     if (a->t.ntiles > 0) {
-        /* the tiles, then the tail's blocks (global_blocks) */
-        const dim3 grid(a->t.ntiles + (a->global_blocks > 0 ? a->global_blocks : 0));
-        if (a->fixed && dw)
-            hipLaunchKernelGGL((push_tile_kernel<ZK_PUSH_OCC, 1, true, ZK_WIN_DEFAULT>), grid, dim3(256), lds, s, *a);
-        else if (a->fixed)
-            hipLaunchKernelGGL((push_tile_kernel<ZK_PUSH_OCC, 1, true>), grid, dim3(256), lds, s, *a);
-        else if (a->waves == 8)
-            hipLaunchKernelGGL((push_tile_kernel<8, 1, false>), grid, dim3(256), lds, s, *a);
-        else if (a->waves == 2)
-            hipLaunchKernelGGL((push_tile_kernel<1, 2, false>), grid, dim3(256), lds, s, *a);
-        else
-            hipLaunchKernelGGL((push_tile_kernel<1, 1, false>), grid, dim3(256), lds, s, *a);
+        /* float-deposit variants: 0 lets the compiler keep every value in
+         * registers (about 6 waves per SIMD); 8 asks for 8 waves per SIMD at
+         * the price of a few register spills; 2 pushes two particles per
+         * thread and iteration */
+        const int nt = a->fixed ? tile_threads(a->t.ntiles) : 256;
+        const tile_kernel fn = a->fixed ? (default_window(a->t) ? fixed_kernel<ZK_WIN_DEFAULT>(nt) : fixed_kernel<0>(nt))
+                               : a->waves == 8 ? (tile_kernel)push_tile_kernel<8, 1, false>
+                               : a->waves == 2 ? (tile_kernel)push_tile_kernel<1, 2, false>
+                                               : (tile_kernel)push_tile_kernel<1, 1, false>;
+        const int e = allow_lds((const void *)fn, lds);
+        if (e) return e;
+        /* the tail's blocks, then the tiles */
+        hipLaunchKernelGGL(fn, dim3(a->global_blocks + a->t.ntiles), dim3(nt), lds, s, *a);
     } else if (a->global_blocks > 0) {
         hipLaunchKernelGGL(push_global_kernel, dim3(a->global_blocks), dim3(256), 0, s, *a);
     }
@@ -153,17 +176,12 @@ extern "C" int zk_push_species(const zk_push_multi *m, zk_stream_t s)
     if (m->n < 1 || m->n > ZK_FUSE_MAX || !a->fixed) return (int)hipErrorInvalidValue;
     const int n = a->t.WX * a->t.WY;
     const size_t lds = (size_t)6 * n * sizeof(float) + (size_t)3 * n * 8;
-    const bool dw = default_window(a->t);
-    const void *fn = dw ? (const void *)push_species_kernel<ZK_WIN_DEFAULT> : (const void *)push_species_kernel<0>;
-    if (lds > 65536) {
-        const int e = (int)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e) return e;
-    }
     if (a->t.ntiles > 0) {
-        if (dw)
-            hipLaunchKernelGGL(push_species_kernel<ZK_WIN_DEFAULT>, dim3(a->t.ntiles), dim3(256), lds, s, *m);
-        else
-            hipLaunchKernelGGL(push_species_kernel<0>, dim3(a->t.ntiles), dim3(256), lds, s, *m);
+        const int nt = tile_threads(a->t.ntiles);
+        const species_kernel fn = default_window(a->t) ? set_kernel<ZK_WIN_DEFAULT>(nt) : set_kernel<0>(nt);
+        const int e = allow_lds((const void *)fn, lds);
+        if (e) return e;
+        hipLaunchKernelGGL(fn, dim3(a->t.ntiles), dim3(nt), lds, s, *m);
     }
     for (int k = 0; k < m->n; k++)
         if (m->s[k].global_blocks > 0)

@@ -37,6 +37,9 @@ struct Win {
     __device__ int n() const { return WC > 0 ? WC * WC : n_; }
 };
 
+constexpr int ZK_WIN_DEFAULT = 25; /* 16 x 16 tiles, 3-cell margin */
+inline bool default_window(const zk_tiles &t) { return t.WX == ZK_WIN_DEFAULT && t.WY == ZK_WIN_DEFAULT; }
+
 /* Field sources: node (a, b) in the source's index space. */
 template <int WC = 0>
 struct LdsFieldsT : Win<WC> {
@@ -612,27 +615,47 @@ struct SpeciesSet {
 };
 
 /* Tile pass.  The workgroup stages the fields of its window and clears
- * the current window once, pushes the tile's particles of each species in
- * turn, and stores the window once: with several species the staging and
- * the window store (0.12 ms of a 2048^2 launch) are not repeated per
- * species.  PAIR = 2 pushes two particles per thread and iteration: the
- * gathers and Boris pushes of both are independent and interleave, which
- * hides LDS and arithmetic latency at the price of registers.  FX selects
- * the fixed-point window (LdsCurrentFxT) instead of float LDS atomics. */
-template <int PAIR = 1, bool FX = false, class Set, int WC = 0>
+ * the current window once, pushes the tile's particles of every species and
+ * stores the window once: with several species the staging and the window
+ * store (0.12 ms of a 2048^2 launch) are not repeated per species.
+ *
+ * Workgroups of more than 256 threads, for grids whose tiles do not fill the
+ * GPU, deal their waves to the species (wave w of nw takes species
+ * w ns / nw), so that the species' loops, each a chain of loads, gathers and
+ * LDS atomics, run side by side.  Workgroups of 256 threads push one species
+ * after the other with all waves (dealing the waves there: 2048^2 run 104.0
+ * -> 107.1 ms).  Either way the tile costs three barriers whatever the number
+ * of species; the out-of-window lists are always dealt.
+ *
+ * PAIR = 2 pushes two particles per thread and iteration: the gathers and
+ * Boris pushes of both are independent and interleave, which hides LDS and
+ * arithmetic latency at the price of registers.  FX selects the fixed-point
+ * window (LdsCurrentFxT) instead of float LDS atomics. */
+template <int PAIR = 1, bool FX = false, class Set, int WC = 0, int NT = 256>
 __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
 {
     extern __shared__ float sm[];
-    __shared__ double red[16];
-    __shared__ int ndead_blk, nlist;
-    __shared__ int nls[ZK_FUSE_MAX];    /* out-of-window list lengths per species */
-    __shared__ double ekin[ZK_FUSE_MAX]; /* energy partials per species */
+    constexpr int nw = NT / ZK_WAVE;
+    constexpr bool DEAL = NT > 256;
+    __shared__ double wkin[(DEAL ? 1 : ZK_FUSE_MAX) * nw]; /* energy per wave (and species) */
+    __shared__ double wfar[nw];          /* energy of the out-of-window particles per wave */
+    __shared__ int nls[ZK_FUSE_MAX];     /* out-of-window list lengths per species */
+    __shared__ int ndeads[ZK_FUSE_MAX];  /* particles removed per species */
     __shared__ unsigned long long nsl[ZK_FUSE_MAX]; /* sorting push: stayers | leavers << 32 */
     const zk_push_args &a0 = S[0];
     const int ns = S.n();
     const zk_tiles &t = a0.t;
-    if (threadIdx.x == 0) ndead_blk = nlist = 0;
-    if (threadIdx.x < ZK_FUSE_MAX) nsl[threadIdx.x] = 0ull;
+    if (threadIdx.x < ZK_FUSE_MAX) {
+        nsl[threadIdx.x] = 0ull;
+        nls[threadIdx.x] = ndeads[threadIdx.x] = 0;
+    }
+    /* the species of this wave, and the wave's place among those that share it */
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ZK_WAVE));
+    const int mine = w * ns / nw;
+    const int w0 = (mine * nw + ns - 1) / ns, w1 = ((mine + 1) * nw + ns - 1) / ns;
+    /* threads that share a species' loop, and this one's place among them */
+    const int bs = DEAL ? (w1 - w0) * ZK_WAVE : NT;
+    const int tid = (int)threadIdx.x - (DEAL ? w0 * ZK_WAVE : 0);
 
     const int tx0 = (tile % t.ntx) * t.TX, ty0 = (tile / t.ntx) * t.TY;
     const TileBox box = {tx0, min(tx0 + t.TX, t.nx), ty0, min(ty0 + t.TY, t.ny)};
@@ -643,7 +666,7 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
     unsigned long long *jx = (unsigned long long *)(sm + 6 * n); /* FX: 3 n integers */
     /* stage the window of E and B; nodes outside the guard-inclusive
      * buffer are never read by an in-window particle */
-    for (int m = threadIdx.x; m < n; m += blockDim.x) {
+    for (int m = threadIdx.x; m < n; m += NT) {
         const int gx = ox + m % t.WX, gy = oy + m / t.WX;
         const bool in = gx >= -1 && gx <= t.nx + 1 && gy >= -1 && gy <= t.ny + 1;
         const int g = 3 * ((gx + 1) + (gy + 1) * a0.nrow);
@@ -678,15 +701,13 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
     } else {
         lj.j = jl;
     }
-    int fx_count = 0; /* slots of the tile over all species of the launch */
-    for (int sp = 0; sp < S.n(); sp++) {
+    int ndead = 0;
+    for (int sp = DEAL ? mine : 0; sp < (DEAL ? mine + 1 : ns); sp++) {
         const zk_push_args &a = S[sp];
         const Consts k = {a.tem, a.dt_dx, a.dt_dy, a.qnx, a.qny, a.q};
         zk_parts P = a.p;
         double kin = 0.0;
-        int ndead = 0;
         const int i0 = a.tile_off[tile], i1 = a.tile_n ? i0 + a.tile_n[tile] : a.tile_off[tile + 1];
-        fx_count += i1 - i0;
         const SortSlots ss = SortSlots::of(a, tile);
         if (PAIR == 1) {
             /* Each thread pushes particles i, i + bs, i + 2 bs, ... with the
@@ -704,7 +725,7 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
                 const int lx = c.ix - tx0, ly = c.iy - ty0;
                 const bool inside = lx >= -t.H && lx < t.TX + t.H && ly >= -t.H && ly < t.TY + t.H;
                 const bool live = i >= i0 && i < i1 && c.ix != ZK_DEAD;
-                list_out(a.ovf_list, i0, i, live && !inside, &nlist);
+                list_out(a.ovf_list, i0, i, live && !inside, &nls[sp]);
                 if constexpr (FX && ZK_DEFER_CROSSING) {
                     /* deposits of cell-crossing particles are deferred (DepQueue) */
                     const bool go = live && inside;
@@ -752,8 +773,8 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
              * wave's 64 consecutive slots cover exactly two 128-byte lines
              * of every array (up to 31 slots of the previous tile are
              * loaded and left alone): 1.98 -> 1.94 ms per 2048^2 launch. */
-            const int bs = blockDim.x, last = i1 - 1;
-            int i = (i0 & ~31) + threadIdx.x;
+            const int last = i1 - 1;
+            int i = (i0 & ~31) + tid;
             if (i1 > i0) {
                 /* The loop runs while any lane of the wave has a slot: the
                  * deferred deposits move data between the wave's lanes, so
@@ -774,8 +795,8 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
             }
             if constexpr (FX && ZK_DEFER_CROSSING) dq.flush(lj, k);
         } else {
-            for (int i = i0 + threadIdx.x; i < i1; i += 2 * blockDim.x) {
-                const int j = i + blockDim.x;
+            for (int i = i0 + tid; i < i1; i += 2 * bs) {
+                const int j = i + bs;
                 const bool hasb = j < i1;
                 Part ca = load_part(P, i);
                 Part cb = hasb ? load_part(P, j) : ca;
@@ -783,8 +804,8 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
                 const bool ina = lxa >= -t.H && lxa < t.TX + t.H && lya >= -t.H && lya < t.TY + t.H;
                 const bool inb = lxb >= -t.H && lxb < t.TX + t.H && lyb >= -t.H && lyb < t.TY + t.H;
                 const bool livea = ca.ix != ZK_DEAD, liveb = hasb && cb.ix != ZK_DEAD;
-                list_out(a.ovf_list, i0, i, livea && !ina, &nlist);
-                list_out(a.ovf_list, i0, j, liveb && !inb, &nlist);
+                list_out(a.ovf_list, i0, i, livea && !ina, &nls[sp]);
+                list_out(a.ovf_list, i0, j, liveb && !inb, &nls[sp]);
                 const bool pa = livea && ina, pb = liveb && inb;
                 /* a particle that is not pushed here moves at a safe cell */
                 const int cia = pa ? ca.ix - ox : t.H + 1, cja = pa ? ca.iy - oy : t.H + 1;
@@ -821,19 +842,30 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
                 }
             }
         }
-        __syncthreads();
-        /* the tile's particles outside its window: global path, by this block
-         * (gathers from the guard-inclusive grids, atomics into Jov); with
-         * several species after all main loops, below */
-        const int nl = nlist;
-        if (ns > 1) {
-            if (threadIdx.x == 0) nls[sp] = nl;
-        } else if (nl > 0) {
+        /* energy per wave, summed per tile below in a fixed order */
+        for (int o = ZK_WAVE / 2; o > 0; o >>= 1) kin += __shfl_down(kin, o, ZK_WAVE);
+        if (__lane_id() == 0) wkin[(DEAL ? 0 : sp * nw) + w] = kin;
+        if (ndead) atomicAdd(&ndeads[sp], ndead);
+        ndead = 0;
+    }
+    __syncthreads();
+    /* the tile's particles outside its window: global path, by the waves
+     * dealt to their species, so that the species' chains of dependent
+     * global accesses run side by side (gathers from the guard-inclusive
+     * grids, atomics into Jov).  Whole waves per round: the sorting store
+     * needs every lane. */
+    {
+        const zk_push_args &a = S[mine];
+        const int nl = nls[mine], stride = (w1 - w0) * ZK_WAVE, first = (int)threadIdx.x - w0 * ZK_WAVE;
+        double kin = 0.0;
+        if (nl > 0) {
+            const Consts k = {a.tem, a.dt_dx, a.dt_dy, a.qnx, a.qny, a.q};
+            const zk_parts P = a.p;
             const GlobalFields gf = {a.E, a.B, a.nrow};
             const GlobalCurrent gj = GlobalCurrent::of(a);
-            /* whole waves per round: the sorting store needs every lane */
-            for (int qb = 0; qb < nl; qb += blockDim.x) {
-                const int q = qb + (int)threadIdx.x;
+            const int i0 = a.tile_off[tile];
+            for (int qb = 0; qb < nl; qb += stride) {
+                const int q = qb + first;
                 int i = 0;
                 Part c = {ZK_DEAD, 0, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
                 if (q < nl) {
@@ -848,93 +880,48 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
                     if (!a.sorting) store_part(P, i, c);
                 }
                 if (a.sorting) {
-                    const int sd = sort_reserve(ss, c.ix != ZK_DEAD, box.has(c.ix, c.iy), &nsl[sp]);
+                    const SortSlots ss = SortSlots::of(a, tile);
+                    const int sd = sort_reserve(ss, c.ix != ZK_DEAD, box.has(c.ix, c.iy), &nsl[mine]);
                     sort_write(a, sd, i, c);
                 }
             }
-            if (threadIdx.x == 0) atomicAdd(&a.ctr->n_overflow, nl);
+            for (int o = ZK_WAVE / 2; o > 0; o >>= 1) kin += __shfl_down(kin, o, ZK_WAVE);
+            if (ndead) atomicAdd(&ndeads[mine], ndead);
         }
-        /* per-tile energy partial (summed in fixed order by zk_spec_finalize) */
-        const double e = zk_block_sum(kin, red);
-        if (threadIdx.x == 0) {
-            if (ns > 1) ekin[sp] = e;
-            else a.epart[tile] = e;
-        }
-        if (ndead) atomicAdd(&ndead_blk, ndead);
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            if (ndead_blk) atomicAdd(&a.ctr->n_dead, ndead_blk);
-            ndead_blk = nlist = 0;
-        }
-        __syncthreads();
+        if (__lane_id() == 0) wfar[w] = kin;
     }
-    if (ns > 1) {
-        /* each species' out-of-window particles on its own wave, so that
-         * their chains of dependent global accesses run side by side
-         * (one species after the other, they took 3 % of the launch) */
-        const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ZK_WAVE));
-        if (w < ns) {
-            const zk_push_args &a = S[w];
-            const int nl = nls[w];
-            double kin = 0.0;
-            int ndead = 0;
-            if (nl > 0) {
-                const Consts k = {a.tem, a.dt_dx, a.dt_dy, a.qnx, a.qny, a.q};
-                const zk_parts P = a.p;
-                const GlobalFields gf = {a.E, a.B, a.nrow};
-                const GlobalCurrent gj = GlobalCurrent::of(a);
-                const int i0 = a.tile_off[tile];
-                for (int qb = 0; qb < nl; qb += ZK_WAVE) {
-                    const int q = qb + (int)__lane_id();
-                    int i = 0;
-                    Part c = {ZK_DEAD, 0, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-                    if (q < nl) {
-                        i = a.ovf_list[i0 + q];
-                        c = load_part(P, i);
-                        int di, dj;
-                        gj.touch(c.ix + 1, c.iy + 1);
-                        kin += push_one(gf, gj, c.ix + 1, c.iy + 1, c.x, c.y, c.ux, c.uy, c.uz, di, dj, k);
-                        c.ix += di;
-                        c.iy += dj;
-                        if (boundaries(c.ix, c.iy, t.nx, t.ny, a.moving_window, a.shift, a.open_y)) ndead++;
-                        if (!a.sorting) store_part(P, i, c);
-                    }
-                    if (a.sorting) {
-                        const SortSlots sw = SortSlots::of(a, tile);
-                        const int sd = sort_reserve(sw, c.ix != ZK_DEAD, box.has(c.ix, c.iy), &nsl[w]);
-                        sort_write(a, sd, i, c);
-                    }
-                }
-                for (int o = ZK_WAVE / 2; o > 0; o >>= 1) {
-                    kin += __shfl_down(kin, o, ZK_WAVE);
-                    ndead += __shfl_down(ndead, o, ZK_WAVE);
-                }
-            }
-            if (__lane_id() == 0) {
-                a.epart[tile] = ekin[w] + kin;
-                if (nl > 0) atomicAdd(&a.ctr->n_overflow, nl);
-                if (ndead) atomicAdd(&a.ctr->n_dead, ndead);
-            }
-        }
-    }
-    /* sorting push: the slots taken per species */
     __syncthreads();
     if ((int)threadIdx.x < ns) {
-        const zk_push_args &a = S[threadIdx.x];
+        const int sq = threadIdx.x;
+        const zk_push_args &a = S[sq];
+        const int v0 = (sq * nw + ns - 1) / ns, v1 = ((sq + 1) * nw + ns - 1) / ns;
+        double e = 0.0;
+        for (int v = DEAL ? v0 : 0; v < (DEAL ? v1 : nw); v++) e += wkin[(DEAL ? 0 : sq * nw) + v];
+        for (int v = v0; v < v1; v++) e += wfar[v];
+        a.epart[tile] = e;
+        if (nls[sq] > 0) atomicAdd(&a.ctr->n_overflow, nls[sq]);
+        if (ndeads[sq]) atomicAdd(&a.ctr->n_dead, ndeads[sq]);
+        /* sorting push: the slots taken */
         if (a.sorting) {
             const int cap = (a.tile_off[tile + 1] >> 1) - (a.tile_off[tile] >> 1);
-            const int nl = (int)(unsigned)(nsl[threadIdx.x] >> 32);
-            a.sstay[tile] = (int)(unsigned)nsl[threadIdx.x];
+            const int nl = (int)(unsigned)(nsl[sq] >> 32);
+            a.sstay[tile] = (int)(unsigned)nsl[sq];
             a.sleave[tile] = min(nl, cap);
             if (nl > cap) atomicAdd(&a.ctr->n_unplaced, nl - cap);
         }
     }
     /* a tile too large for the windows' exact range is counted (the host
      * stops the run when it reads the counter) */
-    if (FX && threadIdx.x == 0 && fx_count > ZK_FX_TILE_MAX) atomicAdd(&a0.ctr->n_fx_range, 1);
+    if (FX && threadIdx.x == 0) {
+        int slots = 0;
+        for (int q = 0; q < ns; q++)
+            slots += (S[q].tile_n ? S[q].tile_off[tile] + S[q].tile_n[tile] : S[q].tile_off[tile + 1]) -
+                     S[q].tile_off[tile];
+        if (slots > ZK_FX_TILE_MAX) atomicAdd(&a0.ctr->n_fx_range, 1);
+    }
     /* store the current window of this tile */
     float *dst = a0.region + (size_t)tile * 3 * n;
-    for (int m = threadIdx.x; m < 3 * n; m += blockDim.x) {
+    for (int m = threadIdx.x; m < 3 * n; m += NT) {
         const float v = FX ? (float)zk_fx_read(jx[m]) * a0.fx_unscale : jl[m];
         dst[m] = a0.fresh ? v : dst[m] + v;
     }

@@ -376,6 +376,7 @@ typedef struct zk_bsim {
     float *E[2], *B[2], *J[2];
     float *region;
     long long *Jov;
+    unsigned char *jflag;
     float jov_unscale;
     int ecur, jcur, npass, deposited;
     int nx, ny, nrow;
@@ -398,22 +399,29 @@ typedef struct zk_bspec {
     int ocur;
     int *cnt, *cursor, *stay, *nbr, *tailn; /* re-sort scratch (zk_sort_tiles) */
     double qm, dx0, dx1;
+    /* its entry in the push arguments of its simulation, when one launch
+     * pushes all species of it (set < 0: pushed on its own) */
+    int fset, fk;
 } zk_bspec;
 
 /* Item tables hold (descriptor index, block index) pairs of ints; the
  * launches are one workgroup per item. */
 int zk_batch_fill_jov(const zk_bsim *sims, const int *items, int n, zk_stream_t s);
 int zk_batch_prepare_push(size_t lds);
+int zk_batch_default_window(const zk_tiles *t);
+/* fused push: one workgroup per tile of a simulation, sets[item] the
+ * arguments of its species (buffers kept current by zk_batch_end_step) */
+int zk_batch_push_sets(const zk_push_multi *sets, const int *items, int n, size_t lds, int win, zk_stream_t s);
 int zk_batch_push(const zk_bspec *specs, const zk_bsim *sims, const int *tile_items, int ntile,
-                  const int *global_items, int nglobal, size_t lds, int waves, int fixed, zk_stream_t s);
+                  const int *global_items, int nglobal, size_t lds, int win, int waves, int fixed, zk_stream_t s);
 int zk_batch_finalize(const zk_bspec *specs, int nspecs, zk_stream_t s);
 int zk_batch_reduce_blocks(const zk_bsim *M); /* blocks of the current fold of one simulation */
 int zk_batch_current(const zk_bsim *sims, const int *reduce_items, int nreduce, const int *node_items, int n,
                      int max_passes, zk_stream_t s);
 int zk_batch_fields(const zk_bsim *sims, const int *yee_items, int nyee, zk_stream_t s);
 int zk_batch_sort(const zk_bspec *specs, int nspecs, const int *items, int n, zk_stream_t s);
-int zk_batch_end_step(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_stream_t s);
-int zk_batch_end_step_sorted(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_stream_t s);
+int zk_batch_end_step(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_push_multi *sets, int sorted,
+                      zk_stream_t s);
 /* output-node tiles of the Yee kernel */
 #define ZK_YEE_BX 32
 #define ZK_YEE_BY 16
