@@ -101,6 +101,23 @@ __global__ void __launch_bounds__(1024) finalize_set_kernel(zk_finalize_set f)
     finalize_body(f.ctr[k], f.epart[k], f.nparts[k], f.qm[k], f.dx0[k], f.dx1[k]);
 }
 
+/* For every float x of [first, first + n) (as bit patterns): whether
+ * rcp_ge1, sqrt_ge1 and div_ge1(a, x) differ from the correctly rounded
+ * results of the compiler's own division and square root. */
+__global__ void rounding_kernel(unsigned first, unsigned n, float a, unsigned long long *bad)
+{
+    unsigned long long r = 0, s = 0, d = 0;
+    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const float x = __uint_as_float(first + i);
+        r += rcp_ge1(x) != 1.0f / x;
+        s += sqrt_ge1(x) != sqrtf(x);
+        d += div_ge1(a, x) != a / x;
+    }
+    if (r) atomicAdd(&bad[0], r);
+    if (s) atomicAdd(&bad[1], s);
+    if (d) atomicAdd(&bad[2], d);
+}
+
 __global__ void rescale_fx_kernel(long long *p, size_t n, int shift)
 {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
@@ -209,6 +226,21 @@ extern "C" int zk_stamp_end(zk_stamp st, zk_stream_t s)
 {
     hipLaunchKernelGGL(stamp_kernel, dim3(1), dim3(64), 0, s, st);
     ZK_LAUNCH_CHECK();
+}
+
+extern "C" int zk_rounding_check(unsigned first, unsigned n, float a, unsigned long long bad[3])
+{
+    unsigned long long *d = nullptr;
+    int e = (int)hipMalloc((void **)&d, 3 * sizeof(*d));
+    if (e) return e;
+    e = (int)hipMemcpy(d, bad, 3 * sizeof(*d), hipMemcpyHostToDevice);
+    if (!e) {
+        hipLaunchKernelGGL(rounding_kernel, dim3(4096), dim3(256), 0, nullptr, first, n, a, d);
+        e = (int)hipGetLastError();
+    }
+    if (!e) e = (int)hipMemcpy(bad, d, 3 * sizeof(*d), hipMemcpyDeviceToHost);
+    (void)hipFree(d);
+    return e;
 }
 
 extern "C" int zk_rescale_fx(long long *p, size_t n, int shift, zk_stream_t s)

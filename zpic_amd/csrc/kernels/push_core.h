@@ -11,13 +11,6 @@
 #include "common.h"
 #include "finalize_core.h"
 
-
-/* 1: the fixed-point push defers the deposits of cell-crossing particles
- * to a per-wave queue (DepQueue); 0: every lane runs deposit() in place */
-#ifndef ZK_DEFER_CROSSING
-#define ZK_DEFER_CROSSING 1
-#endif
-
 namespace zk {
 
 struct Seg {
@@ -40,37 +33,52 @@ struct Win {
 constexpr int ZK_WIN_DEFAULT = 25; /* 16 x 16 tiles, 3-cell margin */
 inline bool default_window(const zk_tiles &t) { return t.WX == ZK_WIN_DEFAULT && t.WY == ZK_WIN_DEFAULT; }
 
-/* Field sources: node (a, b) in the source's index space. */
+/* Field sources.  row(a, b) is the place of node (a, b) in the source's
+ * index space, left() and below() its neighbours, and get<c, i, j>() the
+ * value of component c (E, then B) i nodes to its right and j rows up.
+ *
+ * In LDS the six components of a row lie side by side (row b, component c,
+ * node a): one multiply-add forms a particle's address and all but two of
+ * its 24 values are immediate offsets of it or of its three neighbours.
+ * With a plane per component ten more additions formed addresses. */
 template <int WC = 0>
 struct LdsFieldsT : Win<WC> {
     const float *f;
-    __device__ float at(int p, int a, int b) const { return f[p * this->n() + a + b * this->w()]; }
-    __device__ float ex(int a, int b) const { return at(0, a, b); }
-    __device__ float ey(int a, int b) const { return at(1, a, b); }
-    __device__ float ez(int a, int b) const { return at(2, a, b); }
-    __device__ float bx(int a, int b) const { return at(3, a, b); }
-    __device__ float by(int a, int b) const { return at(4, a, b); }
-    __device__ float bz(int a, int b) const { return at(5, a, b); }
+    typedef const float *at;
+    __device__ at row(int a, int b) const { return f + __umul24(b, 6 * this->w()) + a; }
+    __device__ at left(at p, bool on) const { return p - (on ? 1 : 0); }
+    __device__ at below(at p, bool on) const { return p - (on ? 6 * this->w() : 0); }
+    template <int C, int I, int J>
+    __device__ float get(at p) const
+    {
+        return p[(6 * J + C) * this->w() + I];
+    }
 };
 
 struct GlobalFields {
     const float *E, *B;
     int nrow;
-    __device__ float ex(int a, int b) const { return E[3 * (a + b * nrow) + 0]; }
-    __device__ float ey(int a, int b) const { return E[3 * (a + b * nrow) + 1]; }
-    __device__ float ez(int a, int b) const { return E[3 * (a + b * nrow) + 2]; }
-    __device__ float bx(int a, int b) const { return B[3 * (a + b * nrow) + 0]; }
-    __device__ float by(int a, int b) const { return B[3 * (a + b * nrow) + 1]; }
-    __device__ float bz(int a, int b) const { return B[3 * (a + b * nrow) + 2]; }
+    typedef int at;
+    __device__ at row(int a, int b) const { return a + b * nrow; }
+    __device__ at left(at p, bool on) const { return p - (on ? 1 : 0); }
+    __device__ at below(at p, bool on) const { return p - (on ? nrow : 0); }
+    template <int C, int I, int J>
+    __device__ float get(at p) const
+    {
+        return (C < 3 ? E : B)[3 * (p + I + J * nrow) + C % 3];
+    }
 };
 
-/* Current sinks. */
+/* Current sinks: row(a, b) as above, add<c, i, j>() adds to component c. */
 template <int WC = 0>
 struct LdsCurrentT : Win<WC> {
     float *j;
-    __device__ void add(int a, int b, int c, float v) const
+    typedef float *at;
+    __device__ at row(int a, int b) const { return j + __umul24(b, this->w()) + a; }
+    template <int C, int I, int J>
+    __device__ void add(at p, float v) const
     {
-        atomicAdd(&j[c * this->n() + a + b * this->w()], v);
+        atomicAdd(&p[C * this->n() + J * this->w() + I], v);
     }
 };
 
@@ -85,9 +93,12 @@ template <int WC = 0>
 struct LdsCurrentFxT : Win<WC> {
     unsigned long long *j;
     float scale;
-    __device__ void add(int a, int b, int c, float v) const
+    typedef unsigned long long *at;
+    __device__ at row(int a, int b) const { return j + __umul24(b, this->w()) + a; }
+    template <int C, int I, int J>
+    __device__ void add(at p, float v) const
     {
-        atomicAdd(&j[c * this->n() + a + b * this->w()], zk_fx_raw(v, scale));
+        atomicAdd(&p[C * this->n() + J * this->w() + I], zk_fx_raw(v, scale));
     }
 };
 
@@ -120,33 +131,37 @@ struct GlobalCurrent {
         flag[x0 + y1] = 1;
         flag[x1 + y1] = 1;
     }
-    __device__ void add(int a, int b, int c, float v) const
+    typedef unsigned long long *at;
+    __device__ at row(int a, int b) const { return (unsigned long long *)&J[3 * (a + b * nrow)]; }
+    template <int C, int I, int Jr>
+    __device__ void add(at p, float v) const
     {
-        atomicAdd((unsigned long long *)&J[3 * (a + b * nrow) + c], zk_fx(v, scale));
+        atomicAdd(&p[3 * (I + Jr * nrow) + C], zk_fx(v, scale));
     }
 };
 
 /* Bilinear gather on the staggered mesh (em2d/particles.c:1029-1071);
  * (i, j) is the particle's cell in the source index space. */
+template <int C, class F>
+__device__ inline float bilinear(const F &S, typename F::at p, float wx, float wy)
+{
+    return (S.template get<C, 0, 0>(p) * (1.0f - wx) + S.template get<C, 1, 0>(p) * wx) * (1.0f - wy) +
+           (S.template get<C, 0, 1>(p) * (1.0f - wx) + S.template get<C, 1, 1>(p) * wx) * wy;
+}
+
 template <class F>
 __device__ inline void gather(const F &S, int i, int j, float wx, float wy, float e[3], float b[3])
 {
-    const int ih = i + ((wx < 0.5f) ? -1 : 0);
-    const int jh = j + ((wy < 0.5f) ? -1 : 0);
-    const float wxh = wx + ((wx < 0.5f) ? 0.5f : -0.5f);
-    const float wyh = wy + ((wy < 0.5f) ? 0.5f : -0.5f);
-    e[0] = (S.ex(ih, j) * (1.0f - wxh) + S.ex(ih + 1, j) * wxh) * (1.0f - wy) +
-           (S.ex(ih, j + 1) * (1.0f - wxh) + S.ex(ih + 1, j + 1) * wxh) * wy;
-    e[1] = (S.ey(i, jh) * (1.0f - wx) + S.ey(i + 1, jh) * wx) * (1.0f - wyh) +
-           (S.ey(i, jh + 1) * (1.0f - wx) + S.ey(i + 1, jh + 1) * wx) * wyh;
-    e[2] = (S.ez(i, j) * (1.0f - wx) + S.ez(i + 1, j) * wx) * (1.0f - wy) +
-           (S.ez(i, j + 1) * (1.0f - wx) + S.ez(i + 1, j + 1) * wx) * wy;
-    b[0] = (S.bx(i, jh) * (1.0f - wx) + S.bx(i + 1, jh) * wx) * (1.0f - wyh) +
-           (S.bx(i, jh + 1) * (1.0f - wx) + S.bx(i + 1, jh + 1) * wx) * wyh;
-    b[1] = (S.by(ih, j) * (1.0f - wxh) + S.by(ih + 1, j) * wxh) * (1.0f - wy) +
-           (S.by(ih, j + 1) * (1.0f - wxh) + S.by(ih + 1, j + 1) * wxh) * wy;
-    b[2] = (S.bz(ih, jh) * (1.0f - wxh) + S.bz(ih + 1, jh) * wxh) * (1.0f - wyh) +
-           (S.bz(ih, jh + 1) * (1.0f - wxh) + S.bz(ih + 1, jh + 1) * wxh) * wyh;
+    const bool lx = wx < 0.5f, ly = wy < 0.5f;
+    const float wxh = wx + (lx ? 0.5f : -0.5f);
+    const float wyh = wy + (ly ? 0.5f : -0.5f);
+    const typename F::at p = S.row(i, j), px = S.left(p, lx), py = S.below(p, ly), pxy = S.below(px, ly);
+    e[0] = bilinear<0>(S, px, wxh, wy);
+    e[1] = bilinear<1>(S, py, wx, wyh);
+    e[2] = bilinear<2>(S, p, wx, wy);
+    b[0] = bilinear<3>(S, py, wx, wyh);
+    b[1] = bilinear<4>(S, px, wxh, wy);
+    b[2] = bilinear<5>(S, pxy, wxh, wyh);
 }
 
 /* Cut segment s at the y cell edge crossed (dj = +-1) into s and t
@@ -186,21 +201,22 @@ __device__ inline void ysplit(Seg &s, Seg &t, int dj)
 template <class D>
 __device__ inline void deposit_seg(const D &J, const Seg &g, float qnx, float qny)
 {
+    const typename D::at p = J.row(g.ix, g.iy);
     const float ax0 = 1.0f - g.x0, ax1 = 1.0f - g.x1;
     const float jx = qnx * g.dx, jy = qny * g.dy;
     const float jxh = jx * (0.5f * (g.y0 + g.y1));
     const float jyh = jy * (0.5f * (g.x0 + g.x1));
-    J.add(g.ix, g.iy, 0, jx - jxh);
-    J.add(g.ix, g.iy + 1, 0, jxh);
-    J.add(g.ix, g.iy, 1, jy - jyh);
-    J.add(g.ix + 1, g.iy, 1, jyh);
+    J.template add<0, 0, 0>(p, jx - jxh);
+    J.template add<0, 0, 1>(p, jxh);
+    J.template add<1, 0, 0>(p, jy - jyh);
+    J.template add<1, 1, 0>(p, jyh);
     const float c = __builtin_fmaf(0.5f, g.y1, g.y0), d = __builtin_fmaf(-0.5f, g.y0, g.y1);
     const float qa = g.qvz * (1.5f - c), qb = g.qvz * (0.5f - d);
     const float qc = g.qvz * c, qd = g.qvz * d;
-    J.add(g.ix, g.iy, 2, __builtin_fmaf(ax0, qa, ax1 * qb));
-    J.add(g.ix + 1, g.iy, 2, __builtin_fmaf(g.x0, qa, g.x1 * qb));
-    J.add(g.ix, g.iy + 1, 2, __builtin_fmaf(ax0, qc, ax1 * qd));
-    J.add(g.ix + 1, g.iy + 1, 2, __builtin_fmaf(g.x0, qc, g.x1 * qd));
+    J.template add<2, 0, 0>(p, __builtin_fmaf(ax0, qa, ax1 * qb));
+    J.template add<2, 1, 0>(p, __builtin_fmaf(g.x0, qa, g.x1 * qb));
+    J.template add<2, 0, 1>(p, __builtin_fmaf(ax0, qc, ax1 * qd));
+    J.template add<2, 1, 1>(p, __builtin_fmaf(g.x0, qc, g.x1 * qd));
 }
 
 /* Split the motion at cell edges into up to three segments and deposit
@@ -297,7 +313,7 @@ __device__ inline void deposit_in_cell(const D &J, int ix, int iy, float x0, flo
  * the split arithmetic runs on (nearly) full waves.  The fixed-point sums
  * of the window do not depend on the order of the contributions, so J is
  * unchanged.  Window-local cells fit 8 bits each (windows are at most
- * 73 nodes per side), di + 1 and dj + 1 2 bits each. */
+ * 73 nodes per side). */
 struct DepQueue {
     float x0, y0, dx, dy, qvz;
     int code;
@@ -310,28 +326,26 @@ struct DepQueue {
     {
         if (n == 0) return;
         if ((int)__lane_id() < n) {
-            const int ci = code & 0xff, cj = (code >> 8) & 0xff;
-            const int di = ((code >> 16) & 3) - 1, dj = ((code >> 18) & 3) - 1;
-            deposit(J, ci, cj, di, dj, x0, y0, dx, dy, k.qnx, k.qny, qvz);
+            const float x1 = x0 + dx, y1 = y0 + dy;
+            const int di = (x1 >= 1.0f) - (x1 < 0.0f), dj = (y1 >= 1.0f) - (y1 < 0.0f);
+            deposit(J, code & 0xff, code >> 8, di, dj, x0, y0, dx, dy, k.qnx, k.qny, qvz);
         }
         n = 0;
     }
 
-    /* called by every lane of the wave; lanes with `cross` append */
+    /* called by every lane of the wave; the lanes of m append */
     template <class D>
-    __device__ void push(bool cross, int ci, int cj, int di, int dj, float px, float py, float mx, float my,
-                         float pq, const D &J, const Consts &k)
+    __device__ void push(unsigned long long m, int ci, int cj, float px, float py, float mx, float my, float pq,
+                         const D &J, const Consts &k)
     {
-        const unsigned long long m = __ballot(cross);
         const int add = __popcll(m);
         if (add == 0) return;
         if (n + add > ZK_WAVE) flush(J, k);
-        const int lane = __lane_id();
-        const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+        const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, n));
         /* lanes that do not append send to a lane outside [n, n + add) */
-        const int dst = ((cross ? n + rank : n + add) & (ZK_WAVE - 1)) * 4;
-        const int c = ci | (cj << 8) | ((di + 1) << 16) | ((dj + 1) << 18);
-        const bool take = lane >= n && lane < n + add;
+        const int dst = (__builtin_amdgcn_inverse_ballot_w64(m) ? rank : n + add) * 4;
+        const int c = ci | (cj << 8);
+        const bool take = __builtin_amdgcn_inverse_ballot_w64((~0ull >> (ZK_WAVE - add)) << n);
         const float rx0 = __int_as_float(__builtin_amdgcn_ds_permute(dst, __float_as_int(px)));
         const float ry0 = __int_as_float(__builtin_amdgcn_ds_permute(dst, __float_as_int(py)));
         const float rdx = __int_as_float(__builtin_amdgcn_ds_permute(dst, __float_as_int(mx)));
@@ -382,41 +396,73 @@ __device__ inline void store_part(const zk_parts &P, int i, const Part &c)
     zk_at(P.uz, o) = c.uz;
 }
 
-/* IEEE division a / b and square root of x for the Boris push, where the
- * divisors are >= 1 and the square-root arguments are >= 1: the sequences
- * of the correctly rounded hardware expansions (reciprocal and square-root
- * estimates refined by fused multiply-adds), without the operand scaling
- * and special-value fix-ups that only denormal, infinite, zero or
- * extreme-exponent operands need.  For finite operands in those ranges
- * the results are the correctly rounded ones, bit for bit. */
+/* A particle as it is stored, with its packed cell. */
+struct Slot {
+    int cell;
+    float x, y, ux, uy, uz;
+};
+
+__device__ inline Slot load_slot(const zk_parts &P, int i)
+{
+    const unsigned o = (unsigned)i * 4u;
+    return {zk_at(P.cell, o), zk_at(P.x, o), zk_at(P.y, o), zk_at(P.ux, o), zk_at(P.uy, o), zk_at(P.uz, o)};
+}
+
+__device__ inline void store_slot(const zk_parts &P, int i, const Slot &c)
+{
+    const unsigned o = (unsigned)i * 4u;
+    zk_at(P.cell, o) = c.cell;
+    zk_at(P.x, o) = c.x;
+    zk_at(P.y, o) = c.y;
+    zk_at(P.ux, o) = c.ux;
+    zk_at(P.uy, o) = c.uy;
+    zk_at(P.uz, o) = c.uz;
+}
+
+/* registers whose contents do not matter, without an instruction to set them */
+__device__ inline void any_value(float &a, float &b, float &c) { asm volatile("" : "=v"(a), "=v"(b), "=v"(c)); }
+
+/* Correctly rounded reciprocal, division and square root for the Boris
+ * push, whose divisors and square-root arguments are at least 1: hardware
+ * estimates refined by fused multiply-adds, without the operand scaling and
+ * special-value fix-ups that only denormal, infinite, zero or
+ * extreme-exponent operands need.
+ *
+ * On gfx950 one Newton step of the reciprocal estimate gives the correctly
+ * rounded 1 / b for every float b in [1, 2^126), and one residual step on
+ * x rsq(x) the correctly rounded square root for every x in [1, 2^127)
+ * (checked for all of them, tests/test_gpu_rounding.py).  With y = 1 / b
+ * correctly rounded, q = a y is within 1.5 units of the quotient, one
+ * residual step makes it a faithful rounding, and one more the correctly
+ * rounded quotient (Markstein's theorem).  The shorter sequences take 19
+ * of the push's 420 issue slots per particle. */
+__device__ inline float rcp_ge1(float b)
+{
+    const float y = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+
 __device__ inline float div_ge1(float a, float b)
 {
-    float y = __builtin_amdgcn_rcpf(b);
-    const float e = __builtin_fmaf(-b, y, 1.0f);
-    y = __builtin_fmaf(e, y, y);
+    const float y = rcp_ge1(b);
     float q = a * y;
-    float r = __builtin_fmaf(-b, q, a);
-    q = __builtin_fmaf(r, y, q);
-    r = __builtin_fmaf(-b, q, a);
-    return __builtin_fmaf(r, y, q);
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
 }
 
 __device__ inline float sqrt_ge1(float x)
 {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float sm = __int_as_float(__float_as_int(s) - 1), sp = __int_as_float(__float_as_int(s) + 1);
-    float r = (__builtin_fmaf(-sm, s, x) <= 0.0f) ? sm : s;
-    r = (__builtin_fmaf(-sp, s, x) > 0.0f) ? sp : r;
-    return r;
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
 }
 
 /* Motion of one particle whose cell is (ci, cj) in the sources' index
- * space: gather, Boris push, displacement (mx, my), cells crossed (di, dj)
- * and q v_z; returns the time-centred kinetic energy term
- * (em2d/particles.c:1125-1228). */
+ * space: gather, Boris push, displacement (mx, my) and q v_z; returns the
+ * time-centred kinetic energy term (em2d/particles.c:1125-1228). */
 template <class F>
 __device__ inline double move_one(const F &S, int ci, int cj, float x, float y, float &ux, float &uy, float &uz,
-                                  float &mx, float &my, float &qvz, int &di, int &dj, const Consts &k)
+                                  float &mx, float &my, float &qvz, const Consts &k)
 {
     float e[3], b[3];
     gather(S, ci, cj, x, y, e, b);
@@ -431,7 +477,7 @@ __device__ inline double move_one(const F &S, int ci, int cj, float x, float y, 
     b[0] *= tg;
     b[1] *= tg;
     b[2] *= tg;
-    const float s2 = div_ge1(2.0f, 1.0f + b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
+    const float s2 = 2.0f * rcp_ge1(1.0f + b[0] * b[0] + b[1] * b[1] + b[2] * b[2]); /* the doubling is exact */
     const float vx = ax + ay * b[2] - az * b[1];
     const float vy = ay + az * b[0] - ax * b[2];
     const float vz = az + ax * b[1] - ay * b[0];
@@ -445,14 +491,18 @@ __device__ inline double move_one(const F &S, int ci, int cj, float x, float y, 
     uy = ay + e[1];
     uz = az + e[2];
 
-    const float rg = div_ge1(1.0f, sqrt_ge1(1.0f + ux * ux + uy * uy + uz * uz));
+    const float rg = rcp_ge1(sqrt_ge1(1.0f + ux * ux + uy * uy + uz * uz));
     mx = k.dt_dx * rg * ux;
     my = k.dt_dy * rg * uy;
-    const float x1 = x + mx, y1 = y + my;
-    di = (x1 >= 1.0f) - (x1 < 0.0f);
-    dj = (y1 >= 1.0f) - (y1 < 0.0f);
     qvz = k.q * uz * rg;
     return kin;
+}
+
+/* cells crossed on the way to offsets (x1, y1) (ltrim, em2d/particles.c:1081-1084) */
+__device__ inline void crossed(float x1, float y1, int &di, int &dj)
+{
+    di = (x1 >= 1.0f) - (x1 < 0.0f);
+    dj = (y1 >= 1.0f) - (y1 < 0.0f);
 }
 
 /* Push one particle: move_one, the deposit of its motion, and its new cell
@@ -462,8 +512,9 @@ __device__ inline double push_one(const F &S, const D &J, int ci, int cj, float 
                                   float &ux, float &uy, float &uz, int &di, int &dj, const Consts &k)
 {
     float mx, my, qvz;
-    const double kin = move_one(S, ci, cj, x, y, ux, uy, uz, mx, my, qvz, di, dj, k);
+    const double kin = move_one(S, ci, cj, x, y, ux, uy, uz, mx, my, qvz, k);
     float x1 = x + mx, y1 = y + my;
+    crossed(x1, y1, di, dj);
     x1 -= di;
     y1 -= dj;
     deposit(J, ci, cj, di, dj, x, y, mx, my, k.qnx, k.qny, qvz);
@@ -499,18 +550,17 @@ __device__ inline bool boundaries(int &ix, int &iy, int nx, int ny, int mw, int 
     return false;
 }
 
-/* List the live particles outside the window in the tile's own range of
- * ovf_list (one LDS atomic per wave). */
-__device__ inline void list_out(int *ovf_list, int i0, int i, bool out_here, int *nlist)
+/* List the particles of the lanes in `out`, live and outside the window, in
+ * the tile's own range of ovf_list (one LDS atomic per wave). */
+__device__ inline void list_out(int *ovf_list, int i0, int i, unsigned long long out, int *nlist)
 {
-    const unsigned long long out = __ballot(out_here);
     if (out) {
         const int lane = __lane_id();
         int base = 0;
         const int leader = __ffsll((long long)out) - 1;
         if (lane == leader) base = atomicAdd(nlist, __popcll(out));
         base = __shfl(base, leader, ZK_WAVE);
-        if (out_here) ovf_list[i0 + base + __popcll(out & ((1ull << lane) - 1ull))] = i;
+        if (out >> lane & 1) ovf_list[i0 + base + __popcll(out & ((1ull << lane) - 1ull))] = i;
     }
 }
 
@@ -667,15 +717,16 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
     /* stage the window of E and B; nodes outside the guard-inclusive
      * buffer are never read by an in-window particle */
     for (int m = threadIdx.x; m < n; m += NT) {
-        const int gx = ox + m % t.WX, gy = oy + m / t.WX;
+        const int u = m % t.WX, v = m / t.WX, l = u + 6 * t.WX * v;
+        const int gx = ox + u, gy = oy + v;
         const bool in = gx >= -1 && gx <= t.nx + 1 && gy >= -1 && gy <= t.ny + 1;
         const int g = 3 * ((gx + 1) + (gy + 1) * a0.nrow);
-        fl[0 * n + m] = in ? a0.E[g + 0] : 0.0f;
-        fl[1 * n + m] = in ? a0.E[g + 1] : 0.0f;
-        fl[2 * n + m] = in ? a0.E[g + 2] : 0.0f;
-        fl[3 * n + m] = in ? a0.B[g + 0] : 0.0f;
-        fl[4 * n + m] = in ? a0.B[g + 1] : 0.0f;
-        fl[5 * n + m] = in ? a0.B[g + 2] : 0.0f;
+        fl[l + 0 * t.WX] = in ? a0.E[g + 0] : 0.0f;
+        fl[l + 1 * t.WX] = in ? a0.E[g + 1] : 0.0f;
+        fl[l + 2 * t.WX] = in ? a0.E[g + 2] : 0.0f;
+        fl[l + 3 * t.WX] = in ? a0.B[g + 0] : 0.0f;
+        fl[l + 4 * t.WX] = in ? a0.B[g + 1] : 0.0f;
+        fl[l + 5 * t.WX] = in ? a0.B[g + 2] : 0.0f;
         if (FX) {
             jx[0 * n + m] = 0ull;
             jx[1 * n + m] = 0ull;
@@ -721,51 +772,70 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
              * one particle ahead, 1.03-1.05 ms with two; three ahead spills.) */
             DepQueue dq;
             dq.init();
-            auto step = [&](Part &c, int i) {
-                const int lx = c.ix - tx0, ly = c.iy - ty0;
-                const bool inside = lx >= -t.H && lx < t.TX + t.H && ly >= -t.H && ly < t.TY + t.H;
-                const bool live = i >= i0 && i < i1 && c.ix != ZK_DEAD;
-                list_out(a.ovf_list, i0, i, live && !inside, &nls[sp]);
-                if constexpr (FX && ZK_DEFER_CROSSING) {
+            /* cells a particle of the window can reach in this step lie on the
+             * grid, and nothing else than its motion changes its cell */
+            const bool plain = !a.moving_window && !a.open_y && !a.sorting && tx0 > t.H && ty0 > t.H &&
+                               tx0 + t.TX + t.H < t.nx && ty0 + t.TY + t.H < t.ny;
+            const unsigned spanx = t.TX + 2 * t.H, spany = t.TY + 2 * t.H, slots = i1 - i0;
+            auto step = [&](Slot &c, int i) {
+                /* the predicates are kept as wave masks: every one is a single
+                 * comparison, and their combination costs no vector work */
+                const int cx = c.cell & ((1 << P.cbits) - 1), cy = c.cell >> P.cbits;
+                const unsigned ci = cx - ox, cj = cy - oy;
+                const unsigned long long live = __builtin_amdgcn_ballot_w64(c.cell >= 0) &
+                                                __builtin_amdgcn_ballot_w64((unsigned)(i - i0) < slots);
+                const unsigned long long inside = __builtin_amdgcn_ballot_w64(ci - 1u < spanx) &
+                                                  __builtin_amdgcn_ballot_w64(cj - 1u < spany);
+                list_out(a.ovf_list, i0, i, live & ~inside, &nls[sp]);
+                if constexpr (FX) {
                     /* deposits of cell-crossing particles are deferred (DepQueue) */
-                    const bool go = live && inside;
-                    const int ci = c.ix - ox, cj = c.iy - oy;
-                    float mx = 0.0f, my = 0.0f, qvz = 0.0f;
-                    int di = 0, dj = 0;
-                    if (go) kin += move_one(lf, ci, cj, c.x, c.y, c.ux, c.uy, c.uz, mx, my, qvz, di, dj, k);
-                    const bool cross = go && (di != 0 || dj != 0);
-                    /* the particle after the step */
-                    Part nc = c;
+                    const bool go = __builtin_amdgcn_inverse_ballot_w64(live & inside);
+                    float mx, my, qvz;
+                    any_value(mx, my, qvz); /* of lanes that do not push: never used */
+                    bool cross = false;
+                    Part nc;                /* the particle after a sorting step */
+                    nc.ix = ZK_DEAD;
+                    nc.iy = 0;
                     if (go) {
-                        float x1 = c.x + mx, y1 = c.y + my;
-                        x1 -= di;
-                        y1 -= dj;
-                        nc.x = x1;
-                        nc.y = y1;
-                        nc.ix += di;
-                        nc.iy += dj;
-                        if (boundaries(nc.ix, nc.iy, t.nx, t.ny, a.moving_window, a.shift, a.open_y)) ndead++;
-                    }
-                    int sd = -1;
-                    if (a.sorting)
-                        sd = sort_reserve(ss, go && nc.ix != ZK_DEAD, box.has(nc.ix, nc.iy), &nsl[sp]);
-                    if (go && !cross) deposit_in_cell(lj, ci, cj, c.x, c.y, mx, my, k.qnx, k.qny, qvz);
-                    dq.push(cross, ci, cj, di, dj, c.x, c.y, mx, my, qvz, lj, k);
-                    if (a.sorting) sort_write(a, sd, i, nc);
-                    else if (go) store_part(P, i, nc);
-                } else {
-                    const bool go = live && inside;
-                    if (go) {
-                        int di, dj;
-                        kin += push_one(lf, lj, c.ix - ox, c.iy - oy, c.x, c.y, c.ux, c.uy, c.uz, di, dj, k);
-                        c.ix += di;
-                        c.iy += dj;
-                        if (boundaries(c.ix, c.iy, t.nx, t.ny, a.moving_window, a.shift, a.open_y)) ndead++;
-                        if (!a.sorting) store_part(P, i, c);
+                        kin += move_one(lf, ci, cj, c.x, c.y, c.ux, c.uy, c.uz, mx, my, qvz, k);
+                        const float x1 = c.x + mx, y1 = c.y + my;
+                        /* cells crossed: at most one per axis */
+                        const float fi = __builtin_amdgcn_fmed3f(__builtin_floorf(x1), -1.0f, 1.0f);
+                        const float fj = __builtin_amdgcn_fmed3f(__builtin_floorf(y1), -1.0f, 1.0f);
+                        cross = (fi != 0.0f) | (fj != 0.0f);
+                        const int di = (int)fi, dj = (int)fj;
+                        Slot s = {0, x1 - fi, y1 - fj, c.ux, c.uy, c.uz};
+                        if (plain) {
+                            s.cell = c.cell + di + (dj << P.cbits);
+                            store_slot(P, i, s);
+                        } else {
+                            int ix = cx + di, iy = cy + dj;
+                            if (boundaries(ix, iy, t.nx, t.ny, a.moving_window, a.shift, a.open_y)) ndead++;
+                            s.cell = zk_cell(ix, iy, P.cbits);
+                            if (!a.sorting) store_slot(P, i, s);
+                            nc = {ix, iy, s.x, s.y, s.ux, s.uy, s.uz};
+                        }
+                        if (!cross) deposit_in_cell(lj, ci, cj, c.x, c.y, mx, my, k.qnx, k.qny, qvz);
                     }
                     if (a.sorting) {
-                        const int sd = sort_reserve(ss, go && c.ix != ZK_DEAD, box.has(c.ix, c.iy), &nsl[sp]);
-                        sort_write(a, sd, i, c);
+                        const int sd = sort_reserve(ss, nc.ix != ZK_DEAD, box.has(nc.ix, nc.iy), &nsl[sp]);
+                        sort_write(a, sd, i, nc);
+                    }
+                    dq.push(__builtin_amdgcn_ballot_w64(cross), ci, cj, c.x, c.y, mx, my, qvz, lj, k);
+                } else {
+                    Part q = {cx, cy, c.x, c.y, c.ux, c.uy, c.uz};
+                    const bool go = __builtin_amdgcn_inverse_ballot_w64(live & inside);
+                    if (go) {
+                        int di, dj;
+                        kin += push_one(lf, lj, ci, cj, q.x, q.y, q.ux, q.uy, q.uz, di, dj, k);
+                        q.ix += di;
+                        q.iy += dj;
+                        if (boundaries(q.ix, q.iy, t.nx, t.ny, a.moving_window, a.shift, a.open_y)) ndead++;
+                        if (!a.sorting) store_part(P, i, q);
+                    }
+                    if (a.sorting) {
+                        const int sd = sort_reserve(ss, go && q.ix != ZK_DEAD, box.has(q.ix, q.iy), &nsl[sp]);
+                        sort_write(a, sd, i, q);
                     }
                 }
             };
@@ -780,20 +850,20 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
                  * deferred deposits move data between the wave's lanes, so
                  * no lane may leave the loop early.  Lanes past the range
                  * load its last particle and leave it alone. */
-                Part ca, cb, cc;
-                ca = load_part(P, min(i, last));
-                cb = load_part(P, min(i + bs, last));
+                Slot ca, cb, cc;
+                ca = load_slot(P, min(i, last));
+                cb = load_slot(P, min(i + bs, last));
                 int wave0 = __builtin_amdgcn_readfirstlane(i - (int)__lane_id());
                 for (; wave0 < i1; i += 3 * bs, wave0 += 3 * bs) {
-                    cc = load_part(P, min(i + 2 * bs, last));
+                    cc = load_slot(P, min(i + 2 * bs, last));
                     step(ca, i);
-                    ca = load_part(P, min(i + 3 * bs, last));
+                    ca = load_slot(P, min(i + 3 * bs, last));
                     step(cb, i + bs);
-                    cb = load_part(P, min(i + 4 * bs, last));
+                    cb = load_slot(P, min(i + 4 * bs, last));
                     step(cc, i + 2 * bs);
                 }
             }
-            if constexpr (FX && ZK_DEFER_CROSSING) dq.flush(lj, k);
+            if constexpr (FX) dq.flush(lj, k);
         } else {
             for (int i = i0 + tid; i < i1; i += 2 * bs) {
                 const int j = i + bs;
@@ -804,16 +874,18 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
                 const bool ina = lxa >= -t.H && lxa < t.TX + t.H && lya >= -t.H && lya < t.TY + t.H;
                 const bool inb = lxb >= -t.H && lxb < t.TX + t.H && lyb >= -t.H && lyb < t.TY + t.H;
                 const bool livea = ca.ix != ZK_DEAD, liveb = hasb && cb.ix != ZK_DEAD;
-                list_out(a.ovf_list, i0, i, livea && !ina, &nls[sp]);
-                list_out(a.ovf_list, i0, j, liveb && !inb, &nls[sp]);
+                list_out(a.ovf_list, i0, i, __ballot(livea && !ina), &nls[sp]);
+                list_out(a.ovf_list, i0, j, __ballot(liveb && !inb), &nls[sp]);
                 const bool pa = livea && ina, pb = liveb && inb;
                 /* a particle that is not pushed here moves at a safe cell */
                 const int cia = pa ? ca.ix - ox : t.H + 1, cja = pa ? ca.iy - oy : t.H + 1;
                 const int cib = pb ? cb.ix - ox : t.H + 1, cjb = pb ? cb.iy - oy : t.H + 1;
                 float mxa, mya, qa, mxb, myb, qb;
                 int dia, dja, dib, djb;
-                const double ka = move_one(lf, cia, cja, ca.x, ca.y, ca.ux, ca.uy, ca.uz, mxa, mya, qa, dia, dja, k);
-                const double kb = move_one(lf, cib, cjb, cb.x, cb.y, cb.ux, cb.uy, cb.uz, mxb, myb, qb, dib, djb, k);
+                const double ka = move_one(lf, cia, cja, ca.x, ca.y, ca.ux, ca.uy, ca.uz, mxa, mya, qa, k);
+                const double kb = move_one(lf, cib, cjb, cb.x, cb.y, cb.ux, cb.uy, cb.uz, mxb, myb, qb, k);
+                crossed(ca.x + mxa, ca.y + mya, dia, dja);
+                crossed(cb.x + mxb, cb.y + myb, dib, djb);
                 if (pa) {
                     float x1 = ca.x + mxa, y1 = ca.y + mya;
                     x1 -= dia;

@@ -156,6 +156,10 @@ typedef struct zk_push_multi {
 int zk_fill_f32(float *p, size_t n, float v, zk_stream_t s);
 /* reads the clock into a phase's end on its own */
 int zk_stamp_end(zk_stamp st, zk_stream_t s);
+/* bad[k] += floats with bit patterns first .. first + n - 1 whose reciprocal,
+ * square root or quotient a / x in the push is not the correctly rounded one
+ * (a check for the tests; waits for the GPU) */
+int zk_rounding_check(unsigned first, unsigned n, float a, unsigned long long bad[3]);
 /* divide the n fixed-point values of p by 2^shift (arithmetic shift) */
 int zk_rescale_fx(long long *p, size_t n, int shift, zk_stream_t s);
 int zk_push(const zk_push_args *a, zk_stream_t s);
