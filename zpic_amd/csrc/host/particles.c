@@ -701,45 +701,23 @@ static int sort_readback(struct zpic_dev_species *d)
     return c.n_unplaced + c.n_overfull;
 }
 
-/* Full sort into the other buffer set: `spread` for an unsorted upload
- * (counting sort with cell interleaving), else the re-sort of tile ranges
- * plus a tail; with `slack` the new ranges keep free slots for the staged
- * re-sorts that follow. */
-static void sort_now_from(t_species *s, int spread, int slack, const int *before);
-static void sort_now(t_species *s, int spread, int slack)
+/* Room for the free slots a sort with `slack` leaves (they only serve the
+ * staged re-sort; mode 2: one per range); returns the slack to use. */
+static int sort_slack(struct zpic_dev_species *d, int slack)
 {
-    sort_now_from(s, spread, slack, s->dev->counted ? s->dev->tile_n : NULL);
-}
-
-/* before: the tile counts of the previous sort (NULL: unknown) */
-static void sort_now_from(t_species *s, int spread, int slack, const int *before)
-{
-    struct zpic_dev_species *d = s->dev;
-    /* free slots only serve the staged re-sort (mode 2: one per range) */
-    if (slack) slack = zpic_staged_sort() == 2 ? 2 : zpic_staged_sort() ? 1 : 0;
+    if (!slack) return 0;
+    slack = zpic_staged_sort() == 2 ? 2 : zpic_staged_sort() ? 1 : 0;
     if (slack) {
         const int want = layout_slots(d->np_live, d->t.ntiles);
         if (want > d->cap) grow_sets(d, want);
     }
-    const int other = 1 - d->cur;
-    zpic_ktimer_begin(ZPIC_T_SORT);
-    if (spread) {
-        ZCHECK(zk_sort(&d->set[d->cur], &d->set[other], d->ctr, d->cnt, d->tile_off, d->cursor, d->tile_n, &d->t,
-                       d->np_upper, spread, slack, d->cap, zpic_stream()));
-    } else {
-        /* the particles are in tile ranges (plus a tail): keep the stayers */
-        ZCHECK(zk_sort_tiles(&d->set[d->cur], &d->set[other], d->ctr, d->cnt, d->stay, d->nbr, d->tailn, d->tile_off,
-                             d->counted ? d->tile_n : NULL, before, d->tile_off2, d->tile_n2, d->cursor, &d->t,
-                             d->tail_upper, slack, d->cap, zpic_phase_stamp(ZPIC_T_SPEC), zpic_stream()));
-        int *tmp = d->tile_off;
-        d->tile_off = d->tile_off2;
-        d->tile_off2 = tmp;
-        tmp = d->tile_n;
-        d->tile_n = d->tile_n2;
-        d->tile_n2 = tmp;
-    }
-    zpic_ktimer_end(ZPIC_T_SORT);
-    d->cur = other;
+    return slack;
+}
+
+/* The species' particles are in the other set, sorted. */
+static void sort_done(struct zpic_dev_species *d, int slack)
+{
+    d->cur = 1 - d->cur;
     d->moved_since_sort = 0;
     d->steps_since_sort = 0;
     d->probe_ready = 0;
@@ -752,6 +730,70 @@ static void sort_now_from(t_species *s, int spread, int slack, const int *before
         d->counted = 1;
         d->n_slack = 0;
     }
+}
+
+/* Full re-sort of the tile ranges (plus a tail) of n species into their
+ * other buffer sets; with `slack` the new ranges keep free slots for the
+ * staged re-sorts that follow, sized by the growth since the counts
+ * `before` (NULL: those of each species' last sort). */
+static void resort(t_species *const *list, int n, int slack, const int *before)
+{
+    zk_resort_set m;
+    int got[ZK_FUSE_MAX];
+    memset(&m, 0, sizeof(m));
+    m.n = n;
+    for (int k = 0; k < n; k++) {
+        struct zpic_dev_species *d = list[k]->dev;
+        got[k] = sort_slack(d, slack);
+        zk_resort_args *a = &m.s[k];
+        a->src = d->set[d->cur];
+        a->dst = d->set[1 - d->cur];
+        a->ctr = d->ctr;
+        a->move = d->cnt;
+        a->stay = d->stay;
+        a->nbr = d->nbr;
+        a->tailn = d->tailn;
+        a->old_off = d->tile_off;
+        a->old_n = d->counted ? d->tile_n : NULL;
+        a->before = before ? before : a->old_n;
+        a->new_off = d->tile_off2;
+        a->new_n = d->tile_n2;
+        a->cursor = d->cursor;
+        a->t = d->t;
+        a->tail_upper = d->tail_upper;
+        a->slack = got[k];
+        a->cap_slots = d->cap;
+    }
+    zpic_ktimer_begin(ZPIC_T_SORT);
+    ZCHECK(zk_sort_tiles(&m, zpic_phase_stamp(ZPIC_T_SPEC), zpic_stream()));
+    zpic_ktimer_end(ZPIC_T_SORT);
+    for (int k = 0; k < n; k++) {
+        struct zpic_dev_species *d = list[k]->dev;
+        int *tmp = d->tile_off;
+        d->tile_off = d->tile_off2;
+        d->tile_off2 = tmp;
+        tmp = d->tile_n;
+        d->tile_n = d->tile_n2;
+        d->tile_n2 = tmp;
+        sort_done(d, got[k]);
+    }
+}
+
+/* Sort of one species: `spread` for an unsorted upload (counting sort with
+ * cell interleaving), else the re-sort. */
+static void sort_now(t_species *s, int spread, int slack)
+{
+    struct zpic_dev_species *d = s->dev;
+    if (!spread) {
+        resort(&s, 1, slack, NULL);
+        return;
+    }
+    slack = sort_slack(d, slack);
+    zpic_ktimer_begin(ZPIC_T_SORT);
+    ZCHECK(zk_sort(&d->set[d->cur], &d->set[1 - d->cur], d->ctr, d->cnt, d->tile_off, d->cursor, d->tile_n, &d->t,
+                   d->np_upper, spread, slack, d->cap, zpic_stream()));
+    zpic_ktimer_end(ZPIC_T_SORT);
+    sort_done(d, slack);
 }
 
 /* Whether the push of this step may sort (staged re-sort): the fixed-point
@@ -778,7 +820,7 @@ static void resort_staged(t_species *s)
         g_staged[1]++;
         /* sized by the growth since the sort before the staged one (the
          * counts the staged re-sort left in sstay) */
-        sort_now_from(s, 0, 1, d->sstay);
+        resort(&s, 1, 1, d->sstay);
     }
 }
 
@@ -1302,14 +1344,17 @@ void zpic_spec_advance_all(t_species *spec, int n, t_emf *emf, t_current *cur)
             for (int k = 0; k < n; k++)
                 if (staged[k]) resort_staged(&spec[k]);
             for (int k = 0; k < n; k++) push_done(&spec[k], move[k], m.s[k].global_blocks, cur->dev);
+            t_species *list[ZK_FUSE_MAX];
+            int nl = 0;
             for (int k = 0; k < n; k++) {
                 if (staged[k]) {
                     spec[k].dev->moved_since_sort = 0;
                     spec[k].dev->steps_since_sort = 0;
                 } else if (due[k]) {
-                    sort_now(&spec[k], 0, 1);
+                    list[nl++] = &spec[k];
                 }
             }
+            if (nl > 0) resort(list, nl, 1, NULL);
             for (int k = 0; k < n; k++) probe_prefetch(&spec[k]);
             for (int k = 0; k < n; k++) extra |= staged[k];
             zpic_phase_end(ZPIC_T_SPEC, extra);

@@ -143,25 +143,21 @@ __global__ void __launch_bounds__(256) yee_batch(const zk_bsim *sims, const int 
 /* The re-sort of the single-simulation path (zk_sort_tiles: stayers in
  * order, movers by neighbour slot), one workgroup per (species, tile)
  * item; batch members have no unsorted tail (no moving window). */
-__global__ void snapshot_batch(const zk_bspec *specs)
-{
-    const zk_bspec &S = specs[blockIdx.x];
-    if (sorts_now(S)) S.offs[S.ocur][S.a.t.ntiles + 1] = S.a.ctr->np_total;
-}
-
 __global__ void __launch_bounds__(ZK_SORT_THREADS) count_batch(const zk_bspec *specs, const int *items)
 {
     const zk_bspec &S = specs[items[2 * blockIdx.x]];
     if (!sorts_now(S)) return;
     const zk_parts &p = S.set[S.pcur];
-    count_stay_body(p.cell, p.cbits, S.offs[S.ocur], nullptr, S.stay, S.cnt, S.nbr, S.tailn, S.a.t, items[2 * blockIdx.x + 1],
-                    S.a.t.ntiles);
+    count_stay_body(p.cell, p.cbits, S.offs[S.ocur], nullptr, &S.a.ctr->np_total, S.stay, S.cnt, S.nbr, S.tailn, S.a.t,
+                    items[2 * blockIdx.x + 1], S.a.t.ntiles);
 }
 
 __global__ void __launch_bounds__(1024) scan_batch(const zk_bspec *specs)
 {
     const zk_bspec &S = specs[blockIdx.x];
     if (!sorts_now(S)) return;
+    if (threadIdx.x == 0) S.offs[S.ocur][S.a.t.ntiles + 1] = S.a.ctr->np_total;
+    __syncthreads();
     scan_stay_body(S.stay, S.cnt, S.tailn, S.offs[1 - S.ocur], nullptr, S.cursor, S.a.ctr, S.a.t.ntiles, 0, 0);
 }
 
@@ -289,7 +285,6 @@ extern "C" int zk_batch_fields(const zk_bsim *sims, const int *yee_items, int ny
 extern "C" int zk_batch_sort(const zk_bspec *specs, int nspecs, const int *items, int n, zk_stream_t s)
 {
     if (nspecs <= 0) return 0;
-    hipLaunchKernelGGL(snapshot_batch, dim3(nspecs), dim3(1), 0, s, specs);
     LAUNCH_ITEMS(count_batch, n, specs, items);
     hipLaunchKernelGGL(scan_batch, dim3(nspecs), dim3(1024), 0, s, specs);
     LAUNCH_ITEMS(scatter_batch, n, specs, items);

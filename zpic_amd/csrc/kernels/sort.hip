@@ -54,25 +54,39 @@ __global__ void scatter_indirect(zk_parts src, zk_parts dst, const int *n_old, i
     scatter_body(src, dst, n_old, cursor, off, t, spread, blockIdx.x, gridDim.x, tile_n);
 }
 
-__global__ void __launch_bounds__(ZK_SORT_THREADS)
-    count_stay_kernel(const int *__restrict__ cell, int cbits, const int *old_off, const int *old_n, int *stay,
-                      int *move, int *nbr, int *tailn, zk_tiles t)
+/* The species of block b of a launch over all species of a set, and its
+ * block among theirs. */
+__device__ inline int sort_species(const zk_resort_set &m, int &b)
 {
-    count_stay_body(cell, cbits, old_off, old_n, stay, move, nbr, tailn, t, blockIdx.x, gridDim.x);
+    int k = 0;
+    while (k + 1 < m.n && b >= m.s[k].blocks) b -= m.s[k++].blocks;
+    return k;
 }
 
-__global__ void __launch_bounds__(1024) scan_stay_kernel(const int *stay, int *move, int *tailn, int *new_off,
-                                                         int *new_n, int *cursor, zk_spec_ctr *ctr, int ntiles,
-                                                         int slack, int cap_slots, const int *old_n)
+__global__ void __launch_bounds__(ZK_SORT_THREADS) count_stay_kernel(zk_resort_set m)
 {
-    scan_stay_body(stay, move, tailn, new_off, new_n, cursor, ctr, ntiles, slack, cap_slots, old_n);
+    int b = blockIdx.x;
+    const zk_resort_args &a = m.s[sort_species(m, b)];
+    count_stay_body(a.src.cell, a.src.cbits, a.old_off, a.old_n, &a.ctr->np_total, a.stay, a.move, a.nbr, a.tailn, a.t,
+                    b, a.blocks);
 }
 
-__global__ void __launch_bounds__(ZK_SORT_THREADS)
-    scatter_stay_kernel(zk_parts src, zk_parts dst, const int *old_off, const int *old_n, const int *new_off,
-                        const int *stay, const int *nbr, int *cursor, zk_tiles t, zk_stamp st)
+/* one block per species; keeps the slot count before the sort for the
+ * scatter that follows */
+__global__ void __launch_bounds__(1024) scan_stay_kernel(zk_resort_set m)
 {
-    scatter_stay_body(src, dst, old_off, old_n, new_off, stay, nbr, cursor, t, blockIdx.x, gridDim.x);
+    const zk_resort_args &a = m.s[blockIdx.x];
+    if (threadIdx.x == 0) a.old_off[a.t.ntiles + 1] = a.ctr->np_total;
+    __syncthreads();
+    scan_stay_body(a.stay, a.move, a.tailn, a.new_off, a.new_n, a.cursor, a.ctr, a.t.ntiles, a.slack, a.cap_slots,
+                   a.before);
+}
+
+__global__ void __launch_bounds__(ZK_SORT_THREADS) scatter_stay_kernel(zk_resort_set m, zk_stamp st)
+{
+    int b = blockIdx.x;
+    const zk_resort_args &a = m.s[sort_species(m, b)];
+    scatter_stay_body(a.src, a.dst, a.old_off, a.old_n, a.new_off, a.stay, a.nbr, a.cursor, a.t, b, a.blocks);
     zk_stamp_last(st);
 }
 
@@ -199,27 +213,32 @@ extern "C" int zk_sort(const zk_parts *src, const zk_parts *dst, zk_spec_ctr *ct
     ZK_LAUNCH_CHECK();
 }
 
-/* Sort of a tile-sorted input (ranges old_off, plus an unsorted tail of
- * at most tail_upper slots): one workgroup per source tile keeps the
- * particles that stay in their tile in order at the front of its new
- * range with coalesced writes; particles that changed tile (and the tail)
- * are appended to their new tile. */
-extern "C" int zk_sort_tiles(const zk_parts *src, const zk_parts *dst, zk_spec_ctr *ctr, int *move, int *stay,
-                             int *nbr, int *tailn, int *old_off, const int *old_n, const int *before,
-                             int *new_off, int *new_n, int *cursor, const zk_tiles *t, int tail_upper, int slack,
-                             int cap_slots, zk_stamp st, zk_stream_t s)
+/* Sort of tile-sorted inputs (ranges old_off, plus an unsorted tail of at
+ * most tail_upper slots): one workgroup per source tile keeps the particles
+ * that stay in their tile in order at the front of its new range with
+ * coalesced writes; particles that changed tile (and the tail) are appended
+ * to their new tile.  The species of a simulation are sorted by the same
+ * three launches: with four launches each (one to keep the slot count),
+ * two species took 43 us on a 32 x 32 grid, nearly all of it the launches'
+ * own time. */
+extern "C" int zk_sort_tiles(const zk_resort_set *m, zk_stamp st, zk_stream_t s)
 {
-    const unsigned tb = tail_upper > 0 ? grid_for(tail_upper, 1024, 4096) : 0;
-    const unsigned g = (unsigned)t->ntiles + tb;
-    hipLaunchKernelGGL(snapshot_kernel, dim3(1), dim3(1), 0, s, ctr, old_off + t->ntiles + 1);
-    hipLaunchKernelGGL(count_stay_kernel, dim3(g), dim3(ZK_SORT_THREADS), 0, s, src->cell, src->cbits, old_off, old_n,
-                       stay, move, nbr, tailn, *t);
-    hipLaunchKernelGGL(scan_stay_kernel, dim3(1), dim3(1024), 0, s, stay, move, tailn, new_off, new_n, cursor, ctr,
-                       t->ntiles, slack, cap_slots, before);
-    hipLaunchKernelGGL(scatter_stay_kernel, dim3(g), dim3(ZK_SORT_THREADS), 0, s, *src, *dst, old_off, old_n,
-                       new_off, stay, nbr, cursor, *t, st);
-    if (t->ntiles > 0 && new_n && slack)
-        hipLaunchKernelGGL(mark_free_kernel, dim3(t->ntiles), dim3(256), 0, s, dst->cell, new_off, new_n);
+    if (m->n < 1 || m->n > ZK_FUSE_MAX) return (int)hipErrorInvalidValue;
+    zk_resort_set r = *m;
+    unsigned g = 0;
+    for (int k = 0; k < r.n; k++) {
+        zk_resort_args &a = r.s[k];
+        a.blocks = a.t.ntiles + (a.tail_upper > 0 ? (int)grid_for(a.tail_upper, 1024, 4096) : 0);
+        g += (unsigned)a.blocks;
+    }
+    if (g > 0) hipLaunchKernelGGL(count_stay_kernel, dim3(g), dim3(ZK_SORT_THREADS), 0, s, r);
+    hipLaunchKernelGGL(scan_stay_kernel, dim3(r.n), dim3(1024), 0, s, r);
+    if (g > 0) hipLaunchKernelGGL(scatter_stay_kernel, dim3(g), dim3(ZK_SORT_THREADS), 0, s, r, st);
+    for (int k = 0; k < r.n; k++) {
+        const zk_resort_args &a = r.s[k];
+        if (a.t.ntiles > 0 && a.new_n && a.slack)
+            hipLaunchKernelGGL(mark_free_kernel, dim3(a.t.ntiles), dim3(256), 0, s, a.dst.cell, a.new_off, a.new_n);
+    }
     ZK_LAUNCH_CHECK();
 }
 

@@ -287,10 +287,11 @@ __device__ inline int range_end(const int *off, const int *n, int t) { return n 
  * tile b (stay[b], and per wave in nbr) and its movers per neighbour slot,
  * reserving their runs (nbr, move); farther movers count in tailn.  Blocks
  * beyond count chunks of the tail into tailn.  old_off[ntiles] is the end
- * of the tile ranges, old_off[ntiles + 1] the slot count in use. */
+ * of the tile ranges, *np_slots the slot count in use (old_off[ntiles + 1]
+ * for the scatter). */
 __device__ inline void count_stay_body(const int *__restrict__ cell, int cbits, const int *__restrict__ old_off,
-                                       const int *__restrict__ old_n, int *stay, int *move, int *nbr, int *tailn,
-                                       const zk_tiles &t, const int block, const int nblocks)
+                                       const int *__restrict__ old_n, const int *np_slots, int *stay, int *move,
+                                       int *nbr, int *tailn, const zk_tiles &t, const int block, const int nblocks)
 {
     __shared__ int lc[9], wst[ZK_SORT_THREADS / ZK_WAVE];
     const int lane = __lane_id();
@@ -333,7 +334,7 @@ __device__ inline void count_stay_body(const int *__restrict__ cell, int cbits, 
             nbr[ZK_NBR * block + threadIdx.x] = c ? atomicAdd(&move[nbr_tile(threadIdx.x, block, t)], c) : 0;
         }
     } else {
-        const int n0 = old_off[t.ntiles], n1 = old_off[t.ntiles + 1];
+        const int n0 = old_off[t.ntiles], n1 = *np_slots;
         const int stride = (nblocks - t.ntiles) * blockDim.x;
         for (int base = n0 + (block - t.ntiles) * blockDim.x; base < n1; base += stride) {
             const int i = base + threadIdx.x;

@@ -188,15 +188,27 @@ int zk_spec_finalize_set(const zk_finalize_set *f, zk_stream_t s);
 int zk_sort(const zk_parts *src, const zk_parts *dst, zk_spec_ctr *ctr,
                    int *cnt, int *off, int *cursor, int *tile_n, const zk_tiles *t,
                    int np_upper, int spread, int slack, int cap_slots, zk_stream_t s);
-/* re-sort of a tile-sorted input: old_off (ntiles + 2, the last entry
- * scratch) and old_n -> new_off (ntiles + 1) and new_n; `before` (or NULL)
- * the counts of the previous sort, whose growth sizes the free slots; move
- * and tailn (ntiles, zero on entry and exit), stay and cursor (ntiles),
- * nbr (13 ntiles) */
-int zk_sort_tiles(const zk_parts *src, const zk_parts *dst, zk_spec_ctr *ctr, int *move, int *stay, int *nbr,
-                  int *tailn, int *old_off, const int *old_n, const int *before, int *new_off, int *new_n,
-                  int *cursor, const zk_tiles *t, int tail_upper, int slack, int cap_slots, zk_stamp st,
-                  zk_stream_t s);
+/* Re-sort of the tile-sorted sets of n species of one simulation in three
+ * launches: old_off (ntiles + 2, the last entry receives the slot count
+ * before the sort) and old_n -> new_off (ntiles + 1) and new_n; `before` (or
+ * NULL) the counts of the previous sort, whose growth sizes the free slots;
+ * move and tailn (ntiles, zero on entry and exit), stay and cursor
+ * (ntiles), nbr (13 ntiles); at most tail_upper slots of unsorted tail */
+typedef struct zk_resort_args {
+    zk_parts src, dst;
+    zk_spec_ctr *ctr;
+    int *move, *stay, *nbr, *tailn, *old_off;
+    const int *old_n, *before;
+    int *new_off, *new_n, *cursor;
+    zk_tiles t;
+    int tail_upper, slack, cap_slots;
+    int blocks;                 /* set by zk_sort_tiles */
+} zk_resort_args;
+typedef struct zk_resort_set {
+    zk_resort_args s[ZK_FUSE_MAX];
+    int n;
+} zk_resort_set;
+int zk_sort_tiles(const zk_resort_set *m, zk_stamp st, zk_stream_t s);
 /* Second half of a staged re-sort, after a push with `sorting` set: the
  * staged leavers of every tile (sleave[t] of them in the staging region of
  * dst) go to the free slots of their new tile's range behind its sstay[t]
