@@ -53,14 +53,12 @@ struct zpic_diff {
     int **pos;
     float *lE, *lB, *lJ, *aE, *aB, *Lam, *region;
     int splits;        /* workgroups per tile in the reverse push */
-    unsigned *amax;    /* [ns] running maxima of the gathered-field adjoints (float bits) */
+    size_t nmax;
+    unsigned *amax;    /* [nmax] running maxima of the gathered-field adjoints per window slot (float bits) */
     float *out;        /* device staging of one species' adjoints by id */
     int forward_done;
     int iter0;
 };
-
-/* workgroups the reverse push aims for (tiles times splits) */
-#define ZPIC_ADJ_BLOCKS 1024
 
 #define CS(D, c, k) (&(D)->cs[(size_t)(c) * (D)->ns + (k)])
 
@@ -159,6 +157,26 @@ static void records_free(zpic_diff *D)
 /* record slot of step n of the segment starting at s0 */
 static int rslot(const zpic_diff *D, int n, int s0) { return D->record ? n : n - s0; }
 
+/* Workgroups per tile of the reverse push: the number, up to 8, at which the
+ * launch takes the least time when every workgroup holds its place for the
+ * same time, the share of its tile plus the staging of its windows, and the
+ * GPU takes ZK_ADJ_RESIDENT at once.  The staging is put at a sixteenth of a
+ * whole tile (16 passes over 256 particles in 4096, about one pass's time). */
+static int adj_splits(int items)
+{
+    int best = 1;
+    double tbest = 0.0;
+    for (int s = 1; s <= 8 && items > 0; s++) {
+        const double rounds = (double)(((long long)items * s + ZK_ADJ_RESIDENT - 1) / ZK_ADJ_RESIDENT);
+        const double t = rounds * (1.0 / s + 1.0 / 16.0);
+        if (s == 1 || t < tbest) {
+            best = s;
+            tbest = t;
+        }
+    }
+    return best;
+}
+
 zpic_diff *zpic_diff_new(t_simulation *sim, int nsteps, int ckpt, int loss_first, int loss_last)
 {
     if (!sim || !sim->emf.dev) zpic_fatal("zpic_diff_new: simulation was not created with sim_new");
@@ -231,11 +249,12 @@ zpic_diff *zpic_diff_new(t_simulation *sim, int nsteps, int ckpt, int loss_first
     D->aE = zpic_dmalloc(gb);
     D->aB = zpic_dmalloc(gb);
     D->Lam = zpic_dmalloc(gb);
-    /* enough workgroups to fill the GPU on small grids (a few per CU) */
-    D->splits = t->ntiles > 0 ? (ZPIC_ADJ_BLOCKS + t->ntiles - 1) / t->ntiles : 1;
-    if (D->splits > 8) D->splits = 8;
-    D->region = zpic_dmalloc(sizeof(float) * 6 * (size_t)t->WX * t->WY * t->ntiles * D->splits);
-    D->amax = zpic_dmalloc(sizeof(unsigned) * (size_t)(D->ns > 0 ? D->ns : 1));
+    const int nset = D->ns < ZK_FUSE_MAX ? D->ns : ZK_FUSE_MAX; /* species of one launch */
+    D->splits = adj_splits(nset * t->ntiles);
+    const size_t slots = (size_t)t->ntiles * D->splits;
+    D->region = zpic_dmalloc(sizeof(float) * 6 * (size_t)t->WX * t->WY * slots * (nset > 0 ? nset : 1));
+    D->nmax = slots * (D->ns > 0 ? D->ns : 1);
+    D->amax = zpic_dmalloc(sizeof(unsigned) * D->nmax);
     D->out = zpic_dmalloc(sizeof(float) * 5 * (size_t)npmax);
     return D;
 }
@@ -383,7 +402,7 @@ void zpic_diff_backward(zpic_diff *D, float *dE, float *dB, float *const *dpart)
     ZCHECK(zk_fill_f32(D->lE, 3 * D->nodes, 0.0f, st));
     ZCHECK(zk_fill_f32(D->lB, 3 * D->nodes, 0.0f, st));
     for (int k = 0; k < D->ns; k++) vec_zero(&D->lam[k], D->np[k]);
-    ZCHECK(zk_fill_f32((float *)D->amax, (size_t)(D->ns > 0 ? D->ns : 1), 0.0f, st));
+    ZCHECK(zk_fill_f32((float *)D->amax, D->nmax, 0.0f, st));
 
     for (int c = D->nck - 1; c >= 0; c--) {
         const int s0 = c * D->ckpt, s1 = (s0 + D->ckpt < D->nsteps) ? s0 + D->ckpt : D->nsteps;
@@ -413,34 +432,40 @@ void zpic_diff_backward(zpic_diff *D, float *dE, float *dB, float *const *dpart)
             ZCHECK(zk_adj_fields(D->lE, D->lB, D->lJ, D->aE, D->aB, nx, ny, nrow, sim->dt, emf->dx[0], emf->dx[1],
                                  st));
             ZCHECK(zk_adj_images(D->lJ, D->Lam, nx, ny, nrow, st));
-            for (int k = 0; k < D->ns; k++) {
-                t_species *s = &sim->species[k];
-                struct zpic_dev_species *d = s->dev;
+            for (int k0 = 0; k0 < D->ns; k0 += ZK_FUSE_MAX) {
                 zk_adj_push_args a;
                 memset(&a, 0, sizeof(a));
-                a.p = D->rp[(size_t)r * D->ns + k];
-                a.tile_off = CS(D, c, k)->tile_off;
+                a.ns = D->ns - k0 < ZK_FUSE_MAX ? D->ns - k0 : ZK_FUSE_MAX;
                 a.E = D->rE[r];
                 a.B = D->rB[r];
                 a.lam = D->Lam;
                 a.nrow = nrow;
-                a.lin = D->lam[k];
-                a.lout = D->lam2[k];
-                a.amax = D->amax + k;
                 a.region = D->region;
                 a.lE = D->lE;
                 a.lB = D->lB;
-                a.t = d->t;
-                a.ovf_list = d->ovf_list;
+                a.t = sim->current.dev->t;
                 a.splits = D->splits;
-                /* the push constants of spec_advance */
-                a.tem = 0.5 * s->dt / s->m_q;
-                a.dt_dx = s->dt / s->dx[0];
-                a.dt_dy = s->dt / s->dx[1];
-                a.qnx = s->q * s->dx[0] / s->dt;
-                a.qny = s->q * s->dx[1] / s->dt;
-                a.q = s->q;
+                a.amax = D->amax + (size_t)k0 * a.t.ntiles * D->splits;
+                for (int i = 0; i < a.ns; i++) {
+                    const int k = k0 + i;
+                    const t_species *s = &sim->species[k];
+                    zk_adj_spec *o = &a.s[i];
+                    o->p = D->rp[(size_t)r * D->ns + k];
+                    o->tile_off = CS(D, c, k)->tile_off;
+                    o->lin = D->lam[k];
+                    o->lout = D->lam2[k];
+                    o->ovf_list = s->dev->ovf_list;
+                    /* the push constants of spec_advance */
+                    o->tem = 0.5 * s->dt / s->m_q;
+                    o->dt_dx = s->dt / s->dx[0];
+                    o->dt_dy = s->dt / s->dx[1];
+                    o->qnx = s->q * s->dx[0] / s->dt;
+                    o->qny = s->q * s->dx[1] / s->dt;
+                    o->q = s->q;
+                }
                 ZCHECK(zk_adj_push(&a, st));
+            }
+            for (int k = 0; k < D->ns; k++) {
                 const zk_adj_vec tmp = D->lam[k];
                 D->lam[k] = D->lam2[k];
                 D->lam2[k] = tmp;

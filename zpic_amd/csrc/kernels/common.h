@@ -64,6 +64,41 @@ __device__ inline int zk_cell_ix(int c, int cbits) { return c < 0 ? ZK_DEAD : (c
 __device__ inline int zk_cell_iy(int c, int cbits) { return c >> cbits; }
 __device__ inline int zk_cell(int ix, int iy, int cbits) { return ix == ZK_DEAD ? -1 : (ix | (iy << cbits)); }
 
+/* Correctly rounded reciprocal, division and square root for the Boris
+ * push, whose divisors and square-root arguments are at least 1: hardware
+ * estimates refined by fused multiply-adds, without the operand scaling and
+ * special-value fix-ups that only denormal, infinite, zero or
+ * extreme-exponent operands need.
+ *
+ * On gfx950 one Newton step of the reciprocal estimate gives the correctly
+ * rounded 1 / b for every float b in [1, 2^126), and one residual step on
+ * x rsq(x) the correctly rounded square root for every x in [1, 2^127)
+ * (checked for all of them, tests/test_gpu_rounding.py).  With y = 1 / b
+ * correctly rounded, q = a y is within 1.5 units of the quotient, one
+ * residual step makes it a faithful rounding, and one more the correctly
+ * rounded quotient (Markstein's theorem).  The shorter sequences take 19
+ * of the push's 420 issue slots per particle. */
+__device__ inline float rcp_ge1(float b)
+{
+    const float y = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+
+__device__ inline float div_ge1(float a, float b)
+{
+    const float y = rcp_ge1(b);
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+
+__device__ inline float sqrt_ge1(float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+}
+
 /* Clock readings of a timed phase (zk_clock): zk_stamp_first at the start of
  * a launch, zk_stamp_last at its end; every thread may call them. */
 __device__ inline void zk_stamp_first(const zk_stamp &s)

@@ -422,41 +422,6 @@ __device__ inline void store_slot(const zk_parts &P, int i, const Slot &c)
 /* registers whose contents do not matter, without an instruction to set them */
 __device__ inline void any_value(float &a, float &b, float &c) { asm volatile("" : "=v"(a), "=v"(b), "=v"(c)); }
 
-/* Correctly rounded reciprocal, division and square root for the Boris
- * push, whose divisors and square-root arguments are at least 1: hardware
- * estimates refined by fused multiply-adds, without the operand scaling and
- * special-value fix-ups that only denormal, infinite, zero or
- * extreme-exponent operands need.
- *
- * On gfx950 one Newton step of the reciprocal estimate gives the correctly
- * rounded 1 / b for every float b in [1, 2^126), and one residual step on
- * x rsq(x) the correctly rounded square root for every x in [1, 2^127)
- * (checked for all of them, tests/test_gpu_rounding.py).  With y = 1 / b
- * correctly rounded, q = a y is within 1.5 units of the quotient, one
- * residual step makes it a faithful rounding, and one more the correctly
- * rounded quotient (Markstein's theorem).  The shorter sequences take 19
- * of the push's 420 issue slots per particle. */
-__device__ inline float rcp_ge1(float b)
-{
-    const float y = __builtin_amdgcn_rcpf(b);
-    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-}
-
-__device__ inline float div_ge1(float a, float b)
-{
-    const float y = rcp_ge1(b);
-    float q = a * y;
-    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
-    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
-}
-
-__device__ inline float sqrt_ge1(float x)
-{
-    const float y = __builtin_amdgcn_rsqf(x);
-    const float s = x * y;
-    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
-}
-
 /* Motion of one particle whose cell is (ci, cj) in the sources' index
  * space: gather, Boris push, displacement (mx, my) and q v_z; returns the
  * time-centred kinetic energy term (em2d/particles.c:1125-1228). */

@@ -20,23 +20,28 @@ typedef struct zk_adj_vec {
     float *lx, *ly, *lux, *luy, *luz;
 } zk_adj_vec;
 
-typedef struct zk_adj_push_args {
+typedef struct zk_adj_spec {
     zk_parts p;                 /* particle state at the start of the step (read) */
     const int *tile_off;        /* [ntiles + 1] tile ranges of p */
+    zk_adj_vec lin;             /* particle adjoints after the step (read) */
+    zk_adj_vec lout;            /* particle adjoints before the step (written) */
+    int *ovf_list;              /* slots outside their tile window, listed at the start
+                                   of the listing workgroup's share of the tile range */
+    float tem, dt_dx, dt_dy, qnx, qny, q;
+} zk_adj_spec;
+
+typedef struct zk_adj_push_args {
+    zk_adj_spec s[ZK_FUSE_MAX];
+    int ns;                     /* species (1 to ZK_FUSE_MAX) */
     const float *E, *B;         /* fields at the start of the step */
     const float *lam;           /* adjoint of the raw current, per buffer node */
     int nrow;
-    zk_adj_vec lin;             /* particle adjoints after the step (read) */
-    zk_adj_vec lout;            /* particle adjoints before the step (written) */
-    float *region;              /* [ntiles * splits][6][WY][WX] field-adjoint windows */
+    float *region;              /* [ns * ntiles * splits][6][WY][WX] field-adjoint windows */
     float *lE, *lB;             /* field adjoints (accumulated) */
     zk_tiles t;
-    int *ovf_list;              /* slots outside their tile window, listed at the start
-                                   of the listing workgroup's share of the tile range */
     int splits;                 /* workgroups per tile (>= 1) */
-    unsigned *amax;             /* float bits: running maximum of the gathered-field
-                                   adjoints of this species (0 at the start) */
-    float tem, dt_dx, dt_dy, qnx, qny, q;
+    unsigned *amax;             /* [ns * ntiles * splits] float bits: running maximum of the
+                                   gathered-field adjoints of a window slot (0 at the start) */
 } zk_adj_push_args;
 
 /* dst = src for the seven particle arrays (and ids when both have them) */
@@ -53,8 +58,10 @@ int zk_adj_fields(float *lE, float *lB, float *lJ, float *aE, float *aB, int nx,
 /* Reverse of the periodic current fold: lam(node) = sum of lJ over the
  * buffer nodes with the same periodic image */
 int zk_adj_images(const float *lJ, float *lam, int nx, int ny, int nrow, zk_stream_t s);
-/* Reverse of the particle push of one species (tile pass, global pass,
- * field-adjoint windows added into lE, lB) */
+/* Reverse of the particle push of a set of species (tile pass, listed
+ * particles, field-adjoint windows added into lE, lB) */
+/* workgroups of zk_adj_push that the GPU holds at once */
+#define ZK_ADJ_RESIDENT 768
 int zk_adj_push(const zk_adj_push_args *a, zk_stream_t s);
 /* dst[i] = src[pos[ids_dst[i]]] with pos[ids_src[k]] = k: particle
  * adjoints carried from one particle order to another */
