@@ -15,11 +15,6 @@
 
 #include "zpic_zdf.h"
 
-/* 0: one launch per filter pass (for comparisons) */
-#ifndef ZPIC_SMOOTH_X_FUSE
-#define ZPIC_SMOOTH_X_FUSE 1
-#endif
-
 void current_new(t_current *c, int nx[], float box[], float dt)
 {
     /* em2d/current.c:30-79 */
@@ -241,30 +236,14 @@ void current_update(t_current *c)
     int axis[maxp];
     float sa[maxp], sb[maxp];
     const int np = zpic_current_passes(c, axis, sa, sb, maxp);
-    if (ZPIC_SMOOTH_X_FUSE && np == 2 && axis[0] == 0 && axis[1] == 1 && !d->open_y) {
-        /* one x and one y pass: one launch */
-        ZCHECK(zk_smooth_xy(d->J[d->jcur], d->J[1 - d->jcur], c->nx[0], c->nx[1], c->nrow, sa[0], sb[0], sa[1], sb[1],
-                            !c->moving_window, zpic_stream()));
-        d->jcur = 1 - d->jcur;
-        zpic_ktimer_end(ZPIC_T_CURRENT);
-        c->iter++;
-        d->host_valid = 0;
-        return;
-    }
     for (int k = 0; k < np;) {
-        /* consecutive x passes run in one launch */
-        int run = 1;
-        while (ZPIC_SMOOTH_X_FUSE && k + run < np && run < ZK_MAX_PASSES && axis[k] == 0 && axis[k + run] == 0)
-            run++;
-        if (axis[k] == 0 && run > 1) {
-            ZCHECK(zk_smooth_x_passes(d->J[d->jcur], d->J[1 - d->jcur], c->nx[0], c->nx[1], c->nrow, run, sa + k,
-                                      sb + k, !c->moving_window, zpic_stream()));
-            k += run;
-        } else {
-            ZCHECK(zk_smooth(d->J[d->jcur], d->J[1 - d->jcur], c->nx[0], c->nx[1], c->nrow, axis[k], sa[k], sb[k],
-                             !c->moving_window, d->open_y, zpic_stream()));
-            k++;
-        }
+        /* x passes and the y passes behind them in one launch */
+        int n1 = 0, n2 = 0;
+        while (k + n1 < np && n1 < ZK_MAX_PASSES && axis[k + n1] == 0) n1++;
+        while (k + n1 + n2 < np && n2 < ZK_MAX_Y_PASSES && axis[k + n1 + n2] == 1) n2++;
+        ZCHECK(zk_smooth(d->J[d->jcur], d->J[1 - d->jcur], c->nx[0], c->nx[1], c->nrow, n1, n2, sa + k, sb + k,
+                         !c->moving_window, d->open_y, zpic_stream()));
+        k += n1 + n2;
         d->jcur = 1 - d->jcur;
     }
     zpic_ktimer_end(ZPIC_T_CURRENT);

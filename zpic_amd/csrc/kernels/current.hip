@@ -12,7 +12,7 @@
  * One thread per output node; contributions are summed in a fixed order,
  * so the result does not depend on scheduling.
  *
- * zk_smooth applies one [sa, sb, sa] pass along x or y with the guard
+ * zk_smooth applies [sa, sb, sa] passes along x and then y with the guard
  * handling of kernel_x / kernel_y (em2d/current.c:316-413).
  */
 #include "current_core.h"
@@ -47,118 +47,140 @@ __global__ void __launch_bounds__(256) reduce_kernel(zk_reduce_args a, int nbx, 
     }
 }
 
-__global__ void smooth_kernel(const float *__restrict__ in, float *__restrict__ out, int nx, int ny, int nrow,
-                              int axis, float sa, float sb, int periodic_x, int open_y)
-{
-    smooth_node(in, out, nx, ny, nrow, axis, sa, sb, periodic_x, blockIdx.x * blockDim.x + threadIdx.x, open_y);
-}
-
-__global__ void smooth_xy_kernel(const float *__restrict__ in, float *__restrict__ out, int nx, int ny, int nrow,
-                                 float sax, float sbx, float say, float sby, int periodic_x)
-{
-    smooth_xy_node(in, out, nx, ny, nrow, sax, sbx, say, sby, periodic_x, blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-/* Consecutive x passes in one launch: a block stages SX_R buffer rows of
- * SX_W output columns plus npass columns on each side in LDS and applies
- * every pass there (the valid region shrinks by one column per pass), with
- * the arithmetic and guard handling of kernel_x (em2d/current.c:316-354)
- * pass after pass: interior rows only; with periodic x every column is the
- * image of an interior one (the reference refreshes the guards from their
- * images after each pass); with a moving window the guard columns keep
- * their values.  Bit-identical to the single-pass launches. */
-constexpr int SX_W = 256, SX_R = 4, SX_MAXP = ZK_MAX_PASSES;
-
+/* Filter passes of one launch: n1 along x, then n2 along y. */
 struct SmoothPasses {
-    float sa[SX_MAXP], sb[SX_MAXP];
-    int n;
+    float sa[ZK_MAX_PASSES + ZK_MAX_Y_PASSES], sb[ZK_MAX_PASSES + ZK_MAX_Y_PASSES];
+    int n1, n2;
 };
 
-__global__ void __launch_bounds__(256) smooth_x_passes_kernel(const float *__restrict__ in, float *__restrict__ out,
-                                                              int nx, int ny, int nrow, SmoothPasses ps,
-                                                              int periodic_x)
+__device__ inline float lane_below(float v)
 {
-    extern __shared__ float sx[];
-    const int P = ps.n, W = SX_W + 2 * P;
-    float *bufA = sx, *bufB = sx + 3 * SX_R * W;
-    const int bw = nx + 3, bh = ny + 3;
-    const int c0 = blockIdx.x * SX_W, r0 = blockIdx.y * SX_R;
-    /* stage: local column m <-> buffer column c0 - P + m, raw i = that - 1 */
-    for (int e = threadIdx.x; e < SX_R * W; e += blockDim.x) {
-        const int r = e / W, m = e % W;
-        const int bj = r0 + r, b = c0 - P + m;
-        float v0 = 0.0f, v1 = 0.0f, v2 = 0.0f;
-        if (bj < bh) {
-            const int j = bj - 1;
-            const bool interior_row = j >= 0 && j < ny;
-            int src = b;
-            if (interior_row && periodic_x) src = zk_wrap(b - 1, nx) + 1;
-            if (src >= 0 && src < bw) {
-                const float *q = in + 3 * ((size_t)src + (size_t)bj * nrow);
-                v0 = q[0];
-                v1 = q[1];
-                v2 = q[2];
-            }
-        }
-        float *d = bufA + 3 * e;
-        d[0] = v0;
-        d[1] = v1;
-        d[2] = v2;
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138 /* wave_shr:1 */, 0xf, 0xf, true));
+}
+
+__device__ inline float lane_above(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
+}
+
+/* All filter passes of a step (kernel_x and kernel_y passes,
+ * em2d/current.c:316-459) in one launch and in registers: a wave holds ROWS
+ * rows of 64 columns, a column per lane, and applies the x passes with lane
+ * shifts and the y passes along the rows.  Every pass spends one column or
+ * row of margin on each side, so 64 - 2 n1 columns and ROWS - 2 n2 rows are
+ * written.
+ *
+ * The passes are a few operations on J, which the caches hold on all but the
+ * largest grids: what they cost is launches and, inside one, waiting; the
+ * lane shifts need neither LDS nor barriers.  97 x 61 cells, 3 x and 3 y
+ * passes: 5.1 us, where x passes in LDS and a launch per y pass took 19.3;
+ * 1500 x 128, 5 x passes: 4.4 us instead of 15.4; 2048 x 2048, one of each:
+ * 24.7 us for 100 MB.
+ *
+ * The arithmetic and guard handling are those of the passes one after the
+ * other, so J is the same bit for bit.  x passes filter interior rows only,
+ * and there every column of a periodic axis is the image of an interior one;
+ * with a moving window the guard columns keep their values.  y passes filter
+ * interior columns only; on a periodic axis every row is the image of an
+ * interior one, except that the first y pass reads the guard rows -1 and ny
+ * as the x passes left them, unfiltered; with open y boundaries the guard
+ * rows keep their values. */
+template <int ROWS>
+__global__ void __launch_bounds__(64) smooth_kernel(const float *__restrict__ in, float *__restrict__ out, int nx,
+                                                    int ny, int nrow, SmoothPasses ps, int periodic_x, int open_y)
+{
+    const int lane = threadIdx.x;
+    const int n1 = ps.n1, n2 = ps.n2;
+    const bool ring = !open_y && n2 > 0; /* rows are images of interior rows */
+    const int b = (int)blockIdx.x * (64 - 2 * n1) - n1 + lane, i = b - 1;
+    const int r0 = (int)blockIdx.y * (ROWS - 2 * n2); /* first output buffer row */
+    const int jt = r0 - 1 - n2;                       /* raw row of v[0] */
+    const int c0 = ring ? zk_wrap(jt, ny) : jt;       /* and its image */
+    const bool in_x = i >= 0 && i < nx;
+    const bool col = b >= 0 && b < nx + 3;
+    const int bi = periodic_x ? zk_wrap(i, nx) + 1 : b;
+    float v[ROWS][3];
+#pragma unroll
+    for (int r = 0, c = c0; r < ROWS; r++, c = ring && c + 1 == ny ? 0 : c + 1) {
+        const bool inner = c >= 0 && c < ny;
+        const bool ok = inner ? periodic_x || col : c >= -1 && c <= ny + 1 && col;
+        const float *q = in + (ok ? 3 * ((size_t)(inner ? bi : b) + (size_t)(c + 1) * nrow) : 0);
+        v[r][0] = ok ? q[0] : 0.0f;
+        v[r][1] = ok ? q[1] : 0.0f;
+        v[r][2] = ok ? q[2] : 0.0f;
     }
-    __syncthreads();
-    float *cur = bufA, *nxt = bufB;
-    for (int p = 0; p < P; p++) {
+    /* the guard rows the first y pass reads, if it reaches the seam */
+    float lo[3] = {0.0f, 0.0f, 0.0f}, up[3] = {0.0f, 0.0f, 0.0f};
+    const bool seam = ring && (c0 == 0 || c0 + ROWS >= ny);
+    if (seam && in_x) {
+        const float *q = in + 3 * (size_t)b, *w = in + 3 * ((size_t)b + (size_t)(ny + 1) * nrow);
+        for (int c = 0; c < 3; c++) {
+            lo[c] = q[c];
+            up[c] = w[c];
+        }
+    }
+    for (int p = 0; p < n1; p++) {
         const float sa = ps.sa[p], sb = ps.sb[p];
-        for (int e = threadIdx.x; e < SX_R * W; e += blockDim.x) {
-            const int r = e / W, m = e % W;
-            const int bj = r0 + r, b = c0 - P + m;
-            const int j = bj - 1, i = b - 1;
-            const bool interior_row = j >= 0 && j < ny;
-            const bool live = interior_row && (periodic_x || (i >= 0 && i < nx)) && m > 0 && m < W - 1;
-            const float *c = cur + 3 * e;
-            float *o = nxt + 3 * e;
-            if (live) {
-                stencil(sa, sb, c - 3, c, c + 3, o);
-            } else {
-                o[0] = c[0];
-                o[1] = c[1];
-                o[2] = c[2];
+        const bool live = periodic_x || in_x;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const float l[3] = {lane_below(v[r][0]), lane_below(v[r][1]), lane_below(v[r][2])};
+            const float u[3] = {lane_above(v[r][0]), lane_above(v[r][1]), lane_above(v[r][2])};
+            float o[3];
+            stencil(sa, sb, l, v[r], u, o);
+            const bool f = live && (ring || (jt + r >= 0 && jt + r < ny));
+#pragma unroll
+            for (int c = 0; c < 3; c++) v[r][c] = f ? o[c] : v[r][c];
+        }
+    }
+    for (int p = 0; p < n2; p++) {
+        const float sa = ps.sa[n1 + p], sb = ps.sb[n1 + p];
+        const bool guards = p == 0 && seam;
+        float below[3] = {v[0][0], v[0][1], v[0][2]};
+        int cr = c0;
+#pragma unroll
+        for (int r = 1; r < ROWS - 1; r++) {
+            cr = ring && cr + 1 == ny ? 0 : cr + 1;
+            float l[3] = {below[0], below[1], below[2]}, u[3] = {v[r + 1][0], v[r + 1][1], v[r + 1][2]};
+            if (guards) {
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    l[c] = cr == 0 ? lo[c] : l[c];
+                    u[c] = cr == ny - 1 ? up[c] : u[c];
+                }
+            }
+            float o[3];
+            stencil(sa, sb, l, v[r], u, o);
+            const bool f = in_x && (ring || (jt + r >= 0 && jt + r < ny));
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                below[c] = v[r][c];
+                v[r][c] = f ? o[c] : v[r][c];
             }
         }
-        __syncthreads();
-        float *t = cur;
-        cur = nxt;
-        nxt = t;
     }
-    for (int e = threadIdx.x; e < SX_R * SX_W; e += blockDim.x) {
-        const int r = e / SX_W, m = e % SX_W;
-        const int bj = r0 + r, b = c0 + m;
-        if (bj >= bh || b >= bw) continue;
-        const float *c = cur + 3 * (r * W + m + P);
+    if (lane < n1 || lane >= 64 - n1 || !col) return;
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        const int bj = jt + r + 1;
+        if (r < n2 || r >= ROWS - n2 || bj >= ny + 3) continue;
         float *o = out + 3 * ((size_t)b + (size_t)bj * nrow);
-        o[0] = c[0];
-        o[1] = c[1];
-        o[2] = c[2];
+        o[0] = v[r][0];
+        o[1] = v[r][1];
+        o[2] = v[r][2];
     }
+}
+
+template <int ROWS>
+void smooth_launch(const float *in, float *out, int nx, int ny, int nrow, const SmoothPasses &ps, int periodic_x,
+                   int open_y, hipStream_t s)
+{
+    const int w = 64 - 2 * ps.n1, h = ROWS - 2 * ps.n2;
+    hipLaunchKernelGGL(smooth_kernel<ROWS>, dim3((nx + 3 + w - 1) / w, (ny + 3 + h - 1) / h), dim3(64), 0, s, in, out,
+                       nx, ny, nrow, ps, periodic_x, open_y);
 }
 
 } // namespace
-
-extern "C" int zk_smooth_x_passes(const float *in, float *out, int nx, int ny, int nrow, int npass, const float *sa,
-                                  const float *sb, int periodic_x, zk_stream_t s)
-{
-    if (npass < 1 || npass > SX_MAXP) return (int)hipErrorInvalidValue;
-    SmoothPasses ps;
-    ps.n = npass;
-    for (int k = 0; k < npass; k++) {
-        ps.sa[k] = sa[k];
-        ps.sb[k] = sb[k];
-    }
-    const size_t lds = (size_t)2 * 3 * SX_R * (SX_W + 2 * npass) * sizeof(float);
-    dim3 grid((nx + 3 + SX_W - 1) / SX_W, (ny + 3 + SX_R - 1) / SX_R);
-    hipLaunchKernelGGL(smooth_x_passes_kernel, grid, dim3(256), lds, s, in, out, nx, ny, nrow, ps, periodic_x);
-    ZK_LAUNCH_CHECK();
-}
 
 extern "C" int zk_current_clears(const zk_tiles *t) { return reduce_span(*t) != 0; }
 
@@ -174,20 +196,28 @@ extern "C" int zk_current_reduce(const zk_reduce_args *a, zk_stream_t s)
     ZK_LAUNCH_CHECK();
 }
 
-extern "C" int zk_smooth(const float *in, float *out, int nx, int ny, int nrow, int axis, float sa, float sb,
-                                int periodic_x, int open_y, zk_stream_t s)
+extern "C" int zk_smooth(const float *in, float *out, int nx, int ny, int nrow, int n1, int n2, const float *sa,
+                         const float *sb, int periodic_x, int open_y, zk_stream_t s)
 {
-    const int nodes = (nx + 3) * (ny + 3);
-    hipLaunchKernelGGL(smooth_kernel, dim3((nodes + 255) / 256), dim3(256), 0, s, in, out, nx, ny, nrow, axis, sa, sb,
-                       periodic_x, open_y);
-    ZK_LAUNCH_CHECK();
-}
-
-extern "C" int zk_smooth_xy(const float *in, float *out, int nx, int ny, int nrow, float sax, float sbx, float say,
-                            float sby, int periodic_x, zk_stream_t s)
-{
-    const int nodes = (nx + 3) * (ny + 3);
-    hipLaunchKernelGGL(smooth_xy_kernel, dim3((nodes + 255) / 256), dim3(256), 0, s, in, out, nx, ny, nrow, sax, sbx,
-                       say, sby, periodic_x);
+    if (n1 < 0 || n2 < 0 || n1 > ZK_MAX_PASSES || n2 > ZK_MAX_Y_PASSES || n1 + n2 < 1)
+        return (int)hipErrorInvalidValue;
+    SmoothPasses ps;
+    ps.n1 = n1;
+    ps.n2 = n2;
+    for (int k = 0; k < n1 + n2; k++) {
+        ps.sa[k] = sa[k];
+        ps.sb[k] = sb[k];
+    }
+    /* the fewest rows a wave that leave at least `least` to write: a wave's
+     * time grows with its rows, so two where the GPU has waves to spare (97 x
+     * 61 cells, 3 y passes: 5.1 us with 8 rows, 9.2 with 16), four where the
+     * rows of the margin are read and filtered in time that other waves could
+     * use (from about 2500 waves on) */
+    const int least = (size_t)(nx + 3) * (ny + 3) < (1u << 18) ? 2 : 4;
+    const int rows = 2 * n2 + least;
+    if (rows <= 4) smooth_launch<4>(in, out, nx, ny, nrow, ps, periodic_x, open_y, s);
+    else if (rows <= 8) smooth_launch<8>(in, out, nx, ny, nrow, ps, periodic_x, open_y, s);
+    else if (rows <= 16) smooth_launch<16>(in, out, nx, ny, nrow, ps, periodic_x, open_y, s);
+    else smooth_launch<32>(in, out, nx, ny, nrow, ps, periodic_x, open_y, s);
     ZK_LAUNCH_CHECK();
 }

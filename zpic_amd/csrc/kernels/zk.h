@@ -248,16 +248,12 @@ typedef struct zk_reduce_args {
 /* whether the reduction of this tiling clears Jov_next (and reads flags) */
 int zk_current_clears(const zk_tiles *t);
 int zk_current_reduce(const zk_reduce_args *a, zk_stream_t s);
-int zk_smooth(const float *in, float *out, int nx, int ny, int nrow, int axis,
-                     float sa, float sb, int periodic_x, int open_y, zk_stream_t s);
-/* npass (<= ZK_MAX_PASSES) consecutive x passes in one launch, bit-identical
- * to npass zk_smooth launches along x */
-/* one x pass, then one y pass with periodic y, in one launch (the same
- * values as two zk_smooth launches) */
-int zk_smooth_xy(const float *in, float *out, int nx, int ny, int nrow, float sax, float sbx, float say, float sby,
-                 int periodic_x, zk_stream_t s);
-int zk_smooth_x_passes(const float *in, float *out, int nx, int ny, int nrow, int npass, const float *sa,
-                       const float *sb, int periodic_x, zk_stream_t s);
+/* n1 (<= ZK_MAX_PASSES) filter passes along x, then n2 (<= ZK_MAX_Y_PASSES)
+ * along y; sa and sb hold the weights of the n1 + n2 passes in that order */
+#define ZK_MAX_PASSES 16
+#define ZK_MAX_Y_PASSES 12
+int zk_smooth(const float *in, float *out, int nx, int ny, int nrow, int n1, int n2, const float *sa, const float *sb,
+              int periodic_x, int open_y, zk_stream_t s);
 
 /* fields */
 /* One field step, guard cells of the outputs included (periodic_x: along
@@ -378,7 +374,6 @@ int zk_init_rng_emit(const zk_init_args *a, long long nat, int per, const int *t
 int zk_init_mean(const zk_init_args *a, float *mean, int nkeys, zk_stream_t s);
 
 /* ---- batches of independent simulations (batch.hip) ---- */
-#define ZK_MAX_PASSES 16
 
 /* Yee constants: (dt/2)/dx, (dt/2)/dy, dt/dx, dt/dy, dt, and the Mur
  * coefficient (dt - dy)/(dt + dy) of open y boundaries */
