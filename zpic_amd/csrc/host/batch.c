@@ -271,7 +271,7 @@ static void build_items(zpic_batch *b, table *T)
     GRID_PHASE(b->fill, zk_red_blocks_x(M->nx) * zk_red_blocks_y(M->ny));
     GRID_PHASE(b->fold, zk_batch_reduce_blocks(M));
     GRID_PHASE(b->node, blocks_of((size_t)(M->nx + 3) * (M->ny + 3), 256));
-    GRID_PHASE(b->yee, ((M->nx + 3 + ZK_YEE_BX - 1) / ZK_YEE_BX) * ((M->ny + 3 + ZK_YEE_BY - 1) / ZK_YEE_BY));
+    GRID_PHASE(b->yee, (zk_yee_units(M->nx, M->ny, ZK_YEE_R) + 3) / 4);
 #undef GRID_PHASE
 
     /* particle phases: species by particles per tile (the tile pass) or

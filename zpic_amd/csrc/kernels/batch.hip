@@ -135,9 +135,10 @@ __global__ void __launch_bounds__(256) yee_batch(const zk_bsim *sims, const int 
 {
     const int s = items[2 * blockIdx.x], t = items[2 * blockIdx.x + 1];
     const zk_bsim &M = sims[s];
-    const int ntx = (M.nx + 3 + BX - 1) / BX;
-    yee_tile(M.E[M.ecur], M.B[M.ecur], j_after(M, M.npass), M.E[1 - M.ecur], M.B[1 - M.ecur], M.nx, M.ny, M.nrow,
-             M.yk, t % ntx, t / ntx, 1);
+    const int u = 4 * t + (int)(threadIdx.x / 64);
+    if (u >= zk_yee_units(M.nx, M.ny, ZK_YEE_R)) return;
+    yee_rows<ZK_YEE_R>(M.E[M.ecur], M.B[M.ecur], j_after(M, M.npass), M.E[1 - M.ecur], M.B[1 - M.ecur], M.nx, M.ny,
+                       M.nrow, M.yk, u, 1);
 }
 
 /* The re-sort of the single-simulation path (zk_sort_tiles: stayers in

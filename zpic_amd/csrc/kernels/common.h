@@ -115,6 +115,17 @@ __device__ inline void zk_stamp_last(const zk_stamp &s)
     s.clk->t1[s.slot] = wall_clock64();
 }
 
+/* Value of the lane one below / above (0 past the ends of the wave). */
+__device__ inline float lane_below(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138 /* wave_shr:1 */, 0xf, 0xf, true));
+}
+
+__device__ inline float lane_above(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
+}
+
 /* Floor modulo for periodic wrap. */
 __device__ inline int zk_wrap(int i, int n)
 {

@@ -53,16 +53,6 @@ struct SmoothPasses {
     int n1, n2;
 };
 
-__device__ inline float lane_below(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138 /* wave_shr:1 */, 0xf, 0xf, true));
-}
-
-__device__ inline float lane_above(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
-}
-
 /* All filter passes of a step (kernel_x and kernel_y passes,
  * em2d/current.c:316-459) in one launch and in registers: a wave holds ROWS
  * rows of 64 columns, a column per lane, and applies the x passes with lane

@@ -31,13 +31,16 @@ static __device__ __align__(256) float scratch[2 * ZK_NOALLOC_CHARGE_MAX];
 
 namespace {
 
+template <int R>
 __global__ void __launch_bounds__(256) yee_kernel(const float *__restrict__ E, const float *__restrict__ B,
                                                   const float *__restrict__ J, float *__restrict__ Eo,
                                                   float *__restrict__ Bo, int nx, int ny, int nrow, YeeK k,
-                                                  int periodic_x, int open_y, int shift, zk_stamp st)
+                                                  int periodic_x, int open_y, int shift, int units, zk_stamp st)
 {
     zk_stamp_first(st);
-    yee_tile(E, B, J, Eo, Bo, nx, ny, nrow, k, blockIdx.x, blockIdx.y, periodic_x, open_y, shift);
+    /* contiguous runs of units per XCD: neighbours share their margins in L2 */
+    const int u = zk_xcd_item(blockIdx.x, gridDim.x) * (blockDim.x / 64) + threadIdx.x / 64;
+    if (u < units) yee_rows<R>(E, B, J, Eo, Bo, nx, ny, nrow, k, u, periodic_x, open_y, shift);
     zk_stamp_last(st);
 }
 
@@ -445,9 +448,13 @@ extern "C" int zk_yee(const float *E, const float *B, const float *J, float *Eo,
     k.dty = dt / dy;
     k.dt = dt;
     k.mur_y = (dt - dy) / (dt + dy);
-    dim3 grid((nx + 3 + BX - 1) / BX, (ny + 3 + BY - 1) / BY);
-    hipLaunchKernelGGL(yee_kernel, grid, dim3(256), 0, s, E, B, J, Eo, Bo, nx, ny, nrow, k, periodic_x,
-                       open_y, shift, st);
+    const int r = zk_yee_rows(nx, ny), units = zk_yee_units(nx, ny, r);
+    if (r == ZK_YEE_R_SMALL)
+        hipLaunchKernelGGL(yee_kernel<ZK_YEE_R_SMALL>, dim3(units), dim3(64), 0, s, E, B, J, Eo, Bo, nx, ny, nrow, k,
+                           periodic_x, open_y, shift, units, st);
+    else
+        hipLaunchKernelGGL(yee_kernel<ZK_YEE_R>, dim3((units + 3) / 4), dim3(256), 0, s, E, B, J, Eo, Bo, nx, ny, nrow,
+                           k, periodic_x, open_y, shift, units, st);
     ZK_LAUNCH_CHECK();
 }
 

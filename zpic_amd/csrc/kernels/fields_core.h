@@ -10,27 +10,8 @@
 namespace zk {
 
 
-constexpr int BX = ZK_YEE_BX, BY = ZK_YEE_BY; /* output nodes per tile */
-/* rows staged below the first output row: two, so that the whole step of E
- * is known one row below the outputs (the upper Mur boundary needs it) */
-constexpr int OY = 2;
-constexpr int LX = BX + 3, LY = BY + OY + 2;
-
 typedef zk_yee_k YeeK; /* (dt/2)/dx, (dt/2)/dy, dt/dx, dt/dy, dt, Mur coefficient along y */
 
-/* One BX x BY tile of output nodes, tile (tx, ty) of the buffer.  The
- * half and whole steps update the staged B and E in place: a node's new
- * value depends on its own old value and on neighbours of the other field,
- * which the previous step finished before the barrier (three LDS arrays
- * instead of five).
- *
- * open_y: first-order Mur absorbing boundaries at the y edges, after the
- * whole step of E and before the second half step of B, as the reference's
- * one-dimensional code applies them along x (em1d/emf.c:379-406, 548-561):
- * the tangential components Ex, Ez of the guard rows j = -1 and j = ny
- * become E_in(n) + S (E_in(n+1) - E_guard(n)) with E_in the adjacent
- * interior row (0, ny - 1) and S = (dt - dy) / (dt + dy); the old values
- * are read from the input buffer E, which the kernel does not write. */
 /* shift: the step ends in a window move (em2d/emf.c:646-676): every node
  * is written one column to the left, the leftmost guard column's values
  * are dropped and raw columns nx - 1 .. nx + 1 are zeroed, as the
@@ -66,84 +47,108 @@ __device__ inline void yee_store(float *__restrict__ Eo, float *__restrict__ Bo,
     }
 }
 
-__device__ inline void yee_tile(const float *__restrict__ E, const float *__restrict__ B,
-                                const float *__restrict__ J, float *__restrict__ Eo, float *__restrict__ Bo, int nx,
-                                int ny, int nrow, const YeeK &k, const int tx, const int ty, const int periodic_x,
-                                const int open_y = 0, const int shift = 0)
+/* One field step of R output rows by ZK_YEE_W output columns, unit `u` of the
+ * buffer (units in rows of zk_yee_units_x(nx)), by one wave: a column per
+ * lane, the rows in registers.  A half step of B reaches one column right
+ * and one row up, the whole step of E one left and one down, so the wave
+ * reads one column and row below its outputs and two above.
+ *
+ * The step is a few operations per byte: what bounds it is the reads and
+ * writes on large grids and the latency of one read elsewhere.  Lane shifts
+ * need neither LDS nor barriers, and all loads are under way before the
+ * first is used.  2000 x 512 cells: 14.3 us for 62 MB (20.3 with tiles in
+ * LDS), 256 x 256: 5.4 (6.4), 2048 x 2048: 67.7 for 252 MB (73.4).
+ *
+ * The half and whole steps update B and E in place: a node's new value
+ * depends on its own old value and on neighbours of the other field.
+ *
+ * open_y: first-order Mur absorbing boundaries at the y edges, after the
+ * whole step of E and before the second half step of B, as the reference's
+ * one-dimensional code applies them along x (em1d/emf.c:379-406, 548-561):
+ * the tangential components Ex, Ez of the guard rows j = -1 and j = ny
+ * become E_in(n) + S (E_in(n+1) - E_guard(n)) with E_in the adjacent
+ * interior row (0, ny - 1) and S = (dt - dy) / (dt + dy); the old values
+ * are read from the input buffer E, which the kernel does not write.  The
+ * top unit ends at the last row (and repeats rows of the one below), so
+ * that row ny - 1 is in a wave that writes row ny. */
+template <int R>
+__device__ inline void yee_rows(const float *__restrict__ E, const float *__restrict__ B, const float *__restrict__ J,
+                                float *__restrict__ Eo, float *__restrict__ Bo, int nx, int ny, int nrow,
+                                const YeeK &k, const int u, const int periodic_x, const int open_y = 0,
+                                const int shift = 0)
 {
-    __shared__ float e[3][LY][LX], b[3][LY][LX], jj[3][LY][LX];
     const int bw = nx + 3, bh = ny + 3;
-    const int bi0 = tx * BX, bj0 = ty * BY;
-    const int tid = threadIdx.x;
-    /* local (u, v) <-> buffer node (bi0 - 1 + u, bj0 - OY + v), raw node
-     * (bi0 - 2 + u, bj0 - OY - 1 + v) */
-    for (int m = tid; m < LX * LY; m += blockDim.x) {
-        const int u = m % LX, v = m / LX;
-        const int bi = bi0 - 1 + u, bj = bj0 - OY + v;
-        const bool in = bi >= 0 && bi < bw && bj >= 0 && bj < bh;
-        const size_t g = 3 * ((size_t)bi + (size_t)bj * nrow);
+    const int lane = __lane_id();
+    const int ux = zk_yee_units_x(nx);
+    const int c0 = u % ux * ZK_YEE_W, bi = c0 - 1 + lane, i = bi - 1;
+    const int bj0 = open_y ? max(0, min(u / ux * R, bh - R)) : u / ux * R; /* first output row */
+    const int j0 = bj0 - 2;                                               /* raw row of e[0], b[0] */
+    const bool col = bi >= 0 && bi < bw;
+    float e[R + 3][3], b[R + 2][3], jj[R + 2][3];
+#pragma unroll
+    for (int v = 0; v < R + 3; v++) {
+        const int bj = bj0 - 1 + v;
+        const bool in = col && bj >= 0 && bj < bh;
+        const size_t g = in ? 3 * ((size_t)bi + (size_t)bj * nrow) : 0;
+#pragma unroll
         for (int c = 0; c < 3; c++) {
-            e[c][v][u] = in ? E[g + c] : 0.0f;
-            b[c][v][u] = in ? B[g + c] : 0.0f;
-            jj[c][v][u] = in ? J[g + c] : 0.0f;
+            e[v][c] = in ? E[g + c] : 0.0f;
+            if (v < R + 2) b[v][c] = in ? B[g + c] : 0.0f;
+            if (v > 0 && v < R + 2) jj[v][c] = in ? J[g + c] : 0.0f;
         }
     }
-    __syncthreads();
-    /* B1 = B + dt/2 * (-curl E) on u in [0, LX-1), v in [0, LY-1) */
-    for (int m = tid; m < (LX - 1) * (LY - 1); m += blockDim.x) {
-        const int u = m % (LX - 1), v = m / (LX - 1);
-        const int i = bi0 - 2 + u, j = bj0 - OY - 1 + v; /* raw indices */
-        if (i >= -1 && i <= nx && j >= -1 && j <= ny) {
-            b[0][v][u] += (-k.dty2 * (e[2][v + 1][u] - e[2][v][u]));
-            b[1][v][u] += (k.dtx2 * (e[2][v][u + 1] - e[2][v][u]));
-            b[2][v][u] += (-k.dtx2 * (e[1][v][u + 1] - e[1][v][u]) + k.dty2 * (e[0][v + 1][u] - e[0][v][u]));
+    const bool half_x = i >= -1 && i <= nx, whole_x = i >= 0 && i <= nx + 1;
+    /* B1 = B + dt/2 * (-curl E) */
+#pragma unroll
+    for (int v = 0; v < R + 2; v++) {
+        const bool f = half_x && j0 + v >= -1 && j0 + v <= ny;
+        const float ea1 = lane_above(e[v][1]), ea2 = lane_above(e[v][2]);
+        const float x = b[v][0] + (-k.dty2 * (e[v + 1][2] - e[v][2]));
+        const float y = b[v][1] + (k.dtx2 * (ea2 - e[v][2]));
+        const float z = b[v][2] + (-k.dtx2 * (ea1 - e[v][1]) + k.dty2 * (e[v + 1][0] - e[v][0]));
+        b[v][0] = f ? x : b[v][0];
+        b[v][1] = f ? y : b[v][1];
+        b[v][2] = f ? z : b[v][2];
+    }
+    /* E1 = E + dt * (curl B1 - J) */
+#pragma unroll
+    for (int v = 1; v < R + 2; v++) {
+        const bool f = whole_x && j0 + v >= 0 && j0 + v <= ny + 1;
+        const float bb1 = lane_below(b[v][1]), bb2 = lane_below(b[v][2]);
+        const float x = e[v][0] + ((+k.dty * (b[v][2] - b[v - 1][2])) - k.dt * jj[v][0]);
+        const float y = e[v][1] + ((-k.dtx * (b[v][2] - bb2)) - k.dt * jj[v][1]);
+        const float z = e[v][2] + ((+k.dtx * (b[v][1] - bb1) - k.dty * (b[v][0] - b[v - 1][0])) - k.dt * jj[v][2]);
+        e[v][0] = f ? x : e[v][0];
+        e[v][1] = f ? y : e[v][1];
+        e[v][2] = f ? z : e[v][2];
+    }
+    if (open_y && (bj0 == 0 || bj0 + R >= ny + 1)) {
+#pragma unroll
+        for (int v = 1; v < R + 2; v++) {
+            const int jb = j0 + v;
+            if ((jb != -1 && jb != ny) || !col) continue;
+            const int d = jb == -1 ? 1 : -1; /* towards the interior */
+            const size_t gb = 3 * ((size_t)bi + (size_t)(jb + 1) * nrow);
+            const size_t gi = 3 * ((size_t)bi + (size_t)(jb + 1 + d) * nrow);
+            const float up0 = e[v + 1][0], up2 = e[v + 1][2], dn0 = e[v - 1][0], dn2 = e[v - 1][2];
+            e[v][0] = E[gi + 0] + k.mur_y * ((d > 0 ? up0 : dn0) - E[gb + 0]);
+            e[v][2] = E[gi + 2] + k.mur_y * ((d > 0 ? up2 : dn2) - E[gb + 2]);
         }
     }
-    __syncthreads();
-    /* E1 = E + dt * (curl B1 - J) on u in [1, LX-1), v in [1, LY-1) */
-    for (int m = tid; m < (LX - 2) * (LY - 2); m += blockDim.x) {
-        const int u = 1 + m % (LX - 2), v = 1 + m / (LX - 2);
-        const int i = bi0 - 2 + u, j = bj0 - OY - 1 + v;
-        if (i >= 0 && i <= nx + 1 && j >= 0 && j <= ny + 1) {
-            e[0][v][u] += (+k.dty * (b[2][v][u] - b[2][v - 1][u])) - k.dt * jj[0][v][u];
-            e[1][v][u] += (-k.dtx * (b[2][v][u] - b[2][v][u - 1])) - k.dt * jj[1][v][u];
-            e[2][v][u] += (+k.dtx * (b[1][v][u] - b[1][v][u - 1]) - k.dty * (b[0][v][u] - b[0][v - 1][u])) -
-                          k.dt * jj[2][v][u];
-        }
-    }
-    __syncthreads();
-    if (open_y) {
-        /* Mur rows among this tile's outputs (raw rows bj0 - 1 .. bj0 + BY - 2) */
-        for (int s = 0; s < 2; s++) {
-            const int jb = s ? ny : -1, jin = s ? ny - 1 : 0;
-            if (jb < bj0 - 1 || jb >= bj0 - 1 + BY) continue;
-            const int v = jb - (bj0 - OY - 1), vin = v + (jin - jb);
-            for (int u = 1 + tid; u < BX + 1; u += blockDim.x) {
-                const int bi = bi0 - 1 + u;
-                if (bi >= bw) continue;
-                const size_t gb = 3 * ((size_t)bi + (size_t)(jb + 1) * nrow);
-                const size_t gi = 3 * ((size_t)bi + (size_t)(jin + 1) * nrow);
-                e[0][v][u] = E[gi + 0] + k.mur_y * (e[0][vin][u] - E[gb + 0]);
-                e[2][v][u] = E[gi + 2] + k.mur_y * (e[2][vin][u] - E[gb + 2]);
-            }
-        }
-        __syncthreads();
-    }
-    /* tiles holding guards, or nodes that guards are images of */
-    const bool edge = (periodic_x && (bi0 <= 2 || bi0 + BX > nx)) || (!open_y && (bj0 <= 2 || bj0 + BY > ny));
-    /* B2 = B1 + dt/2 * (-curl E1) and outputs on u in [1, BX+1), v in [OY, BY+OY) */
-    for (int m = tid; m < BX * BY; m += blockDim.x) {
-        const int u = 1 + m % BX, v = OY + m / BX;
-        const int bi = bi0 - 1 + u, bj = bj0 - OY + v;
-        if (bi >= bw || bj >= bh) continue;
-        const int i = bi - 1, j = bj - 1;
-        float bx = b[0][v][u], by = b[1][v][u], bz = b[2][v][u];
-        if (i >= -1 && i <= nx && j >= -1 && j <= ny) {
-            bx += (-k.dty2 * (e[2][v + 1][u] - e[2][v][u]));
-            by += (k.dtx2 * (e[2][v][u + 1] - e[2][v][u]));
-            bz += (-k.dtx2 * (e[1][v][u + 1] - e[1][v][u]) + k.dty2 * (e[0][v + 1][u] - e[0][v][u]));
-        }
-        const float bn[3] = {bx, by, bz}, en[3] = {e[0][v][u], e[1][v][u], e[2][v][u]};
+    /* units holding guards, or nodes that guards are images of */
+    const bool edge = (periodic_x && (c0 <= 2 || c0 + ZK_YEE_W > nx)) || (!open_y && (bj0 <= 2 || bj0 + R > ny));
+    /* B2 = B1 + dt/2 * (-curl E1) and outputs */
+#pragma unroll
+    for (int v = 1; v < R + 1; v++) {
+        const int bj = bj0 - 1 + v, j = bj - 1;
+        const bool f = half_x && j >= -1 && j <= ny;
+        const float ea1 = lane_above(e[v][1]), ea2 = lane_above(e[v][2]);
+        const float x = b[v][0] + (-k.dty2 * (e[v + 1][2] - e[v][2]));
+        const float y = b[v][1] + (k.dtx2 * (ea2 - e[v][2]));
+        const float z = b[v][2] + (-k.dtx2 * (ea1 - e[v][1]) + k.dty2 * (e[v + 1][0] - e[v][0]));
+        if (lane < 1 || lane > ZK_YEE_W || bi >= bw || bj >= bh) continue;
+        const float bn[3] = {f ? x : b[v][0], f ? y : b[v][1], f ? z : b[v][2]};
+        const float en[3] = {e[v][0], e[v][1], e[v][2]};
         if (!edge) {
             yee_store(Eo, Bo, nx, nrow, bi, bj, en, bn, shift);
             continue;

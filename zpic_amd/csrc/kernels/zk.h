@@ -433,9 +433,29 @@ int zk_batch_fields(const zk_bsim *sims, const int *yee_items, int nyee, zk_stre
 int zk_batch_sort(const zk_bspec *specs, int nspecs, const int *items, int n, zk_stream_t s);
 int zk_batch_end_step(zk_bsim *sims, int nsims, zk_bspec *specs, int nspecs, zk_push_multi *sets, int sorted,
                       zk_stream_t s);
-/* output-node tiles of the Yee kernel */
-#define ZK_YEE_BX 32
-#define ZK_YEE_BY 16
+/* work of the field step: units of ZK_YEE_W columns by a few rows, one wave
+ * each.  More rows re-read fewer margins, fewer make more waves: 2048 x 2048
+ * cells take 67.7 us with 8 rows and 70.9 with 4, 2000 x 512 17.8 and 14.3,
+ * 4000 x 256 20.4 and 18.9, so ZK_YEE_R rows from ZK_YEE_LARGE nodes on,
+ * ZK_YEE_R_SMALL below (batch members, many to a launch: ZK_YEE_R) */
+#define ZK_YEE_W 61
+#define ZK_YEE_R 8
+#define ZK_YEE_R_SMALL 4
+#define ZK_YEE_LARGE (1 << 21)
+#ifdef __HIPCC__
+#define ZK_HD __host__ __device__
+#else
+#define ZK_HD
+#endif
+ZK_HD static inline int zk_yee_rows(int nx, int ny)
+{
+    return (long long)(nx + 3) * (ny + 3) < ZK_YEE_LARGE ? ZK_YEE_R_SMALL : ZK_YEE_R;
+}
+ZK_HD static inline int zk_yee_units_x(int nx) { return (nx + 3 + ZK_YEE_W - 1) / ZK_YEE_W; }
+ZK_HD static inline int zk_yee_units(int nx, int ny, int rows)
+{
+    return zk_yee_units_x(nx) * ((ny + 3 + rows - 1) / rows);
+}
 
 #ifdef __cplusplus
 }
