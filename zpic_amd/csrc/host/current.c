@@ -26,7 +26,7 @@ void current_new(t_current *c, int nx[], float box[], float dt)
         c->dx[d] = box[d] / nx[d];
     }
     c->nrow = nx[0] + 3;
-    c->J_buf = calloc(zpic_grid_nodes(c->nx), sizeof(float3));
+    c->J_buf = zpic_host_grid(zpic_grid_nodes(c->nx) * sizeof(float3));
     if (!c->J_buf) zpic_fatal("out of host memory for the current grid");
     c->J = c->J_buf + 1 + c->nrow;
     c->smooth.xtype = NONE;

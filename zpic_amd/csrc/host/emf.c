@@ -27,8 +27,8 @@ void emf_new(t_emf *emf, int nx[], float box[], const float dt)
     }
     emf->nrow = nx[0] + 3;
     const size_t nodes = zpic_grid_nodes(emf->nx);
-    emf->E_buf = calloc(nodes, sizeof(float3));
-    emf->B_buf = calloc(nodes, sizeof(float3));
+    emf->E_buf = zpic_host_grid(nodes * sizeof(float3));
+    emf->B_buf = zpic_host_grid(nodes * sizeof(float3));
     if (!emf->E_buf || !emf->B_buf) zpic_fatal("out of host memory for the field grids");
     emf->E = emf->E_buf + 1 + emf->nrow;
     emf->B = emf->B_buf + 1 + emf->nrow;
@@ -42,6 +42,7 @@ void emf_new(t_emf *emf, int nx[], float box[], const float dt)
     emf->dev = calloc(1, sizeof(struct zpic_dev_emf));
     emf->dev->host_dirty = 1;
     emf->dev->host_valid = 1;
+    zpic_stage_hold(1);
 }
 
 void emf_delete(t_emf *emf)
@@ -63,6 +64,7 @@ void emf_delete(t_emf *emf)
         zpic_dfree(d->energy6);
         free(d);
         emf->dev = NULL;
+        zpic_stage_hold(-1);
     }
     free(emf->E_buf);
     free(emf->B_buf);

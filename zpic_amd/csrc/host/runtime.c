@@ -5,10 +5,14 @@
  * (process-global timers and RNG, em2d/particles.c:26-27, em2d/emf.c:27,
  * em2d/random.c:16-17), so one process-wide stream carries all work.
  */
+#define _DEFAULT_SOURCE /* madvise */
 #include <math.h>
+#include <pthread.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <stdlib.h>
+#include <string.h>
+#include <sys/mman.h>
 
 #include <hip/hip_runtime_api.h>
 
@@ -205,8 +209,116 @@ void zpic_h2d(void *dst, const void *src, size_t bytes)
     ZCHECK(hipStreamSynchronize(zpic_stream()));
 }
 
+/* Large reads into ordinary memory.  The runtime's own copy stages them with
+ * one host thread, about 19 GB/s for the grids of a simulation; here
+ * STAGE_THREADS threads each keep two page-locked chunks, one filled by the
+ * GPU while the other is copied out: E, B and J of 2000 x 512 cells (37 MB)
+ * in 1.0 ms instead of 1.9, of 2048 x 2048 (151 MB) in 3 ms instead of 8.6.
+ *
+ * The chunks are allocated by the first large read and belong to the live
+ * simulations (zpic_stage_hold): the last one to be deleted gives them back.
+ * A read that finds them taken, or too small a read, uses the plain copy. */
+#define STAGE_THREADS 4
+#define STAGE_CHUNK ((size_t)1 << 21)
+#define STAGE_MIN ((size_t)1 << 23) /* 3 MB grids gain nothing (512 x 512), 13 MB ones half */
+
+static struct {
+    pthread_mutex_t lock;
+    int holders, busy;
+    char *buf; /* STAGE_THREADS pairs of chunks */
+    hipEvent_t ev[2 * STAGE_THREADS];
+} g_stage = {.lock = PTHREAD_MUTEX_INITIALIZER};
+
+typedef struct {
+    char *dst;
+    const char *src;
+    size_t bytes, chunk;
+    int first; /* chunks first, first + STAGE_THREADS, ... */
+    hipStream_t stream;
+} stage_job;
+
+/* GPU copy of chunk c into a page-locked chunk (no-op past the end) */
+static void stage_issue(const stage_job *j, size_t c, int slot)
+{
+    const size_t off = c * j->chunk;
+    if (off >= j->bytes) return;
+    const size_t n = j->bytes - off < j->chunk ? j->bytes - off : j->chunk;
+    ZCHECK(hipMemcpyAsync(g_stage.buf + slot * STAGE_CHUNK, j->src + off, n, hipMemcpyDeviceToHost, j->stream));
+    ZCHECK(hipEventRecord(g_stage.ev[slot], j->stream));
+}
+
+static void *stage_run(void *arg)
+{
+    const stage_job *j = arg;
+    ZCHECK(hipSetDevice(g_device));
+    size_t c = (size_t)j->first;
+    int slot = 2 * j->first;
+    stage_issue(j, c, slot);
+    stage_issue(j, c + STAGE_THREADS, slot + 1);
+    for (; c * j->chunk < j->bytes; c += STAGE_THREADS, slot ^= 1) {
+        const size_t off = c * j->chunk;
+        ZCHECK(hipEventSynchronize(g_stage.ev[slot]));
+        memcpy(j->dst + off, g_stage.buf + slot * STAGE_CHUNK, j->bytes - off < j->chunk ? j->bytes - off : j->chunk);
+        stage_issue(j, c + 2 * STAGE_THREADS, slot);
+    }
+    return NULL;
+}
+
+/* with the lock held, no read running */
+static void stage_free(void)
+{
+    if (!g_stage.buf) return;
+    zpic_pinned_free(g_stage.buf);
+    g_stage.buf = NULL;
+    for (int k = 0; k < 2 * STAGE_THREADS; k++) ZCHECK(hipEventDestroy(g_stage.ev[k]));
+}
+
+void zpic_stage_hold(int n)
+{
+    pthread_mutex_lock(&g_stage.lock);
+    g_stage.holders += n;
+    if (g_stage.holders == 0 && !g_stage.busy) stage_free();
+    pthread_mutex_unlock(&g_stage.lock);
+}
+
+/* 1: the read was done */
+static int staged_d2h(void *dst, const void *src, size_t bytes)
+{
+    if (bytes < STAGE_MIN) return 0;
+    pthread_mutex_lock(&g_stage.lock);
+    const int mine = g_stage.holders > 0 && !g_stage.busy;
+    if (mine) g_stage.busy = 1;
+    pthread_mutex_unlock(&g_stage.lock);
+    if (!mine) return 0;
+    const hipStream_t stream = zpic_stream();
+    if (!g_stage.buf) {
+        g_stage.buf = zpic_pinned_alloc(2 * STAGE_THREADS * STAGE_CHUNK);
+        for (int k = 0; k < 2 * STAGE_THREADS; k++) g_stage.ev[k] = zpic_event_new_read();
+    }
+    /* at least two chunks a thread, so that copies and reads overlap */
+    size_t chunk = (bytes / (2 * STAGE_THREADS) + 4095) / 4096 * 4096;
+    if (chunk > STAGE_CHUNK) chunk = STAGE_CHUNK;
+    stage_job job[STAGE_THREADS];
+    pthread_t th[STAGE_THREADS];
+    int started[STAGE_THREADS];
+    for (int k = STAGE_THREADS - 1; k >= 0; k--) {
+        job[k] = (stage_job){dst, src, bytes, chunk, k, stream};
+        started[k] = k > 0 && pthread_create(&th[k], NULL, stage_run, &job[k]) == 0;
+    }
+    for (int k = 0; k < STAGE_THREADS; k++)
+        if (!started[k]) stage_run(&job[k]);
+    for (int k = 1; k < STAGE_THREADS; k++)
+        if (started[k]) pthread_join(th[k], NULL);
+    pthread_mutex_lock(&g_stage.lock);
+    g_stage.busy = 0;
+    if (g_stage.holders == 0) stage_free();
+    pthread_mutex_unlock(&g_stage.lock);
+    return 1;
+}
+
 void zpic_d2h(void *dst, const void *src, size_t bytes)
 {
+    if (staged_d2h(dst, src, bytes)) return;
     if (bytes) ZCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, zpic_stream()));
     ZCHECK(hipStreamSynchronize(zpic_stream()));
 }
@@ -219,6 +331,14 @@ void zpic_d2h_async(void *dst, const void *src, size_t bytes)
 void zpic_d2d_async(void *dst, const void *src, size_t bytes)
 {
     if (bytes) ZCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, zpic_stream()));
+}
+
+void *zpic_host_grid(size_t bytes)
+{
+    void *p = calloc(1, bytes > 0 ? bytes : 1);
+    const size_t page = 4096, a = ((size_t)p + page - 1) / page * page;
+    if (p && bytes >= STAGE_MIN) madvise((void *)a, ((size_t)p + bytes - a) / page * page, MADV_HUGEPAGE);
+    return p;
 }
 
 void zpic_sync(void)

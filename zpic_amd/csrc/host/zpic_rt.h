@@ -24,6 +24,9 @@ void zpic_dfree(void *p);
 void zpic_h2d(void *dst, const void *src, size_t bytes);      /* synchronous */
 void zpic_d2h(void *dst, const void *src, size_t bytes);      /* synchronous */
 void zpic_d2d_async(void *dst, const void *src, size_t bytes); /* on the stream */
+/* zeroed host grid (calloc; NULL when out of memory); large ones ask for huge
+ * pages, which the first read from the device fills several times faster */
+void *zpic_host_grid(size_t bytes);
 void zpic_sync(void);
 void zpic_h2d_async(void *dst, const void *src, size_t bytes); /* host buffer must outlive the copy */
 void zpic_d2h_async(void *dst, const void *src, size_t bytes); /* into page-locked memory; wait on an
@@ -31,6 +34,8 @@ void zpic_d2h_async(void *dst, const void *src, size_t bytes); /* into page-lock
 
 /* page-locked host memory (copies from it run asynchronously) and events
  * on the library's stream that the host can wait for */
+/* +1 / -1: a simulation begins / ends (page-locked chunks of large reads) */
+void zpic_stage_hold(int n);
 void *zpic_pinned_alloc(size_t bytes);
 void zpic_pinned_free(void *p);
 void *zpic_pinned_device(void *p); /* device address of page-locked memory */
