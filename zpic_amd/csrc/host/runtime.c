@@ -323,11 +323,6 @@ void zpic_d2h(void *dst, const void *src, size_t bytes)
     ZCHECK(hipStreamSynchronize(zpic_stream()));
 }
 
-void zpic_d2h_async(void *dst, const void *src, size_t bytes)
-{
-    if (bytes) ZCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, zpic_stream()));
-}
-
 void zpic_d2d_async(void *dst, const void *src, size_t bytes)
 {
     if (bytes) ZCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, zpic_stream()));
@@ -592,6 +587,19 @@ void *zpic_pinned_alloc(size_t bytes)
     void *p = NULL;
     ZCHECK(hipHostMalloc(&p, bytes > 0 ? bytes : 1, hipHostMallocMapped | hipHostMallocCoherent));
     return p;
+}
+
+/* The word is written by work on the stream that was launched before.  A
+ * short wait is spent looking at the word; then the stream's end is waited
+ * for, by which the word must be there. */
+void zpic_wait_word(const unsigned *word, unsigned value)
+{
+    for (int i = 0; i < 1 << 16; i++) {
+        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == value) return;
+        __builtin_ia32_pause();
+    }
+    zpic_sync();
+    if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != value) zpic_fatal("counters asked of the device did not arrive");
 }
 
 void *zpic_pinned_device(void *p)

@@ -35,8 +35,7 @@ __global__ void __launch_bounds__(256) reduce_kernel(zk_reduce_args a, int nbx, 
     const int b = (int)blockIdx.x - RED_FIN;
     if (b < 0) {
         const int k = blockIdx.x;
-        if (k < a.fin.n)
-            finalize_body(a.fin.ctr[k], a.fin.epart[k], a.fin.nparts[k], a.fin.qm[k], a.fin.dx0[k], a.fin.dx1[k]);
+        if (k < a.fin.n) finalize_set_body(a.fin, k);
         return;
     }
     if constexpr (N == 0) {

@@ -32,6 +32,25 @@ __device__ inline void finalize_body(zk_spec_ctr *ctr, const double *epart, int 
     }
 }
 
+/* Species k of the set; the counters also go to the host where asked for.
+ * One wave stores them word by word, each lane makes its word visible to
+ * the host, and then lane 0 stores the sequence number that completes
+ * them. */
+__device__ inline void finalize_set_body(const zk_finalize_set &f, int k)
+{
+    finalize_body(f.ctr[k], f.epart[k], f.nparts[k], f.qm[k], f.dx0[k], f.dx1[k]);
+    if (!f.probe[k]) return;
+    __syncthreads();
+    if (threadIdx.x >= ZK_WAVE) return;
+    static_assert(sizeof(zk_spec_ctr) % 4 == 0 && sizeof(zk_spec_ctr) / 4 <= ZK_WAVE, "one word a lane");
+    if (threadIdx.x < sizeof(zk_spec_ctr) / 4)
+        __hip_atomic_store((unsigned *)&f.probe[k]->c + threadIdx.x, ((const unsigned *)f.ctr[k])[threadIdx.x],
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    if (threadIdx.x == 0)
+        __hip_atomic_store(&f.probe[k]->seq, f.seq[k], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 } // namespace zk
 
 #endif

@@ -98,7 +98,7 @@ __global__ void stamp_kernel(zk_stamp st) { zk_stamp_last(st); }
 __global__ void __launch_bounds__(1024) finalize_set_kernel(zk_finalize_set f)
 {
     const int k = blockIdx.x;
-    finalize_body(f.ctr[k], f.epart[k], f.nparts[k], f.qm[k], f.dx0[k], f.dx1[k]);
+    finalize_set_body(f, k);
 }
 
 /* For every float x of [first, first + n) (as bit patterns): whether

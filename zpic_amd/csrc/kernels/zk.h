@@ -166,10 +166,20 @@ int zk_push(const zk_push_args *a, zk_stream_t s);
 /* fused tile pass over m->n species (fixed-point windows), then the
  * global pass of each species that has an unsorted tail */
 int zk_push_species(const zk_push_multi *m, zk_stream_t s);
-/* energy and push count of up to ZK_FUSE_MAX species in one launch */
+/* Counters of a species in page-locked host memory, for the host to read
+ * without a copy or an event behind the work it waits for: complete once
+ * seq has the value asked for. */
+typedef struct zk_probe {
+    zk_spec_ctr c;
+    unsigned seq;
+} zk_probe;
+/* energy and push count of up to ZK_FUSE_MAX species in one launch, and
+ * their counters to probe[k] (device address; NULL: none) with seq[k] */
 typedef struct zk_finalize_set {
     int n;
     zk_spec_ctr *ctr[ZK_FUSE_MAX];
+    zk_probe *probe[ZK_FUSE_MAX];
+    unsigned seq[ZK_FUSE_MAX];
     const double *epart[ZK_FUSE_MAX];
     int nparts[ZK_FUSE_MAX];
     double qm[ZK_FUSE_MAX], dx0[ZK_FUSE_MAX], dx1[ZK_FUSE_MAX];
