@@ -209,29 +209,45 @@ int zpic_current_passes(const t_current *c, int axis[], float sa[], float sb[], 
     return n;
 }
 
+/* Arguments of the fold of a step; returns whether it clears the other
+ * overflow grid. */
+static int reduce_args(t_current *c, zk_reduce_args *a)
+{
+    struct zpic_dev_current *d = c->dev;
+    a->region = d->fresh ? NULL : d->region;
+    a->Jov = d->Jov2[d->jov_cur];
+    a->jflag = d->jov_state[d->jov_cur] == ZPIC_JOV_DIRTY ? NULL : d->jflag[d->jov_cur];
+    const int other = 1 - d->jov_cur;
+    const int clears = d->jov_state[other] == ZPIC_JOV_FLAGGED && zk_current_clears(&d->t);
+    a->Jov_next = clears ? d->Jov2[other] : NULL;
+    a->jflag_next = clears ? d->jflag[other] : NULL;
+    a->jov_unscale = zpic_current_jov_unscale(c);
+    a->J = d->J[d->jcur];
+    a->nrow = c->nrow;
+    a->t = d->t;
+    a->periodic_x = !c->moving_window;
+    a->open_y = d->open_y;
+    a->fin = d->fin;
+    return clears;
+}
+
+/* after the launch that folds */
+static void reduce_done(t_current *c, int cleared)
+{
+    struct zpic_dev_current *d = c->dev;
+    if (cleared) d->jov_state[1 - d->jov_cur] = ZPIC_JOV_CLEAN;
+    fin_done(d);
+}
+
 void current_update(t_current *c)
 {
     zpic_current_ensure(c, NULL);
     struct zpic_dev_current *d = c->dev;
     zk_reduce_args a;
-    a.region = d->fresh ? NULL : d->region;
-    a.Jov = d->Jov2[d->jov_cur];
-    a.jflag = d->jov_state[d->jov_cur] == ZPIC_JOV_DIRTY ? NULL : d->jflag[d->jov_cur];
-    const int other = 1 - d->jov_cur;
-    const int clears = d->jov_state[other] == ZPIC_JOV_FLAGGED && zk_current_clears(&d->t);
-    a.Jov_next = clears ? d->Jov2[other] : NULL;
-    a.jflag_next = clears ? d->jflag[other] : NULL;
-    a.jov_unscale = zpic_current_jov_unscale(c);
-    a.J = d->J[d->jcur];
-    a.nrow = c->nrow;
-    a.t = d->t;
-    a.periodic_x = !c->moving_window;
-    a.open_y = d->open_y;
-    a.fin = d->fin;
+    const int clears = reduce_args(c, &a);
     zpic_ktimer_begin(ZPIC_T_CURRENT);
     ZCHECK(zk_current_reduce(&a, zpic_stream()));
-    if (clears) d->jov_state[other] = ZPIC_JOV_CLEAN;
-    fin_done(d);
+    reduce_done(c, clears);
     const int maxp = 2 * (c->smooth.xlevel > 0 ? c->smooth.xlevel : 0) + 2;
     int axis[maxp];
     float sa[maxp], sb[maxp];
@@ -249,6 +265,29 @@ void current_update(t_current *c)
     zpic_ktimer_end(ZPIC_T_CURRENT);
     c->iter++;
     d->host_valid = 0;
+}
+
+int zpic_current_field_args(t_current *c, zk_field_args *f)
+{
+    zpic_current_ensure(c, NULL);
+    const struct zpic_dev_current *d = c->dev;
+    const int maxp = 2 * (c->smooth.xlevel > 0 ? c->smooth.xlevel : 0) + 2;
+    if (maxp > ZK_MAX_PASSES + ZK_MAX_Y_PASSES) return 0;
+    int axis[maxp];
+    const int np = zpic_current_passes(c, axis, f->sa, f->sb, maxp);
+    f->n1 = f->n2 = 0;
+    while (f->n1 < np && axis[f->n1] == 0) f->n1++;
+    while (f->n1 + f->n2 < np && axis[f->n1 + f->n2] == 1) f->n2++;
+    if (!zk_field_step_ok(&d->t, f->n1, f->n2, d->open_y)) return 0;
+    reduce_args(c, &f->r);
+    return 1;
+}
+
+void zpic_current_field_done(t_current *c, const zk_field_args *f)
+{
+    reduce_done(c, f->r.jflag_next != NULL);
+    c->iter++;
+    c->dev->host_valid = 0;
 }
 
 void current_sync_host(t_current *c)

@@ -448,11 +448,10 @@ const float *zpic_emf_particle_B(t_emf *emf)
 
 /* ---- time step (em2d/emf.c:688-716) ---- */
 
-void emf_advance(t_emf *emf, const t_current *ccur)
+/* The field step of emf_advance: with cf the launch also folds and filters
+ * the current. */
+static void advance(t_emf *emf, t_current *cur, zk_field_args *cf)
 {
-    t_current *cur = (t_current *)ccur;
-    zpic_emf_ensure(emf);
-    zpic_current_ensure(cur, NULL);
     struct zpic_dev_emf *d = emf->dev;
     const zk_stamp st = zpic_phase_begin(ZPIC_T_EMF);
     const int o = 1 - d->cur;
@@ -463,11 +462,22 @@ void emf_advance(t_emf *emf, const t_current *ccur)
     const int move = emf->moving_window && ((emf->iter + 1) * emf->dt) > emf->dx[0] * (emf->n_move + 1);
     const int fused = move && zpic_window_shift_fusion() && emf->ext_fld.E_type == EMF_FLD_TYPE_NONE &&
                       emf->ext_fld.B_type == EMF_FLD_TYPE_NONE;
-    zpic_ktimer_begin(ZPIC_T_FIELD);
-    ZCHECK(zk_yee(d->E[d->cur], d->B[d->cur], zpic_current_J(cur), d->E[o], d->B[o], emf->nx[0], emf->nx[1],
-                  emf->nrow, emf->dt, emf->dx[0], emf->dx[1], !emf->moving_window, d->open_y, fused, st,
-                  zpic_stream()));
-    zpic_ktimer_end(ZPIC_T_FIELD);
+    if (cf) {
+        cf->E = d->E[d->cur];
+        cf->B = d->B[d->cur];
+        cf->Eo = d->E[o];
+        cf->Bo = d->B[o];
+        cf->shift = fused;
+        cf->stamp = st;
+        ZCHECK(zk_field_step(cf, emf->dt, emf->dx[0], emf->dx[1], zpic_stream()));
+        zpic_current_field_done(cur, cf);
+    } else {
+        zpic_ktimer_begin(ZPIC_T_FIELD);
+        ZCHECK(zk_yee(d->E[d->cur], d->B[d->cur], zpic_current_J(cur), d->E[o], d->B[o], emf->nx[0], emf->nx[1],
+                      emf->nrow, emf->dt, emf->dx[0], emf->dx[1], !emf->moving_window, d->open_y, fused, st,
+                      zpic_stream()));
+        zpic_ktimer_end(ZPIC_T_FIELD);
+    }
     d->cur = o;
     part_fields(emf);
     emf->iter += 1;
@@ -483,6 +493,30 @@ void emf_advance(t_emf *emf, const t_current *ccur)
     zpic_phase_end(ZPIC_T_EMF, (move && !fused) || emf->ext_fld.E_type != EMF_FLD_TYPE_NONE ||
                                    emf->ext_fld.B_type != EMF_FLD_TYPE_NONE);
     d->host_valid = 0;
+}
+
+void emf_advance(t_emf *emf, const t_current *ccur)
+{
+    t_current *cur = (t_current *)ccur;
+    zpic_emf_ensure(emf);
+    zpic_current_ensure(cur, NULL);
+    advance(emf, cur, NULL);
+}
+
+void zpic_update_advance(t_current *cur, t_emf *emf)
+{
+    zk_field_args f;
+    zpic_emf_ensure(emf);
+    zpic_current_ensure(cur, NULL);
+    const int same = cur->nx[0] == emf->nx[0] && cur->nx[1] == emf->nx[1] && cur->nrow == emf->nrow &&
+                     cur->moving_window == emf->moving_window && cur->dev->open_y == emf->dev->open_y;
+    /* the kernel timers tell the current's launches from the fields' */
+    if (same && !zpic_kernel_timing_on() && zpic_current_field_args(cur, &f)) {
+        advance(emf, cur, &f);
+        return;
+    }
+    current_update(cur);
+    advance(emf, cur, NULL);
 }
 
 double emf_time(void) { return zpic_timer_total(ZPIC_T_EMF); }

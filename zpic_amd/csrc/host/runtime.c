@@ -517,6 +517,8 @@ double zpic_timer_total(int w)
     return g_timer[w].total;
 }
 
+int zpic_kernel_timing_on(void) { return g_ktiming; }
+
 void zpic_ktimer_begin(int w)
 {
     if (g_ktiming) zpic_timer_begin(w);

@@ -21,8 +21,8 @@ void sim_iter(t_simulation *sim)
      * pushed by one launch (same results up to the FP32 rounding of the
      * current windows) */
     zpic_spec_advance_all(sim->species, sim->n_species, &sim->emf, &sim->current);
-    current_update(&sim->current);
-    emf_advance(&sim->emf, &sim->current);
+    /* current_update and emf_advance */
+    zpic_update_advance(&sim->current, &sim->emf);
 }
 
 void sim_timings(t_simulation *sim, uint64_t t0, uint64_t t1)

@@ -164,5 +164,12 @@ void zpic_spec_settle(struct zpic_dev_species *d);
 void zpic_spec_sync_energy(t_species *s);
 void zpic_spec_sort(t_species *s); /* tile sort of the device particles now */
 int zpic_current_passes(const t_current *c, int axis[], float sa[], float sb[], int max);
+/* Arguments of the launch that folds and filters the current and takes the
+ * field step (0: the grid or the passes need separate launches), and the
+ * bookkeeping after it. */
+int zpic_current_field_args(t_current *c, zk_field_args *f);
+void zpic_current_field_done(t_current *c, const zk_field_args *f);
+/* current_update and emf_advance, in one launch where that is faster */
+void zpic_update_advance(t_current *cur, t_emf *emf);
 
 #endif

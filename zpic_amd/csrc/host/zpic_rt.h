@@ -78,6 +78,7 @@ enum {
     ZPIC_T_FIELD = 5,
     ZPIC_NTIMERS = 6
 };
+int zpic_kernel_timing_on(void);
 void zpic_ktimer_begin(int which); /* no-op unless kernel timing is on */
 void zpic_ktimer_end(int which);
 void zpic_timer_begin(int which);

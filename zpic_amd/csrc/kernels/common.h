@@ -99,20 +99,30 @@ __device__ inline float sqrt_ge1(float x)
     return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
 }
 
-/* Clock readings of a timed phase (zk_clock): zk_stamp_first at the start of
- * a launch, zk_stamp_last at its end; every thread may call them. */
-__device__ inline void zk_stamp_first(const zk_stamp &s)
+/* Clock readings of a timed phase (zk_clock), by one thread: zk_stamp_open at
+ * the start of its first launch, zk_stamp_close at the end of each. */
+__device__ inline void zk_stamp_open(const zk_stamp &s)
 {
-    if (!s.clk || !s.open || blockIdx.x + blockIdx.y != 0 || threadIdx.x != 0) return;
+    if (!s.clk || !s.open) return;
     const int o = 1 - s.slot;
     if (s.clk->t1[o] > s.clk->t0[o]) s.clk->total += s.clk->t1[o] - s.clk->t0[o];
     s.clk->t0[s.slot] = wall_clock64();
 }
 
+__device__ inline void zk_stamp_close(const zk_stamp &s)
+{
+    if (s.clk) s.clk->t1[s.slot] = wall_clock64();
+}
+
+/* The same for a whole launch: every thread may call them. */
+__device__ inline void zk_stamp_first(const zk_stamp &s)
+{
+    if (blockIdx.x + blockIdx.y == 0 && threadIdx.x == 0) zk_stamp_open(s);
+}
+
 __device__ inline void zk_stamp_last(const zk_stamp &s)
 {
-    if (!s.clk || blockIdx.x + 1 != gridDim.x || blockIdx.y + 1 != gridDim.y || threadIdx.x != 0) return;
-    s.clk->t1[s.slot] = wall_clock64();
+    if (blockIdx.x + 1 == gridDim.x && blockIdx.y + 1 == gridDim.y && threadIdx.x == 0) zk_stamp_close(s);
 }
 
 /* Value of the lane one below / above (0 past the ends of the wave). */

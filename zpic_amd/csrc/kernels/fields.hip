@@ -20,7 +20,9 @@
  */
 #include <mutex>
 
+#include "current_core.h"
 #include "fields_core.h"
+#include "finalize_core.h"
 
 using namespace zk;
 
@@ -42,6 +44,136 @@ __global__ void __launch_bounds__(256) yee_kernel(const float *__restrict__ E, c
     const int u = zk_xcd_item(blockIdx.x, gridDim.x) * (blockDim.x / 64) + threadIdx.x / 64;
     if (u < units) yee_rows<R>(E, B, J, Eo, Bo, nx, ny, nrow, k, u, periodic_x, open_y, shift);
     zk_stamp_last(st);
+}
+
+/* Waves of a workgroup of field_step_kernel, a staged row each, and the rows
+ * that leaves to write: fewer waves start sooner, more spend fewer on the
+ * rows of the margin. */
+__host__ __device__ inline int field_rows(int waves, int n2, int open_y) { return waves - 1 - open_y - 2 * n2; }
+inline int field_waves(int n2, int open_y) { return field_rows(8, n2, open_y) >= 4 ? 8 : 16; }
+__host__ __device__ inline int field_cols(int n1) { return 64 - (n1 > 1 ? n1 : 1) - (n1 > 1 ? n1 + 1 : 2); }
+
+/* Current fold, filter passes and field step in one launch, bit for bit the
+ * separate kernels' results.
+ *
+ * On grids of up to a few hundred cells a side each of those kernels takes 4
+ * to 6 us, of which its loads and arithmetic are a fraction: the rest is
+ * starting, waiting for one chain of loads and draining, and about 3.5 us
+ * pass between two launches.  Here the chains run once and side by side: a
+ * wave starts the loads of E and B, sums the windows for its row of J (a
+ * column per lane), filters along x by lane shifts, along y through LDS, and
+ * takes the field step of its row.  Rows and columns of the margins are
+ * computed by every workgroup that needs them, which is why larger grids
+ * keep the separate launches.  32 x 32 cells: 8.9 us for fold and step, 11.7
+ * and a gap in two launches; 256 x 256, a pass each way: 10.0 us, 16.1 and
+ * two gaps in three; 1500 x 128, 5 x passes: 12.3 us instead of 15.9.
+ *
+ * Workgroups in order: one per species whose push is to be finished, those
+ * that clear the flagged blocks of the next overflow grid (a wave per
+ * block), and the field_cols x field_rows units of the buffer.
+ *
+ * The passes' guard handling is smooth_kernel's; the raw guard rows that the
+ * first y pass reads equal their images' raw rows (both are folded alike),
+ * which the neighbouring waves hold. */
+template <int N, int X>
+__global__ void __launch_bounds__(1024) field_step_kernel(zk_field_args f)
+{
+    extern __shared__ float fs[];
+    const int waves = blockDim.x / 64, lane = threadIdx.x % 64;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+    int u = (int)blockIdx.x - f.r.fin.n;
+    if (u < 0) {
+        finalize_set_body(f.r.fin, blockIdx.x);
+        return;
+    }
+    const int nx = f.r.t.nx, ny = f.r.t.ny, nrow = f.r.nrow;
+    if (u < f.clears) {
+        const int nbx = zk_red_blocks_x(nx), b = u * waves + w;
+        if (b >= nbx * zk_red_blocks_y(ny) || !f.r.jflag_next[b]) return;
+        for (int k = lane; k < ZK_RED_BX * ZK_RED_BY; k += 64) {
+            const int bi = b % nbx * ZK_RED_BX + k % ZK_RED_BX, bj = b / nbx * ZK_RED_BY + k / ZK_RED_BX;
+            if (bi >= nx + 3 || bj >= ny + 3) continue;
+            long long *z = f.r.Jov_next + 3 * ((size_t)bi + (size_t)bj * nrow);
+            z[0] = z[1] = z[2] = 0;
+        }
+        if (lane == 0) f.r.jflag_next[b] = 0;
+        return;
+    }
+    u -= f.clears;
+    const int n1 = f.n1, n2 = f.n2, px = f.r.periodic_x, oy = f.r.open_y;
+    const int l0 = n1 > 1 ? n1 : 1, cols = field_cols(n1), rows = field_rows(waves, n2, X);
+    const int ux = (nx + 3 + cols - 1) / cols;
+    const int c0 = u % ux * cols, bi = c0 - l0 + lane, i = bi - 1;
+    const int r0 = u / ux * rows;            /* first buffer row to write */
+    const int j = r0 - 1 - n2 - X + w;       /* this wave's raw row */
+    const bool ring = !oy && n2 > 0;         /* rows are images of interior rows */
+    const int cr = ring ? zk_wrap(j, ny) : j;
+    const bool inner = cr >= 0 && cr < ny, in_x = i >= 0 && i < nx, col = bi >= 0 && bi < nx + 3;
+    const bool out = w >= n2 + X && w < n2 + X + rows && j + 1 < ny + 3;
+    YeeRows<1, X> y;
+    if (out) y.load(f.E, f.B, nx, ny, nrow, bi, j + 1);
+    float s[3] = {0.0f, 0.0f, 0.0f};
+    if (inner ? px || col : cr >= -1 && cr <= ny + 1 && col)
+        reduce_sum<N>(f.r, inner && px ? zk_wrap(i, nx) : i, cr, s);
+    /* LDS: the rows before the x passes (for the first y pass), then two
+     * buffers in turn */
+    const int plane = 3 * 64 * waves, own = 3 * (64 * w + lane);
+    float *raw = fs, *cur = fs + plane, *nxt = fs + 2 * plane;
+    if (n2 > 0)
+        for (int c = 0; c < 3; c++) raw[own + c] = s[c];
+    const bool live_x = (px || in_x) && (ring || inner);
+    for (int p = 0; p < n1; p++) {
+        const float l[3] = {lane_below(s[0]), lane_below(s[1]), lane_below(s[2])};
+        const float a[3] = {lane_above(s[0]), lane_above(s[1]), lane_above(s[2])};
+        float o[3];
+        stencil(f.sa[p], f.sb[p], l, s, a, o);
+        for (int c = 0; c < 3; c++) s[c] = live_x ? o[c] : s[c];
+    }
+    for (int c = 0; c < 3; c++) cur[own + c] = s[c];
+    __syncthreads();
+    const bool live_y = in_x && (ring || inner) && w > 0 && w < waves - 1;
+    for (int p = 0; p < n2; p++) {
+        if (live_y) {
+            const float *l = (p == 0 && ring && cr == 0 ? raw : cur) + own - 3 * 64;
+            const float *a = (p == 0 && ring && cr == ny - 1 ? raw : cur) + own + 3 * 64;
+            float o[3];
+            stencil(f.sa[n1 + p], f.sb[n1 + p], l, s, a, o);
+            for (int c = 0; c < 3; c++) s[c] = o[c];
+        }
+        for (int c = 0; c < 3; c++) nxt[own + c] = s[c];
+        __syncthreads();
+        float *t = cur;
+        cur = nxt;
+        nxt = t;
+    }
+    if (!out) return;
+    if (u == 0 && w == n2 + X && lane == 0) zk_stamp_open(f.stamp);
+    for (int c = 0; c < 3; c++) {
+        if (X) y.jj[1][c] = cur[own - 3 * 64 + c];
+        y.jj[1 + X][c] = s[c];
+        y.jj[2 + X][c] = cur[own + 3 * 64 + c];
+    }
+    if (lane >= l0 && lane < l0 + cols && col) {
+        float *o = f.r.J + 3 * ((size_t)bi + (size_t)(j + 1) * nrow);
+        o[0] = s[0];
+        o[1] = s[1];
+        o[2] = s[2];
+    }
+    y.step(f.E, f.Eo, f.Bo, nx, ny, nrow, f.k, bi, j + 1, l0, cols, c0, px, oy, f.shift);
+    if (blockIdx.x + 1 == gridDim.x && w == n2 + X && lane == 0) zk_stamp_close(f.stamp);
+}
+
+YeeK yee_constants(float dt, float dx, float dy)
+{
+    YeeK k;
+    const float dt2 = dt / 2.0f;
+    k.dtx2 = dt2 / dx;
+    k.dty2 = dt2 / dy;
+    k.dtx = dt / dx;
+    k.dty = dt / dy;
+    k.dt = dt;
+    k.mur_y = (dt - dy) / (dt + dy);
+    return k;
 }
 
 __global__ void guard_kernel(float *E, float *B, int nx, int ny, int nrow, int periodic_x, int open_y)
@@ -440,14 +572,7 @@ extern "C" int zk_yee(const float *E, const float *B, const float *J, float *Eo,
                              int nrow, float dt, float dx, float dy, int periodic_x, int open_y, int shift, zk_stamp st,
                       zk_stream_t s)
 {
-    YeeK k;
-    const float dt2 = dt / 2.0f;
-    k.dtx2 = dt2 / dx;
-    k.dty2 = dt2 / dy;
-    k.dtx = dt / dx;
-    k.dty = dt / dy;
-    k.dt = dt;
-    k.mur_y = (dt - dy) / (dt + dy);
+    const YeeK k = yee_constants(dt, dx, dy);
     const int r = zk_yee_rows(nx, ny), units = zk_yee_units(nx, ny, r);
     if (r == ZK_YEE_R_SMALL)
         hipLaunchKernelGGL(yee_kernel<ZK_YEE_R_SMALL>, dim3(units), dim3(64), 0, s, E, B, J, Eo, Bo, nx, ny, nrow, k,
@@ -455,6 +580,37 @@ extern "C" int zk_yee(const float *E, const float *B, const float *J, float *Eo,
     else
         hipLaunchKernelGGL(yee_kernel<ZK_YEE_R>, dim3((units + 3) / 4), dim3(256), 0, s, E, B, J, Eo, Bo, nx, ny, nrow,
                            k, periodic_x, open_y, shift, units, st);
+    ZK_LAUNCH_CHECK();
+}
+
+/* From here on the separate launches read each window and node once and cost
+ * no more: 256 x 256 cells 10.0 us in one launch, 16.1 in three; 512 x 512
+ * the same with the gap between two; 2000 x 512 22.2 and 22.0, the run 1.5 %
+ * longer in one; 2048 x 2048 210 and 175. */
+#define ZK_FIELD_STEP_NODES (1 << 19)
+
+extern "C" int zk_field_step_ok(const zk_tiles *t, int n1, int n2, int open_y)
+{
+    return reduce_span(*t) != 0 && n1 <= ZK_MAX_PASSES && n2 <= ZK_MAX_Y_PASSES && field_rows(16, n2, open_y) >= 4 &&
+           (long long)(t->nx + 3) * (t->ny + 3) < ZK_FIELD_STEP_NODES;
+}
+
+extern "C" int zk_field_step(const zk_field_args *args, float dt, float dx, float dy, zk_stream_t s)
+{
+    zk_field_args f = *args;
+    const int nx = f.r.t.nx, ny = f.r.t.ny, oy = f.r.open_y != 0;
+    if (!zk_field_step_ok(&f.r.t, f.n1, f.n2, oy) || f.n1 < 0 || f.n2 < 0) return (int)hipErrorInvalidValue;
+    f.k = yee_constants(dt, dx, dy);
+    const int waves = field_waves(f.n2, oy), rows = field_rows(waves, f.n2, oy), cols = field_cols(f.n1);
+    f.clears = f.r.jflag_next ? (zk_red_blocks_x(nx) * zk_red_blocks_y(ny) + waves - 1) / waves : 0;
+    const int units = (nx + 3 + cols - 1) / cols * ((ny + 3 + rows - 1) / rows);
+    const dim3 grid(f.r.fin.n + f.clears + units), block(64 * waves);
+    const size_t lds = sizeof(float) * 3 * 3 * 64 * waves;
+    const int span = reduce_span(f.r.t);
+    if (span == 2 && !oy) hipLaunchKernelGGL((field_step_kernel<2, 0>), grid, block, lds, s, f);
+    else if (span == 2) hipLaunchKernelGGL((field_step_kernel<2, 1>), grid, block, lds, s, f);
+    else if (!oy) hipLaunchKernelGGL((field_step_kernel<3, 0>), grid, block, lds, s, f);
+    else hipLaunchKernelGGL((field_step_kernel<3, 1>), grid, block, lds, s, f);
     ZK_LAUNCH_CHECK();
 }
 

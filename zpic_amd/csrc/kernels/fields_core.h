@@ -47,11 +47,11 @@ __device__ inline void yee_store(float *__restrict__ Eo, float *__restrict__ Bo,
     }
 }
 
-/* One field step of R output rows by ZK_YEE_W output columns, unit `u` of the
- * buffer (units in rows of zk_yee_units_x(nx)), by one wave: a column per
- * lane, the rows in registers.  A half step of B reaches one column right
- * and one row up, the whole step of E one left and one down, so the wave
- * reads one column and row below its outputs and two above.
+/* One field step of R rows of the buffer from row bj0 on, by one wave: a
+ * column per lane (buffer column bi), the rows in registers.  A half step of
+ * B reaches one column right and one row up, the whole step of E one left
+ * and one down, so the wave reads one column and row below its outputs and
+ * two above; X = 1: one more row below.
  *
  * The step is a few operations per byte: what bounds it is the reads and
  * writes on large grids and the latency of one read elsewhere.  Lane shifts
@@ -68,103 +68,137 @@ __device__ inline void yee_store(float *__restrict__ Eo, float *__restrict__ Bo,
  * the tangential components Ex, Ez of the guard rows j = -1 and j = ny
  * become E_in(n) + S (E_in(n+1) - E_guard(n)) with E_in the adjacent
  * interior row (0, ny - 1) and S = (dt - dy) / (dt + dy); the old values
- * are read from the input buffer E, which the kernel does not write.  The
- * top unit ends at the last row (and repeats rows of the one below), so
- * that row ny - 1 is in a wave that writes row ny. */
+ * are read from the input buffer E, which the kernel does not write.  A wave
+ * that writes row ny needs the whole step on row ny - 1: either the row is
+ * one of its own or X is 1. */
+template <int R, int X>
+struct YeeRows {
+    float e[R + 3 + X][3], b[R + 2 + X][3], jj[R + 2 + X][3]; /* row v is buffer row bj0 - 1 - X + v */
+
+    __device__ void load(const float *__restrict__ E, const float *__restrict__ B, int nx, int ny, int nrow, int bi,
+                         int bj0)
+    {
+#pragma unroll
+        for (int v = 0; v < R + 3 + X; v++) {
+            const int bj = bj0 - 1 - X + v;
+            const bool in = bi >= 0 && bi < nx + 3 && bj >= 0 && bj < ny + 3;
+            const size_t g = in ? 3 * ((size_t)bi + (size_t)bj * nrow) : 0;
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                e[v][c] = in ? E[g + c] : 0.0f;
+                if (v < R + 2 + X) b[v][c] = in ? B[g + c] : 0.0f;
+            }
+        }
+    }
+
+    __device__ void load_j(const float *__restrict__ J, int nx, int ny, int nrow, int bi, int bj0)
+    {
+#pragma unroll
+        for (int v = 1; v < R + 2 + X; v++) {
+            const int bj = bj0 - 1 - X + v;
+            const bool in = bi >= 0 && bi < nx + 3 && bj >= 0 && bj < ny + 3;
+            const size_t g = in ? 3 * ((size_t)bi + (size_t)bj * nrow) : 0;
+#pragma unroll
+            for (int c = 0; c < 3; c++) jj[v][c] = in ? J[g + c] : 0.0f;
+        }
+    }
+
+    /* the step, and the R rows of lanes [l0, l0 + w), whose first holds
+     * buffer column c0, to Eo and Bo */
+    __device__ void step(const float *__restrict__ E, float *__restrict__ Eo, float *__restrict__ Bo, int nx, int ny,
+                         int nrow, const YeeK &k, int bi, int bj0, int l0, int w, int c0, int periodic_x, int open_y,
+                         int shift)
+    {
+        const int lane = __lane_id();
+        const int bw = nx + 3, bh = ny + 3;
+        const int i = bi - 1, j0 = bj0 - 2 - X; /* raw column, raw row of e[0] */
+        const bool half_x = i >= -1 && i <= nx, whole_x = i >= 0 && i <= nx + 1;
+        /* B1 = B + dt/2 * (-curl E) */
+#pragma unroll
+        for (int v = 0; v < R + 2 + X; v++) {
+            const bool f = half_x && j0 + v >= -1 && j0 + v <= ny;
+            const float ea1 = lane_above(e[v][1]), ea2 = lane_above(e[v][2]);
+            const float x = b[v][0] + (-k.dty2 * (e[v + 1][2] - e[v][2]));
+            const float y = b[v][1] + (k.dtx2 * (ea2 - e[v][2]));
+            const float z = b[v][2] + (-k.dtx2 * (ea1 - e[v][1]) + k.dty2 * (e[v + 1][0] - e[v][0]));
+            b[v][0] = f ? x : b[v][0];
+            b[v][1] = f ? y : b[v][1];
+            b[v][2] = f ? z : b[v][2];
+        }
+        /* E1 = E + dt * (curl B1 - J) */
+#pragma unroll
+        for (int v = 1; v < R + 2 + X; v++) {
+            const bool f = whole_x && j0 + v >= 0 && j0 + v <= ny + 1;
+            const float bb1 = lane_below(b[v][1]), bb2 = lane_below(b[v][2]);
+            const float x = e[v][0] + ((+k.dty * (b[v][2] - b[v - 1][2])) - k.dt * jj[v][0]);
+            const float y = e[v][1] + ((-k.dtx * (b[v][2] - bb2)) - k.dt * jj[v][1]);
+            const float z = e[v][2] + ((+k.dtx * (b[v][1] - bb1) - k.dty * (b[v][0] - b[v - 1][0])) - k.dt * jj[v][2]);
+            e[v][0] = f ? x : e[v][0];
+            e[v][1] = f ? y : e[v][1];
+            e[v][2] = f ? z : e[v][2];
+        }
+        if (open_y && (bj0 <= X || bj0 + R >= ny + 1)) {
+#pragma unroll
+            for (int v = 1; v < R + 2 + X; v++) {
+                const int jb = j0 + v;
+                if ((jb != -1 && jb != ny) || bi < 0 || bi >= bw) continue;
+                const int d = jb == -1 ? 1 : -1; /* towards the interior */
+                const size_t gb = 3 * ((size_t)bi + (size_t)(jb + 1) * nrow);
+                const size_t gi = 3 * ((size_t)bi + (size_t)(jb + 1 + d) * nrow);
+                const float up0 = e[v + 1][0], up2 = e[v + 1][2], dn0 = e[v - 1][0], dn2 = e[v - 1][2];
+                e[v][0] = E[gi + 0] + k.mur_y * ((d > 0 ? up0 : dn0) - E[gb + 0]);
+                e[v][2] = E[gi + 2] + k.mur_y * ((d > 0 ? up2 : dn2) - E[gb + 2]);
+            }
+        }
+        /* rows holding guards, or nodes that guards are images of */
+        const bool edge = (periodic_x && (c0 <= 2 || c0 + w > nx)) || (!open_y && (bj0 <= 2 || bj0 + R > ny));
+        /* B2 = B1 + dt/2 * (-curl E1) and outputs */
+#pragma unroll
+        for (int v = 1 + X; v < R + 1 + X; v++) {
+            const int bj = bj0 - 1 - X + v, j = bj - 1;
+            const bool f = half_x && j >= -1 && j <= ny;
+            const float ea1 = lane_above(e[v][1]), ea2 = lane_above(e[v][2]);
+            const float x = b[v][0] + (-k.dty2 * (e[v + 1][2] - e[v][2]));
+            const float y = b[v][1] + (k.dtx2 * (ea2 - e[v][2]));
+            const float z = b[v][2] + (-k.dtx2 * (ea1 - e[v][1]) + k.dty2 * (e[v + 1][0] - e[v][0]));
+            if (lane < l0 || lane >= l0 + w || bi >= bw || bj >= bh) continue;
+            const float bn[3] = {f ? x : b[v][0], f ? y : b[v][1], f ? z : b[v][2]};
+            const float en[3] = {e[v][0], e[v][1], e[v][2]};
+            if (!edge) {
+                yee_store(Eo, Bo, nx, nrow, bi, bj, en, bn, shift);
+                continue;
+            }
+            /* the images of an interior index c on a periodic axis of n cells:
+             * c - n when that is the lower guard, c, and c + n, ... up to n + 1 */
+            const bool cy = !open_y;
+            if ((periodic_x && (i < 0 || i >= nx)) || (cy && (j < 0 || j >= ny))) continue;
+            for (int gj = cy && j - ny >= -1 ? j - ny : j; gj <= ny + 1; gj += ny) {
+                for (int gi = periodic_x && i - nx >= -1 ? i - nx : i; gi <= nx + 1; gi += nx) {
+                    yee_store(Eo, Bo, nx, nrow, gi + 1, gj + 1, en, bn, shift);
+                    if (!periodic_x) break;
+                }
+                if (!cy) break;
+            }
+        }
+    }
+};
+
+/* Unit u of the buffer: R rows by ZK_YEE_W columns, units in rows of
+ * zk_yee_units_x(nx).  With open y the top units end at the last row (and
+ * repeat rows of those below), which keeps rows ny - 1 and ny together. */
 template <int R>
 __device__ inline void yee_rows(const float *__restrict__ E, const float *__restrict__ B, const float *__restrict__ J,
                                 float *__restrict__ Eo, float *__restrict__ Bo, int nx, int ny, int nrow,
                                 const YeeK &k, const int u, const int periodic_x, const int open_y = 0,
                                 const int shift = 0)
 {
-    const int bw = nx + 3, bh = ny + 3;
-    const int lane = __lane_id();
     const int ux = zk_yee_units_x(nx);
-    const int c0 = u % ux * ZK_YEE_W, bi = c0 - 1 + lane, i = bi - 1;
-    const int bj0 = open_y ? max(0, min(u / ux * R, bh - R)) : u / ux * R; /* first output row */
-    const int j0 = bj0 - 2;                                               /* raw row of e[0], b[0] */
-    const bool col = bi >= 0 && bi < bw;
-    float e[R + 3][3], b[R + 2][3], jj[R + 2][3];
-#pragma unroll
-    for (int v = 0; v < R + 3; v++) {
-        const int bj = bj0 - 1 + v;
-        const bool in = col && bj >= 0 && bj < bh;
-        const size_t g = in ? 3 * ((size_t)bi + (size_t)bj * nrow) : 0;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            e[v][c] = in ? E[g + c] : 0.0f;
-            if (v < R + 2) b[v][c] = in ? B[g + c] : 0.0f;
-            if (v > 0 && v < R + 2) jj[v][c] = in ? J[g + c] : 0.0f;
-        }
-    }
-    const bool half_x = i >= -1 && i <= nx, whole_x = i >= 0 && i <= nx + 1;
-    /* B1 = B + dt/2 * (-curl E) */
-#pragma unroll
-    for (int v = 0; v < R + 2; v++) {
-        const bool f = half_x && j0 + v >= -1 && j0 + v <= ny;
-        const float ea1 = lane_above(e[v][1]), ea2 = lane_above(e[v][2]);
-        const float x = b[v][0] + (-k.dty2 * (e[v + 1][2] - e[v][2]));
-        const float y = b[v][1] + (k.dtx2 * (ea2 - e[v][2]));
-        const float z = b[v][2] + (-k.dtx2 * (ea1 - e[v][1]) + k.dty2 * (e[v + 1][0] - e[v][0]));
-        b[v][0] = f ? x : b[v][0];
-        b[v][1] = f ? y : b[v][1];
-        b[v][2] = f ? z : b[v][2];
-    }
-    /* E1 = E + dt * (curl B1 - J) */
-#pragma unroll
-    for (int v = 1; v < R + 2; v++) {
-        const bool f = whole_x && j0 + v >= 0 && j0 + v <= ny + 1;
-        const float bb1 = lane_below(b[v][1]), bb2 = lane_below(b[v][2]);
-        const float x = e[v][0] + ((+k.dty * (b[v][2] - b[v - 1][2])) - k.dt * jj[v][0]);
-        const float y = e[v][1] + ((-k.dtx * (b[v][2] - bb2)) - k.dt * jj[v][1]);
-        const float z = e[v][2] + ((+k.dtx * (b[v][1] - bb1) - k.dty * (b[v][0] - b[v - 1][0])) - k.dt * jj[v][2]);
-        e[v][0] = f ? x : e[v][0];
-        e[v][1] = f ? y : e[v][1];
-        e[v][2] = f ? z : e[v][2];
-    }
-    if (open_y && (bj0 == 0 || bj0 + R >= ny + 1)) {
-#pragma unroll
-        for (int v = 1; v < R + 2; v++) {
-            const int jb = j0 + v;
-            if ((jb != -1 && jb != ny) || !col) continue;
-            const int d = jb == -1 ? 1 : -1; /* towards the interior */
-            const size_t gb = 3 * ((size_t)bi + (size_t)(jb + 1) * nrow);
-            const size_t gi = 3 * ((size_t)bi + (size_t)(jb + 1 + d) * nrow);
-            const float up0 = e[v + 1][0], up2 = e[v + 1][2], dn0 = e[v - 1][0], dn2 = e[v - 1][2];
-            e[v][0] = E[gi + 0] + k.mur_y * ((d > 0 ? up0 : dn0) - E[gb + 0]);
-            e[v][2] = E[gi + 2] + k.mur_y * ((d > 0 ? up2 : dn2) - E[gb + 2]);
-        }
-    }
-    /* units holding guards, or nodes that guards are images of */
-    const bool edge = (periodic_x && (c0 <= 2 || c0 + ZK_YEE_W > nx)) || (!open_y && (bj0 <= 2 || bj0 + R > ny));
-    /* B2 = B1 + dt/2 * (-curl E1) and outputs */
-#pragma unroll
-    for (int v = 1; v < R + 1; v++) {
-        const int bj = bj0 - 1 + v, j = bj - 1;
-        const bool f = half_x && j >= -1 && j <= ny;
-        const float ea1 = lane_above(e[v][1]), ea2 = lane_above(e[v][2]);
-        const float x = b[v][0] + (-k.dty2 * (e[v + 1][2] - e[v][2]));
-        const float y = b[v][1] + (k.dtx2 * (ea2 - e[v][2]));
-        const float z = b[v][2] + (-k.dtx2 * (ea1 - e[v][1]) + k.dty2 * (e[v + 1][0] - e[v][0]));
-        if (lane < 1 || lane > ZK_YEE_W || bi >= bw || bj >= bh) continue;
-        const float bn[3] = {f ? x : b[v][0], f ? y : b[v][1], f ? z : b[v][2]};
-        const float en[3] = {e[v][0], e[v][1], e[v][2]};
-        if (!edge) {
-            yee_store(Eo, Bo, nx, nrow, bi, bj, en, bn, shift);
-            continue;
-        }
-        /* the images of an interior index c on a periodic axis of n cells:
-         * c - n when that is the lower guard, c, and c + n, ... up to n + 1 */
-        const bool cy = !open_y;
-        if ((periodic_x && (i < 0 || i >= nx)) || (cy && (j < 0 || j >= ny))) continue;
-        for (int gj = cy && j - ny >= -1 ? j - ny : j; gj <= ny + 1; gj += ny) {
-            for (int gi = periodic_x && i - nx >= -1 ? i - nx : i; gi <= nx + 1; gi += nx) {
-                yee_store(Eo, Bo, nx, nrow, gi + 1, gj + 1, en, bn, shift);
-                if (!periodic_x) break;
-            }
-            if (!cy) break;
-        }
-    }
+    const int c0 = u % ux * ZK_YEE_W, bi = c0 - 1 + (int)__lane_id();
+    const int bj0 = open_y ? max(0, min(u / ux * R, ny + 3 - R)) : u / ux * R;
+    YeeRows<R, 0> y;
+    y.load(E, B, nx, ny, nrow, bi, bj0);
+    y.load_j(J, nx, ny, nrow, bi, bj0);
+    y.step(E, Eo, Bo, nx, ny, nrow, k, bi, bj0, 1, ZK_YEE_W, c0, periodic_x, open_y, shift);
 }
 
 /* Guard nodes take the value of their image: x (unless the window moves)

@@ -265,6 +265,25 @@ int zk_current_reduce(const zk_reduce_args *a, zk_stream_t s);
 int zk_smooth(const float *in, float *out, int nx, int ny, int nrow, int n1, int n2, const float *sa, const float *sb,
               int periodic_x, int open_y, zk_stream_t s);
 
+/* zk_current_reduce, zk_smooth and zk_yee of one step in one launch, for
+ * grids small enough to be bound by launches (same J, E and B bit for bit);
+ * zk_field_step_ok: whether it takes this grid and these passes */
+typedef struct zk_yee_k {
+    float dtx2, dty2, dtx, dty, dt, mur_y;
+} zk_yee_k;
+typedef struct zk_field_args {
+    zk_reduce_args r;
+    const float *E, *B;
+    float *Eo, *Bo;
+    zk_yee_k k;                 /* set by zk_field_step */
+    int shift, n1, n2;
+    float sa[ZK_MAX_PASSES + ZK_MAX_Y_PASSES], sb[ZK_MAX_PASSES + ZK_MAX_Y_PASSES];
+    int clears;                 /* set by zk_field_step: workgroups that clear Jov_next */
+    zk_stamp stamp;             /* of the field step */
+} zk_field_args;
+int zk_field_step_ok(const zk_tiles *t, int n1, int n2, int open_y);
+int zk_field_step(const zk_field_args *f, float dt, float dx, float dy, zk_stream_t s);
+
 /* fields */
 /* One field step, guard cells of the outputs included (periodic_x: along
  * x; along y unless open_y).  open_y: first-order Mur absorbing boundaries at the y edges; shift: the
@@ -387,9 +406,6 @@ int zk_init_mean(const zk_init_args *a, float *mean, int nkeys, zk_stream_t s);
 
 /* Yee constants: (dt/2)/dx, (dt/2)/dy, dt/dx, dt/dy, dt, and the Mur
  * coefficient (dt - dy)/(dt + dy) of open y boundaries */
-typedef struct zk_yee_k {
-    float dtx2, dty2, dtx, dty, dt, mur_y;
-} zk_yee_k;
 
 /* One simulation of a batch.  ecur/jcur select the current E,B and J
  * buffers and are advanced on the device at the end of every step. */
