@@ -362,21 +362,43 @@ void emf_set_ext_fld(t_emf *const emf, t_emf_ext_fld *ext)
 
 /* ---- device residency ---- */
 
-static void part_fields(t_emf *emf)
+/* the external fields of the grid, in zk_ext's form */
+static void ext_args(t_emf *emf, zk_ext *x)
 {
     struct zpic_dev_emf *d = emf->dev;
-    const size_t nodes = zpic_grid_nodes(emf->nx);
-    const t_emf_ext_fld *x = &emf->ext_fld;
-    if (x->E_type != EMF_FLD_TYPE_NONE) {
-        if (!d->Ep) d->Ep = zpic_dmalloc(sizeof(float3) * nodes);
-        ZCHECK(zk_add_ext(d->E[d->cur], x->E_type == EMF_FLD_TYPE_CUSTOM ? d->Eext : NULL, x->E_0.x, x->E_0.y,
-                          x->E_0.z, d->Ep, nodes, zpic_stream()));
+    const t_emf_ext_fld *f = &emf->ext_fld;
+    const size_t bytes = sizeof(float3) * zpic_grid_nodes(emf->nx);
+    memset(x, 0, sizeof(*x));
+    if (f->E_type != EMF_FLD_TYPE_NONE) {
+        if (!d->Ep) d->Ep = zpic_dmalloc(bytes);
+        x->out[0] = d->Ep;
+        x->grid[0] = f->E_type == EMF_FLD_TYPE_CUSTOM ? d->Eext : NULL;
+        x->uniform[0][0] = f->E_0.x;
+        x->uniform[0][1] = f->E_0.y;
+        x->uniform[0][2] = f->E_0.z;
     }
-    if (x->B_type != EMF_FLD_TYPE_NONE) {
-        if (!d->Bp) d->Bp = zpic_dmalloc(sizeof(float3) * nodes);
-        ZCHECK(zk_add_ext(d->B[d->cur], x->B_type == EMF_FLD_TYPE_CUSTOM ? d->Bext : NULL, x->B_0.x, x->B_0.y,
-                          x->B_0.z, d->Bp, nodes, zpic_stream()));
+    if (f->B_type != EMF_FLD_TYPE_NONE) {
+        if (!d->Bp) d->Bp = zpic_dmalloc(bytes);
+        x->out[1] = d->Bp;
+        x->grid[1] = f->B_type == EMF_FLD_TYPE_CUSTOM ? d->Bext : NULL;
+        x->uniform[1][0] = f->B_0.x;
+        x->uniform[1][1] = f->B_0.y;
+        x->uniform[1][2] = f->B_0.z;
     }
+}
+
+/* the particles' fields from the fields as they are (the field step writes
+ * them itself) */
+static void part_fields(t_emf *emf)
+{
+    const struct zpic_dev_emf *d = emf->dev;
+    const float *F[2] = {d->E[d->cur], d->B[d->cur]};
+    zk_ext x;
+    ext_args(emf, &x);
+    for (int k = 0; k < 2; k++)
+        if (x.out[k])
+            ZCHECK(zk_add_ext(F[k], x.grid[k], x.uniform[k][0], x.uniform[k][1], x.uniform[k][2], x.out[k],
+                              zpic_grid_nodes(emf->nx), zpic_stream()));
 }
 
 void zpic_emf_ensure(t_emf *emf)
@@ -462,7 +484,10 @@ static void advance(t_emf *emf, t_current *cur, zk_field_args *cf)
     const int move = emf->moving_window && ((emf->iter + 1) * emf->dt) > emf->dx[0] * (emf->n_move + 1);
     const int fused = move && zpic_window_shift_fusion() && emf->ext_fld.E_type == EMF_FLD_TYPE_NONE &&
                       emf->ext_fld.B_type == EMF_FLD_TYPE_NONE;
+    zk_ext ext;
+    ext_args(emf, &ext);
     if (cf) {
+        cf->ext = ext;
         cf->E = d->E[d->cur];
         cf->B = d->B[d->cur];
         cf->Eo = d->E[o];
@@ -473,13 +498,12 @@ static void advance(t_emf *emf, t_current *cur, zk_field_args *cf)
         zpic_current_field_done(cur, cf);
     } else {
         zpic_ktimer_begin(ZPIC_T_FIELD);
-        ZCHECK(zk_yee(d->E[d->cur], d->B[d->cur], zpic_current_J(cur), d->E[o], d->B[o], emf->nx[0], emf->nx[1],
-                      emf->nrow, emf->dt, emf->dx[0], emf->dx[1], !emf->moving_window, d->open_y, fused, st,
-                      zpic_stream()));
+        ZCHECK(zk_yee_ext(d->E[d->cur], d->B[d->cur], zpic_current_J(cur), d->E[o], d->B[o], emf->nx[0], emf->nx[1],
+                          emf->nrow, emf->dt, emf->dx[0], emf->dx[1], !emf->moving_window, d->open_y, fused, &ext, st,
+                          zpic_stream()));
         zpic_ktimer_end(ZPIC_T_FIELD);
     }
     d->cur = o;
-    part_fields(emf);
     emf->iter += 1;
     if (fused) {
         emf->n_move++;
@@ -490,8 +514,7 @@ static void advance(t_emf *emf, t_current *cur, zk_field_args *cf)
         d->cur = m;
         emf->n_move++;
     }
-    zpic_phase_end(ZPIC_T_EMF, (move && !fused) || emf->ext_fld.E_type != EMF_FLD_TYPE_NONE ||
-                                   emf->ext_fld.B_type != EMF_FLD_TYPE_NONE);
+    zpic_phase_end(ZPIC_T_EMF, move && !fused);
     d->host_valid = 0;
 }
 

@@ -33,16 +33,17 @@ static __device__ __align__(256) float scratch[2 * ZK_NOALLOC_CHARGE_MAX];
 
 namespace {
 
-template <int R>
+template <int R, bool EXT>
 __global__ void __launch_bounds__(256) yee_kernel(const float *__restrict__ E, const float *__restrict__ B,
                                                   const float *__restrict__ J, float *__restrict__ Eo,
                                                   float *__restrict__ Bo, int nx, int ny, int nrow, YeeK k,
-                                                  int periodic_x, int open_y, int shift, int units, zk_stamp st)
+                                                  int periodic_x, int open_y, int shift, int units, zk_ext ext,
+                                                  zk_stamp st)
 {
     zk_stamp_first(st);
     /* contiguous runs of units per XCD: neighbours share their margins in L2 */
     const int u = zk_xcd_item(blockIdx.x, gridDim.x) * (blockDim.x / 64) + threadIdx.x / 64;
-    if (u < units) yee_rows<R>(E, B, J, Eo, Bo, nx, ny, nrow, k, u, periodic_x, open_y, shift);
+    if (u < units) yee_rows<R>(E, B, J, Eo, Bo, nx, ny, nrow, k, u, periodic_x, open_y, shift, EXT ? ext : zk_ext());
     zk_stamp_last(st);
 }
 
@@ -159,7 +160,7 @@ __global__ void __launch_bounds__(1024) field_step_kernel(zk_field_args f)
         o[1] = s[1];
         o[2] = s[2];
     }
-    y.step(f.E, f.Eo, f.Bo, nx, ny, nrow, f.k, bi, j + 1, l0, cols, c0, px, oy, f.shift);
+    y.step(f.E, f.Eo, f.Bo, nx, ny, nrow, f.k, bi, j + 1, l0, cols, c0, px, oy, f.shift, f.ext);
     if (blockIdx.x + 1 == gridDim.x && w == n2 + X && lane == 0) zk_stamp_close(f.stamp);
 }
 
@@ -568,19 +569,30 @@ extern "C" int zk_pha(const zk_parts *p, int np_upper, const zk_spec_ctr *ctr, i
     ZK_LAUNCH_CHECK();
 }
 
-extern "C" int zk_yee(const float *E, const float *B, const float *J, float *Eo, float *Bo, int nx, int ny,
-                             int nrow, float dt, float dx, float dy, int periodic_x, int open_y, int shift, zk_stamp st,
-                      zk_stream_t s)
+extern "C" int zk_yee_ext(const float *E, const float *B, const float *J, float *Eo, float *Bo, int nx, int ny,
+                          int nrow, float dt, float dx, float dy, int periodic_x, int open_y, int shift,
+                          const zk_ext *ext, zk_stamp st, zk_stream_t s)
 {
+    if (shift && (ext->out[0] || ext->out[1])) return (int)hipErrorInvalidValue;
     const YeeK k = yee_constants(dt, dx, dy);
     const int r = zk_yee_rows(nx, ny), units = zk_yee_units(nx, ny, r);
-    if (r == ZK_YEE_R_SMALL)
-        hipLaunchKernelGGL(yee_kernel<ZK_YEE_R_SMALL>, dim3(units), dim3(64), 0, s, E, B, J, Eo, Bo, nx, ny, nrow, k,
-                           periodic_x, open_y, shift, units, st);
-    else
-        hipLaunchKernelGGL(yee_kernel<ZK_YEE_R>, dim3((units + 3) / 4), dim3(256), 0, s, E, B, J, Eo, Bo, nx, ny, nrow,
-                           k, periodic_x, open_y, shift, units, st);
+    const bool x = ext->out[0] || ext->out[1];
+#define YEE(R, X, WAVES)                                                                                              \
+    hipLaunchKernelGGL((yee_kernel<R, X>), dim3((units + WAVES - 1) / WAVES), dim3(64 * WAVES), 0, s, E, B, J, Eo,    \
+                       Bo, nx, ny, nrow, k, periodic_x, open_y, shift, units, *ext, st)
+    if (r == ZK_YEE_R_SMALL && x) YEE(ZK_YEE_R_SMALL, true, 1);
+    else if (r == ZK_YEE_R_SMALL) YEE(ZK_YEE_R_SMALL, false, 1);
+    else if (x) YEE(ZK_YEE_R, true, 4);
+    else YEE(ZK_YEE_R, false, 4);
+#undef YEE
     ZK_LAUNCH_CHECK();
+}
+
+extern "C" int zk_yee(const float *E, const float *B, const float *J, float *Eo, float *Bo, int nx, int ny, int nrow,
+                      float dt, float dx, float dy, int periodic_x, int open_y, int shift, zk_stamp st, zk_stream_t s)
+{
+    const zk_ext none = {};
+    return zk_yee_ext(E, B, J, Eo, Bo, nx, ny, nrow, dt, dx, dy, periodic_x, open_y, shift, &none, st, s);
 }
 
 /* From here on the separate launches read each window and node once and cost
@@ -599,7 +611,9 @@ extern "C" int zk_field_step(const zk_field_args *args, float dt, float dx, floa
 {
     zk_field_args f = *args;
     const int nx = f.r.t.nx, ny = f.r.t.ny, oy = f.r.open_y != 0;
-    if (!zk_field_step_ok(&f.r.t, f.n1, f.n2, oy) || f.n1 < 0 || f.n2 < 0) return (int)hipErrorInvalidValue;
+    if (!zk_field_step_ok(&f.r.t, f.n1, f.n2, oy) || f.n1 < 0 || f.n2 < 0 ||
+        (f.shift && (f.ext.out[0] || f.ext.out[1])))
+        return (int)hipErrorInvalidValue;
     f.k = yee_constants(dt, dx, dy);
     const int waves = field_waves(f.n2, oy), rows = field_rows(waves, f.n2, oy), cols = field_cols(f.n1);
     f.clears = f.r.jflag_next ? (zk_red_blocks_x(nx) * zk_red_blocks_y(ny) + waves - 1) / waves : 0;

@@ -23,9 +23,18 @@ typedef zk_yee_k YeeK; /* (dt/2)/dx, (dt/2)/dy, dt/dx, dt/dy, dt, Mur coefficien
  * (a launch of 3.5-4.5 us at any grid size: 11 % of a 32 x 32 step's
  * kernels, 5 % of a vacuum step at 2000 x 512).  Tiles away from the edges
  * keep the plain store. */
+/* ext: the fields the particles see, E and B plus the external ones
+ * (em2d/emf.c:432-470), are written with them (a launch of 2.6 us for each
+ * of the two, and one for the phase's clock, on a 97 x 61 grid). */
 __device__ inline void yee_store(float *__restrict__ Eo, float *__restrict__ Bo, int nx, int nrow, int bi, int bj,
-                                 const float *e, const float *b, int shift)
+                                 const float *e, const float *b, int shift, const zk_ext &ext)
 {
+    for (int f = 0; f < 2; f++) {
+        if (!ext.out[f]) continue;
+        const size_t g = 3 * ((size_t)bi + (size_t)bj * nrow);
+        for (int c = 0; c < 3; c++)
+            ext.out[f][g + c] = (f ? b[c] : e[c]) + (ext.grid[f] ? ext.grid[f][g + c] : ext.uniform[f][c]);
+    }
     if (shift) {
         /* buffer column bi goes to bi - 1 (raw i - 1); raw columns from
          * nx - 1 on are zero, the last one written by the last node */
@@ -107,7 +116,7 @@ struct YeeRows {
      * buffer column c0, to Eo and Bo */
     __device__ void step(const float *__restrict__ E, float *__restrict__ Eo, float *__restrict__ Bo, int nx, int ny,
                          int nrow, const YeeK &k, int bi, int bj0, int l0, int w, int c0, int periodic_x, int open_y,
-                         int shift)
+                         int shift, const zk_ext &ext)
     {
         const int lane = __lane_id();
         const int bw = nx + 3, bh = ny + 3;
@@ -165,7 +174,7 @@ struct YeeRows {
             const float bn[3] = {f ? x : b[v][0], f ? y : b[v][1], f ? z : b[v][2]};
             const float en[3] = {e[v][0], e[v][1], e[v][2]};
             if (!edge) {
-                yee_store(Eo, Bo, nx, nrow, bi, bj, en, bn, shift);
+                yee_store(Eo, Bo, nx, nrow, bi, bj, en, bn, shift, ext);
                 continue;
             }
             /* the images of an interior index c on a periodic axis of n cells:
@@ -174,7 +183,7 @@ struct YeeRows {
             if ((periodic_x && (i < 0 || i >= nx)) || (cy && (j < 0 || j >= ny))) continue;
             for (int gj = cy && j - ny >= -1 ? j - ny : j; gj <= ny + 1; gj += ny) {
                 for (int gi = periodic_x && i - nx >= -1 ? i - nx : i; gi <= nx + 1; gi += nx) {
-                    yee_store(Eo, Bo, nx, nrow, gi + 1, gj + 1, en, bn, shift);
+                    yee_store(Eo, Bo, nx, nrow, gi + 1, gj + 1, en, bn, shift, ext);
                     if (!periodic_x) break;
                 }
                 if (!cy) break;
@@ -190,7 +199,7 @@ template <int R>
 __device__ inline void yee_rows(const float *__restrict__ E, const float *__restrict__ B, const float *__restrict__ J,
                                 float *__restrict__ Eo, float *__restrict__ Bo, int nx, int ny, int nrow,
                                 const YeeK &k, const int u, const int periodic_x, const int open_y = 0,
-                                const int shift = 0)
+                                const int shift = 0, const zk_ext &ext = zk_ext())
 {
     const int ux = zk_yee_units_x(nx);
     const int c0 = u % ux * ZK_YEE_W, bi = c0 - 1 + (int)__lane_id();
@@ -198,7 +207,7 @@ __device__ inline void yee_rows(const float *__restrict__ E, const float *__rest
     YeeRows<R, 0> y;
     y.load(E, B, nx, ny, nrow, bi, bj0);
     y.load_j(J, nx, ny, nrow, bi, bj0);
-    y.step(E, Eo, Bo, nx, ny, nrow, k, bi, bj0, 1, ZK_YEE_W, c0, periodic_x, open_y, shift);
+    y.step(E, Eo, Bo, nx, ny, nrow, k, bi, bj0, 1, ZK_YEE_W, c0, periodic_x, open_y, shift, ext);
 }
 
 /* Guard nodes take the value of their image: x (unless the window moves)

@@ -271,11 +271,20 @@ int zk_smooth(const float *in, float *out, int nx, int ny, int nrow, int n1, int
 typedef struct zk_yee_k {
     float dtx2, dty2, dtx, dty, dt, mur_y;
 } zk_yee_k;
+/* External fields: the field step also writes out[0] = E + external, out[1]
+ * = B + external (NULL: not) with the external field a grid or uniform; not
+ * together with a shift. */
+typedef struct zk_ext {
+    float *out[2];
+    const float *grid[2];       /* NULL: uniform */
+    float uniform[2][3];
+} zk_ext;
 typedef struct zk_field_args {
     zk_reduce_args r;
     const float *E, *B;
     float *Eo, *Bo;
     zk_yee_k k;                 /* set by zk_field_step */
+    zk_ext ext;
     int shift, n1, n2;
     float sa[ZK_MAX_PASSES + ZK_MAX_Y_PASSES], sb[ZK_MAX_PASSES + ZK_MAX_Y_PASSES];
     int clears;                 /* set by zk_field_step: workgroups that clear Jov_next */
@@ -292,6 +301,9 @@ int zk_field_step(const zk_field_args *f, float dt, float dx, float dy, zk_strea
 int zk_yee(const float *E, const float *B, const float *J, float *Eo, float *Bo,
                   int nx, int ny, int nrow, float dt, float dx, float dy, int periodic_x, int open_y, int shift,
                   zk_stamp st, zk_stream_t s);
+int zk_yee_ext(const float *E, const float *B, const float *J, float *Eo, float *Bo, int nx, int ny, int nrow,
+               float dt, float dx, float dy, int periodic_x, int open_y, int shift, const zk_ext *ext, zk_stamp st,
+               zk_stream_t s);
 int zk_field_guards(float *E, float *B, int nx, int ny, int nrow, int periodic_x,
                            int open_y, zk_stream_t s);
 int zk_move_window(const float *E, const float *B, float *Eo, float *Bo, int nx,
