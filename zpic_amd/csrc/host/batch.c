@@ -469,6 +469,7 @@ void zpic_batch_run(zpic_batch *b, int steps)
             struct zpic_dev_current *dc = sim->current.dev;
             struct zpic_dev_emf *de = sim->emf.dev;
             dc->jcur = (dc->jcur + b->hsims[i].npass) & 1;
+            dc->jzero = 0;
             sim->current.iter++;
             de->cur ^= 1;
             sim->emf.iter++;

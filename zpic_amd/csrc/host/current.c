@@ -126,6 +126,7 @@ void zpic_current_ensure(t_current *c, const zk_tiles *t)
         d->region = zpic_dmalloc(sizeof(float) * 3 * (size_t)tt.WX * (size_t)tt.WY * (size_t)tt.ntiles);
         ZCHECK(zk_fill_f32(d->J[0], 3 * nodes, 0.0f, zpic_stream()));
         d->jcur = 0;
+        d->jzero = 1;
         d->ready = 1;
     } else if (t && (t->TX != d->t.TX || t->TY != d->t.TY || t->H != d->t.H || t->nx != d->t.nx ||
                      t->ny != d->t.ny)) {
@@ -231,10 +232,27 @@ static int reduce_args(t_current *c, zk_reduce_args *a)
     return clears;
 }
 
+/* whether the step's deposits are all zero: none was made */
+static int no_current(const struct zpic_dev_current *d)
+{
+    return d->fresh && d->jov_state[d->jov_cur] == ZPIC_JOV_CLEAN;
+}
+
+int zpic_current_idle(t_current *c)
+{
+    struct zpic_dev_current *d = c->dev;
+    if (!d->jzero || !no_current(d)) return 0;
+    zpic_current_settle(d);
+    c->iter++;
+    d->host_valid = 0;
+    return 1;
+}
+
 /* after the launch that folds */
 static void reduce_done(t_current *c, int cleared)
 {
     struct zpic_dev_current *d = c->dev;
+    d->jzero = no_current(d);
     if (cleared) d->jov_state[1 - d->jov_cur] = ZPIC_JOV_CLEAN;
     fin_done(d);
 }
@@ -243,6 +261,7 @@ void current_update(t_current *c)
 {
     zpic_current_ensure(c, NULL);
     struct zpic_dev_current *d = c->dev;
+    if (zpic_current_idle(c)) return;
     zk_reduce_args a;
     const int clears = reduce_args(c, &a);
     zpic_ktimer_begin(ZPIC_T_CURRENT);
@@ -298,7 +317,8 @@ void current_sync_host(t_current *c)
     d->host_valid = 1;
 }
 
-const float *zpic_current_J(t_current *c) { return c->dev->J[c->dev->jcur]; }
+/* NULL: zero everywhere */
+const float *zpic_current_J(t_current *c) { return c->dev->jzero ? NULL : c->dev->J[c->dev->jcur]; }
 
 void current_report(const t_current *cc, const int jc)
 {

@@ -533,6 +533,10 @@ void zpic_update_advance(t_current *cur, t_emf *emf)
     zpic_current_ensure(cur, NULL);
     const int same = cur->nx[0] == emf->nx[0] && cur->nx[1] == emf->nx[1] && cur->nrow == emf->nrow &&
                      cur->moving_window == emf->moving_window && cur->dev->open_y == emf->dev->open_y;
+    if (zpic_current_idle(cur)) {
+        advance(emf, cur, NULL);
+        return;
+    }
     /* the kernel timers tell the current's launches from the fields' */
     if (same && !zpic_kernel_timing_on() && zpic_current_field_args(cur, &f)) {
         advance(emf, cur, &f);

@@ -114,6 +114,7 @@ struct zpic_dev_current {
     int jov_k;            /* Jov holds multiples of 2^(jov_k - 40) */
     int jov_set;          /* jov_k was set by a species */
     int fresh;            /* no deposit since current_zero */
+    int jzero;            /* J[jcur] is zero at every node */
     int pref[3];          /* preferred tile (tx, ty, halo), 0: process-wide setting */
     int open_y;           /* no fold along y (open y boundaries) */
     /* pushes whose energy and push count the next current_update finishes
@@ -164,6 +165,9 @@ void zpic_spec_settle(struct zpic_dev_species *d);
 void zpic_spec_sync_energy(t_species *s);
 void zpic_spec_sort(t_species *s); /* tile sort of the device particles now */
 int zpic_current_passes(const t_current *c, int axis[], float sa[], float sb[], int max);
+/* The step's current is zero and so is J: nothing to fold (em2d/current.c:
+ * 171-183 adds and filters zeros); does the rest of current_update. */
+int zpic_current_idle(t_current *c);
 /* Arguments of the launch that folds and filters the current and takes the
  * field step (0: the grid or the passes need separate launches), and the
  * bookkeeping after it. */

@@ -100,12 +100,13 @@ struct YeeRows {
         }
     }
 
+    /* J NULL: zero */
     __device__ void load_j(const float *__restrict__ J, int nx, int ny, int nrow, int bi, int bj0)
     {
 #pragma unroll
         for (int v = 1; v < R + 2 + X; v++) {
             const int bj = bj0 - 1 - X + v;
-            const bool in = bi >= 0 && bi < nx + 3 && bj >= 0 && bj < ny + 3;
+            const bool in = J && bi >= 0 && bi < nx + 3 && bj >= 0 && bj < ny + 3;
             const size_t g = in ? 3 * ((size_t)bi + (size_t)bj * nrow) : 0;
 #pragma unroll
             for (int c = 0; c < 3; c++) jj[v][c] = in ? J[g + c] : 0.0f;
