@@ -428,10 +428,13 @@ void zpic_diff_backward(zpic_diff *D, float *dE, float *dB, float *const *dpart)
         }
         for (int n = s1 - 1; n >= s0; n--) {
             const int r = rslot(D, n, s0);
-            if (in_loss(D, n + 1)) ZCHECK(zk_adj_loss(D->lB, D->rB[r + 1], nx, ny, nrow, scale, st));
-            ZCHECK(zk_adj_fields(D->lE, D->lB, D->lJ, D->aE, D->aB, nx, ny, nrow, sim->dt, emf->dx[0], emf->dx[1],
-                                 st));
-            ZCHECK(zk_adj_images(D->lJ, D->Lam, nx, ny, nrow, st));
+            ZCHECK(zk_adj_fields(D->lE, D->lB, in_loss(D, n + 1) ? D->rB[r + 1] : NULL, scale, D->aE, D->aB, D->lJ,
+                                 D->Lam, nx, ny, nrow, sim->dt, emf->dx[0], emf->dx[1], st));
+            float *const e = D->lE, *const b = D->lB;
+            D->lE = D->aE;
+            D->lB = D->aB;
+            D->aE = e;
+            D->aB = b;
             for (int k0 = 0; k0 < D->ns; k0 += ZK_FUSE_MAX) {
                 zk_adj_push_args a;
                 memset(&a, 0, sizeof(a));

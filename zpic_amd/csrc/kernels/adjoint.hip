@@ -37,6 +37,7 @@
  * others, through the global grids with atomics.
  */
 #include "common.h"
+#include "reduce_index.h"
 #include "zk_adjoint.h"
 
 namespace {
@@ -51,139 +52,279 @@ struct Grid {
     __device__ size_t at(int i, int j) const { return 3 * ((size_t)(i + 1) + (size_t)(j + 1) * nrow); }
 };
 
-__device__ inline int wrapi(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
-
-/* adjoint of the guard copies: guard adjoints move to their images */
-__global__ void adj_guards_kernel(const float *__restrict__ lEo, const float *__restrict__ lBo, float *__restrict__ aE,
-                                  float *__restrict__ aB, Grid g)
-{
-    const int bw = g.nx + 3, bh = g.ny + 3;
-    const int node = blockIdx.x * blockDim.x + threadIdx.x;
-    if (node >= bw * bh) return;
-    const int i = node % bw - 1, j = node / bw - 1;
-    float e[3] = {0.f, 0.f, 0.f}, b[3] = {0.f, 0.f, 0.f};
-    if (i >= 0 && i < g.nx && j >= 0 && j < g.ny) {
-        /* every buffer node whose image is (i, j): offsets 0, +-n */
-        for (int dj = -1; dj <= 1; dj++) {
-            const int jj = j + dj * g.ny;
-            if (jj < -1 || jj > g.ny + 1) continue;
-            for (int di = -1; di <= 1; di++) {
-                const int ii = i + di * g.nx;
-                if (ii < -1 || ii > g.nx + 1) continue;
-                const size_t s = g.at(ii, jj);
-                for (int c = 0; c < 3; c++) {
-                    e[c] += lEo[s + c];
-                    b[c] += lBo[s + c];
-                }
-            }
-        }
-    }
-    const size_t d = g.at(i, j);
-    for (int c = 0; c < 3; c++) {
-        aE[d + c] = e[c];
-        aB[d + c] = b[c];
-    }
-}
-
 /* B node (i, j) is updated by the half steps when i, j in [-1, n] */
 __device__ inline bool in_rb(const Grid &g, int i, int j) { return i >= -1 && i <= g.nx && j >= -1 && j <= g.ny; }
 /* E node (i, j) is updated by the full step when i, j in [0, n + 1] */
 __device__ inline bool in_re(const Grid &g, int i, int j) { return i >= 0 && i <= g.nx + 1 && j >= 0 && j <= g.ny + 1; }
 
-/* E adjoint += transpose of the B half step (B += dt/2 (-curl E)) applied
- * to the B adjoint aB, at E node (i, j). */
-__device__ inline void curl_e_t(const Grid &g, const float *aB, int i, int j, float dtx2, float dty2, float out[3])
-{
-    float x = 0.f, y = 0.f, z = 0.f;
-    if (in_rb(g, i, j)) {
+/* nodes (i, j) in the buffer that share an image with no other */
+__device__ inline bool single(const Grid &g, int i, int j) { return i >= 2 && i <= g.nx - 2 && j >= 2 && j <= g.ny - 2; }
+
+/* The adjoints after a step as its reverse reads them, stage by stage from
+ * the output fields back. */
+struct AdjFields {
+    const float *E, *B; /* adjoints of the output fields */
+    const float *F;     /* NULL, or the output B: its loss term is added */
+    float scale;
+    Grid g;
+    float dtx2, dty2, dtx, dty, dt;
+
+    __device__ void at_e(int i, int j, float o[3]) const
+    {
         const size_t s = g.at(i, j);
-        /* Bx(i,j) += -dty2 (Ez(i,j+1) - Ez(i,j)); By(i,j) += dtx2 (Ez(i+1,j) - Ez(i,j));
-         * Bz(i,j) += -dtx2 (Ey(i+1,j) - Ey(i,j)) + dty2 (Ex(i,j+1) - Ex(i,j)) */
-        z += dty2 * aB[s + 0] - dtx2 * aB[s + 1];
-        y += dtx2 * aB[s + 2];
-        x += -dty2 * aB[s + 2];
+        for (int c = 0; c < 3; c++) o[c] = E[s + c];
     }
-    if (in_rb(g, i, j - 1)) {
-        const size_t s = g.at(i, j - 1);
-        z += -dty2 * aB[s + 0];
-        x += dty2 * aB[s + 2];
-    }
-    if (in_rb(g, i - 1, j)) {
-        const size_t s = g.at(i - 1, j);
-        z += dtx2 * aB[s + 1];
-        y += -dtx2 * aB[s + 2];
-    }
-    out[0] = x;
-    out[1] = y;
-    out[2] = z;
-}
 
-/* second half step: aE += (dB/dE)^T aB (aB is the adjoint of the output B) */
-__global__ void adj_bhalf2_kernel(float *__restrict__ aE, const float *__restrict__ aB, Grid g, float dtx2, float dty2)
-{
-    const int bw = g.nx + 3, bh = g.ny + 3;
-    const int node = blockIdx.x * blockDim.x + threadIdx.x;
-    if (node >= bw * bh) return;
-    const int i = node % bw - 1, j = node / bw - 1;
-    float t[3];
-    curl_e_t(g, aB, i, j, dtx2, dty2, t);
-    const size_t d = g.at(i, j);
-    aE[d + 0] += t[0];
-    aE[d + 1] += t[1];
-    aE[d + 2] += t[2];
-}
+    __device__ void at_b(int i, int j, float o[3]) const
+    {
+        const size_t s = g.at(i, j);
+        const bool loss = F && i >= 0 && i < g.nx && j >= 0 && j < g.ny;
+        for (int c = 0; c < 3; c++) o[c] = loss ? B[s + c] + scale * F[s + c] : B[s + c];
+    }
 
-/* full E step: lE = aE; aB += (dE/dB)^T aE; lJ = -dt aE on its range */
-__global__ void adj_efull_kernel(const float *__restrict__ aE, float *__restrict__ aB, float *__restrict__ lE,
-                                 float *__restrict__ lJ, Grid g, float dtx, float dty, float dt)
-{
-    const int bw = g.nx + 3, bh = g.ny + 3;
-    const int node = blockIdx.x * blockDim.x + threadIdx.x;
-    if (node >= bw * bh) return;
-    const int i = node % bw - 1, j = node / bw - 1;
-    const size_t d = g.at(i, j);
-    /* Ex(i,j) += dty (Bz(i,j) - Bz(i,j-1)); Ey(i,j) += -dtx (Bz(i,j) - Bz(i-1,j));
+    /* adjoint of the guard copies: an interior node takes the adjoints of
+     * every buffer node that is its image (offsets 0, +-n, and 2 n on an axis
+     * of one cell), a guard none */
+    template <bool MAG>
+    __device__ void guards(int i, int j, float o[3]) const
+    {
+        o[0] = o[1] = o[2] = 0.0f;
+        if (i < 0 || i >= g.nx || j < 0 || j >= g.ny) return;
+        if (single(g, i, j)) {
+            if (MAG) at_b(i, j, o);
+            else at_e(i, j, o);
+            return;
+        }
+        for (int dj = -1; dj <= 2; dj++) {
+            const int jj = j + dj * g.ny;
+            if (jj < -1 || jj > g.ny + 1) continue;
+            for (int di = -1; di <= 2; di++) {
+                const int ii = i + di * g.nx;
+                if (ii < -1 || ii > g.nx + 1) continue;
+                float v[3];
+                if (MAG) at_b(ii, jj, v);
+                else at_e(ii, jj, v);
+                for (int c = 0; c < 3; c++) o[c] += v[c];
+            }
+        }
+    }
+
+    /* E adjoint += transpose of the B half step (B += dt/2 (-curl E)) applied
+     * to the B adjoints at (i, j), (i, j - 1) and (i - 1, j):
+     * Bx(i,j) += -dty2 (Ez(i,j+1) - Ez(i,j)); By(i,j) += dtx2 (Ez(i+1,j) - Ez(i,j));
+     * Bz(i,j) += -dtx2 (Ey(i+1,j) - Ey(i,j)) + dty2 (Ex(i,j+1) - Ex(i,j)) */
+    __device__ void half_t(int i, int j, const float b[3], const float bd[3], const float bl[3], float e[3]) const
+    {
+        float x = 0.f, y = 0.f, z = 0.f;
+        if (in_rb(g, i, j)) {
+            z += dty2 * b[0] - dtx2 * b[1];
+            y += dtx2 * b[2];
+            x += -dty2 * b[2];
+        }
+        if (in_rb(g, i, j - 1)) {
+            z += -dty2 * bd[0];
+            x += dty2 * bd[2];
+        }
+        if (in_rb(g, i - 1, j)) {
+            z += dtx2 * bl[1];
+            y += -dtx2 * bl[2];
+        }
+        e[0] += x;
+        e[1] += y;
+        e[2] += z;
+    }
+
+    /* E adjoint before the second half step */
+    __device__ void e1(int i, int j, float o[3]) const
+    {
+        float b[3], bd[3], bl[3];
+        guards<false>(i, j, o);
+        guards<true>(i, j, b);
+        guards<true>(i, j - 1, bd);
+        guards<true>(i - 1, j, bl);
+        half_t(i, j, b, bd, bl, o);
+    }
+
+    /* B adjoint before the whole step of E, from the E adjoints after it at
+     * (i, j), (i, j + 1) and (i + 1, j):
+     * Ex(i,j) += dty (Bz(i,j) - Bz(i,j-1)); Ey(i,j) += -dtx (Bz(i,j) - Bz(i-1,j));
      * Ez(i,j) += dtx (By(i,j) - By(i-1,j)) - dty (Bx(i,j) - Bx(i,j-1)); E -= dt J */
-    float bx = 0.f, by = 0.f, bz = 0.f;
-    if (in_re(g, i, j)) {
-        bz += dty * aE[d + 0] - dtx * aE[d + 1];
-        by += dtx * aE[d + 2];
-        bx += -dty * aE[d + 2];
+    __device__ void b1(int i, int j, const float e[3], const float eu[3], const float er[3], float o[3]) const
+    {
+        guards<true>(i, j, o);
+        whole_t(i, j, e, eu, er, o);
     }
-    if (in_re(g, i, j + 1) && j + 1 <= g.ny + 1) {
-        const size_t s = g.at(i, j + 1);
-        bz += -dty * aE[s + 0];
-        bx += dty * aE[s + 2];
-    }
-    if (in_re(g, i + 1, j) && i + 1 <= g.nx + 1) {
-        const size_t s = g.at(i + 1, j);
-        bz += dtx * aE[s + 1];
-        by += -dtx * aE[s + 2];
-    }
-    aB[d + 0] += bx;
-    aB[d + 1] += by;
-    aB[d + 2] += bz;
-    const bool r = in_re(g, i, j);
-    for (int c = 0; c < 3; c++) {
-        lE[d + c] = aE[d + c];
-        lJ[d + c] = r ? -dt * aE[d + c] : 0.0f;
-    }
-}
 
-/* first half step: lB = aB; lE += (dB/dE)^T aB */
-__global__ void adj_bhalf1_kernel(float *__restrict__ lE, const float *__restrict__ aB, float *__restrict__ lB, Grid g,
-                                  float dtx2, float dty2)
+    __device__ void whole_t(int i, int j, const float e[3], const float eu[3], const float er[3], float o[3]) const
+    {
+        float bx = 0.f, by = 0.f, bz = 0.f;
+        if (in_re(g, i, j)) {
+            bz += dty * e[0] - dtx * e[1];
+            by += dtx * e[2];
+            bx += -dty * e[2];
+        }
+        if (in_re(g, i, j + 1)) {
+            bz += -dty * eu[0];
+            bx += dty * eu[2];
+        }
+        if (in_re(g, i + 1, j)) {
+            bz += dtx * er[1];
+            by += -dtx * er[2];
+        }
+        o[0] += bx;
+        o[1] += by;
+        o[2] += bz;
+    }
+
+    /* adjoint of the current at node (i, j) of its range */
+    __device__ void current(int i, int j, const float e[3], float o[3]) const
+    {
+        const bool r = in_re(g, i, j);
+        for (int c = 0; c < 3; c++) o[c] = r ? -dt * e[c] : 0.0f;
+    }
+};
+
+/* The reverse of the field step at one node per thread, for any grid: the
+ * adjoints of the input fields, and lJ, the adjoint of the current.  The
+ * middle stages are formed at the seven nodes around the own that they are
+ * needed at. */
+__global__ void __launch_bounds__(256) adj_fields_node_kernel(AdjFields a, float *__restrict__ lE,
+                                                              float *__restrict__ lB, float *__restrict__ lJ)
 {
+    const Grid &g = a.g;
     const int bw = g.nx + 3, bh = g.ny + 3;
     const int node = blockIdx.x * blockDim.x + threadIdx.x;
     if (node >= bw * bh) return;
     const int i = node % bw - 1, j = node / bw - 1;
-    float t[3];
-    curl_e_t(g, aB, i, j, dtx2, dty2, t);
+    float e[3], eu[3], er[3], ed[3], erd[3], el[3], elu[3];
+    a.e1(i, j, e);
+    a.e1(i, j + 1, eu);
+    a.e1(i + 1, j, er);
+    a.e1(i, j - 1, ed);
+    a.e1(i + 1, j - 1, erd);
+    a.e1(i - 1, j, el);
+    a.e1(i - 1, j + 1, elu);
+    float b[3], bd[3], bl[3], s[3];
+    a.b1(i, j, e, eu, er, b);
+    a.b1(i, j - 1, ed, e, erd, bd);
+    a.b1(i - 1, j, el, elu, e, bl);
+    a.current(i, j, e, s);
+    a.half_t(i, j, b, bd, bl, e);
     const size_t d = g.at(i, j);
     for (int c = 0; c < 3; c++) {
-        lE[d + c] += t[c];
-        lB[d + c] = aB[d + c];
+        lE[d + c] = e[c];
+        lB[d + c] = b[c];
+        lJ[d + c] = s[c];
+    }
+}
+
+/* The same for grids of at least 3 x 3 cells, by waves of 64 columns and
+ * ADJ_R output rows in registers (lanes 2 to 62 write): neighbours along x
+ * are lane shifts, and the loads of all rows are under way together.
+ *
+ * Stage by stage over the grid (loss, guards, half step, whole step, half
+ * step) each launch took 5 us on 256 x 256 cells, nearly all of it its own
+ * time; this launch takes 7.3, and a thread per node as above, whose loads
+ * wait for one another, 54. */
+constexpr int ADJ_R = 4, ADJ_W = 61;
+
+__global__ void __launch_bounds__(64) adj_fields_kernel(AdjFields a, float *__restrict__ lE, float *__restrict__ lB,
+                                                        float *__restrict__ lJ)
+{
+    constexpr int R = ADJ_R;
+    const Grid &g = a.g;
+    const int lane = threadIdx.x;
+    const int i = (int)blockIdx.x * ADJ_W - 3 + lane, j0 = (int)blockIdx.y * R - 1; /* raw; row v is j0 - 2 + v */
+    const bool in_x = i >= 0 && i < g.nx;
+    int xs[2] = {0, 0};
+    const int nix = in_x ? zk::axis_images(i, g.nx, 1, xs) : 0;
+    /* adjoints of the guard copies: sums over a node's images in order */
+    float ge[R + 3][3], gb[R + 3][3];
+#pragma unroll
+    for (int v = 0; v < R + 3; v++) {
+        const int j = j0 - 2 + v;
+        const bool in = in_x && j >= 0 && j < g.ny;
+        int ys[2] = {0, 0};
+        if (j >= 0 && j < g.ny) zk::axis_images(j, g.ny, 1, ys);
+        const size_t s = in ? g.at(xs[0], ys[0]) : 0;
+        const bool loss = in && a.F && xs[0] >= 0 && ys[0] >= 0;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const float e = a.E[s + c], b = a.B[s + c], f = loss ? a.F[s + c] : 0.0f;
+            ge[v][c] = in ? e : 0.0f;
+            gb[v][c] = !in ? 0.0f : loss ? b + a.scale * f : b;
+        }
+    }
+    if (__any(nix > 1)) {
+        float te[R + 3][3], tb[R + 3][3];
+#pragma unroll
+        for (int v = 0; v < R + 3; v++) {
+            const int j = j0 - 2 + v;
+            const bool in = nix > 1 && j >= 0 && j < g.ny;
+            int ys[2] = {0, 0};
+            if (j >= 0 && j < g.ny) zk::axis_images(j, g.ny, 1, ys);
+            const size_t s = in ? g.at(xs[1], ys[0]) : 0;
+            const bool loss = in && a.F && xs[1] < g.nx && ys[0] >= 0;
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const float e = a.E[s + c], b = a.B[s + c], f = loss ? a.F[s + c] : 0.0f;
+                te[v][c] = in ? e : 0.0f;
+                tb[v][c] = !in ? 0.0f : loss ? b + a.scale * f : b;
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < R + 3; v++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                ge[v][c] += te[v][c];
+                gb[v][c] += tb[v][c];
+            }
+    }
+#pragma unroll
+    for (int v = 0; v < R + 3; v++) {
+        const int j = j0 - 2 + v;
+        int ys[2];
+        if (j < 0 || j >= g.ny || zk::axis_images(j, g.ny, 1, ys) < 2) continue;
+        for (int k = 0; k < 2; k++) {
+            if (k >= nix) break;
+            float e[3], b[3];
+            a.at_e(xs[k], ys[1], e);
+            a.at_b(xs[k], ys[1], b);
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                ge[v][c] += e[c];
+                gb[v][c] += b[c];
+            }
+        }
+    }
+    /* E before the second half step, rows 1 to R + 2 */
+#pragma unroll
+    for (int v = 1; v < R + 3; v++) {
+        const float bl[3] = {lane_below(gb[v][0]), lane_below(gb[v][1]), lane_below(gb[v][2])};
+        a.half_t(i, j0 - 2 + v, gb[v], gb[v - 1], bl, ge[v]);
+    }
+    /* B before the whole step, rows 1 to R + 1 */
+#pragma unroll
+    for (int v = 1; v < R + 2; v++) {
+        const float er[3] = {lane_above(ge[v][0]), lane_above(ge[v][1]), lane_above(ge[v][2])};
+        a.whole_t(i, j0 - 2 + v, ge[v], ge[v + 1], er, gb[v]);
+    }
+    /* E before the first half step, rows 2 to R + 1, and outputs */
+#pragma unroll
+    for (int v = 2; v < R + 2; v++) {
+        const int j = j0 - 2 + v;
+        float e[3] = {ge[v][0], ge[v][1], ge[v][2]}, s[3];
+        const float bl[3] = {lane_below(gb[v][0]), lane_below(gb[v][1]), lane_below(gb[v][2])};
+        a.current(i, j, e, s);
+        a.half_t(i, j, gb[v], gb[v - 1], bl, e);
+        if (lane < 2 || lane >= 2 + ADJ_W || i > g.nx + 1 || j > g.ny + 1) continue;
+        const size_t d = g.at(i, j);
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            lE[d + c] = e[c];
+            lB[d + c] = gb[v][c];
+            lJ[d + c] = s[c];
+        }
     }
 }
 
@@ -195,12 +336,12 @@ __global__ void adj_images_kernel(const float *__restrict__ lJ, float *__restric
     const int node = blockIdx.x * blockDim.x + threadIdx.x;
     if (node >= bw * bh) return;
     const int i = node % bw - 1, j = node / bw - 1;
-    const int ci = wrapi(i, g.nx), cj = wrapi(j, g.ny);
+    const int ci = zk_wrap(i, g.nx), cj = zk_wrap(j, g.ny);
     float s[3] = {0.f, 0.f, 0.f};
-    for (int dj = -1; dj <= 1; dj++) {
+    for (int dj = -1; dj <= 2; dj++) {
         const int jj = cj + dj * g.ny;
         if (jj < -1 || jj > g.ny + 1) continue;
-        for (int di = -1; di <= 1; di++) {
+        for (int di = -1; di <= 2; di++) {
             const int ii = ci + di * g.nx;
             if (ii < -1 || ii > g.nx + 1) continue;
             const size_t q = g.at(ii, jj);
@@ -919,25 +1060,20 @@ extern "C" int zk_adj_loss(float *lB, const float *B, int nx, int ny, int nrow, 
     ZK_LAUNCH_CHECK();
 }
 
-extern "C" int zk_adj_fields(float *lE, float *lB, float *lJ, float *aE, float *aB, int nx, int ny, int nrow, float dt,
-                             float dx, float dy, zk_stream_t s)
+extern "C" int zk_adj_fields(const float *lE, const float *lB, const float *F, float scale, float *lE_in,
+                             float *lB_in, float *lJ, float *lam, int nx, int ny, int nrow, float dt, float dx, float dy,
+                             zk_stream_t s)
 {
-    const Grid g = {nx, ny, nrow};
-    const unsigned nb = grid_of((size_t)(nx + 3) * (ny + 3));
     /* constants of the forward step (zk_yee) */
     const float dt2 = dt / 2.0f;
-    const float dtx2 = dt2 / dx, dty2 = dt2 / dy, dtx = dt / dx, dty = dt / dy;
-    hipLaunchKernelGGL(adj_guards_kernel, dim3(nb), dim3(256), 0, s, lE, lB, aE, aB, g);
-    hipLaunchKernelGGL(adj_bhalf2_kernel, dim3(nb), dim3(256), 0, s, aE, aB, g, dtx2, dty2);
-    hipLaunchKernelGGL(adj_efull_kernel, dim3(nb), dim3(256), 0, s, aE, aB, lE, lJ, g, dtx, dty, dt);
-    hipLaunchKernelGGL(adj_bhalf1_kernel, dim3(nb), dim3(256), 0, s, lE, aB, lB, g, dtx2, dty2);
-    ZK_LAUNCH_CHECK();
-}
-
-extern "C" int zk_adj_images(const float *lJ, float *lam, int nx, int ny, int nrow, zk_stream_t s)
-{
-    const Grid g = {nx, ny, nrow};
-    hipLaunchKernelGGL(adj_images_kernel, dim3(grid_of((size_t)(nx + 3) * (ny + 3))), dim3(256), 0, s, lJ, lam, g);
+    const AdjFields a = {lE, lB, F, scale, {nx, ny, nrow}, dt2 / dx, dt2 / dy, dt / dx, dt / dy, dt};
+    const unsigned nb = grid_of((size_t)(nx + 3) * (ny + 3));
+    if (nx < 3 || ny < 3)
+        hipLaunchKernelGGL(adj_fields_node_kernel, dim3(nb), dim3(256), 0, s, a, lE_in, lB_in, lJ);
+    else
+        hipLaunchKernelGGL(adj_fields_kernel, dim3((nx + 3 + ADJ_W - 1) / ADJ_W, (ny + 3 + ADJ_R - 1) / ADJ_R),
+                           dim3(64), 0, s, a, lE_in, lB_in, lJ);
+    hipLaunchKernelGGL(adj_images_kernel, dim3(nb), dim3(256), 0, s, lJ, lam, a.g);
     ZK_LAUNCH_CHECK();
 }
 

@@ -50,14 +50,13 @@ int zk_copy_parts(const zk_parts *dst, const zk_parts *src, int n, zk_stream_t s
 int zk_copy_pair(float *a, const float *sa, float *b, const float *sb, size_t n, zk_stream_t s);
 /* lB(interior) += scale * B(interior) */
 int zk_adj_loss(float *lB, const float *B, int nx, int ny, int nrow, float scale, zk_stream_t s);
-/* Reverse of zk_yee + zk_field_guards (periodic): on entry lE, lB hold the
- * adjoints of the step's output fields, on exit those of its input fields;
- * lJ receives the adjoint of the current.  aE, aB are scratch grids. */
-int zk_adj_fields(float *lE, float *lB, float *lJ, float *aE, float *aB, int nx, int ny, int nrow, float dt,
-                  float dx, float dy, zk_stream_t s);
-/* Reverse of the periodic current fold: lam(node) = sum of lJ over the
- * buffer nodes with the same periodic image */
-int zk_adj_images(const float *lJ, float *lam, int nx, int ny, int nrow, zk_stream_t s);
+/* Reverse of the field step (periodic) and of the periodic current fold: lE,
+ * lB hold the adjoints of the step's output fields, lE_in, lB_in (other
+ * buffers) receive those of its input fields, lJ that of the current and lam
+ * that of the raw current (per buffer node).  F: NULL, or the step's output B, whose loss term
+ * scale * B is first added to lB on the interior. */
+int zk_adj_fields(const float *lE, const float *lB, const float *F, float scale, float *lE_in, float *lB_in,
+                  float *lJ, float *lam, int nx, int ny, int nrow, float dt, float dx, float dy, zk_stream_t s);
 /* Reverse of the particle push of a set of species (tile pass, listed
  * particles, field-adjoint windows added into lE, lB) */
 /* workgroups of zk_adj_push that the GPU holds at once */
