@@ -48,7 +48,6 @@ namespace {
 
 struct Grid {
     int nx, ny, nrow;
-    __device__ bool in_buf(int i, int j) const { return i >= -1 && i <= nx + 1 && j >= -1 && j <= ny + 1; }
     __device__ size_t at(int i, int j) const { return 3 * ((size_t)(i + 1) + (size_t)(j + 1) * nrow); }
 };
 

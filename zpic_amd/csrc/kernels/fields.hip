@@ -4,16 +4,20 @@
  * zk_yee fuses the three half/whole steps of the reference emf_advance
  * (em2d/emf.c:688-698): B += dt/2 curl E over i,j in [-1,n] (yee_b,
  * :500-522), E += dt (curl B - J) over [0,n+1] (yee_e, :531-562), and
- * B += dt/2 curl E again, into one pass over LDS tiles.  Each node is
- * computed with the reference's expressions and update ranges, so with the
- * same J the result is bit-identical.  Inputs and outputs are distinct
+ * B += dt/2 curl E again, into one pass with rows in registers.  Each node
+ * is computed with the reference's expressions and update ranges, so with
+ * the same J the result is bit-identical.  Inputs and outputs are distinct
  * buffers (the host swaps them).  The guard cells of the outputs are
- * written by the nodes they are images of (emf_update_gc, :573-637).
+ * written by the nodes they are images of (emf_update_gc, :573-637), and
+ * with external fields the same pass writes the fields seen by particles
+ * (emf_update_part_fld, :838-914).  zk_field_step folds and filters the
+ * current in the same launch (current.hip's kernels on their own).
  *
  * zk_field_guards copies guard cells from their periodic images on its own
  * (grids edited outside the step); zk_move_window shifts the grid one cell left
  * and clears the last columns (emf_move_window, :648-675); zk_add_ext
- * forms the fields seen by particles (emf_update_part_fld, :838-914);
+ * forms the fields seen by particles on its own (grids edited outside the
+ * step);
  * zk_emf_energy sums E_c^2 and B_c^2 in FP64 (emf_get_energy, :729-750);
  * zk_charge deposits the CIC charge density (spec_deposit_charge,
  * em2d/particles.c:1289-1324, before its boundary fold).
