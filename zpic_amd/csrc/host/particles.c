@@ -749,6 +749,7 @@ static void resort(t_species *const *list, int n, int slack, const int *before)
         a->ctr = d->ctr;
         a->move = d->cnt;
         a->stay = d->stay;
+        a->ticket = d->stay + d->t.ntiles;
         a->nbr = d->nbr;
         a->tailn = d->tailn;
         a->old_off = d->tile_off;
@@ -882,7 +883,8 @@ void zpic_species_ensure(t_species *s)
         zpic_h2d(d->ctr, &zero, sizeof(zero));
         d->tile_off = zpic_dmalloc(sizeof(int) * (size_t)(d->t.ntiles + 2));
         d->tile_off2 = zpic_dmalloc(sizeof(int) * (size_t)(d->t.ntiles + 2));
-        d->stay = zpic_dmalloc(sizeof(int) * (size_t)d->t.ntiles);
+        d->stay = zpic_dmalloc(sizeof(int) * (size_t)(d->t.ntiles + 1)); /* and the re-sort's ticket */
+        ZCHECK(zk_fill_f32((float *)(d->stay + d->t.ntiles), 1, 0.0f, zpic_stream()));
         d->nbr = zpic_dmalloc(sizeof(int) * 13 * (size_t)d->t.ntiles);
         d->tailn = zpic_dmalloc(sizeof(int) * (size_t)d->t.ntiles);
         ZCHECK(zk_fill_f32((float *)d->tailn, (size_t)d->t.ntiles, 0.0f, zpic_stream())); /* int zeros */

@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(ZK_SORT_THREADS) scatter_batch(const zk_bspec 
 {
     const zk_bspec &S = specs[items[2 * blockIdx.x]];
     if (!sorts_now(S)) return;
-    scatter_stay_body(S.set[S.pcur], S.set[1 - S.pcur], S.offs[S.ocur], nullptr, S.offs[1 - S.ocur], S.stay, S.nbr, S.cursor,
+    scatter_stay_body(S.set[S.pcur], S.set[1 - S.pcur], S.offs[S.ocur], nullptr, ScannedDest{S.offs[1 - S.ocur], S.cursor}, S.stay, S.nbr,
                       S.a.t, items[2 * blockIdx.x + 1], S.a.t.ntiles);
 }
 

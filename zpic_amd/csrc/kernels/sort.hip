@@ -67,6 +67,12 @@ __global__ void __launch_bounds__(ZK_SORT_THREADS) count_stay_kernel(zk_resort_s
 {
     int b = blockIdx.x;
     const zk_resort_args &a = m.s[sort_species(m, b)];
+    if (m.local) {
+        /* what the scan launch leaves for the scatter otherwise: the slot
+         * count before the sort, and cursors */
+        if (threadIdx.x == 0 && b == 0) a.old_off[a.t.ntiles + 1] = a.ctr->np_total;
+        if (threadIdx.x == 0 && b < a.t.ntiles) a.cursor[b] = 0;
+    }
     count_stay_body(a.src.cell, a.src.cbits, a.old_off, a.old_n, &a.ctr->np_total, a.stay, a.move, a.nbr, a.tailn, a.t,
                     b, a.blocks);
 }
@@ -86,7 +92,53 @@ __global__ void __launch_bounds__(ZK_SORT_THREADS) scatter_stay_kernel(zk_resort
 {
     int b = blockIdx.x;
     const zk_resort_args &a = m.s[sort_species(m, b)];
-    scatter_stay_body(a.src, a.dst, a.old_off, a.old_n, a.new_off, a.stay, a.nbr, a.cursor, a.t, b, a.blocks);
+    scatter_stay_body(a.src, a.dst, a.old_off, a.old_n, ScannedDest{a.new_off, a.cursor}, a.stay, a.nbr, a.t, b,
+                      a.blocks);
+    zk_stamp_last(st);
+}
+
+/* The scatter with the scan of the tile counts in every workgroup: up to
+ * ZK_SCAN_LOCAL tiles, no free slots.  A scan launch takes 6.5 us for any
+ * number of them, and 3.5 pass before and after it; reading and scanning the
+ * counts costs a workgroup about 2 us: 32 x 32 cells 790 -> 766 us for 20
+ * steps, 128 x 128 2040 -> 1986 for 50.  The species' first
+ * workgroup leaves the offsets, counts and counters; move and tailn, which
+ * all read, are cleared by the last to have read them (ticket, zero on entry
+ * and exit). */
+__global__ void __launch_bounds__(ZK_SORT_THREADS) scatter_scan_kernel(zk_resort_set m, zk_stamp st)
+{
+    __shared__ int off[ZK_SCAN_LOCAL], front[ZK_SCAN_LOCAL], last;
+    int b = blockIdx.x;
+    const zk_resort_args &a = m.s[sort_species(m, b)];
+    const int n = a.t.ntiles;
+    const int total = resort_scan(a.stay, a.move, a.tailn, n, off, front);
+    int before = 0;
+    if (threadIdx.x == 0) before = atomicAdd(a.ticket, 1);
+    if (b == 0) {
+        for (int t = threadIdx.x; t < n; t += blockDim.x) {
+            a.new_off[t] = off[t];
+            if (a.new_n) a.new_n[t] = (t + 1 < n ? off[t + 1] : total) - off[t];
+        }
+        if (threadIdx.x == 0) {
+            a.new_off[n] = total;
+            zk_spec_ctr &c = *a.ctr;
+            c.np_total = total;
+            c.n_sorted = total;
+            c.n_dead = 0;
+            c.n_slack = 0;
+            c.n_unplaced = 0;
+            c.n_overfull = 0;
+            c.ovf_sorted = c.n_overflow;
+        }
+    }
+    scatter_stay_body(a.src, a.dst, a.old_off, a.old_n, LocalDest{off, front, a.cursor}, a.stay, a.nbr, a.t, b,
+                      a.blocks);
+    if (threadIdx.x == 0) last = before == a.blocks - 1;
+    __syncthreads();
+    if (last) {
+        for (int t = threadIdx.x; t < n; t += blockDim.x) a.move[t] = a.tailn[t] = 0;
+        if (threadIdx.x == 0) *a.ticket = 0;
+    }
     zk_stamp_last(st);
 }
 
@@ -226,12 +278,18 @@ extern "C" int zk_sort_tiles(const zk_resort_set *m, zk_stamp st, zk_stream_t s)
     if (m->n < 1 || m->n > ZK_FUSE_MAX) return (int)hipErrorInvalidValue;
     zk_resort_set r = *m;
     unsigned g = 0;
+    r.local = 1;
     for (int k = 0; k < r.n; k++) {
         zk_resort_args &a = r.s[k];
+        if (a.slack || !a.ticket || a.t.ntiles < 1 || a.t.ntiles > ZK_SCAN_LOCAL) r.local = 0;
         a.blocks = a.t.ntiles + (a.tail_upper > 0 ? (int)grid_for(a.tail_upper, 1024, 4096) : 0);
         g += (unsigned)a.blocks;
     }
     if (g > 0) hipLaunchKernelGGL(count_stay_kernel, dim3(g), dim3(ZK_SORT_THREADS), 0, s, r);
+    if (r.local) {
+        hipLaunchKernelGGL(scatter_scan_kernel, dim3(g), dim3(ZK_SORT_THREADS), 0, s, r, st);
+        ZK_LAUNCH_CHECK();
+    }
     hipLaunchKernelGGL(scan_stay_kernel, dim3(r.n), dim3(1024), 0, s, r);
     if (g > 0) hipLaunchKernelGGL(scatter_stay_kernel, dim3(g), dim3(ZK_SORT_THREADS), 0, s, r, st);
     for (int k = 0; k < r.n; k++) {

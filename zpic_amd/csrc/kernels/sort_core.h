@@ -422,16 +422,74 @@ __device__ inline void copy_part(const zk_parts &src, const zk_parts &dst, int i
     if (src.id) dst.id[d] = src.id[i];
 }
 
+/* Where the particles of a tile go: from a scan launch before (offsets and
+ * the next slot behind the movers in global memory) ... */
+struct ScannedDest {
+    const int *new_off;
+    int *cursor;
+    __device__ int start(int tile) const { return new_off[tile]; }
+    /* a slot behind the movers of tile `key` (-1: none); all 64 lanes */
+    __device__ int reserve(int key) const { return zk_run_reserve(key, cursor); }
+};
+
+/* ... or from the workgroup's own scan (resort_scan): offsets and the ends
+ * of the movers in LDS, slots behind them counted from 0 in cursor. */
+struct LocalDest {
+    const int *off, *front;
+    int *cursor;
+    __device__ int start(int tile) const { return off[tile]; }
+    __device__ int reserve(int key) const
+    {
+        const int r = zk_run_reserve(key, cursor);
+        return key >= 0 ? front[key] + r : r;
+    }
+};
+
+/* Tiles up to which every workgroup of the scatter scans the tile counts
+ * itself: one a thread.  With up to four a thread the 800 tiles of a 1500 x
+ * 128 grid gained nothing (the run 1.4 % longer). */
+#define ZK_SCAN_LOCAL ZK_SORT_THREADS
+
+/* scan_stay_body's offsets (no free slots) in LDS: off[t] the exclusive scan
+ * of stay + move + tailn, front[t] = off[t] + stay[t] + move[t]; returns the
+ * total.  ZK_SORT_THREADS threads, ntiles <= ZK_SCAN_LOCAL. */
+__device__ inline int resort_scan(const int *stay, const int *move, const int *tailn, int ntiles, int *off, int *front)
+{
+    __shared__ int wsum[ZK_SORT_THREADS / ZK_WAVE];
+    const int lane = __lane_id(), w = threadIdx.x / ZK_WAVE;
+    const int t = threadIdx.x;
+    const int st = t < ntiles ? stay[t] : 0, mv = t < ntiles ? move[t] : 0, tl = t < ntiles ? tailn[t] : 0;
+    const int sum = st + mv + tl;
+    int x = sum; /* inclusive scan within the wave */
+    for (int o = 1; o < ZK_WAVE; o <<= 1) {
+        const int y = __shfl_up(x, o, ZK_WAVE);
+        if (lane >= o) x += y;
+    }
+    if (lane == ZK_WAVE - 1) wsum[w] = x;
+    __syncthreads();
+    int run = x - sum, total = 0;
+    for (int k = 0; k < ZK_SORT_THREADS / ZK_WAVE; k++) {
+        if (k < w) run += wsum[k];
+        total += wsum[k];
+    }
+    if (t < ntiles) {
+        off[t] = run;
+        front[t] = run + st + mv;
+    }
+    __syncthreads();
+    return total;
+}
+
 /* Block b < ntiles (ZK_SORT_THREADS threads) moves source tile b:
- * stayers to new_off[b] + their rank among the tile's stayers (contiguous,
+ * stayers to the tile's start + their rank among the tile's stayers (contiguous,
  * in order), movers to their slot's run; blocks beyond move chunks of the
  * tail.  Every lane loads its particle before the slot bookkeeping, so the
  * loads are in flight during it. */
+template <class D>
 __device__ inline void scatter_stay_body(const zk_parts &src, const zk_parts &dst, const int *__restrict__ old_off,
-                                         const int *__restrict__ old_n, const int *__restrict__ new_off,
-                                         const int *__restrict__ stay,
-                                         const int *__restrict__ nbr, int *cursor, const zk_tiles &t,
-                                         const int block, const int nblocks)
+                                         const int *__restrict__ old_n, const D &dest,
+                                         const int *__restrict__ stay, const int *__restrict__ nbr,
+                                         const zk_tiles &t, const int block, const int nblocks)
 {
     __shared__ int lc[9], run0[9];
     const int lane = __lane_id();
@@ -439,12 +497,12 @@ __device__ inline void scatter_stay_body(const zk_parts &src, const zk_parts &ds
         if (threadIdx.x < 9) {
             const int d = nbr_tile(threadIdx.x, block, t);
             lc[threadIdx.x] = 0;
-            run0[threadIdx.x] = new_off[d] + stay[d] + nbr[ZK_NBR * block + threadIdx.x];
+            run0[threadIdx.x] = dest.start(d) + stay[d] + nbr[ZK_NBR * block + threadIdx.x];
         }
         const int nw = ZK_SORT_THREADS / ZK_WAVE, w = threadIdx.x / ZK_WAVE;
         int wlo, whi;
         wave_piece(old_off[block], range_end(old_off, old_n, block), w, nw, &wlo, &whi);
-        int placed = new_off[block];
+        int placed = dest.start(block);
         for (int k = 0; k < w; k++) placed += nbr[ZK_NBR * block + 9 + k];
         __syncthreads();
         const unsigned long long lt = (1ull << lane) - 1ull;
@@ -476,7 +534,7 @@ __device__ inline void scatter_stay_body(const zk_parts &src, const zk_parts &ds
                 const int r = wave_slot_add(slot, lc);
                 if (slot >= 0) d = run0[slot] + r;
                 const bool far = key >= 0 && !st && slot < 0;
-                const int dm = zk_run_reserve(far ? key : -1, cursor);
+                const int dm = dest.reserve(far ? key : -1);
                 if (far) d = dm;
                 if (key >= 0) {
                     const unsigned od = (unsigned)d * 4u;
@@ -500,7 +558,7 @@ __device__ inline void scatter_stay_body(const zk_parts &src, const zk_parts &ds
                 c = src.cell[i];
                 key = tile_key_cell(c, src.cbits, t);
             }
-            const int dm = zk_run_reserve(key, cursor);
+            const int dm = dest.reserve(key);
             if (key >= 0) copy_part(src, dst, i, dm, c);
         }
     }

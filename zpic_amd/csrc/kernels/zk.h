@@ -199,7 +199,7 @@ int zk_sort(const zk_parts *src, const zk_parts *dst, zk_spec_ctr *ctr,
                    int *cnt, int *off, int *cursor, int *tile_n, const zk_tiles *t,
                    int np_upper, int spread, int slack, int cap_slots, zk_stream_t s);
 /* Re-sort of the tile-sorted sets of n species of one simulation in three
- * launches: old_off (ntiles + 2, the last entry receives the slot count
+ * launches, or two on grids of few tiles: old_off (ntiles + 2, the last entry receives the slot count
  * before the sort) and old_n -> new_off (ntiles + 1) and new_n; `before` (or
  * NULL) the counts of the previous sort, whose growth sizes the free slots;
  * move and tailn (ntiles, zero on entry and exit), stay and cursor
@@ -212,11 +212,13 @@ typedef struct zk_resort_args {
     int *new_off, *new_n, *cursor;
     zk_tiles t;
     int tail_upper, slack, cap_slots;
+    int *ticket;                /* zero on entry and exit (NULL: always three launches) */
     int blocks;                 /* set by zk_sort_tiles */
 } zk_resort_args;
 typedef struct zk_resort_set {
     zk_resort_args s[ZK_FUSE_MAX];
     int n;
+    int local;                  /* set by zk_sort_tiles: no scan launch */
 } zk_resort_set;
 int zk_sort_tiles(const zk_resort_set *m, zk_stamp st, zk_stream_t s);
 /* Second half of a staged re-sort, after a push with `sorting` set: the
