@@ -197,7 +197,9 @@ int spec_overflow_count(t_species *spec);
 
 /* Per-kernel GPU time, measured with HIP events on the library's stream
  * around each launch while enabled.  Classes: 0 push and deposit, 1 tile
- * sort, 2 current reduction and smoothing, 3 field solver. */
+ * sort, 2 current reduction and smoothing, 3 field solver.  Where sim_iter
+ * takes the last two in one launch, it launches them apart while enabled
+ * (same results). */
 enum zpic_kernel_class { ZPIC_K_PUSH = 0, ZPIC_K_SORT = 1, ZPIC_K_CURRENT = 2, ZPIC_K_FIELD = 3 };
 void zpic_kernel_timing(int enable);
 double zpic_kernel_time(int kclass, long long *launches); /* seconds */
