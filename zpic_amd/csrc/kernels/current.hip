@@ -69,7 +69,9 @@ struct SmoothPasses {
  * The arithmetic and guard handling are those of the passes one after the
  * other, so J is the same bit for bit.  x passes filter interior rows only,
  * and there every column of a periodic axis is the image of an interior one;
- * with a moving window the guard columns keep their values.  y passes filter
+ * with a moving window, or without x passes, the guard columns keep their
+ * values (after y passes of an earlier launch they are no images: y passes
+ * leave them unfiltered).  y passes filter
  * interior columns only; on a periodic axis every row is the image of an
  * interior one, except that the first y pass reads the guard rows -1 and ny
  * as the x passes left them, unfiltered; with open y boundaries the guard
@@ -87,12 +89,13 @@ __global__ void __launch_bounds__(64) smooth_kernel(const float *__restrict__ in
     const int c0 = ring ? zk_wrap(jt, ny) : jt;       /* and its image */
     const bool in_x = i >= 0 && i < nx;
     const bool col = b >= 0 && b < nx + 3;
-    const int bi = periodic_x ? zk_wrap(i, nx) + 1 : b;
+    const bool images = periodic_x && n1 > 0; /* columns of inner rows are images of interior columns */
+    const int bi = images ? zk_wrap(i, nx) + 1 : b;
     float v[ROWS][3];
 #pragma unroll
     for (int r = 0, c = c0; r < ROWS; r++, c = ring && c + 1 == ny ? 0 : c + 1) {
         const bool inner = c >= 0 && c < ny;
-        const bool ok = inner ? periodic_x || col : c >= -1 && c <= ny + 1 && col;
+        const bool ok = inner ? images || col : c >= -1 && c <= ny + 1 && col;
         const float *q = in + (ok ? 3 * ((size_t)(inner ? bi : b) + (size_t)(c + 1) * nrow) : 0);
         v[r][0] = ok ? q[0] : 0.0f;
         v[r][1] = ok ? q[1] : 0.0f;
