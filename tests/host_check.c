@@ -1,0 +1,147 @@
+/*
+ * host_check.c - the library's host code on the CPU, with the GPU runtime and
+ * the kernel launches it needs replaced by the few lines below: device memory
+ * is ordinary memory, copies are done at once, and every pointer handed to a
+ * copy or a launch has to lie in a live allocation.  One check per argument;
+ * exit status 0 when it holds, and why not on stderr.
+ */
+#include <pthread.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <hip/hip_runtime_api.h>
+
+#define float3 zpic_float3 /* the runtime's headers have a type of that name */
+#include "zpic_internal.h"
+
+static int failed;
+#define CHECK(c)                                                                                                       \
+    do {                                                                                                               \
+        if (!(c)) {                                                                                                    \
+            fprintf(stderr, "%s:%d: %s\n", __FILE__, __LINE__, #c);                                                    \
+            failed = 1;                                                                                                \
+        }                                                                                                              \
+    } while (0)
+
+/* ---- device memory ---- */
+
+static pthread_mutex_t lock = PTHREAD_MUTEX_INITIALIZER;
+static struct {
+    char *p;
+    size_t n;
+} block[256];
+
+static int live(const void *p, size_t n)
+{
+    int ok = 0;
+    pthread_mutex_lock(&lock);
+    for (int k = 0; k < 256; k++)
+        ok |= block[k].p && (const char *)p >= block[k].p && (const char *)p + n <= block[k].p + block[k].n;
+    pthread_mutex_unlock(&lock);
+    return ok;
+}
+
+hipError_t hipMalloc(void **p, size_t n)
+{
+    *p = calloc(1, n);
+    pthread_mutex_lock(&lock);
+    int k = 0;
+    while (block[k].p) k++;
+    block[k].p = *p;
+    block[k].n = n;
+    pthread_mutex_unlock(&lock);
+    return hipSuccess;
+}
+
+hipError_t hipFree(void *p)
+{
+    pthread_mutex_lock(&lock);
+    for (int k = 0; k < 256; k++)
+        if (block[k].p == p) block[k].p = NULL;
+    pthread_mutex_unlock(&lock);
+    free(p);
+    return hipSuccess;
+}
+
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind kind, hipStream_t s)
+{
+    const int ok = kind == hipMemcpyHostToDevice   ? live(dst, n)
+                   : kind == hipMemcpyDeviceToHost ? live(src, n)
+                                                   : live(dst, n) && live(src, n);
+    CHECK(ok);
+    if (ok) memcpy(dst, src, n);
+    return hipSuccess;
+}
+
+/* ---- the rest of the runtime ---- */
+
+hipError_t hipGetDeviceCount(int *n) { return *n = 1, hipSuccess; }
+hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
+hipError_t hipSetDevice(int d) { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned f) { return *s = (hipStream_t)1, hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { return hipSuccess; }
+hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
+const char *hipGetErrorString(hipError_t e) { return "error"; }
+
+/* ---- launches ---- */
+
+int zk_fill_f32(float *p, size_t n, float v, zk_stream_t s)
+{
+    CHECK(live(p, 4 * n));
+    if (live(p, 4 * n))
+        for (size_t k = 0; k < n; k++) p[k] = v;
+    return 0;
+}
+
+int zk_unpack(const void *aos, int n, const zk_parts *dst, int64_t id0, zk_spec_ctr *ctr, int append, zk_stream_t s)
+{
+    CHECK(live(aos, 28 * (size_t)n) && live(dst->cell, 4 * (size_t)n));
+    ctr->np_total = n;
+    return 0;
+}
+
+int zk_sort(const zk_parts *src, const zk_parts *dst, zk_spec_ctr *ctr, int *cnt, int *off, int *cursor, int *tile_n,
+            const zk_tiles *t, int np_upper, int spread, int slack, int cap_slots, zk_stream_t s)
+{
+    ctr->n_sorted = ctr->np_total;
+    return 0;
+}
+
+int zk_charge(zk_charge_args a, int tail_upper, zk_stream_t s)
+{
+    CHECK(live(a.rho, 4 * (size_t)(a.t.nx + 1) * (a.t.ny + 1)));
+    return 0;
+}
+
+/* ---- checks ---- */
+
+static void species(t_species *s, int nx, int ny)
+{
+    const int n[2] = {nx, ny}, ppc[2] = {1, 1};
+    const float u[3] = {0, 0, 0};
+    float box[2] = {0.1f * nx, 0.1f * ny};
+    spec_new(s, "electrons", -1.0f, ppc, u, u, n, box, 0.07f, NULL);
+}
+
+/* the staging buffer is allocated again after the species' device buffers
+ * were freed to track ids */
+static void staging(void)
+{
+    t_species s;
+    species(&s, 8, 8);
+    float rho[81] = {0};
+    spec_deposit_charge(&s, rho);
+    spec_track_ids(&s);
+    CHECK(s.dev->stage == NULL);
+    spec_deposit_charge(&s, rho);
+    CHECK(live(s.dev->stage, s.dev->stage_cap));
+}
+
+int main(int argc, char **argv)
+{
+    const char *what = argc > 1 ? argv[1] : "";
+    if (!strcmp(what, "staging")) staging();
+    else CHECK(!"a known check");
+    return failed;
+}

@@ -541,6 +541,7 @@ static void species_free_device(struct zpic_dev_species *d)
     d->tile_off = d->cnt = d->cursor = NULL;
     d->epart = NULL;
     d->stage = NULL;
+    d->stage_cap = 0;
     d->ctr = NULL;
     d->ready = 0;
 }
