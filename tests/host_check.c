@@ -81,7 +81,18 @@ hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 hipError_t hipSetDevice(int d) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned f) { return *s = (hipStream_t)1, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { return hipSuccess; }
+static int pinned; /* allocations of page-locked memory and of events */
+hipError_t hipHostMalloc(void **p, size_t n, unsigned f)
+{
+    pinned++;
+    *p = malloc(n);
+    return hipSuccess;
+}
 hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned f) { return pinned++, *e = (hipEvent_t)1, hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t e) { return hipSuccess; }
 const char *hipGetErrorString(hipError_t e) { return "error"; }
 
 /* ---- launches ---- */
@@ -114,6 +125,20 @@ int zk_charge(zk_charge_args a, int tail_upper, zk_stream_t s)
     return 0;
 }
 
+int zk_noalloc_scratch(float **p)
+{
+    static void *scratch;
+    if (!scratch) hipMalloc(&scratch, 8 * (size_t)ZK_NOALLOC_CHARGE_MAX);
+    *p = scratch;
+    return 0;
+}
+
+int zk_add_f32(float *acc, const float *v, size_t n, zk_stream_t s)
+{
+    for (size_t k = 0; k < n; k++) acc[k] += v[k];
+    return 0;
+}
+
 /* ---- checks ---- */
 
 static void species(t_species *s, int nx, int ny)
@@ -138,10 +163,27 @@ static void staging(void)
     CHECK(live(s.dev->stage, s.dev->stage_cap));
 }
 
+/* the charge deposit that allocates nothing, on a grid whose read would
+ * otherwise be staged through page-locked memory */
+static void noalloc(void)
+{
+    t_species s;
+    species(&s, 1500, 1400);
+    zpic_stage_hold(1);
+    zpic_species_ensure(&s);
+    float *rho = malloc(4 * (size_t)1501 * 1401);
+    for (int k = 0; k < 1501 * 1401; k++) rho[k] = 1.0f;
+    pinned = 0;
+    CHECK(spec_deposit_charge_noalloc(&s, rho) == 0);
+    CHECK(pinned == 0);
+    CHECK(rho[1600] == 1.0f);
+}
+
 int main(int argc, char **argv)
 {
     const char *what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "staging")) staging();
+    else if (!strcmp(what, "noalloc")) noalloc();
     else CHECK(!"a known check");
     return failed;
 }

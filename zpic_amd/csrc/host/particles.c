@@ -1455,7 +1455,8 @@ int spec_deposit_charge_noalloc(const t_species *cs, float *charge)
     ZCHECK(zk_fill_f32(rho, n, 0.0f, zpic_stream()));
     ZCHECK(zk_charge(charge_args(s, rho), d->tail_upper, zpic_stream()));
     ZCHECK(zk_add_f32(acc, rho, n, zpic_stream()));
-    zpic_d2h(charge, acc, sizeof(float) * n);
+    /* a staged read may allocate its page-locked chunks */
+    zpic_d2h_plain(charge, acc, sizeof(float) * n);
     if (!s->moving_window)
         for (int j = 0; j < s->nx[1] + 1; j++) charge[j * nrow] += charge[s->nx[0] + j * nrow];
     if (!d->open_y)

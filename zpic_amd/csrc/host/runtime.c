@@ -316,11 +316,15 @@ static int staged_d2h(void *dst, const void *src, size_t bytes)
     return 1;
 }
 
-void zpic_d2h(void *dst, const void *src, size_t bytes)
+void zpic_d2h_plain(void *dst, const void *src, size_t bytes)
 {
-    if (staged_d2h(dst, src, bytes)) return;
     if (bytes) ZCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, zpic_stream()));
     ZCHECK(hipStreamSynchronize(zpic_stream()));
+}
+
+void zpic_d2h(void *dst, const void *src, size_t bytes)
+{
+    if (!staged_d2h(dst, src, bytes)) zpic_d2h_plain(dst, src, bytes);
 }
 
 void zpic_d2d_async(void *dst, const void *src, size_t bytes)

@@ -23,6 +23,7 @@ void *zpic_dmalloc(size_t bytes);
 void zpic_dfree(void *p);
 void zpic_h2d(void *dst, const void *src, size_t bytes);      /* synchronous */
 void zpic_d2h(void *dst, const void *src, size_t bytes);      /* synchronous */
+void zpic_d2h_plain(void *dst, const void *src, size_t bytes); /* the same, one copy: nothing is allocated for it */
 void zpic_d2d_async(void *dst, const void *src, size_t bytes); /* on the stream */
 /* zeroed host grid (calloc; NULL when out of memory); large ones ask for huge
  * pages, which the first read from the device fills several times faster */
