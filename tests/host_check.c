@@ -81,13 +81,15 @@ hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 hipError_t hipSetDevice(int d) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned f) { return *s = (hipStream_t)1, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { return hipSuccess; }
-static int pinned; /* allocations of page-locked memory and of events */
+static int pinned;   /* allocations of page-locked memory and of events */
+static int nopinned; /* page-locked memory has run out */
 hipError_t hipHostMalloc(void **p, size_t n, unsigned f)
 {
     pinned++;
-    *p = malloc(n);
-    return hipSuccess;
+    *p = nopinned ? NULL : malloc(n);
+    return nopinned ? hipErrorOutOfMemory : hipSuccess;
 }
+hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned f) { return pinned++, *e = (hipEvent_t)1, hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { return hipSuccess; }
@@ -179,11 +181,30 @@ static void noalloc(void)
     CHECK(rho[1600] == 1.0f);
 }
 
+/* large reads with and without page-locked memory to stage them in */
+static void reads(void)
+{
+    const size_t n = (size_t)9 << 20;
+    char *src = zpic_dmalloc(n), *dst = malloc(n);
+    for (size_t k = 0; k < n; k++) src[k] = (char)(k * 7 + k / 4096);
+    zpic_stage_hold(1);
+    for (nopinned = 1; nopinned >= 0; nopinned--) {
+        memset(dst, 0, n);
+        zpic_d2h(dst, src, n);
+        CHECK(!memcmp(dst, src, n));
+    }
+    pinned = 0;
+    zpic_d2h(dst, src, n);
+    CHECK(pinned == 0); /* the chunks are kept */
+    zpic_stage_hold(-1);
+}
+
 int main(int argc, char **argv)
 {
     const char *what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "staging")) staging();
     else if (!strcmp(what, "noalloc")) noalloc();
+    else if (!strcmp(what, "reads")) reads();
     else CHECK(!"a known check");
     return failed;
 }

@@ -217,7 +217,8 @@ void zpic_h2d(void *dst, const void *src, size_t bytes)
  *
  * The chunks are allocated by the first large read and belong to the live
  * simulations (zpic_stage_hold): the last one to be deleted gives them back.
- * A read that finds them taken, or too small a read, uses the plain copy. */
+ * A read that finds them taken or no memory for them, or too small a read,
+ * uses the plain copy. */
 #define STAGE_THREADS 4
 #define STAGE_CHUNK ((size_t)1 << 21)
 #define STAGE_MIN ((size_t)1 << 23) /* 3 MB grids gain nothing (512 x 512), 13 MB ones half */
@@ -281,6 +282,27 @@ void zpic_stage_hold(int n)
     pthread_mutex_unlock(&g_stage.lock);
 }
 
+/* by the read that holds the chunks; 0: no page-locked memory to be had */
+static int stage_alloc(void)
+{
+    void *p = NULL;
+    if (hipHostMalloc(&p, 2 * STAGE_THREADS * STAGE_CHUNK, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+        (void)hipGetLastError(); /* not an error of the caller's */
+        return 0;
+    }
+    g_stage.buf = p;
+    for (int k = 0; k < 2 * STAGE_THREADS; k++) g_stage.ev[k] = zpic_event_new_read();
+    return 1;
+}
+
+static void stage_release(void)
+{
+    pthread_mutex_lock(&g_stage.lock);
+    g_stage.busy = 0;
+    if (g_stage.holders == 0) stage_free();
+    pthread_mutex_unlock(&g_stage.lock);
+}
+
 /* 1: the read was done */
 static int staged_d2h(void *dst, const void *src, size_t bytes)
 {
@@ -291,9 +313,9 @@ static int staged_d2h(void *dst, const void *src, size_t bytes)
     pthread_mutex_unlock(&g_stage.lock);
     if (!mine) return 0;
     const hipStream_t stream = zpic_stream();
-    if (!g_stage.buf) {
-        g_stage.buf = zpic_pinned_alloc(2 * STAGE_THREADS * STAGE_CHUNK);
-        for (int k = 0; k < 2 * STAGE_THREADS; k++) g_stage.ev[k] = zpic_event_new_read();
+    if (!g_stage.buf && !stage_alloc()) {
+        stage_release();
+        return 0;
     }
     /* at least two chunks a thread, so that copies and reads overlap */
     size_t chunk = (bytes / (2 * STAGE_THREADS) + 4095) / 4096 * 4096;
@@ -309,10 +331,7 @@ static int staged_d2h(void *dst, const void *src, size_t bytes)
         if (!started[k]) stage_run(&job[k]);
     for (int k = 1; k < STAGE_THREADS; k++)
         if (started[k]) pthread_join(th[k], NULL);
-    pthread_mutex_lock(&g_stage.lock);
-    g_stage.busy = 0;
-    if (g_stage.holders == 0) stage_free();
-    pthread_mutex_unlock(&g_stage.lock);
+    stage_release();
     return 1;
 }
 
