@@ -77,8 +77,9 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind ki
 /* ---- the rest of the runtime ---- */
 
 hipError_t hipGetDeviceCount(int *n) { return *n = 1, hipSuccess; }
-hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
-hipError_t hipSetDevice(int d) { return hipSuccess; }
+static __thread int device; /* current device of the thread; streams are on device 0 */
+hipError_t hipGetDevice(int *d) { return *d = device, hipSuccess; }
+hipError_t hipSetDevice(int d) { return device = d, hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned f) { return *s = (hipStream_t)1, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { return hipSuccess; }
 static int pinned;   /* allocations of page-locked memory and of events */
@@ -91,9 +92,19 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned f)
 }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
-hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned f) { return pinned++, *e = (hipEvent_t)1, hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned f) 
+{
+    CHECK(device == 0); /* an event belongs to the device it is made on */
+    pinned++;
+    *e = (hipEvent_t)1;
+    return hipSuccess;
+}
 hipError_t hipEventDestroy(hipEvent_t e) { return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
+{
+    CHECK(device == 0);
+    return hipSuccess;
+}
 hipError_t hipEventSynchronize(hipEvent_t e) { return hipSuccess; }
 const char *hipGetErrorString(hipError_t e) { return "error"; }
 
@@ -199,12 +210,25 @@ static void reads(void)
     zpic_stage_hold(-1);
 }
 
+/* a large read by a caller that works on another device */
+static void other_device(void)
+{
+    const size_t n = (size_t)9 << 20;
+    char *src = zpic_dmalloc(n), *dst = malloc(n);
+    zpic_stage_hold(1);
+    device = 1;
+    zpic_d2h(dst, src, n);
+    CHECK(device == 1);
+    zpic_stage_hold(-1);
+}
+
 int main(int argc, char **argv)
 {
     const char *what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "staging")) staging();
     else if (!strcmp(what, "noalloc")) noalloc();
     else if (!strcmp(what, "reads")) reads();
+    else if (!strcmp(what, "device")) other_device();
     else CHECK(!"a known check");
     return failed;
 }

@@ -313,7 +313,12 @@ static int staged_d2h(void *dst, const void *src, size_t bytes)
     pthread_mutex_unlock(&g_stage.lock);
     if (!mine) return 0;
     const hipStream_t stream = zpic_stream();
+    /* the events and this thread's copies are on the library's device */
+    int dev = g_device;
+    ZCHECK(hipGetDevice(&dev));
+    if (dev != g_device) ZCHECK(hipSetDevice(g_device));
     if (!g_stage.buf && !stage_alloc()) {
+        if (dev != g_device) ZCHECK(hipSetDevice(dev));
         stage_release();
         return 0;
     }
@@ -331,6 +336,7 @@ static int staged_d2h(void *dst, const void *src, size_t bytes)
         if (!started[k]) stage_run(&job[k]);
     for (int k = 1; k < STAGE_THREADS; k++)
         if (started[k]) pthread_join(th[k], NULL);
+    if (dev != g_device) ZCHECK(hipSetDevice(dev));
     stage_release();
     return 1;
 }
