@@ -463,6 +463,16 @@ __device__ inline double move_one(const F &S, int ci, int cj, float x, float y, 
     return kin;
 }
 
+/* cells crossed along one axis on the way to offset x1, at most one: floor(x1)
+ * held to [-1, 1], and 0 for a NaN.  Each median is its operand with the
+ * clamp to [0, 1], which takes a NaN to 0 and no instruction; one median to
+ * [-1, 1] would take it to -1. */
+__device__ inline float crossed_axis(float x1)
+{
+    return __builtin_amdgcn_fmed3f(__builtin_floorf(x1), 0.0f, 1.0f) -
+           __builtin_amdgcn_fmed3f(__builtin_ceilf(-x1), 0.0f, 1.0f);
+}
+
 /* cells crossed on the way to offsets (x1, y1) (ltrim, em2d/particles.c:1081-1084) */
 __device__ inline void crossed(float x1, float y1, int &di, int &dj)
 {
@@ -764,9 +774,7 @@ __device__ __forceinline__ void push_tile_body(const Set &S, const int tile)
                     if (go) {
                         kin += move_one(lf, ci, cj, c.x, c.y, c.ux, c.uy, c.uz, mx, my, qvz, k);
                         const float x1 = c.x + mx, y1 = c.y + my;
-                        /* cells crossed: at most one per axis */
-                        const float fi = __builtin_amdgcn_fmed3f(__builtin_floorf(x1), -1.0f, 1.0f);
-                        const float fj = __builtin_amdgcn_fmed3f(__builtin_floorf(y1), -1.0f, 1.0f);
+                        const float fi = crossed_axis(x1), fj = crossed_axis(y1);
                         cross = (fi != 0.0f) | (fj != 0.0f);
                         const int di = (int)fi, dj = (int)fj;
                         Slot s = {0, x1 - fi, y1 - fj, c.ux, c.uy, c.uz};
