@@ -1415,7 +1415,12 @@ static zk_charge_args charge_args(const t_species *s, float *rho)
     a.tile_n = d->counted ? d->tile_n : NULL;
     a.ctr = d->ctr;
     a.q = s->q;
-    zpic_fixed_point_scale(s->q, &a.fx_scale, &a.fx_unscale);
+    /* an infinite or NaN charge leaves no weight to the fixed point */
+    const int k = zpic_fixed_point_exp(s->q);
+    a.fx_scale = ldexp(1.0, 44 - k);
+    a.fx_unscale = ldexp(1.0, k - 44);
+    a.fx_min = ldexpf(1.0f, k - 21);
+    a.fx_max = isfinite(s->q) && fabsf(s->q) > a.fx_min ? fabsf(s->q) : a.fx_min;
     a.t = d->t;
     a.rho = rho;
     return a;

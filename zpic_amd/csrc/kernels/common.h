@@ -38,9 +38,9 @@ __device__ inline int zk_xcd_item(int b, int n)
  * FP64; adding 1.5 * 2^52 in the same fused operation rounds it to an
  * integer held in the low mantissa bits, and subtracting the bit pattern
  * of 1.5 * 2^52 (whose low word is zero) leaves its two's complement. */
-__device__ inline unsigned long long zk_fx(float v, float scale)
+__device__ inline unsigned long long zk_fx(float v, double scale)
 {
-    const double r = __builtin_fma((double)v, (double)scale, 6755399441055744.0);
+    const double r = __builtin_fma((double)v, scale, 6755399441055744.0);
     return (unsigned long long)__double_as_longlong(r) - 0x4338000000000000ull;
 }
 

@@ -338,14 +338,27 @@ __device__ inline void charge_global(float *rho, int c, int nrow, float wx, floa
     unsafeAtomicAdd(&rho[c + 1 + nrow], (wx) * (wy) * q);
 }
 
+/* One weight: to window node w where its float is an integer at the fixed
+ * point's scale, 2^44 / Q with Q the power of two at or above |q|, which the
+ * floats of [2^-21 Q, |q|] are; sums of ZK_FX_TILE_MAX of them fit.  Smaller
+ * weights (one corner in some 10^5) would be cut, and a NaN or a weight
+ * beyond |q|, of a particle that is not in its cell, lost: they go to the
+ * grid as they are. */
+__device__ inline void charge_add(const zk_charge_args &a, unsigned long long *w, float *rho, float v)
+{
+    const unsigned lo = __float_as_uint(a.fx_min), hi = __float_as_uint(a.fx_max);
+    if (__float_as_uint(fabsf(v)) - lo <= hi - lo) atomicAdd(w, zk_fx(v, a.fx_scale));
+    else if (v != 0.0f) unsafeAtomicAdd(rho, v);
+}
+
 /* Charge density from tile-sorted particles.  With four global atomics per
  * particle the atomics set the time (512 x 512, 4.2 M particles: 395 us,
  * where reading the particles takes 11 us).  Here `splits` workgroups per
  * tile sum their share in an LDS window of the tile and its H-cell drift
- * margin, in the push's exact fixed point (scale 2^32 / Q), and add each
- * window node to the grid once (16 us).  Particles outside the window, the
- * unsorted tail (the last `tail` workgroups) and tiles beyond the fixed
- * point's range use the global atomics. */
+ * margin, in fixed point, and add each window node to the grid once (16 us).
+ * Particles outside the window, the unsorted tail (the last `tail`
+ * workgroups), weights outside [fx_min, fx_max] (charge_add) and tiles beyond
+ * the fixed point's range use the global atomics. */
 __global__ void __launch_bounds__(256) charge_kernel(zk_charge_args a)
 {
     extern __shared__ unsigned long long win[];
@@ -380,18 +393,19 @@ __global__ void __launch_bounds__(256) charge_kernel(zk_charge_args a)
         const unsigned u = ix - x0, v = iy - y0;
         if (exact && u < (unsigned)(W - 1) && v < (unsigned)(V - 1)) {
             unsigned long long *w = win + u + v * W;
-            atomicAdd(&w[0], zk_fx_raw((1.0f - wx) * (1.0f - wy) * a.q, a.fx_scale));
-            atomicAdd(&w[1], zk_fx_raw((wx) * (1.0f - wy) * a.q, a.fx_scale));
-            atomicAdd(&w[W], zk_fx_raw((1.0f - wx) * (wy) * a.q, a.fx_scale));
-            atomicAdd(&w[W + 1], zk_fx_raw((wx) * (wy) * a.q, a.fx_scale));
+            float *r = a.rho + ix + nrow * iy;
+            charge_add(a, &w[0], &r[0], (1.0f - wx) * (1.0f - wy) * a.q);
+            charge_add(a, &w[1], &r[1], (wx) * (1.0f - wy) * a.q);
+            charge_add(a, &w[W], &r[nrow], (1.0f - wx) * (wy) * a.q);
+            charge_add(a, &w[W + 1], &r[nrow + 1], (wx) * (wy) * a.q);
         } else {
             charge_global(a.rho, ix + nrow * iy, nrow, wx, wy, a.q);
         }
     }
     __syncthreads();
     for (int m = threadIdx.x; m < W * V; m += blockDim.x) {
-        const long long r = zk_fx_read(win[m]);
-        if (r != 0) unsafeAtomicAdd(&a.rho[x0 + m % W + nrow * (y0 + m / W)], (float)r * a.fx_unscale);
+        const long long r = (long long)win[m];
+        if (r != 0) unsafeAtomicAdd(&a.rho[x0 + m % W + nrow * (y0 + m / W)], (float)((double)r * a.fx_unscale));
     }
 }
 

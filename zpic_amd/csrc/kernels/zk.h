@@ -330,7 +330,8 @@ typedef struct zk_charge_args {
     zk_parts p;
     const int *tile_off, *tile_n;
     const zk_spec_ctr *ctr;
-    float q, fx_scale, fx_unscale;
+    float q, fx_min, fx_max;    /* magnitudes of the weights summed in fixed point */
+    double fx_scale, fx_unscale;
     zk_tiles t;
     int splits, tail;
     float *rho;
