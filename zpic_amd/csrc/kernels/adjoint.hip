@@ -676,7 +676,7 @@ __device__ inline float adjoint_one(const S &src, int ci, int cj, float x, float
     const float g = sqrt_ge1(1.0f + usq);
     const float tg = div_ge1(k.tem, g);
     const float tx = f[3] * tg, ty = f[4] * tg, tz = f[5] * tg;
-    const float s2 = 2.0f * rcp_ge1(1.0f + tx * tx + ty * ty + tz * tz);
+    const float s2 = two_over(1.0f + tx * tx + ty * ty + tz * tz);
     const float vx = ax + ay * tz - az * ty;
     const float vy = ay + az * tx - ax * tz;
     const float vz = az + ax * ty - ay * tx;

@@ -67,17 +67,22 @@ __device__ inline int zk_cell(int ix, int iy, int cbits) { return ix == ZK_DEAD 
 /* Correctly rounded reciprocal, division and square root for the Boris
  * push, whose divisors and square-root arguments are at least 1: hardware
  * estimates refined by fused multiply-adds, without the operand scaling and
- * special-value fix-ups that only denormal, infinite, zero or
- * extreme-exponent operands need.
+ * special-value fix-ups that denormal, infinite, zero or extreme-exponent
+ * operands need.
  *
  * On gfx950 one Newton step of the reciprocal estimate gives the correctly
  * rounded 1 / b for every float b in [1, 2^126), and one residual step on
- * x rsq(x) the correctly rounded square root for every x in [1, 2^127)
- * (checked for all of them, tests/test_gpu_rounding.py).  With y = 1 / b
- * correctly rounded, q = a y is within 1.5 units of the quotient, one
- * residual step makes it a faithful rounding, and one more the correctly
- * rounded quotient (Markstein's theorem).  The shorter sequences take 19
- * of the push's 420 issue slots per particle. */
+ * x rsq(x) the correctly rounded square root for every finite x >= 1
+ * (checked for all of them, tests/test_gpu_rounding.py and
+ * test_gpu_extremes.py).  With y = 1 / b correctly rounded, q = a y is within
+ * 1.5 units of the quotient, one residual step makes it a faithful rounding,
+ * and one more the correctly rounded quotient (Markstein's theorem).
+ *
+ * A square root of infinity comes out as the largest float: as a divisor
+ * that gives 0 in rcp_ge1 and div_ge1 (its reciprocal's estimate is below
+ * the smallest normal float, hence 0), as infinity does.  The square root of
+ * a NaN does too: every momentum of such a particle is NaN already.
+ * two_over takes any b >= 1. */
 __device__ inline float rcp_ge1(float b)
 {
     const float y = __builtin_amdgcn_rcpf(b);
@@ -96,7 +101,13 @@ __device__ inline float sqrt_ge1(float x)
 {
     const float y = __builtin_amdgcn_rsqf(x);
     const float s = x * y;
-    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+    return fminf(__builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s), 3.402823466e38f);
+}
+
+__device__ inline float two_over(float b)
+{
+    if (__builtin_expect(!(b < 0x1p126f), 0)) return 2.0f / b;
+    return 2.0f * rcp_ge1(b); /* the doubling is exact */
 }
 
 /* Clock readings of a timed phase (zk_clock), by one thread: zk_stamp_open at

@@ -442,7 +442,7 @@ __device__ inline double move_one(const F &S, int ci, int cj, float x, float y, 
     b[0] *= tg;
     b[1] *= tg;
     b[2] *= tg;
-    const float s2 = 2.0f * rcp_ge1(1.0f + b[0] * b[0] + b[1] * b[1] + b[2] * b[2]); /* the doubling is exact */
+    const float s2 = two_over(1.0f + b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
     const float vx = ax + ay * b[2] - az * b[1];
     const float vy = ay + az * b[0] - ax * b[2];
     const float vz = az + ax * b[1] - ay * b[0];
