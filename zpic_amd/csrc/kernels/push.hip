@@ -200,9 +200,12 @@ extern "C" int zk_push_species(const zk_push_multi *m, zk_stream_t s)
         if (e) return e;
         hipLaunchKernelGGL(fn, dim3(a->t.ntiles), dim3(nt), lds, s, *m);
     }
-    for (int k = 0; k < m->n; k++)
-        if (m->s[k].global_blocks > 0)
-            hipLaunchKernelGGL(push_global_kernel, dim3(m->s[k].global_blocks), dim3(256), 0, s, m->s[k]);
+    for (int k = 0; k < m->n; k++) {
+        if (m->s[k].global_blocks <= 0) continue;
+        zk_push_args g = m->s[k];
+        if (a->t.ntiles > 0) g.stamp.open = 0; /* the tile launch began the phase */
+        hipLaunchKernelGGL(push_global_kernel, dim3(g.global_blocks), dim3(256), 0, s, g);
+    }
     ZK_LAUNCH_CHECK();
 }
 
