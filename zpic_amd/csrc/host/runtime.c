@@ -469,7 +469,7 @@ static void timer_drain_n(int w, int n)
  * clock read in a kernel that runs anyway costs nothing. */
 static zk_clock *g_clock; /* [2] on the device */
 static struct {
-    int slot, open;
+    int used, open; /* slots used since the last zk_clock_fold */
 } g_phase[2];
 
 zk_stamp zpic_phase_begin(int w)
@@ -478,15 +478,18 @@ zk_stamp zpic_phase_begin(int w)
         g_clock = zpic_dmalloc(2 * sizeof(zk_clock));
         ZCHECK(zk_fill_f32((float *)g_clock, 2 * sizeof(zk_clock) / sizeof(float), 0.0f, zpic_stream()));
     }
-    g_phase[w].slot ^= 1;
+    if (g_phase[w].used == ZK_CLOCK_SLOTS) {
+        ZCHECK(zk_clock_fold(g_clock + w, ZK_CLOCK_SLOTS, zpic_stream()));
+        g_phase[w].used = 0;
+    }
+    const zk_stamp st = {g_clock + w, g_phase[w].used++, 1};
     g_phase[w].open = 1;
-    const zk_stamp st = {g_clock + w, g_phase[w].slot, 1};
     return st;
 }
 
 zk_stamp zpic_phase_stamp(int w)
 {
-    const zk_stamp st = {g_phase[w].open ? g_clock + w : NULL, g_phase[w].slot, 0};
+    const zk_stamp st = {g_phase[w].open ? g_clock + w : NULL, g_phase[w].used - 1, 0};
     return st;
 }
 
@@ -499,11 +502,11 @@ void zpic_phase_end(int w, int extra)
 static double phase_total(int w)
 {
     if (!g_clock) return 0.0;
-    zk_clock c;
-    zpic_d2h(&c, g_clock + w, sizeof(c));
-    const int s = g_phase[w].slot;
-    unsigned long long n = c.total;
-    if (c.t1[s] > c.t0[s]) n += c.t1[s] - c.t0[s];
+    /* an open phase keeps its slot */
+    ZCHECK(zk_clock_fold(g_clock + w, g_phase[w].used - g_phase[w].open, zpic_stream()));
+    if (!g_phase[w].open) g_phase[w].used = 0;
+    unsigned long long n;
+    zpic_d2h(&n, &g_clock[w].total, sizeof(n));
     int khz = 0;
     ZCHECK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, g_device));
     return khz > 0 ? (double)n / (1e3 * khz) : 0.0;

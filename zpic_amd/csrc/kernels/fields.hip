@@ -48,7 +48,8 @@ __global__ void __launch_bounds__(256) yee_kernel(const float *__restrict__ E, c
     /* contiguous runs of units per XCD: neighbours share their margins in L2 */
     const int u = zk_xcd_item(blockIdx.x, gridDim.x) * (blockDim.x / 64) + threadIdx.x / 64;
     if (u < units) yee_rows<R>(E, B, J, Eo, Bo, nx, ny, nrow, k, u, periodic_x, open_y, shift, EXT ? ext : zk_ext());
-    zk_stamp_last(st);
+    /* the units are alike: the last end with the last */
+    if (blockIdx.x + 512 >= gridDim.x) zk_stamp_last_waves(st);
 }
 
 /* Waves of a workgroup of field_step_kernel, a staged row each, and the rows
@@ -165,7 +166,7 @@ __global__ void __launch_bounds__(1024) field_step_kernel(zk_field_args f)
         o[2] = s[2];
     }
     y.step(f.E, f.Eo, f.Bo, nx, ny, nrow, f.k, bi, j + 1, l0, cols, c0, px, oy, f.shift, f.ext);
-    if (blockIdx.x + 1 == gridDim.x && w == n2 + X && lane == 0) zk_stamp_close(f.stamp);
+    if (w == n2 + X && lane == 0) zk_stamp_close(f.stamp);
 }
 
 YeeK yee_constants(float dt, float dx, float dy)

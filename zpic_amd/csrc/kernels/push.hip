@@ -94,6 +94,29 @@ __global__ void __launch_bounds__(256) push_global_kernel(zk_push_args a)
 
 __global__ void stamp_kernel(zk_stamp st) { zk_stamp_last(st); }
 
+/* a thread per slot: start to end of the phases of slots 0 .. n - 1 */
+__global__ void __launch_bounds__(ZK_CLOCK_SLOTS) clock_fold_kernel(zk_clock *clk, int n)
+{
+    __shared__ unsigned long long part[ZK_CLOCK_SLOTS];
+    const int k = threadIdx.x;
+    unsigned long long t = 0;
+    if (k < n) {
+        auto &a = clk->at[k];
+        unsigned long long e = 0;
+        for (int x = 0; x < ZK_XCDS; x++) {
+            e = max(e, a.end[x]);
+            a.end[x] = 0;
+        }
+        if (a.start != 0 && e > a.start) t = e - a.start;
+        a.start = 0;
+    }
+    part[k] = t;
+    __syncthreads();
+    if (k > 0) return;
+    for (int i = 1; i < ZK_CLOCK_SLOTS; i++) t += part[i];
+    clk->total += t;
+}
+
 /* one block per species */
 __global__ void __launch_bounds__(1024) finalize_set_kernel(zk_finalize_set f)
 {
@@ -228,6 +251,13 @@ extern "C" int zk_fill_f32(float *p, size_t n, float v, zk_stream_t s)
 extern "C" int zk_stamp_end(zk_stamp st, zk_stream_t s)
 {
     hipLaunchKernelGGL(stamp_kernel, dim3(1), dim3(64), 0, s, st);
+    ZK_LAUNCH_CHECK();
+}
+
+extern "C" int zk_clock_fold(zk_clock *clk, int n, zk_stream_t s)
+{
+    if (n < 0 || n > ZK_CLOCK_SLOTS) return (int)hipErrorInvalidValue;
+    if (n > 0) hipLaunchKernelGGL(clock_fold_kernel, dim3(1), dim3(ZK_CLOCK_SLOTS), 0, s, clk, n);
     ZK_LAUNCH_CHECK();
 }
 

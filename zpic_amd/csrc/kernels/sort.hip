@@ -94,7 +94,7 @@ __global__ void __launch_bounds__(ZK_SORT_THREADS) scatter_stay_kernel(zk_resort
     const zk_resort_args &a = m.s[sort_species(m, b)];
     scatter_stay_body(a.src, a.dst, a.old_off, a.old_n, ScannedDest{a.new_off, a.cursor}, a.stay, a.nbr, a.t, b,
                       a.blocks);
-    zk_stamp_last(st);
+    zk_stamp_last_waves(st);
 }
 
 /* The scatter with the scan of the tile counts in every workgroup: up to
@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(ZK_SORT_THREADS) scatter_scan_kernel(zk_resort
         for (int t = threadIdx.x; t < n; t += blockDim.x) a.move[t] = a.tailn[t] = 0;
         if (threadIdx.x == 0) *a.ticket = 0;
     }
-    zk_stamp_last(st);
+    zk_stamp_last_waves(st);
 }
 
 __global__ void __launch_bounds__(ZK_SORT_THREADS)

@@ -42,13 +42,19 @@ extern "C" {
 #define ZK_FX_TILE_MAX ((1 << 18) - 16)
 
 /* Time the GPU spends in a phase of the step (spec_time, emf_time), kept by
- * the phase's own kernels: the first block of its first launch reads the
- * constant-rate clock into t0[slot] and adds the previous phase's interval
- * to total; the last block of each of its launches reads it into t1[slot].
- * Phases alternate slots, so the two never touch the same entry in one
- * launch. */
+ * the phase's own kernels: the workgroup that begins its first launch reads
+ * the constant-rate clock into start, and every wave of each of its launches,
+ * at its end, into the end of its XCD.  Waves of an XCD share an L2, where
+ * the last of them writes last, so the largest end is the phase's.  A phase
+ * takes a slot; zk_clock_fold adds the intervals of the slots used to total
+ * and clears them. */
+#define ZK_CLOCK_SLOTS 128
+#define ZK_XCDS 8
 typedef struct zk_clock {
-    unsigned long long t0[2], t1[2], total; /* ticks */
+    unsigned long long total;   /* ticks */
+    struct {
+        unsigned long long start, end[ZK_XCDS]; /* 0: none */
+    } at[ZK_CLOCK_SLOTS];
 } zk_clock;
 typedef struct zk_stamp {
     zk_clock *clk;              /* NULL: the launch is not timed */
@@ -156,6 +162,8 @@ typedef struct zk_push_multi {
 int zk_fill_f32(float *p, size_t n, float v, zk_stream_t s);
 /* reads the clock into a phase's end on its own */
 int zk_stamp_end(zk_stamp st, zk_stream_t s);
+/* slots 0 .. n - 1 into total */
+int zk_clock_fold(zk_clock *clk, int n, zk_stream_t s);
 /* bad[k] += floats with bit patterns first .. first + n - 1 whose reciprocal,
  * square root or quotient a / x in the push is not the correctly rounded one
  * (a check for the tests; waits for the GPU) */
