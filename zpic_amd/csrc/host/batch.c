@@ -73,8 +73,7 @@ static void fill_sim(zpic_batch *b, int i)
     }
     M->region = dc->region;
     for (int k = 0; k < sim->n_species; k++) zpic_current_jov_register(cur, sim->species[k].q);
-    zpic_current_jov_tidy(cur);
-    M->Jov = zpic_current_jov(cur, 1);
+    M->Jov = zpic_current_jov(cur);
     M->jflag = dc->jflag[dc->jov_cur];
     M->jov_unscale = zpic_current_jov_unscale(cur);
     M->ecur = de->cur;
@@ -111,7 +110,7 @@ static void fill_spec(zpic_batch *b, int k)
     a->nrow = cur->nrow;
     a->region = dc->region;
     a->fresh = (b->spec_k[k] == 0);
-    a->Jov = zpic_current_jov(cur, 1);
+    a->Jov = zpic_current_jov(cur);
     a->jflag = dc->jflag[dc->jov_cur];
     a->jov_scale = zpic_current_jov_scale(cur);
     a->epart = d->epart;

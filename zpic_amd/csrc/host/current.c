@@ -77,16 +77,10 @@ static void jov_clear(t_current *c, int k)
     d->jov_state[k] = ZPIC_JOV_CLEAN;
 }
 
-void zpic_current_jov_tidy(t_current *c)
-{
-    if (c->dev->jov_state[c->dev->jov_cur] == ZPIC_JOV_DIRTY) jov_clear(c, c->dev->jov_cur);
-}
-
-long long *zpic_current_jov(t_current *c, int flagged)
+long long *zpic_current_jov(t_current *c)
 {
     struct zpic_dev_current *d = c->dev;
-    int *st = &d->jov_state[d->jov_cur];
-    *st = flagged && *st != ZPIC_JOV_DIRTY ? ZPIC_JOV_FLAGGED : ZPIC_JOV_DIRTY;
+    d->jov_state[d->jov_cur] = ZPIC_JOV_FLAGGED;
     return d->Jov2[d->jov_cur];
 }
 
@@ -217,7 +211,7 @@ static int reduce_args(t_current *c, zk_reduce_args *a)
     struct zpic_dev_current *d = c->dev;
     a->region = d->fresh ? NULL : d->region;
     a->Jov = d->Jov2[d->jov_cur];
-    a->jflag = d->jov_state[d->jov_cur] == ZPIC_JOV_DIRTY ? NULL : d->jflag[d->jov_cur];
+    a->jflag = d->jflag[d->jov_cur];
     const int other = 1 - d->jov_cur;
     const int clears = d->jov_state[other] == ZPIC_JOV_FLAGGED && zk_current_clears(&d->t);
     a->Jov_next = clears ? d->Jov2[other] : NULL;

@@ -1147,7 +1147,7 @@ static void push_args(t_species *s, t_emf *emf, t_current *cur, zk_push_args *pa
     a.region = dc->region;
     a.fresh = dc->fresh;
     zpic_current_jov_register(cur, s->q);
-    a.Jov = zpic_current_jov(cur, 1);
+    a.Jov = zpic_current_jov(cur);
     a.jflag = dc->jflag[dc->jov_cur];
     a.jov_scale = zpic_current_jov_scale(cur);
     a.epart = d->epart;

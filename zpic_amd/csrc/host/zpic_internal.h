@@ -92,7 +92,7 @@ struct zpic_dev_species {
 };
 
 enum {
-    ZPIC_JOV_DIRTY = 0,   /* anything: cleared as a whole before it is used */
+    ZPIC_JOV_DIRTY = 0,   /* anything, as allocated: cleared as a whole before its first use */
     ZPIC_JOV_CLEAN = 1,   /* all zero, no flag set */
     ZPIC_JOV_FLAGGED = 2, /* zero but for the flagged blocks */
 };
@@ -150,11 +150,9 @@ const float *zpic_current_J(t_current *cur);
 /* the overflow grid's fixed-point scale covers a species of charge q
  * (raised, with the grid's sums rescaled exactly, when q needs more) */
 void zpic_current_jov_register(t_current *cur, float q);
-/* the overflow grid of this step, about to be deposited to: by a push that
- * flags what it touches, or (flagged 0) by one that does not */
-long long *zpic_current_jov(t_current *cur, int flagged);
-/* its contents are zero but for the flagged blocks afterwards */
-void zpic_current_jov_tidy(t_current *cur);
+/* the overflow grid of this step, about to be deposited to by a push that
+ * flags what it touches */
+long long *zpic_current_jov(t_current *cur);
 float zpic_current_jov_scale(const t_current *cur);   /* 2^(40 - jov_k) */
 float zpic_current_jov_unscale(const t_current *cur); /* 2^(jov_k - 40) */
 

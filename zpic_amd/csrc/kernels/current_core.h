@@ -94,7 +94,7 @@ __device__ inline void reduce_sum(const zk_reduce_args &a, const int i, const in
             const int rx = gx ? rxs[1] : rxs[0];
             const int kx = last_tile(rx, t.H, invx);
             long long o0 = 0, o1 = 0, o2 = 0;
-            if (!a.jflag || a.jflag[(rx + 1) / ZK_RED_BX + (ry + 1) / ZK_RED_BY * zk_red_blocks_x(t.nx)]) {
+            if (a.jflag[(rx + 1) / ZK_RED_BX + (ry + 1) / ZK_RED_BY * zk_red_blocks_x(t.nx)]) {
                 const long long *o = a.Jov + 3 * ((rx + 1) + (size_t)(ry + 1) * a.nrow);
                 o0 = o[0];
                 o1 = o[1];

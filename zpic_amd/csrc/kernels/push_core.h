@@ -123,7 +123,6 @@ struct GlobalCurrent {
      * nearly empty is not read and rewritten every step. */
     __device__ void touch(int ci, int cj) const
     {
-        if (!flag) return;
         const int x0 = (ci - 1) / ZK_RED_BX, x1 = (ci + 2) / ZK_RED_BX;
         const int y0 = (cj - 1) / ZK_RED_BY * nfx, y1 = (cj + 2) / ZK_RED_BY * nfx;
         flag[x0 + y0] = 1;

@@ -121,8 +121,7 @@ typedef struct zk_push_args {
     int fresh;                  /* 1: overwrite region, 0: accumulate    */
     long long *Jov;             /* raw current of out-of-window pushes, 64-bit
                                    fixed point at jov_scale (order-free sums) */
-    unsigned char *jflag;       /* set for the zk_red_blocks of Jov deposited to
-                                   (NULL: not kept) */
+    unsigned char *jflag;       /* set for the zk_red_blocks of Jov deposited to */
     double *epart;              /* energy partials, one per block        */
     zk_tiles t;
     int moving_window;          /* x absorbing + window shift           */
@@ -254,7 +253,7 @@ int zk_unpack_append(const void *aos, int n, const zk_parts *dst, int64_t id0, z
 typedef struct zk_reduce_args {
     const float *region;
     const long long *Jov;
-    const unsigned char *jflag; /* blocks of Jov that may be nonzero (NULL: all) */
+    const unsigned char *jflag; /* blocks of Jov that may be nonzero */
     long long *Jov_next;        /* overflow grid of the next step, cleared here where */
     unsigned char *jflag_next;  /* its flags say so (NULL: not cleared) */
     float jov_unscale;          /* Q_J / 2^40 */
@@ -275,9 +274,8 @@ int zk_current_reduce(const zk_reduce_args *a, zk_stream_t s);
 int zk_smooth(const float *in, float *out, int nx, int ny, int nrow, int n1, int n2, const float *sa, const float *sb,
               int periodic_x, int open_y, zk_stream_t s);
 
-/* zk_current_reduce, zk_smooth and zk_yee of one step in one launch, for
- * grids small enough to be bound by launches (same J, E and B bit for bit);
- * zk_field_step_ok: whether it takes this grid and these passes */
+/* Yee constants: (dt/2)/dx, (dt/2)/dy, dt/dx, dt/dy, dt, and the Mur
+ * coefficient (dt - dy)/(dt + dy) of open y boundaries */
 typedef struct zk_yee_k {
     float dtx2, dty2, dtx, dty, dt, mur_y;
 } zk_yee_k;
@@ -300,6 +298,9 @@ typedef struct zk_field_args {
     int clears;                 /* set by zk_field_step: workgroups that clear Jov_next */
     zk_stamp stamp;             /* of the field step */
 } zk_field_args;
+/* zk_current_reduce, zk_smooth and zk_yee of one step in one launch, for
+ * grids small enough to be bound by launches (same J, E and B bit for bit);
+ * zk_field_step_ok: whether it takes this grid and these passes */
 int zk_field_step_ok(const zk_tiles *t, int n1, int n2, int open_y);
 int zk_field_step(const zk_field_args *f, float dt, float dx, float dy, zk_stream_t s);
 
@@ -426,9 +427,6 @@ int zk_init_rng_emit(const zk_init_args *a, long long nat, int per, const int *t
 int zk_init_mean(const zk_init_args *a, float *mean, int nkeys, zk_stream_t s);
 
 /* ---- batches of independent simulations (batch.hip) ---- */
-
-/* Yee constants: (dt/2)/dx, (dt/2)/dy, dt/dx, dt/dy, dt, and the Mur
- * coefficient (dt - dy)/(dt + dy) of open y boundaries */
 
 /* One simulation of a batch.  ecur/jcur select the current E,B and J
  * buffers and are advanced on the device at the end of every step. */
