@@ -23,9 +23,8 @@
 
 using namespace zk;
 
-/* waves per SIMD the fixed-point tile push is compiled for: 5 (96 VGPRs,
- * 24 bytes per lane spilled) against 4: 512-member scan 146.5 -> 148.3
- * sims/s */
+/* waves per SIMD the fixed-point tile push is compiled for: 5, which allow 96
+ * VGPRs, against 4: 512-member scan 146.5 -> 148.3 sims/s */
 #ifndef ZK_PUSH_OCC
 #define ZK_PUSH_OCC 5
 #endif

@@ -356,7 +356,7 @@ __device__ inline void charge_add(const zk_charge_args &a, unsigned long long *w
  * particle the atomics set the time (512 x 512, 4.2 M particles: 395 us,
  * where reading the particles takes 11 us).  Here `splits` workgroups per
  * tile sum their share in an LDS window of the tile and its H-cell drift
- * margin, in fixed point, and add each window node to the grid once (16 us).
+ * margin, in fixed point, and add each window node to the grid once (20 us).
  * Particles outside the window, the unsorted tail (the last `tail`
  * workgroups), weights outside [fx_min, fx_max] (charge_add) and tiles beyond
  * the fixed point's range use the global atomics. */

@@ -20,28 +20,27 @@
  * windows are summed into J afterwards by current.hip in a fixed order.
  *
  * A particle that has drifted more than H cells out of its tile since the
- * last sort is listed by the tile pass and pushed by a second kernel on the
- * global path: gathers from the guard-inclusive field buffers exactly as
- * the reference indexes them, and deposits into the raw overflow grid
+ * last sort is listed, and pushed on the global path by the same workgroup
+ * after the others: gathers from the guard-inclusive field buffers exactly
+ * as the reference indexes them, and deposits into the raw overflow grid
  * `Jov` with 64-bit fixed-point atomics (exact, order-free sums).  The
- * same kernel pushes the unsorted tail (particles injected by the moving
- * window since the last sort).
+ * unsorted tail (particles injected by the moving window since the last
+ * sort) takes the same path, in workgroups of its own.
  */
 #include "push_core.h"
 
 using namespace zk;
 
-/* waves per SIMD of the single-species tile push: 5 fits 96 VGPRs, with a
- * few values spilled outside the loop (LWFA 4000 x 256: 0.2537 -> 0.2505
- * ms per step against 4 waves) */
+/* waves per SIMD of the single-species tile push: 5 allow 96 VGPRs, of which
+ * it takes 85 or 86 (LWFA 4000 x 256: 0.2537 -> 0.2505 ms per step against 4
+ * waves, when the 96 still left a few values spilled outside the loop) */
 #ifndef ZK_PUSH_OCC
 #define ZK_PUSH_OCC 5
 #endif
-/* waves per SIMD of the fused multi-species push: 5 fits 96 VGPRs, with
- * 16 bytes per lane spilled before the loop and reloaded after it; the
- * extra wave hides more latency (2048^2 Weibel: 5 waves 1.727 ms per
- * launch against 1.750 with 4, when the 5-wave build still reloaded two
- * spilled address terms in the loop; 1.697 ms without them) */
+/* waves per SIMD of the fused multi-species push: 5 allow 96 VGPRs, of which
+ * it takes 87; the extra wave hides more latency (2048^2 Weibel: 5 waves
+ * 1.727 ms per launch against 1.750 with 4, when the 5-wave build still
+ * reloaded two spilled address terms in the loop) */
 #ifndef ZK_SPECIES_OCC
 #define ZK_SPECIES_OCC 5
 #endif
