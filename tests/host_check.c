@@ -222,6 +222,27 @@ static void other_device(void)
     zpic_stage_hold(-1);
 }
 
+/* a slab on a grid whose cells are not square: its particles fit the buffer */
+static void slab(void)
+{
+    const float dx[3] = {0.05f, 0.1f, 0.2f};
+    for (int k = 0; k < 9; k++) {
+        const int n[2] = {130, 70}, ppc[2] = {2, 2};
+        const float u[3] = {0, 0, 0};
+        float box[2] = {dx[k / 3] * n[0], dx[k % 3] * n[1]};
+        t_density d;
+        memset(&d, 0, sizeof(d));
+        d.type = SLAB;
+        d.n = 1.0f;
+        d.start = 0.2f * box[0];
+        d.end = 0.6f * box[0];
+        t_species s;
+        spec_new(&s, "slab", -1.0f, ppc, u, u, n, box, 0.01f, &d);
+        CHECK(s.np == 52 * 70 * 4);
+        CHECK(s.np <= s.np_max);
+    }
+}
+
 int main(int argc, char **argv)
 {
     const char *what = argc > 1 ? argv[1] : "";
@@ -229,6 +250,7 @@ int main(int argc, char **argv)
     else if (!strcmp(what, "noalloc")) noalloc();
     else if (!strcmp(what, "reads")) reads();
     else if (!strcmp(what, "device")) other_device();
+    else if (!strcmp(what, "slab")) slab();
     else CHECK(!"a known check");
     return failed;
 }

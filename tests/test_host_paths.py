@@ -26,7 +26,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["staging", "noalloc", "reads", "device"])
+@pytest.mark.parametrize("what", ["staging", "noalloc", "reads", "device", "slab"])
 def test_host_path(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr

@@ -37,8 +37,10 @@ static float unit_density(float x, void *data)
     return 1.0f;
 }
 
-/* Upper bound of the particles a cell range receives (em2d/particles.c:367-449);
- * the slab's upper edge divides by dx[1], as the reference does. */
+/* Upper bound of the particles a cell range receives (em2d/particles.c:367-449).
+ * The slab's upper edge is a cell along x, as inject_positions has it; the
+ * reference divides it by dx[1], which is too small a bound on cells that are
+ * wider in y. */
 static int inject_bound(const t_species *s, const int r[2][2])
 {
     const int rows = r[1][1] - r[1][0] + 1;
@@ -51,7 +53,7 @@ static int inject_bound(const t_species *s, const int r[2][2])
     }
     case SLAB: {
         int i0 = s->density.start / s->dx[0] - s->n_move;
-        int i1 = s->density.end / s->dx[1] - s->n_move;
+        int i1 = s->density.end / s->dx[0] - s->n_move;
         if (i0 > r[0][1] || i1 < r[0][0]) return 0;
         if (i0 < r[0][0]) i0 = r[0][0];
         if (i1 > r[0][1]) i1 = r[0][1];
